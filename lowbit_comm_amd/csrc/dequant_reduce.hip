@@ -39,7 +39,7 @@ hipError_t launch_reduce_w(int mode, const ReduceArgs &a, hipStream_t stream) {
         case kStreamThrough: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kStreamThrough>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
         case kStream: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kStream>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kVector>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kScalar>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kUnaligned>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }
@@ -88,7 +88,7 @@ hipError_t launch_reduce_quant_w(int mode, const ReduceQuantArgs &a, hipStream_t
     switch (mode) {
         case kStream: hipLaunchKernelGGL((dequant_reduce_quant_kernel<MT, G, W, kStream>), grid, dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((dequant_reduce_quant_kernel<MT, G, W, kVector>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((dequant_reduce_quant_kernel<MT, G, W, kScalar>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((dequant_reduce_quant_kernel<MT, G, W, kUnaligned>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }
@@ -136,7 +136,7 @@ hipError_t launch_decode_op(int mode, const DecodeArgs &a, int world, hipStream_
     switch (mode) {
         case kStream: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kStream>), grid, dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kVector>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kScalar>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kUnaligned>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void ef_update_kernel(const EfArgs a) {
     const TT *__restrict__ restored = static_cast<const TT *>(a.restored);
     RT *__restrict__ residual = static_cast<RT *>(a.residual);
     const int64_t block_first = static_cast<int64_t>(xcd_contiguous_block(BLOCK_ELEMS)) * BLOCK_ELEMS;
-    if (MODE != kScalar && block_first + BLOCK_ELEMS <= a.numel) {
+    if (MODE != kUnaligned && block_first + BLOCK_ELEMS <= a.numel) {
         PT pv[UNROLL][VEC];
         TT tv[UNROLL][VEC];
 #pragma unroll
@@ -212,7 +212,7 @@ hipError_t launch_ef(int mode, const EfArgs &a, hipStream_t stream) {
     switch (mode) {
         case kStream: hipLaunchKernelGGL((ef_update_kernel<PT, TT, RT, kStream>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((ef_update_kernel<PT, TT, RT, kVector>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((ef_update_kernel<PT, TT, RT, kScalar>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((ef_update_kernel<PT, TT, RT, kUnaligned>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }

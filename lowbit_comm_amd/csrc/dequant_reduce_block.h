@@ -58,7 +58,7 @@ template <typename OT, int W, int MODE> constexpr int reduce_store_policy() {
 
 template <int VEC, int MODE>
 __device__ __forceinline__ void load_codes(const int8_t *__restrict__ p, uint32_t (&w)[VEC / 4]) {
-    if constexpr (MODE != kScalar) {
+    if constexpr (MODE != kUnaligned) {
         load_vec<uint32_t, VEC / 4, MODE>(reinterpret_cast<const uint32_t *>(p), w);
     } else {
 #pragma unroll
@@ -90,7 +90,7 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
     OT *new_r = static_cast<OT *>(a.new_residual);
     const bool mean = a.divisor != 1.0f;
 
-    if (MODE != kScalar && block_first + T::BLOCK_ELEMS <= a.numel) {
+    if (MODE != kUnaligned && block_first + T::BLOCK_ELEMS <= a.numel) {
         // ---- interior block: one descriptor per stream over the block's span, 32-bit offsets per lane ----
         constexpr int kCodes = code_policy<OT, W, MODE>();
         constexpr int kLoad = policy_of<MODE>();
@@ -232,7 +232,7 @@ __device__ __forceinline__ void dequant_reduce_quant_block(const ReduceQuantArgs
     uint32_t out_words[VEC / 4];
 #pragma unroll
     for (int k = 0; k < VEC / 4; ++k) out_words[k] = pack4(c[4 * k], c[4 * k + 1], c[4 * k + 2], c[4 * k + 3]);
-    if constexpr (MODE != kScalar) {
+    if constexpr (MODE != kUnaligned) {
         store_vec<uint32_t, VEC / 4, kVector>(reinterpret_cast<uint32_t *>(a.out_codes + e0), out_words);
     } else {
 #pragma unroll
@@ -280,7 +280,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs &a, unsigned block
     const int64_t block_first = static_cast<int64_t>(xcd_contiguous_block(block_x, grid_x, T::BLOCK_ELEMS)) * T::BLOCK_ELEMS;
     if (block_first >= valid) return;
 
-    if (MODE != kScalar && block_first + T::BLOCK_ELEMS <= valid) {
+    if (MODE != kUnaligned && block_first + T::BLOCK_ELEMS <= valid) {
         uint32_t words[UNROLL][VEC / 4];
         float scale[UNROLL];
         int64_t e0[UNROLL];

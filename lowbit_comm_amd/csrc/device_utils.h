@@ -49,8 +49,8 @@ __device__ __forceinline__ unsigned xcd_contiguous_block(int block_elems) {
 }
 constexpr uint32_t kEpsBits = 0x34000000u;  // 2^-23, torch.finfo(float32).eps
 
-// Access modes of the bulk loads and stores.  kScalar: element by element (any
-// alignment).  kVector: one vector instruction per lane (the caller guarantees
+// Access modes of the bulk loads and stores.  kUnaligned: one vector instruction per lane at
+// element alignment, non-temporal loads (any tensor).  kVector: one vector instruction per lane (the caller guarantees
 // N*sizeof(T) alignment), plain cached accesses - for operands that are known to
 // sit in the last-level cache.  kStream: vector instructions with the
 // non-temporal hint on the loads - every tensor here is read once, and when it is
@@ -59,7 +59,7 @@ constexpr uint32_t kEpsBits = 0x34000000u;  // 2^-23, torch.finfo(float32).eps
 // 256 MiB memory-side cache holds; cached loads are ~5 % faster only when
 // everything is resident).  Stores under kStream are chosen per kernel.
 // kStreamThrough (fused reduce only): kStream with write-through stores.
-enum AccessMode { kScalar = 0, kVector = 1, kStream = 2, kStreamThrough = 3 };
+enum AccessMode { kUnaligned = 0, kVector = 1, kStream = 2, kStreamThrough = 3 };
 
 template <typename T, int N>
 using vec_t = T __attribute__((ext_vector_type(N)));
@@ -124,35 +124,58 @@ template <typename T, int N> __device__ __forceinline__ void narrow_all(const fl
     }
 }
 
+// ---- N elements at an address aligned to ALIGN bytes only ----------------------------
+// gfx950's global memory instructions take any address (dword-aligned or not), so a tensor that starts in the middle of
+// a 16-byte line - a chunk of a bucket whose shard size is no multiple of anything, a view - still moves as one vector
+// instruction per lane.  `live` elements exist from `p` on; the rest of dst becomes 0 and is not stored.
+template <typename T, int N, int ALIGN> struct vec_at {
+    typedef vec_t<T, N> type __attribute__((aligned(ALIGN)));
+};
+template <typename T, int N, bool NT, int ALIGN = sizeof(T)>
+__device__ __forceinline__ void load_any(const T *p, T (&dst)[N]) {
+    using V = typename vec_at<T, N, ALIGN>::type;
+    vec_t<T, N> v;
+    if constexpr (NT) v = __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
+    else v = *reinterpret_cast<const V *>(p);
+#pragma unroll
+    for (int i = 0; i < N; ++i) dst[i] = v[i];
+}
+template <typename T, int N, bool NT, int ALIGN = sizeof(T)>
+__device__ __forceinline__ void store_any(T *p, const T (&src)[N]) {
+    using V = typename vec_at<T, N, ALIGN>::type;
+    vec_t<T, N> v;
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = src[i];
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<V *>(p));
+    else *reinterpret_cast<V *>(p) = v;
+}
+template <typename T, int N, bool NT> __device__ __forceinline__ void load_live(const T *p, int64_t live, T (&dst)[N]) {
+    if (live >= N) {
+        load_any<T, N, NT>(p, dst);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) dst[i] = i < live ? p[i] : static_cast<T>(0.0f);
+    }
+}
+template <typename T, int N, bool NT> __device__ __forceinline__ void store_live(T *p, int64_t live, const T (&src)[N]) {
+    if (live >= N) {
+        store_any<T, N, NT>(p, src);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (i < live) p[i] = src[i];
+    }
+}
+
 // ---- N-element contiguous load / store --------------------------------------
 template <typename T, int N, int MODE>
 __device__ __forceinline__ void load_vec(const T *__restrict__ p, T (&dst)[N]) {
-    if constexpr (MODE != kScalar) {
-        using V = vec_t<T, N>;
-        V v;
-        if constexpr (MODE == kStream) v = __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
-        else v = *reinterpret_cast<const V *>(p);
-#pragma unroll
-        for (int i = 0; i < N; ++i) dst[i] = v[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) dst[i] = p[i];
-    }
+    load_any<T, N, MODE == kStream || MODE == kUnaligned, MODE == kUnaligned ? sizeof(T) : N * sizeof(T)>(p, dst);
 }
 
 template <typename T, int N, int MODE>
 __device__ __forceinline__ void store_vec(T *__restrict__ p, const T (&src)[N]) {
-    if constexpr (MODE != kScalar) {
-        using V = vec_t<T, N>;
-        V v;
-#pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = src[i];
-        if constexpr (MODE == kStream) __builtin_nontemporal_store(v, reinterpret_cast<V *>(p));
-        else *reinterpret_cast<V *>(p) = v;
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) p[i] = src[i];
-    }
+    store_any<T, N, MODE == kStream, MODE == kUnaligned ? sizeof(T) : N * sizeof(T)>(p, src);
 }
 
 // Loads / stores N elements as ceil(N*sizeof(T)/16) instructions of at most 16 bytes.

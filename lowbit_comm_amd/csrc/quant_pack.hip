@@ -38,7 +38,7 @@ hipError_t launch_typed(int mode, const QuantArgs &a, int world, hipStream_t str
     switch (mode) {
         case kStream: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStream>), grid, dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kVector>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kScalar>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kUnaligned>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }

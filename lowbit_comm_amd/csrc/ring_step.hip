@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kBlock) void ring_step_kernel(const RingStepArgs a)
     const bool mean = a.divisor != 1.0f;
     const bool emit = a.send_codes != nullptr;  // uniform over the grid
 
-    if (MODE != kScalar && block_first + L::BLOCK_ELEMS <= a.numel) {
+    if (MODE != kUnaligned && block_first + L::BLOCK_ELEMS <= a.numel) {
         // ---- interior block: every tile is full ----
         T xv[UNROLL][VEC];
         uint32_t words[UNROLL][VEC / 4];
@@ -139,7 +139,7 @@ hipError_t launch_ring_g(int mode, const RingStepArgs &a, hipStream_t stream) {
     switch (mode) {
         case kStream: hipLaunchKernelGGL((ring_step_kernel<T, G, kStream, ACC>), grid, dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((ring_step_kernel<T, G, kVector, ACC>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((ring_step_kernel<T, G, kScalar, ACC>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((ring_step_kernel<T, G, kUnaligned, ACC>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
 }
