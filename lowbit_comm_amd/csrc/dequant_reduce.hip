@@ -174,14 +174,20 @@ __global__ __launch_bounds__(kBlock) void ef_update_kernel(const EfArgs a) {
     const TT *__restrict__ restored = static_cast<const TT *>(a.restored);
     RT *__restrict__ residual = static_cast<RT *>(a.residual);
     const int64_t block_first = static_cast<int64_t>(xcd_contiguous_block(BLOCK_ELEMS)) * BLOCK_ELEMS;
-    if (MODE != kUnaligned && block_first + BLOCK_ELEMS <= a.numel) {
+    auto tiles = [&](auto whole) __attribute__((always_inline)) {   // WHOLE: all of the block's elements exist
+        constexpr bool WHOLE = decltype(whole)::value;
         PT pv[UNROLL][VEC];
         TT tv[UNROLL][VEC];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             const int64_t e0 = block_first + (static_cast<int64_t>(u) * kBlock + threadIdx.x) * VEC;
-            load_vec<PT, VEC, MODE>(prepared + e0, pv[u]);
-            load_vec<TT, VEC, MODE>(restored + e0, tv[u]);
+            if constexpr (WHOLE) {
+                load_vec<PT, VEC, MODE>(prepared + e0, pv[u]);
+                load_vec<TT, VEC, MODE>(restored + e0, tv[u]);
+            } else {
+                load_live<PT, VEC, MODE == kStream>(prepared + e0, a.numel - e0, pv[u]);
+                load_live<TT, VEC, MODE == kStream>(restored + e0, a.numel - e0, tv[u]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -189,18 +195,12 @@ __global__ __launch_bounds__(kBlock) void ef_update_kernel(const EfArgs a) {
             RT d[VEC];
 #pragma unroll
             for (int i = 0; i < VEC; ++i) d[i] = narrow<RT>(widen(pv[u][i]) - widen(tv[u][i]));
-            store_vec<RT, VEC, MODE>(residual + e0, d);
+            if constexpr (WHOLE) store_vec<RT, VEC, MODE>(residual + e0, d);
+            else store_live<RT, VEC, MODE == kStream>(residual + e0, a.numel - e0, d);
         }
-        return;
-    }
-    for (int u = 0; u < UNROLL; ++u) {
-        const int64_t e0 = block_first + (static_cast<int64_t>(u) * kBlock + threadIdx.x) * VEC;
-        for (int i = 0; i < VEC; ++i) {
-            const int64_t e = e0 + i;
-            if (e >= a.numel) break;
-            residual[e] = narrow<RT>(widen(prepared[e]) - widen(restored[e]));
-        }
-    }
+    };
+    if (block_first + BLOCK_ELEMS <= a.numel) tiles(std::true_type{});
+    else tiles(std::false_type{});
 }
 
 template <typename PT, typename TT, typename RT>

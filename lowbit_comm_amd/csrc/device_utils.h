@@ -178,41 +178,6 @@ __device__ __forceinline__ void store_vec(T *__restrict__ p, const T (&src)[N]) 
     store_any<T, N, MODE == kStream, MODE == kUnaligned ? sizeof(T) : N * sizeof(T)>(p, src);
 }
 
-// Loads / stores N elements as ceil(N*sizeof(T)/16) instructions of at most 16 bytes.
-template <typename T, int N, int MODE>
-__device__ __forceinline__ void load_wide(const T *__restrict__ p, T (&dst)[N]) {
-    constexpr int PER = 16 / sizeof(T);
-    if constexpr (N <= PER) {
-        load_vec<T, N, MODE>(p, dst);
-    } else {
-        static_assert(N % PER == 0, "whole 16-byte pieces");
-#pragma unroll
-        for (int k = 0; k < N / PER; ++k) {
-            T piece[PER];
-            load_vec<T, PER, MODE>(p + k * PER, piece);
-#pragma unroll
-            for (int i = 0; i < PER; ++i) dst[k * PER + i] = piece[i];
-        }
-    }
-}
-
-template <typename T, int N, int MODE>
-__device__ __forceinline__ void store_wide(T *__restrict__ p, const T (&src)[N]) {
-    constexpr int PER = 16 / sizeof(T);
-    if constexpr (N <= PER) {
-        store_vec<T, N, MODE>(p, src);
-    } else {
-        static_assert(N % PER == 0, "whole 16-byte pieces");
-#pragma unroll
-        for (int k = 0; k < N / PER; ++k) {
-            T piece[PER];
-#pragma unroll
-            for (int i = 0; i < PER; ++i) piece[i] = src[k * PER + i];
-            store_vec<T, PER, MODE>(p + k * PER, piece);
-        }
-    }
-}
-
 // ---- buffer addressing ---------------------------------------------------------
 // A descriptor over [base, base + bytes) held in scalar registers.  Loads and stores through it take a 32-bit
 // byte offset per lane, so a wavefront spends no vector instructions on 64-bit addresses before its first load

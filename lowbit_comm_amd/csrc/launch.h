@@ -136,7 +136,7 @@ struct WireGeneralDecodeArgs {
 
 // Each returns hipSuccess/last launch error, or hipErrorNotSupported when no
 // instantiation exists for the type combination.
-// `mode` is an lbc::AccessMode: 0 element-wise (any alignment), 1 vector, 2 vector + non-temporal.
+// `mode` is an lbc::AccessMode: 0 element alignment, 1 vector, 2 vector + non-temporal.
 hipError_t launch_quant_pack(int x_dtype, int r_dtype, int d_dtype, bool outputs, int group_size, int mode,
                              const QuantArgs &args, int world, hipStream_t stream);
 // Elements one lane owns for that combination (decides the alignment the vector modes need).

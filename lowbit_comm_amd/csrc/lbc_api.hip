@@ -31,8 +31,8 @@ bool aligned_to(const void *p, uintptr_t bytes) { return (reinterpret_cast<uintp
 // torch promotion of two of {f32, f16, bf16}
 int promote(int a, int b) { return a == b ? a : LBC_F32; }
 
-// Access mode of a call (LBC_ACCESS_*): a function of the arguments only, no process state.  Operands that lack
-// the alignment of the vector paths take the element-wise kernels whatever the caller asked for.
+// Access mode of a call (LBC_ACCESS_*): a function of the arguments only, no process state.  Operands that do not
+// start on 16 bytes (codes: on a lane's share of them) take the kernels at element alignment whatever the caller asked for.
 bool valid_access(int access) { return access >= LBC_ACCESS_AUTO && access <= LBC_ACCESS_STREAM; }
 
 int pick_mode(bool aligned, int access) {

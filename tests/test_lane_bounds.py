@@ -68,3 +68,74 @@ def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
         fresh.check(p.float() - want, "new residual")
         prepared.check(p, "prepared")
         x_in.check(x, "input")
+
+
+def payloads_of(world, n, seed, device, g=64):
+    """``world`` payloads covering ``n`` elements: (codes, scales) pairs for the oracle, packed tensors for the kernels."""
+    pairs = [codec_torch.quantize(values(n, torch.float32, seed + r), g) for r in range(world)]
+    return pairs, [codec_torch.pack(*pair).to(device) for pair in pairs]
+
+
+# a workgroup of the decode spans 2048 (fp32) or 4096 (16-bit) outputs, of the reduce half of that from three payloads on
+@pytest.mark.parametrize("n", [1, 7, 66, 1023, 2047, 2049, 4095, 4097, 4096 + 2048 + 5])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_decode_and_reduce_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
+    from lowbit_comm_amd.hip import ops
+
+    t = DTYPES[dtype]
+    pairs, packed = payloads_of(8, n, 100 + n, hip_device)
+    for op in ("none", "sum", "max"):
+        old = values(n, t, n + 1)
+        out = Guarded(n, t, offset, hip_device, old)
+        assert ops.dequant_payload_into(packed[0], out.inside, reduce_op=op)
+        decoded = codec_torch.dequantize(*pairs[0], n, dtype=dtype)
+        want = {"none": decoded, "sum": old + decoded, "max": torch.where(old > decoded, old, decoded)}[op]
+        out.check(want, f"decode {op}")
+    for world in (1, 2, 8):
+        p = values(n, t, n + 2)
+        out, fresh = Guarded(n, t, offset, hip_device), Guarded(n, t, offset, hip_device)
+        prepared = Guarded(n, t, offset, hip_device, p)
+        assert ops.dequant_reduce_into(packed[:world], out.inside, divisor=float(world), prepared=prepared.inside,
+                                       new_residual=fresh.inside)
+        want = codec_torch.reduce_payloads(pairs[:world], n, dtype=dtype, reduce="mean")
+        out.check(want, f"reduce of {world}")
+        fresh.check((p.float() - want.float()).to(t), f"residual of {world}")
+    # shards of an odd bucket: every shard but the first starts off a 16-byte line
+    world, shard = 3, -(-n // 3)
+    shard_pairs, shard_packed = payloads_of(world, shard, 200 + n, hip_device)
+    rows = torch.zeros(world, shard_packed[0].numel() + 4, dtype=torch.uint8, device=hip_device)
+    for row, payload in zip(rows, shard_packed):
+        row[:payload.numel()] = payload
+    out = Guarded(n, t, offset, hip_device)
+    assert ops.dequant_chunks_into(rows, out.inside, shard)
+    out.check(torch.cat([codec_torch.dequantize(*pair, shard, dtype=dtype) for pair in shard_pairs])[:n], "shards")
+
+
+@pytest.mark.parametrize("n", [1, 7, 66, 2047, 2049, 4095, 4097, 8193])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_ring_step_and_feedback_update_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
+    from lowbit_comm_amd.hip import ops
+
+    t = DTYPES[dtype]
+    (pair,), (received,) = payloads_of(1, n, 300 + n, hip_device)
+    start = values(n, t, n + 3)
+    for op in ("sum", "none"):
+        chunk = Guarded(n, t, offset, hip_device, start)
+        send = Guarded(received.numel(), torch.uint8, 3 * offset, hip_device)
+        scales_at = -(-n // 64) * 64
+        if (send.inside.data_ptr() + scales_at) % 4 == 0:        # the payload's scales must lie on 4 bytes
+            assert ops.ring_step_into(received, chunk.inside, send.inside, reduce_op=op, divisor=2.0)
+        else:
+            send = Guarded(received.numel(), torch.uint8, 0, hip_device)
+            assert ops.ring_step_into(received, chunk.inside, send.inside, reduce_op=op, divisor=2.0)
+        decoded = codec_torch.dequantize(*pair, n, dtype=dtype)
+        want = (start + decoded if op == "sum" else decoded) / 2
+        chunk.check(want, f"chunk {op}")
+        send.check(codec_torch.pack(*codec_torch.quantize(want)), f"payload {op}")
+    prepared, restored = values(n, t, n + 4), values(n, t, n + 5)
+    residual = Guarded(n, t, offset, hip_device)
+    assert ops.ef_update_into(Guarded(n, t, offset, hip_device, prepared).inside,
+                              Guarded(n, t, offset, hip_device, restored).inside, residual.inside)
+    residual.check((prepared.float() - restored.float()).to(t), "feedback update")
