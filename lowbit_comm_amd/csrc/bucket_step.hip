@@ -42,7 +42,7 @@ __global__ __launch_bounds__(kBlock) void bucket_step_kernel(const QuantArgs q, 
 
 template <typename XT, typename RT, int VEC, typename OT, int W>
 hipError_t launch_w(int mode, const QuantArgs &q, int quant_world, const ReduceArgs &r, hipStream_t stream) {
-    using QT = quant::quant_tiling<VEC>;
+    using QT = quant::quant_tiling<VEC, quant::quant_unroll<VEC>()>;
     using RTile = reduce::decode_tiling<OT, W>;
     const int64_t padded = (q.shard_numel + 63) / 64 * 64;
     const int64_t quant_grid_x = (padded + QT::BLOCK_ELEMS - 1) / QT::BLOCK_ELEMS;

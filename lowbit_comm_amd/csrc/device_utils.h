@@ -20,6 +20,10 @@ using bf16 = __bf16;
 constexpr int kWave = 64;
 constexpr int kBlock = LBC_BLOCK;
 constexpr int kWavesPerBlock = kBlock / kWave;
+// Wavefronts the chip holds at once (256 CUs of 32).  A launch whose tiles fit them all gives every wavefront one tile:
+// several tiles a wavefront then only leave compute units without work and put the tiles' arithmetic one behind the
+// other.  Beyond that more tiles in flight per wavefront pay, as measured kernel by kernel.
+constexpr int64_t kResidentWaves = 256 * 32;
 
 // Index of the u-th tile a wavefront handles inside its block.  Order 0: the block's
 // wavefronts sweep the block's span together (tile = u * waves + wave); order 1: each

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kBlock) void bucket_pipeline_step_kernel(const Quan
 template <typename T, typename RT, int VEC, int W>
 hipError_t launch_w(int mode, const QuantArgs *q, int quant_world, const ReduceQuantArgs *r, const DecodeArgs *d,
                     int decode_world, hipStream_t stream) {
-    using QT = quant::quant_tiling<VEC>;
+    using QT = quant::quant_tiling<VEC, quant::quant_unroll<VEC>()>;
     using DTile = reduce::decode1_tiling<T>;
     constexpr int G = 64;
     const QuantArgs qa = q ? *q : QuantArgs{};

@@ -21,14 +21,14 @@ namespace {
 
 using namespace quant;
 
-template <typename XT, typename RT, typename DT, int G, int VEC, int MODE>
+template <typename XT, typename RT, typename DT, int G, int VEC, int MODE, int TILES>
 __global__ __launch_bounds__(kBlock) void quant_pack_kernel(const QuantArgs a) {
-    quant_pack_block<XT, RT, DT, G, VEC, MODE>(a, blockIdx.x, gridDim.x, blockIdx.y);
+    quant_pack_block<XT, RT, DT, G, VEC, MODE, TILES>(a, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
-template <typename XT, typename RT, typename DT, int G, int VEC>
-hipError_t launch_typed(int mode, const QuantArgs &a, int world, hipStream_t stream) {
-    using T = quant_tiling<VEC>;
+template <typename XT, typename RT, typename DT, int G, int VEC, int TILES>
+hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t stream) {
+    using T = quant_tiling<VEC, TILES>;
     const int64_t groups = (a.shard_numel + G - 1) / G;
     const int64_t padded = groups * G;
     const int64_t blocks = (padded + T::BLOCK_ELEMS - 1) / T::BLOCK_ELEMS;
@@ -36,11 +36,21 @@ hipError_t launch_typed(int mode, const QuantArgs &a, int world, hipStream_t str
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
     switch (mode) {
-        case kStream: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStream>), grid, dim3(kBlock), 0, stream, a); break;
-        case kVector: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kVector>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kUnaligned>), grid, dim3(kBlock), 0, stream, a); break;
+        case kStream: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStream, TILES>), grid, dim3(kBlock), 0, stream, a); break;
+        case kVector: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kVector, TILES>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kUnaligned, TILES>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
+}
+
+// One tile a wavefront while the tiles fit the chip's wavefront slots (2 Mi elements of four a lane, 4 Mi of eight):
+// one tile against the usual number, us: fp32 10,007 elements 1.9 / 2.3, 65,536 2.1 / 2.4, 1 Mi 2.9 / 3.2, 2 Mi 3.6 / 3.9,
+// 4 Mi 5.7 / 5.5, 6.6 M 8.9 / 7.4; bf16 10,007 2.0 / 2.2, 1 Mi 2.6 / 2.8, 4 Mi 3.8 / 3.9, 13.1 M 9.5 / 8.9; bf16 with an
+// fp32 residual 10,007 2.3 / 3.5, 1 Mi 4.2 / 4.5, 2 Mi 6.0 / 6.3, 6.6 M 15.0 / 14.0.
+template <typename XT, typename RT, typename DT, int G, int VEC>
+hipError_t launch_typed(int mode, const QuantArgs &a, int world, hipStream_t stream) {
+    if (a.numel <= kResidentWaves * kWave * VEC) return launch_tiles<XT, RT, DT, G, VEC, 1>(mode, a, world, stream);
+    return launch_tiles<XT, RT, DT, G, VEC, quant_unroll<VEC>()>(mode, a, world, stream);
 }
 
 template <typename XT, typename RT, typename DT, int VEC>
@@ -66,7 +76,10 @@ hipError_t launch_x(int x_dtype, int r_dtype, int d_dtype, bool outputs, int g, 
         return launch_group<XT, void, float, 4>(g, mode, a, world, s);
     }
     if (r_dtype == x_dtype) {
-        if (d_is_x) return launch_group<XT, XT, XT, WIDE>(g, mode, a, world, s);
+        // Without `restored` and `new_residual` nothing is rounded to DT, so the call is as narrow as its tensors:
+        // 13.1 M bf16 elements with a bf16 residual and their sum as a second output (the all_gather hook's quantize)
+        // take the same 16.5 us either way, 1.3 M 4.4 us with 8 elements a lane and 4.6 us with 4, 131,072 2.9 and 3.1 us.
+        if (d_is_x || !outputs) return launch_group<XT, XT, XT, WIDE>(g, mode, a, world, s);
         return launch_group<XT, XT, float, 4>(g, mode, a, world, s);
     }
     if (r_dtype == kF32) {
@@ -82,7 +95,7 @@ int quant_pack_vec(int x_dtype, int r_dtype, int d_dtype, bool outputs) {
     if (x_dtype == kF32) return 4;
     const bool d_is_x = d_dtype == x_dtype;
     if (r_dtype == kNone) return (!outputs || d_is_x) ? 8 : 4;
-    if (r_dtype == x_dtype) return d_is_x ? 8 : 4;
+    if (r_dtype == x_dtype) return (d_is_x || !outputs) ? 8 : 4;
     return 4;
 }
 

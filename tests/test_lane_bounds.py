@@ -33,8 +33,8 @@ class Guarded:
         assert bool((outside == 0x5A).all()), f"{what}: wrote outside"
 
 
-# a workgroup of the quantize spans 4096 (fp32) or 8192 (16-bit) elements, a lane 4 or 8
-@pytest.mark.parametrize("n", [1, 5, 66, 4095, 4097, 8191, 8193, 2 * 8192 + 3])
+# a workgroup of the quantize spans 1024 elements (4 a lane) or 2048 (8 a lane) of a tensor that the chip holds at once
+@pytest.mark.parametrize("n", [1, 5, 66, 1023, 1025, 2047, 2049, 4097, 8193, 2 * 8192 + 3])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
 def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
@@ -68,6 +68,24 @@ def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
         fresh.check(p.float() - want, "new residual")
         prepared.check(p, "prepared")
         x_in.check(x, "input")
+
+
+# the tile count per wavefront changes where the chip holds no more: 2 Mi elements of four a lane, 4 Mi of eight
+@pytest.mark.parametrize("dtype, residual_type, edge", [("fp32", None, 1 << 21), ("bf16", None, 1 << 22), ("bf16", "fp32", 1 << 21),
+                                                        ("fp16", "fp16", 1 << 22)])
+def test_quantize_on_both_sides_of_the_tile_rule(hip_device, dtype, residual_type, edge):
+    from lowbit_comm_amd.hip import ops
+
+    for n in (edge, edge + 1, edge + 4096 + 5):
+        x = values(n, DTYPES[dtype], n)
+        r = None if residual_type is None else values(n, DTYPES[residual_type], n + 7, 1e-5)
+        p = x if r is None else x + r
+        prepared = Guarded(n, p.dtype, 0, hip_device)
+        payload = Guarded(ops.payload_nbytes(n), torch.uint8, 0, hip_device)
+        assert ops.quant_pack_payload_into(x.to(hip_device), payload.inside, residual=None if r is None else r.to(hip_device),
+                                           prepared_out=prepared.inside)
+        payload.check(codec_torch.pack(*codec_torch.quantize(p)), f"payload of {n}")
+        prepared.check(p, f"prepared of {n}")
 
 
 def payloads_of(world, n, seed, device, g=64):
