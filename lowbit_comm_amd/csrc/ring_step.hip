@@ -24,19 +24,20 @@
 namespace lbc {
 namespace {
 
-// Tiles in flight per wavefront, as measured on 1.6 M to 26 M element chunks: the accumulating step, which reads
-// and writes the chunk, is fastest with one (more wavefronts resident), the write-only steps with four (fp32) or
-// two (16-bit) tiles of loads issued ahead.
-template <typename T, bool ACC> struct ring_tiling {
+// Tiles in flight per wavefront beyond the chip's wavefront slots: one, except for the write-only step on a 16-bit chunk,
+// which keeps two (decode only, 26.2 M bf16 elements 13.6 us with two, 14.2 with one; decode + requantize 15.8 / 16.1).
+// An fp32 chunk's write-only step used to keep four: 26.2 M elements 23.5 us, with one 22.3; 6.6 M 7.8 and 7.0 us.
+template <typename T, bool ACC> constexpr int ring_unroll() { return ACC || sizeof(T) == 4 ? 1 : 2; }
+template <typename T, int TILES> struct ring_tiling {
     static constexpr int VEC = 16 / sizeof(T);
     static constexpr int TILE = kWave * VEC;
-    static constexpr int UNROLL = ACC ? 1 : (sizeof(T) == 4 ? 4 : 2);
+    static constexpr int UNROLL = TILES;
     static constexpr int BLOCK_ELEMS = TILE * kWavesPerBlock * UNROLL;
 };
 
-template <typename T, int G, int MODE, bool ACC>
+template <typename T, int G, int MODE, bool ACC, int TILES>
 __global__ __launch_bounds__(kBlock) void ring_step_kernel(const RingStepArgs a) {
-    using L = ring_tiling<T, ACC>;
+    using L = ring_tiling<T, TILES>;
     constexpr int VEC = L::VEC;
     constexpr int LPG = G / VEC;
     constexpr int UNROLL = L::UNROLL;
@@ -122,20 +123,29 @@ __global__ __launch_bounds__(kBlock) void ring_step_kernel(const RingStepArgs a)
     else tiles(std::false_type{});
 }
 
-template <typename T, int G, bool ACC>
-hipError_t launch_ring_g(int mode, const RingStepArgs &a, hipStream_t stream) {
-    using L = ring_tiling<T, ACC>;
+template <typename T, int G, bool ACC, int TILES>
+hipError_t launch_ring_tiles(int mode, const RingStepArgs &a, hipStream_t stream) {
+    using L = ring_tiling<T, TILES>;
     const int64_t padded = (a.numel + G - 1) / G * G;
     const int64_t blocks = (padded + L::BLOCK_ELEMS - 1) / L::BLOCK_ELEMS;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks));
     switch (mode) {
-        case kStream: hipLaunchKernelGGL((ring_step_kernel<T, G, kStream, ACC>), grid, dim3(kBlock), 0, stream, a); break;
-        case kVector: hipLaunchKernelGGL((ring_step_kernel<T, G, kVector, ACC>), grid, dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((ring_step_kernel<T, G, kUnaligned, ACC>), grid, dim3(kBlock), 0, stream, a); break;
+        case kStream: hipLaunchKernelGGL((ring_step_kernel<T, G, kStream, ACC, TILES>), grid, dim3(kBlock), 0, stream, a); break;
+        case kVector: hipLaunchKernelGGL((ring_step_kernel<T, G, kVector, ACC, TILES>), grid, dim3(kBlock), 0, stream, a); break;
+        default: hipLaunchKernelGGL((ring_step_kernel<T, G, kUnaligned, ACC, TILES>), grid, dim3(kBlock), 0, stream, a); break;
     }
     return hipGetLastError();
+}
+
+// One tile a wavefront while the tiles fit the chip's wavefront slots (decode + requantize, us with one / two tiles: 65,536
+// bf16 elements 2.0 / 2.3, 1 Mi 2.7 / 3.0, 4 Mi 4.1 / 4.3, 6.6 M 5.4 / 5.4).
+template <typename T, int G, bool ACC>
+hipError_t launch_ring_g(int mode, const RingStepArgs &a, hipStream_t stream) {
+    constexpr int TILES = ring_unroll<T, ACC>();
+    if (TILES > 1 && a.numel <= kResidentWaves * ring_tiling<T, 1>::TILE) return launch_ring_tiles<T, G, ACC, 1>(mode, a, stream);
+    return launch_ring_tiles<T, G, ACC, TILES>(mode, a, stream);
 }
 
 template <typename T>

@@ -130,7 +130,8 @@ def test_decode_and_reduce_at_block_ends_and_start_offsets(hip_device, dtype, of
     out.check(torch.cat([codec_torch.dequantize(*pair, shard, dtype=dtype) for pair in shard_pairs])[:n], "shards")
 
 
-@pytest.mark.parametrize("n", [1, 7, 66, 2047, 2049, 4095, 4097, 8193])
+# a workgroup of the ring step spans 1024 (fp32) or 2048 (16-bit) elements, 4096 of a 16-bit chunk above 4 Mi elements
+@pytest.mark.parametrize("n", [1, 7, 66, 1023, 1025, 2047, 2049, 4097, 8193, (1 << 22) + 4095, (1 << 22) + 4097])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
 def test_ring_step_and_feedback_update_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
