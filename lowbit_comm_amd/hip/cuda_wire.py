@@ -14,7 +14,6 @@ from typing import Sequence
 
 import torch
 
-from lowbit_comm_amd.hip.library import load_library
 from lowbit_comm_amd.hip.ops import (MAX_PAYLOADS, REDUCE_OPS, BoundLaunch, _device_tensor, _float_tensor, _ptr,
                                      _require, access_code, num_groups)
 
@@ -39,7 +38,6 @@ def _payload(t: torch.Tensor, name: str, device: torch.device, nbytes: int) -> N
 def bind_quant_pack(x: torch.Tensor, payload: torch.Tensor, *, group_size: int = 64, compact: bool = True,
                     residual: torch.Tensor | None = None, bit: int = 8,
                     access: str | None = None) -> BoundLaunch:
-    lib = load_library()
     code = _float_tensor(x, "input")
     _payload(payload, "output", x.device, payload_nbytes(x.numel(), x.dtype, group_size, bit))
     if residual is not None:
@@ -47,7 +45,7 @@ def bind_quant_pack(x: torch.Tensor, payload: torch.Tensor, *, group_size: int =
         _require(residual.dtype == x.dtype, "input and residual must have the same dtype")
         _require(residual.numel() == x.numel(), "input and residual must have the same number of elements")
     args = (_ptr(x), _ptr(residual), code, x.numel(), group_size, int(bit), int(compact), _ptr(payload))
-    return BoundLaunch(lib.lbc_wire_quant_pack, args + (access_code(access),), x.device, lib, (x, residual, payload))
+    return BoundLaunch("lbc_wire_quant_pack", args + (access_code(access),), x.device, (x, residual, payload))
 
 
 def quant_pack_into(x: torch.Tensor, payload: torch.Tensor, *, group_size: int = 64, compact: bool = True,
@@ -71,7 +69,6 @@ def bind_quant_pack_chunks(x: torch.Tensor, payloads: torch.Tensor, world: int, 
                            compact: bool = True, residual: torch.Tensor | None = None, bit: int = 8,
                            access: str | None = None) -> BoundLaunch:
     """``payloads`` is a ``(world, stride)`` uint8 tensor; row d receives chunk d of ``ceil(numel/world)`` elements."""
-    lib = load_library()
     code = _float_tensor(x, "input")
     _payload_rows(payloads, x.device)
     _require(payloads.shape[0] == world, "payloads must have one row per chunk")
@@ -83,21 +80,20 @@ def bind_quant_pack_chunks(x: torch.Tensor, payloads: torch.Tensor, world: int, 
                  "input and residual must have the same dtype and number of elements")
     args = (_ptr(x), _ptr(residual), code, x.numel(), world, group_size, int(bit), int(compact), _ptr(payloads),
             payloads.stride(0))
-    return BoundLaunch(lib.lbc_wire_quant_pack_chunks, args + (access_code(access),), x.device, lib,
+    return BoundLaunch("lbc_wire_quant_pack_chunks", args + (access_code(access),), x.device,
                        (x, residual, payloads))
 
 
 def bind_dequant(payload: torch.Tensor, out: torch.Tensor, *, numel: int | None = None, group_size: int = 64,
                  compact: bool = True, reduce_op: str = "none", bit: int = 8,
                  access: str | None = None) -> BoundLaunch:
-    lib = load_library()
     code = _float_tensor(out, "output")
     n = out.numel() if numel is None else int(numel)
     _require(0 <= n <= out.numel(), "numel exceeds the output size")
     _require(reduce_op in REDUCE_OPS, f"unsupported reduce op {reduce_op!r}")
     _payload(payload, "input", out.device, payload_nbytes(n, out.dtype, group_size, bit))
     args = (_ptr(payload), n, group_size, int(bit), int(compact), _ptr(out), code, REDUCE_OPS[reduce_op])
-    return BoundLaunch(lib.lbc_wire_dequant, args + (access_code(access),), out.device, lib, (payload, out))
+    return BoundLaunch("lbc_wire_dequant", args + (access_code(access),), out.device, (payload, out))
 
 
 def dequant_into(payload: torch.Tensor, out: torch.Tensor, *, numel: int | None = None, group_size: int = 64,
@@ -110,7 +106,6 @@ def dequant_into(payload: torch.Tensor, out: torch.Tensor, *, numel: int | None 
 
 def bind_dequant_chunks(payloads: torch.Tensor, out: torch.Tensor, shard_numel: int, *, group_size: int = 64,
                         compact: bool = True, bit: int = 8, access: str | None = None) -> BoundLaunch:
-    lib = load_library()
     code = _float_tensor(out, "output")
     _payload_rows(payloads, out.device)
     world = payloads.shape[0]
@@ -118,7 +113,7 @@ def bind_dequant_chunks(payloads: torch.Tensor, out: torch.Tensor, shard_numel: 
     _require(payloads.shape[1] >= payload_nbytes(shard_numel, out.dtype, group_size, bit), "payload rows are too small")
     args = (_ptr(payloads), payloads.stride(0), world, shard_numel, out.numel(), group_size, int(bit), int(compact),
             _ptr(out), code, REDUCE_OPS["none"])
-    return BoundLaunch(lib.lbc_wire_dequant_chunks, args + (access_code(access),), out.device, lib, (payloads, out))
+    return BoundLaunch("lbc_wire_dequant_chunks", args + (access_code(access),), out.device, (payloads, out))
 
 
 def bind_dequant_reduce(payloads: Sequence[torch.Tensor], out: torch.Tensor, *, numel: int | None = None,
@@ -126,7 +121,6 @@ def bind_dequant_reduce(payloads: Sequence[torch.Tensor], out: torch.Tensor, *, 
                         fused_multiply_add: bool = True, prepared: torch.Tensor | None = None,
                         new_residual: torch.Tensor | None = None, access: str | None = None) -> BoundLaunch | None:
     """``None`` when the request has no kernel (more than 8 payloads, group size other than 64)."""
-    lib = load_library()
     _require(len(payloads) > 0, "inputs must not be empty")
     _require(inv_divisor > 0, "inv_divisor must be > 0")
     code = _float_tensor(out, "output")
@@ -148,7 +142,7 @@ def bind_dequant_reduce(payloads: Sequence[torch.Tensor], out: torch.Tensor, *, 
             _require(t.numel() == n, f"{name} must have numel elements")
     args = (pointers, len(payloads), n, group_size, int(compact), float(inv_divisor), int(fused_multiply_add),
             _ptr(out), code, _ptr(prepared), _ptr(new_residual))
-    return BoundLaunch(lib.lbc_wire_dequant_reduce, args + (access_code(access),), device, lib,
+    return BoundLaunch("lbc_wire_dequant_reduce", args + (access_code(access),), device,
                        (tuple(payloads), out, prepared, new_residual))
 
 
@@ -172,7 +166,6 @@ def bind_ring_step(received: torch.Tensor, chunk: torch.Tensor, send: torch.Tens
                    divisor: float = 1.0, access: str | None = None) -> BoundLaunch:
     """One ring / tree hop in this format: ``chunk (op)= decode(received)``, ``chunk *= 1/divisor`` (torch's device
     ``div_``), and - with ``send`` - the payload of the updated chunk, in one launch.  ``chunk`` holds whole groups."""
-    lib = load_library()
     code = _float_tensor(chunk, "chunk")
     n = chunk.numel()
     _require(n % group_size == 0, "numel should be multiple of group_size")
@@ -185,7 +178,7 @@ def bind_ring_step(received: torch.Tensor, chunk: torch.Tensor, send: torch.Tens
         _require(n == 0 or send.data_ptr() != received.data_ptr(), "the payload to send must not alias the received one")
     args = (_ptr(received), _ptr(chunk), code, n, group_size, int(compact), REDUCE_OPS[reduce_op], float(divisor),
             _ptr(send))
-    return BoundLaunch(lib.lbc_wire_ring_step, args + (access_code(access),), chunk.device, lib,
+    return BoundLaunch("lbc_wire_ring_step", args + (access_code(access),), chunk.device,
                        (received, chunk, send))
 
 
@@ -211,7 +204,6 @@ def bind_quant_general(x: torch.Tensor, payload: torch.Tensor, *, group_size: in
                        quant_type: str = "linear", topk: int = 0, stochastic: tuple[int, int] | None = None,
                        compact: bool = False) -> BoundLaunch:
     """``stochastic`` is the (seed, offset) pair of the Philox stream, ``None`` for round-to-nearest."""
-    lib = load_library()
     code = _float_tensor(x, "input")
     kind = _policy(quant_type, bit, topk)
     _require(x.numel() % group_size == 0, "input numel should be multiple of group_size")
@@ -219,7 +211,7 @@ def bind_quant_general(x: torch.Tensor, payload: torch.Tensor, *, group_size: in
     seed, offset = (0, 0) if stochastic is None else (int(stochastic[0]), int(stochastic[1]))
     args = (_ptr(x), code, x.numel(), group_size, int(bit), kind, int(topk), int(stochastic is not None),
             seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, int(compact), _ptr(payload))
-    return BoundLaunch(lib.lbc_wire_quant_general, args, x.device, lib, (x, payload))
+    return BoundLaunch("lbc_wire_quant_general", args, x.device, (x, payload))
 
 
 def quant_general_into(x: torch.Tensor, payload: torch.Tensor, **policy) -> bool:
@@ -230,7 +222,6 @@ def quant_general_into(x: torch.Tensor, payload: torch.Tensor, **policy) -> bool
 def bind_dequant_general(payload: torch.Tensor, out: torch.Tensor, *, group_size: int = 64, bit: int = 8,
                          quant_type: str = "linear", topk: int = 0, compact: bool = False,
                          reduce_op: str = "none") -> BoundLaunch:
-    lib = load_library()
     code = _float_tensor(out, "output")
     kind = _policy(quant_type, bit, topk)
     _require(reduce_op in REDUCE_OPS, f"unsupported reduce op {reduce_op!r}")
@@ -238,7 +229,7 @@ def bind_dequant_general(payload: torch.Tensor, out: torch.Tensor, *, group_size
     _payload(payload, "input", out.device, general_payload_nbytes(out.numel(), out.dtype, group_size, bit, topk))
     args = (_ptr(payload), out.numel(), group_size, int(bit), kind, int(topk), int(compact), _ptr(out), code,
             REDUCE_OPS[reduce_op])
-    return BoundLaunch(lib.lbc_wire_dequant_general, args, out.device, lib, (payload, out))
+    return BoundLaunch("lbc_wire_dequant_general", args, out.device, (payload, out))
 
 
 def dequant_general_into(payload: torch.Tensor, out: torch.Tensor, **policy) -> bool:

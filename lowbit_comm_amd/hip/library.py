@@ -83,6 +83,21 @@ class DequantChunksStage(ctypes.Structure):
 
 
 _library: ctypes.CDLL | None = None
+_host_error: str | None = None
+
+
+def native_host():
+    """The native host side (``lowbit_comm_amd._host``, ``csrc/host_module.cpp``), or ``None`` when it is not built:
+    importing this package needs no build, and :func:`load_library` says what is missing."""
+    global _host_error
+    try:
+        import torch  # noqa: F401  (its libraries first: the module links against them)
+
+        from lowbit_comm_amd import _host
+    except ImportError as exc:
+        _host_error = str(exc)
+        return None
+    return _host
 
 
 def load_library(path: str | Path | None = None) -> ctypes.CDLL:
@@ -109,6 +124,12 @@ def load_library(path: str | Path | None = None) -> ctypes.CDLL:
     if version != ABI_VERSION:
         raise CCDLUnavailableError(f"{target.name} has ABI version {version}, expected {ABI_VERSION}")
     if path is None:
+        host = native_host()
+        if host is None:
+            raise CCDLUnavailableError(f"lowbit_comm_amd._host cannot be loaded (run `make -C lowbit_comm_amd/csrc` or "
+                                       f"__graft_entry__.build()): {_host_error}")
+        if host.abi_version() != ABI_VERSION:
+            raise CCDLUnavailableError(f"lowbit_comm_amd._host was built for another ABI version than {target.name}")
         _library = lib
     return lib
 
