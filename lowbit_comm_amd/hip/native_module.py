@@ -15,7 +15,6 @@ and ignored: the portable format has a single layout.
 from __future__ import annotations
 
 import enum
-import operator
 import threading
 from collections import OrderedDict
 from typing import Sequence
@@ -23,7 +22,9 @@ from typing import Sequence
 import torch
 
 from lowbit_comm_amd.hip import ops
-from lowbit_comm_amd.hip.library import load_library
+from lowbit_comm_amd.hip.library import load_library, native_host
+
+_host = native_host()
 
 
 class QuantType(enum.IntEnum):
@@ -47,8 +48,6 @@ class ReduceOP(enum.IntEnum):
     MIN = 3
 
 
-_IS_CUDA = operator.attrgetter("is_cuda")
-_DTYPE = operator.attrgetter("dtype")
 _TORCH_OF = {DType.FP16: torch.float16, DType.BF16: torch.bfloat16, DType.FP32: torch.float32}
 _OP_NAME = {ReduceOP.NONE: "none", ReduceOP.SUM: "sum", ReduceOP.MAX: "max", ReduceOP.MIN: "min"}
 
@@ -143,35 +142,21 @@ class HipNativeModule:
         return bound
 
     @staticmethod
-    def _spec(tensor):
-        """What a binding depends on, for a contiguous GPU tensor; ``None`` for anything else (the caller then takes
-        the validating path, which names what is wrong)."""
-        if tensor is None:
-            return ()
-        if not isinstance(tensor, torch.Tensor) or not tensor.is_cuda or not tensor.is_contiguous():
-            return None
-        return (tensor.data_ptr(), tensor.dtype, tensor.numel())
+    def _key(tag, policy, *operands):
+        """Memo key of an in-place call: addresses, types and element counts of every operand (tensors, ``None``, a list
+        of payloads) and the policy; ``None`` when an operand is no contiguous GPU tensor (the caller then takes the
+        validating path, which names what is wrong).  One native call: this runs for every bucket."""
+        specs = _host.specs(*operands)
+        return None if specs is None else (tag, specs, policy)
 
-    def _reduce_key(self, tag, inputs, tensors, policy):
-        """Memo key of a fused reduce: payload addresses and sizes, the other tensors' specs, the policy."""
-        if not isinstance(inputs, (list, tuple)) or not 1 <= len(inputs) <= ops.MAX_PAYLOADS:
-            return None
-        specs = []
-        for tensor in tensors:
-            spec = self._spec(tensor)
-            if spec is None:
-                return None
-            specs.append(spec)
-        try:        # loops that stay in C: this runs for every bucket
-            if not (all(map(_IS_CUDA, inputs)) and all(map(torch.Tensor.is_contiguous, inputs))):
-                return None
-            return (tag, tuple(map(torch.Tensor.data_ptr, inputs)), tuple(map(torch.Tensor.numel, inputs)),
-                    tuple(map(_DTYPE, inputs)), tuple(specs), policy)
-        except (TypeError, AttributeError):      # something in the list is not a tensor
-            return None
+    # The portable format pads the last group with zeros while it encodes: the facade need not hand over whole groups.
+    _PADS_THE_LAST_GROUP = True
 
     # ---- quantize ------------------------------------------------------------------------------
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
+        payload = _host.quantize(input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
+        if isinstance(payload, torch.Tensor):
+            return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         output = torch.empty(ops.payload_nbytes(input.numel(), group_size), dtype=torch.uint8, device=input.device)
         self.inplace_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact)
@@ -195,6 +180,10 @@ class HipNativeModule:
         would have computed in a kernel of its own (ccdl_comm/quantization/error_feedback.py:27-36)."""
         if not _policy_supported(group_size, topk, stochastic, bit, quant_type):
             return False
+        key = self._key("quant_pack", group_size, input, output, residual, prepared_out)
+        bound = self._recall(key)
+        if bound is not None:
+            return bound()
         if not isinstance(input, torch.Tensor) or not input.is_cuda:
             raise RuntimeError("input must be a GPU tensor")
         if not input.is_contiguous():
@@ -212,14 +201,19 @@ class HipNativeModule:
         bind = lambda: ops.bind_quant_pack_payload(input.reshape(-1), output, group_size=group_size,  # noqa: E731
                                                    residual=None if residual is None else residual.reshape(-1),
                                                    prepared_out=None if prepared_out is None else prepared_out.reshape(-1))
-        out_spec, r_spec, p_spec = self._spec(output), self._spec(residual), self._spec(prepared_out)
-        if out_spec is None or r_spec is None or p_spec is None:
-            return bind()()
-        key = ("quant_pack", input.data_ptr(), input.dtype, input.numel(), out_spec, r_spec, p_spec, group_size)
-        return self._memoized(key, bind)()
+        return (bind() if key is None else self._memoized(key, bind))()
 
     # ---- dequantize -----------------------------------------------------------------------------
+    def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype):
+        """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
+        all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
+        decoded = _host.dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, ops.access_code(None))
+        return decoded if isinstance(decoded, torch.Tensor) else None
+
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
+        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype)
+        if decoded is not None:
+            return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
         _check_payload(input, "input")
         output = torch.empty(_padded_numel_of(input, group_size), dtype=_TORCH_OF[DType(int(dtype))],
@@ -257,6 +251,12 @@ class HipNativeModule:
             return [buffer.reshape(-1) for buffer in inputs]
         return [_views(buffer, group_size) for buffer in inputs]
 
+    def _dequantize_reduce_shaped(self, inputs, shape, group_size, topk, bit, quant_type, dtype, divisor):
+        """Decode and reduce into a fresh tensor of ``shape`` in one native call; ``None`` as in the decode."""
+        reduced = _host.dequantize_reduce(inputs, shape, dtype, group_size, topk, bit, quant_type, divisor,
+                                          ops.access_code(None))
+        return reduced if isinstance(reduced, torch.Tensor) else None
+
     def dequantize_reduce(self, inputs, group_size, topk, bit, quant_type, dtype, compact):
         _require_policy(group_size, topk, False, bit, quant_type)
         if len(inputs) == 0:
@@ -289,7 +289,7 @@ class HipNativeModule:
         _check_payload(inputs[0], "input")
         flat = output.reshape(-1)
         numel = min(flat.numel(), _padded_numel_of(inputs[0], group_size))
-        key = self._reduce_key("reduce", inputs, (flat,), (group_size, topk, bit, int(quant_type), numel))
+        key = self._key("reduce", (group_size, topk, bit, int(quant_type), numel), inputs, flat)
         bound = self._recall(key)
         if bound is not None:
             if not bound():
@@ -329,8 +329,7 @@ class HipNativeModule:
                                        divisor) -> bool:
         if divisor <= 0:
             raise RuntimeError("divisor must be > 0")
-        key = self._reduce_key("reduce_mean", inputs, (output,),
-                               (group_size, topk, bit, int(quant_type), float(divisor)))
+        key = self._key("reduce_mean", (group_size, topk, bit, int(quant_type), float(divisor)), inputs, output)
         bound = self._recall(key)
         if bound is None:
             if not self._fused_eligible(inputs, output, group_size, topk, bit, quant_type):
@@ -371,8 +370,8 @@ class HipNativeModule:
         """One launch: ``restored = mean/sum of payloads``, ``residual = prepared - restored``."""
         if divisor <= 0:
             raise RuntimeError("divisor must be > 0")
-        key = self._reduce_key("reduce_mean_feedback", inputs, (prepared, restored, residual),
-                               (group_size, topk, bit, int(quant_type), float(divisor)))
+        key = self._key("reduce_mean_feedback", (group_size, topk, bit, int(quant_type), float(divisor)),
+                        inputs, prepared, restored, residual)
         bound = self._recall(key)
         if bound is not None:
             return bound()

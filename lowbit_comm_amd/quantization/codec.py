@@ -37,9 +37,10 @@ def _module_of(extension_status: Any | None) -> object:
 
 
 def _symbol(owner: object, name: str) -> Any:
-    if not hasattr(owner, name):
-        raise CCDLUnavailableError(f"{_MODULE_LABEL} missing required symbol: {name}")
-    return getattr(owner, name)
+    try:
+        return getattr(owner, name)
+    except AttributeError:
+        raise CCDLUnavailableError(f"{_MODULE_LABEL} missing required symbol: {name}") from None
 
 
 def _quant_type(module: object, config: CompressionConfig) -> Any:
@@ -179,7 +180,9 @@ def quantize_tensor(tensor: object, config: CompressionConfig, *, extension_stat
         return output
     if output is not None and _try_quantize_pack(module, tensor, output, residual, config, metadata, quant_type):
         return output
-    prepared = _zero_padded(tensor if residual is None else tensor + residual, config.group_size)
+    prepared = tensor if residual is None else tensor + residual
+    if output is not None or not getattr(module, "_PADS_THE_LAST_GROUP", False):
+        prepared = _zero_padded(prepared, config.group_size)
     policy = (config.group_size, config.topk, config.stochastic, config.bit, quant_type, config.compact)
     if output is not None:
         _symbol(module, "inplace_quantize")(prepared, output, *policy)
@@ -206,6 +209,11 @@ def dequantize_tensor(buffer: object, shape: tuple[int, ...], config: Compressio
     dtype_member = _dtype(module, dtype)
     op = _reduce_op(module, reduce_op)
     if output is None:
+        shaped = getattr(module, "_dequantize_shaped", None)
+        if shaped is not None:          # a module that decodes straight into the shape: nothing to trim afterwards
+            decoded = shaped(buffer, shape, config.group_size, config.topk, config.bit, op, quant_type, dtype_member)
+            if decoded is not None:
+                return decoded
         decoded = _symbol(module, "dequantize")(buffer, config.group_size, config.topk, config.bit, op, quant_type,
                                                 dtype_member, config.compact)
     else:
@@ -225,6 +233,12 @@ def dequantize_reduce_tensors(buffers: list[object], shape: tuple[int, ...], con
     dtype_member = _dtype(module, dtype)
     fused = False
     if output is None:
+        shaped = getattr(module, "_dequantize_reduce_shaped", None)
+        if shaped is not None:
+            decoded = shaped(buffers, shape, config.group_size, config.topk, config.bit, quant_type, dtype_member,
+                             len(buffers) if reduce == "mean" else 1)
+            if decoded is not None:
+                return decoded
         decoded = None
         one_launch = getattr(module, "dequantize_reduce_mean", None) if reduce == "mean" else None
         if one_launch is not None:      # an extension that divides in the reduce launch itself (same bits)
