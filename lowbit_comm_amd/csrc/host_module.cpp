@@ -17,6 +17,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/Context.h>
+#include <ATen/core/Generator.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
@@ -27,6 +29,7 @@
 
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -329,10 +332,10 @@ PyObject *dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
 int payloads_of(PyObject *list, int64_t &nbytes, const uint8_t **pointers, const at::Tensor *&first) {
     PyObject **items;
     Py_ssize_t count;
-    if (PyList_CheckExact(list)) {
+    if (PyList_Check(list)) {
         items = reinterpret_cast<PyListObject *>(list)->ob_item;
         count = PyList_GET_SIZE(list);
-    } else if (PyTuple_CheckExact(list)) {
+    } else if (PyTuple_Check(list)) {
         items = reinterpret_cast<PyTupleObject *>(list)->ob_item;
         count = PyTuple_GET_SIZE(list);
     } else {
@@ -388,6 +391,137 @@ PyObject *dequantize_reduce(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the CUDA extension's format ---------------------------------------------------------------------------------
+bool cuda_policy(const Policy &p) {
+    return valid_group(p.group) && p.topk >= 0 && p.topk <= 2 && (p.bit == 8 || p.bit == 4) && p.quant_type >= LBC_QUANT_LINEAR &&
+           p.quant_type <= LBC_QUANT_E2M1 && (p.quant_type == LBC_QUANT_LINEAR || p.bit == 4);
+}
+bool plain(const Policy &p) { return p.topk == 0 && p.stochastic == 0 && p.quant_type == LBC_QUANT_LINEAR; }
+// bytes of a group: codes, the scale in the tensor's type, with outliers the index word and the outliers themselves
+int64_t cuda_group_bytes(const Policy &p, int type) {
+    return p.group * p.bit / 8 + (type == LBC_F32 ? 4 : 2) * (p.topk == 0 ? 1 : p.topk + 2);
+}
+
+// (seed, offset) of the device's default generator, advanced past `increment` draws rounded up to a multiple of four, as
+// HipCudaWireModule.philox_engine_inputs does it.
+std::pair<uint64_t, uint64_t> philox_inputs(const at::Tensor &x, uint64_t increment) {
+    at::Generator generator = at::globalContext().defaultGenerator(x.device());
+    std::lock_guard<std::mutex> lock(generator.mutex());
+    const uint64_t offset = generator.get_offset();
+    generator.set_offset(offset + (increment + 3) / 4 * 4);
+    return {generator.current_seed(), offset};
+}
+
+// wire_quantize(input, output or None, group_size, topk, stochastic, bit, quant_type, compact, access) -> payload
+PyObject *wire_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Policy p;
+    long compact, access;
+    if (n != 9 || !integer(a[2], p.group) || !integer(a[3], p.topk) || !integer(a[4], p.stochastic) || !integer(a[5], p.bit) ||
+        !integer(a[6], p.quant_type) || !integer(a[7], compact) || !integer(a[8], access))
+        return elsewhere();
+    const at::Tensor *x = gpu_tensor(a[0]);
+    if (x == nullptr || x->numel() == 0 || !cuda_policy(p)) return elsewhere();
+    const int type = code_of(x->scalar_type());
+    const int64_t numel = x->numel();
+    if (type == LBC_NONE || (!plain(p) && numel % p.group != 0)) return elsewhere();
+    const int64_t nbytes = groups_of(numel, p.group) * cuda_group_bytes(p, type);
+    at::Tensor payload;
+    if (a[1] == Py_None) {
+        payload = fresh({nbytes}, at::kByte, *x);
+    } else {
+        const at::Tensor *given = payload_tensor(a[1]);
+        if (given == nullptr || given->numel() != nbytes || !with(*given, *x)) return elsewhere();
+        payload = *given;
+    }
+    uint8_t *base = static_cast<uint8_t *>(payload.data_ptr());
+    const void *data = x->data_ptr();
+    const int g = static_cast<int>(p.group), bit = static_cast<int>(p.bit), inside = compact != 0;
+    std::pair<uint64_t, uint64_t> stream_position{0, 0};
+    if (p.stochastic) stream_position = philox_inputs(*x, static_cast<uint64_t>(numel));
+    const int rc = enqueue(x->get_device(), [&](void *stream) {
+        if (plain(p)) return lbc_wire_quant_pack(data, nullptr, type, numel, g, bit, inside, base, static_cast<int>(access), stream);
+        return lbc_wire_quant_general(data, type, numel, g, bit, static_cast<int>(p.quant_type), static_cast<int>(p.topk), p.stochastic != 0,
+                                      stream_position.first, stream_position.second, inside, base, stream);
+    });
+    if (rc == LBC_OK) return THPVariable_Wrap(std::move(payload));
+    return answer(rc);
+    END_HANDLE_TH_ERRORS
+}
+
+// wire_dequantize(payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact, access) -> tensor of that
+// shape (None: flat, every element the payload holds)
+PyObject *wire_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Policy p{};
+    long dtype, op, compact, access;
+    if (n != 10 || !integer(a[2], dtype) || !integer(a[3], p.group) || !integer(a[4], p.topk) || !integer(a[5], p.bit) ||
+        !integer(a[6], op) || !integer(a[7], p.quant_type) || !integer(a[8], compact) || !integer(a[9], access))
+        return elsewhere();
+    const at::Tensor *payload = payload_tensor(a[0]);
+    if (payload == nullptr || !cuda_policy(p) || op != LBC_REDUCE_NONE || dtype < LBC_F32 || dtype > LBC_BF16) return elsewhere();
+    const int type = static_cast<int>(dtype);
+    const int64_t nbytes = payload->numel(), per_group = cuda_group_bytes(p, type), padded = nbytes / per_group * p.group;
+    c10::SmallVector<int64_t, 5> sizes;
+    int64_t numel;
+    if (nbytes % per_group != 0 || !sizes_of(a[1], padded, sizes, numel) || numel == 0 ||
+        groups_of(numel, p.group) * p.group != padded || (!plain(p) && numel % p.group != 0))
+        return elsewhere();
+    at::Tensor out = fresh(sizes, type_of(dtype), *payload);
+    const uint8_t *base = static_cast<const uint8_t *>(payload->data_ptr());
+    void *data = out.data_ptr();
+    const int g = static_cast<int>(p.group), bit = static_cast<int>(p.bit), inside = compact != 0;
+    const int rc = enqueue(payload->get_device(), [&](void *stream) {
+        if (plain(p)) return lbc_wire_dequant(base, numel, g, bit, inside, data, type, LBC_REDUCE_NONE, static_cast<int>(access), stream);
+        return lbc_wire_dequant_general(base, numel, g, bit, static_cast<int>(p.quant_type), static_cast<int>(p.topk), inside, data, type,
+                                        LBC_REDUCE_NONE, stream);
+    });
+    if (rc == LBC_OK) return THPVariable_Wrap(std::move(out));
+    return answer(rc);
+    END_HANDLE_TH_ERRORS
+}
+
+// wire_reduce(payloads, out, prepared or None, residual or None, group_size, topk, bit, quant_type, compact, divisor,
+// fused multiply-add, access) -> True: out = sum or mean, and with prepared the residual update.  What the extension's
+// fused reduce takes: group 64, plain 8-bit codes, whole groups of outputs.
+PyObject *wire_reduce(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Policy p{};
+    long compact, fma, access;
+    if (n != 12 || !integer(a[4], p.group) || !integer(a[5], p.topk) || !integer(a[6], p.bit) || !integer(a[7], p.quant_type) ||
+        !integer(a[8], compact) || !integer(a[10], fma) || !integer(a[11], access))
+        return elsewhere();
+    const double divisor = PyFloat_AsDouble(a[9]);
+    const at::Tensor *out = gpu_tensor(a[1]);
+    if (out == nullptr || !plain(p) || p.group != 64 || p.bit != 8 || !(divisor > 0.0)) return elsewhere();
+    const int type = code_of(out->scalar_type());
+    if (type == LBC_NONE || out->numel() == 0 || out->numel() % 64 != 0) return elsewhere();
+    int64_t nbytes = out->numel() / 64 * cuda_group_bytes(p, type), numel = out->numel();
+    const uint8_t *bases[LBC_MAX_PAYLOADS];
+    const at::Tensor *first = nullptr;
+    const int world = payloads_of(a[0], nbytes, bases, first);
+    if (world == 0 || !with(*first, *out) || (a[2] == Py_None) != (a[3] == Py_None)) return elsewhere();
+    const void *prepared = nullptr;
+    void *residual = nullptr;
+    if (a[2] != Py_None) {
+        const at::Tensor *before = gpu_tensor(a[2]), *after = gpu_tensor(a[3]);
+        if (before == nullptr || after == nullptr || before->scalar_type() != out->scalar_type() ||
+            after->scalar_type() != out->scalar_type() || !with(*before, *out) || !with(*after, *out) ||
+            before->numel() != after->numel() || groups_of(before->numel(), 64) * 64 != out->numel())
+            return elsewhere();
+        prepared = before->data_ptr();
+        residual = after->data_ptr();
+        numel = before->numel();
+    }
+    void *data = out->data_ptr();
+    const float inverse = 1.0f / static_cast<float>(divisor);
+    return answer(enqueue(out->get_device(), [&](void *stream) {
+        return lbc_wire_dequant_reduce(bases, world, numel, 64, compact != 0, inverse, fma != 0, data, type, prepared, residual,
+                                       static_cast<int>(access), stream);
+    }));
+    END_HANDLE_TH_ERRORS
+}
+
 // specs(objects...) -> (address, type, elements, ...) of every tensor, flattened, None as 0 and a list or tuple as its
 // tensors behind their count; None when one of them is not a contiguous GPU tensor.  What a bound launch depends on.
 bool append_spec(PyObject *o, std::vector<int64_t> &out, bool nested) {
@@ -438,6 +572,9 @@ PyMethodDef kMethods[] = {
     {"quantize", reinterpret_cast<PyCFunction>(quantize), METH_FASTCALL, "Quantize into a fresh portable payload."},
     {"dequantize", reinterpret_cast<PyCFunction>(dequantize), METH_FASTCALL, "Decode a portable payload into a fresh tensor."},
     {"dequantize_reduce", reinterpret_cast<PyCFunction>(dequantize_reduce), METH_FASTCALL, "Decode and reduce portable payloads into a fresh tensor."},
+    {"wire_quantize", reinterpret_cast<PyCFunction>(wire_quantize), METH_FASTCALL, "Quantize into a payload of the CUDA extension's format."},
+    {"wire_dequantize", reinterpret_cast<PyCFunction>(wire_dequantize), METH_FASTCALL, "Decode a payload of that format into a fresh tensor."},
+    {"wire_reduce", reinterpret_cast<PyCFunction>(wire_reduce), METH_FASTCALL, "Fused reduce of payloads of that format, optionally with the residual update."},
     {"specs", reinterpret_cast<PyCFunction>(specs), METH_FASTCALL, "Addresses, types and element counts of contiguous GPU tensors."},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -24,12 +24,10 @@ from typing import Sequence
 import torch
 
 from lowbit_comm_amd.hip import cuda_wire, ops
-from lowbit_comm_amd.hip.library import load_library
+from lowbit_comm_amd.hip.library import load_library, native_host
 from lowbit_comm_amd.hip.native_module import DType, QuantType, ReduceOP, _OP_NAME, _TORCH_OF, _check_payload
 
-FUSED_GROUP_SIZE = 64
-FUSED_BIT = 8
-
+_host = native_host()
 
 _KIND = {int(QuantType.Linear): "linear", int(QuantType.Normal): "normal", int(QuantType.Uniform): "uniform",
          int(QuantType.E3M0): "e3m0", int(QuantType.E2M1): "e2m1"}
@@ -83,6 +81,10 @@ class HipCudaWireModule:
 
     # ---- quantize ------------------------------------------------------------------------------
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
+        payload = _host.wire_quantize(input, None, group_size, topk, stochastic, bit, quant_type, compact,
+                                      ops.access_code(None))
+        if isinstance(payload, torch.Tensor):
+            return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         nbytes = cuda_wire.general_payload_nbytes(input.numel(), input.dtype, group_size, bit, topk)
         output = torch.empty(nbytes, dtype=torch.uint8, device=input.device)
@@ -90,6 +92,10 @@ class HipCudaWireModule:
         return output
 
     def inplace_quantize(self, input, output, group_size, topk, stochastic, bit, quant_type, compact) -> None:
+        if output is not None and isinstance(
+                _host.wire_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact,
+                                    ops.access_code(None)), torch.Tensor):
+            return
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         if _plain(topk, stochastic, quant_type):
             done = self._quantize(input, output, None, group_size, compact, bit)
@@ -160,7 +166,17 @@ class HipCudaWireModule:
                                          compact=bool(compact), residual=flat_residual, bit=bit)
 
     # ---- dequantize -----------------------------------------------------------------------------
+    def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
+        """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
+        all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
+        decoded = _host.wire_dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact,
+                                        ops.access_code(None))
+        return decoded if isinstance(decoded, torch.Tensor) else None
+
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
+        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
+        if decoded is not None:
+            return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
         _check_payload(input, "input")
         torch_dtype = _TORCH_OF[DType(int(dtype))]
@@ -194,39 +210,21 @@ class HipCudaWireModule:
             raise RuntimeError(f"no HIP dequantize kernel for output dtype {output.dtype}")
 
     # ---- dequantize + reduce ------------------------------------------------------------------
-    def _fused_eligible(self, inputs, output, group_size, topk, bit, quant_type) -> bool:
-        """``can_use_fused_dequant_reduce`` (dequant_reduce_kernel.cu:243-262)."""
-        if not 1 <= len(inputs) <= ops.MAX_PAYLOADS:
-            return False
-        if group_size != FUSED_GROUP_SIZE or bit != FUSED_BIT or not _plain(topk, False, quant_type):
-            return False
-        if not isinstance(output, torch.Tensor) or not output.is_cuda or not output.is_contiguous():
-            return False
-        if output.dtype not in ops.DTYPE_CODES or output.numel() == 0 or output.numel() % FUSED_GROUP_SIZE != 0:
-            return False
-        expected = cuda_wire.payload_nbytes(output.numel(), output.dtype, group_size)
-        for buffer in inputs:
-            if not isinstance(buffer, torch.Tensor) or buffer.dtype != torch.uint8 or not buffer.is_cuda:
-                return False
-            if not buffer.is_contiguous() or buffer.device != output.device or buffer.numel() != expected:
-                return False
-        return True
-
-    def _fused(self, inputs, output, compact, inv_divisor, prepared=None, residual=None) -> bool:
-        numel = output.numel() if prepared is None else prepared.numel()
-        return cuda_wire.dequant_reduce_into(
-            [buffer.reshape(-1) for buffer in inputs], output.reshape(-1), numel=numel,
-            group_size=FUSED_GROUP_SIZE, compact=bool(compact), inv_divisor=inv_divisor,
-            fused_multiply_add=self.fused_multiply_add,
-            prepared=None if prepared is None else prepared.reshape(-1),
-            new_residual=None if residual is None else residual.reshape(-1))
+    def _fused(self, inputs, output, group_size, topk, bit, quant_type, compact, divisor, prepared=None,
+               residual=None) -> bool:
+        """The fused reduce where ``can_use_fused_dequant_reduce`` (dequant_reduce_kernel.cu:243-262) allows it: at most
+        8 payloads of the output's size, group 64, plain 8-bit codes, whole groups of outputs.  The divisor becomes its
+        fp32 reciprocal, as in the reference."""
+        inputs = inputs if isinstance(inputs, (list, tuple)) else list(inputs)
+        done = _host.wire_reduce(inputs, output, prepared, residual, group_size, topk, bit, quant_type, compact, divisor,
+                                 self.fused_multiply_add, ops.access_code(None))
+        return bool(done)
 
     def inplace_dequantize_reduce(self, inputs: Sequence[torch.Tensor], output, group_size, topk, bit, quant_type,
                                   compact) -> None:
         if len(inputs) == 0:
             raise RuntimeError("inputs must not be empty")
-        if self._fused_eligible(inputs, output, group_size, topk, bit, quant_type) and \
-                self._fused(inputs, output, compact, 1.0):
+        if self._fused(inputs, output, group_size, topk, bit, quant_type, compact, 1.0):
             return
         for i, buffer in enumerate(inputs):                      # pybind.cpp:44-55
             self.inplace_dequantize(buffer, output, group_size, topk, bit,
@@ -246,10 +244,7 @@ class HipCudaWireModule:
                                        divisor) -> bool:
         if divisor <= 0:
             raise RuntimeError("divisor must be > 0")
-        if not self._fused_eligible(inputs, output, group_size, topk, bit, quant_type):
-            return False
-        inv = float(torch.tensor(1.0, dtype=torch.float32) / torch.tensor(float(divisor), dtype=torch.float32))
-        return self._fused(inputs, output, compact, inv)
+        return self._fused(inputs, output, group_size, topk, bit, quant_type, compact, divisor)
 
     # ---- error feedback -------------------------------------------------------------------------
     def inplace_error_feedback_update(self, prepared, restored, residual) -> None:
@@ -288,12 +283,9 @@ class HipCudaWireModule:
             raise RuntimeError("prepared and residual must have the same dtype")
         if prepared.device != restored.device or prepared.device != residual.device:
             raise RuntimeError("prepared, restored and residual must be on the same device")
-        if not self._fused_eligible(inputs, restored, group_size, topk, bit, quant_type):
-            return False                                        # eligibility is judged on `restored` (:381)
-        if -(-prepared.numel() // FUSED_GROUP_SIZE) * FUSED_GROUP_SIZE != restored.numel():
-            return False           # the kernel derives the group count from prepared.numel() (:387, :170)
-        inv = float(torch.tensor(1.0, dtype=torch.float32) / torch.tensor(float(divisor), dtype=torch.float32))
-        return self._fused(inputs, restored, compact, inv, prepared, residual)
+        # eligibility is judged on `restored` (:381), and the kernel derives the group count from prepared.numel()
+        # (:387, :170): it has to be restored's
+        return self._fused(inputs, restored, group_size, topk, bit, quant_type, compact, divisor, prepared, residual)
 
     def dequantize_reduce_update_error_feedback(self, inputs, prepared, residual, group_size, topk, bit, quant_type,
                                                 dtype, compact, divisor):

@@ -204,14 +204,14 @@ class HipNativeModule:
         return (bind() if key is None else self._memoized(key, bind))()
 
     # ---- dequantize -----------------------------------------------------------------------------
-    def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype):
+    def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
         """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
         all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
         decoded = _host.dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype)
+        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
         if decoded is not None:
             return decoded
         _require_policy(group_size, topk, False, bit, quant_type)

@@ -211,7 +211,8 @@ def dequantize_tensor(buffer: object, shape: tuple[int, ...], config: Compressio
     if output is None:
         shaped = getattr(module, "_dequantize_shaped", None)
         if shaped is not None:          # a module that decodes straight into the shape: nothing to trim afterwards
-            decoded = shaped(buffer, shape, config.group_size, config.topk, config.bit, op, quant_type, dtype_member)
+            decoded = shaped(buffer, shape, config.group_size, config.topk, config.bit, op, quant_type, dtype_member,
+                             config.compact)
             if decoded is not None:
                 return decoded
         decoded = _symbol(module, "dequantize")(buffer, config.group_size, config.topk, config.bit, op, quant_type,
