@@ -19,6 +19,8 @@
 // issued before the arithmetic.  Group strides of 66 or 68 bytes leave code words only 2- or
 // 4-byte aligned; gfx950 global memory instructions accept that, so all accesses here are typed
 // with element alignment only and there is no separate path for unaligned tensors.
+#include <type_traits>
+
 #include "device_utils.h"
 #include "launch.h"
 #include "wire_common.h"
@@ -36,13 +38,13 @@ namespace {
 // ---------------------------------------------------------------------------
 // quantize + pack (optionally x + residual), `world` chunks via blockIdx.y
 // ---------------------------------------------------------------------------
-template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int NT>
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int NT, int TILES>
 __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs a) {
     constexpr int PNT = COMPACT ? kPlain : NT;
     using W = wire<T, BIT>;
     constexpr int VEC = W::VEC;
     constexpr int LPG = G / VEC;
-    constexpr int UNROLL = 4;
+    constexpr int UNROLL = TILES;
     constexpr int BLOCK_ELEMS = W::TILE * kWavesPerBlock * UNROLL;
     static_assert(LPG >= 1 && LPG <= 16, "a group must fit one DPP row");
 
@@ -89,15 +91,24 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
         for (int i = 0; i < VEC; ++i) c[i] = c[i] < -L ? -L : (c[i] > L ? L : c[i]);
     };
 
-    if (block_first + BLOCK_ELEMS <= valid) {
+    // One pass over the block's tiles, every load issued before the first use.  WHOLE: all of the block's elements are
+    // live; otherwise a lane's vector is cut short where the chunk ends, and what lies behind counts as zeros
+    // (walked element by element, the last block bounded every small tensor: 10,048 bf16 elements 2.5 us, now 2.0 us).
+    auto tiles = [&](auto whole) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole)::value;
         T xv[UNROLL][VEC];
         T rv[UNROLL][VEC];
         int64_t e0[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             e0[u] = block_first + static_cast<int64_t>(tile_in_block<UNROLL>(u, wave)) * W::TILE + lane * VEC;
-            load_elems<T, VEC, NT>(x + e0[u], xv[u]);
-            if constexpr (HAS_R) load_elems<T, VEC, NT>(r + e0[u], rv[u]);
+            if constexpr (WHOLE) {
+                load_elems<T, VEC, NT>(x + e0[u], xv[u]);
+                if constexpr (HAS_R) load_elems<T, VEC, NT>(r + e0[u], rv[u]);
+            } else {
+                load_live<T, VEC, NT == kNonTemporal>(x + e0[u], valid - e0[u], xv[u]);
+                if constexpr (HAS_R) load_live<T, VEC, NT == kNonTemporal>(r + e0[u], valid - e0[u], rv[u]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -105,16 +116,19 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
             uint32_t m = 0;   // largest magnitude pattern; above the pattern of infinity when the lane holds a NaN
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
-                float v = widen(xv[u][i]);
-                if constexpr (HAS_R) v = round_through<T>(v + widen(rv[u][i]));
-                p[i] = v;
-                const uint32_t bits = as_u32(v) & 0x7FFFFFFFu;
+                p[i] = widen(xv[u][i]);
+                if constexpr (HAS_R) p[i] += widen(rv[u][i]);
+            }
+            if constexpr (HAS_R) round_through_all<T, VEC>(p);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                const uint32_t bits = as_u32(p[i]) & 0x7FFFFFFFu;
                 m = bits > m ? bits : m;
             }
             const int64_t group = e0[u] / G;
             const int k0 = static_cast<int>(e0[u] - group * G);
             float absmax;
-            float multiplier = group_multiplier(m, absmax);
+            float multiplier = group_multiplier(m, absmax);   // every lane of the row takes part
             Raw stored = __builtin_bit_cast(Raw, narrow<T>(absmax));
             bool wide_codes = false;   // wavefront-uniform: codes may leave [-LEVELS, LEVELS]
             if (__ballot(m > 0x7F800000u) != 0) {   // a NaN somewhere in the wavefront: rare, and uniform
@@ -140,6 +154,7 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
             if (wide_codes) clamp_codes(c);
             uint32_t words[W::WORDS];
             pack_codes<T, BIT, VEC, W::WORDS>(c, words);
+            if (!WHOLE && e0[u] >= padded) continue;   // a lane's elements lie inside the padded range together
             // Interleaved 16-bit payloads leave as misaligned 8-byte stores here.  Re-slicing a pair of 66-byte groups
             // into aligned dwords across lanes (store_group_pair16, what the ring's gather hop does) measured slower in
             // this kernel at every size, with operands rotated through 700 MB: 26.2 M bf16 elements 15.8 us as it is,
@@ -150,71 +165,41 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
             store_piece<T, BIT, PNT, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words);
             if ((lane & (LPG - 1)) == 0) *reinterpret_cast<Raw *>(payload + at.scale(group)) = stored;
         }
-        return;
-    }
-
-    // ---- edge block: ragged tail and zero padding, element-wise ----------------
-    for (int u = 0; u < UNROLL; ++u) {
-        const int64_t e0 = block_first + static_cast<int64_t>(tile_in_block<UNROLL>(u, wave)) * W::TILE + lane * VEC;
-        if (e0 - lane * VEC >= padded) break;  // wavefront-uniform
-        float p[VEC];
-        T held[VEC];
-        uint32_t m = 0;
-        bool has_nan = false;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-            const int64_t e = e0 + i;
-            float v = 0.0f;
-            held[i] = narrow<T>(0.0f);
-            if (e < valid) {
-                held[i] = x[e];
-                v = widen(x[e]);
-                if constexpr (HAS_R) v = round_through<T>(v + widen(r[e]));
-            }
-            p[i] = v;
-            uint32_t bits = as_u32(v) & 0x7FFFFFFFu;
-            has_nan |= bits > 0x7F800000u;
-            bits = bits > 0x7F800000u ? 0u : bits;
-            m = bits > m ? bits : m;
-        }
-        const int64_t group = e0 / G;
-        const int k0 = static_cast<int>(e0 - group * G);
-        float absmax;
-        float multiplier = group_multiplier(m, absmax);   // every lane of the row takes part
-        Raw stored = __builtin_bit_cast(Raw, narrow<T>(absmax));
-        bool wide_codes = false;
-        if constexpr (!HAS_R) {
-            if (resets && __ballot(has_nan) != 0) {
-                const uint32_t scale_raw = scan_scale(held, group, k0);
-                multiplier = multiplier_of(value_of<T>(scale_raw));
-                stored = static_cast<Raw>(scale_raw);
-                wide_codes = true;
-            }
-        }
-        if (e0 < padded) {   // the lane's VEC elements lie inside the padded range together: whole words again
-            int c[VEC];
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) c[i] = cvt_i32(__builtin_rintf(p[i] * multiplier));
-            if (wide_codes) clamp_codes(c);
-            uint32_t words[W::WORDS];
-            pack_codes<T, BIT, VEC, W::WORDS>(c, words);
-            store_piece<T, BIT, kPlain, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words);
-            if ((lane & (LPG - 1)) == 0) *reinterpret_cast<Raw *>(payload + at.scale(group)) = stored;
-        }
-    }
+    };
+    if (block_first + BLOCK_ELEMS <= valid) tiles(std::true_type{});
+    else tiles(std::false_type{});
 }
 
-template <typename T, int G, int BIT, bool HAS_R, bool COMPACT>
-hipError_t launch_wire_quant_c(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
-    constexpr int BLOCK_ELEMS = wire<T, BIT>::TILE * kWavesPerBlock * 4;
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int TILES>
+hipError_t launch_wire_quant_tiles(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
+    constexpr int BLOCK_ELEMS = wire<T, BIT>::TILE * kWavesPerBlock * TILES;
     const int64_t groups = (a.shard_numel + G - 1) / G;
     const int64_t blocks = (groups * G + BLOCK_ELEMS - 1) / BLOCK_ELEMS;
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    if (mode == kStream) hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kNonTemporal>), grid, dim3(kBlock), 0, stream, a);
-    else hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kPlain>), grid, dim3(kBlock), 0, stream, a);
+    if (mode == kStream) hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kNonTemporal, TILES>), grid, dim3(kBlock), 0, stream, a);
+    else hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kPlain, TILES>), grid, dim3(kBlock), 0, stream, a);
     return hipGetLastError();
+}
+
+// Tiles in flight per wavefront: one while they fit the chip's wavefront slots (us with one / four tiles: 10,048 fp32
+// elements 1.9 / 2.6, 1 Mi 2.9 / 3.2, 2 Mi 3.5 / 4.0; bf16 10,048 2.0 / 2.5, 1 Mi 2.6 / 3.1, 4 Mi 3.7 / 4.4).  Beyond, two
+// where a residual is read as well (13.1 M fp32 19.9 us, 20.7 with four; bf16 12.6 / 13.1), and without one four - for a
+// 16-bit tensor two until there are twice the slots (6.6 M bf16 5.3 us with two, 6.0 with four; 13.1 M 9.3 / 9.1; fp32
+// 6.6 M 7.8 / 7.6, 26.2 M 23.3 / 22.1).
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT>
+hipError_t launch_wire_quant_c(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
+    constexpr int64_t kOneEach = kResidentWaves * wire<T, BIT>::TILE;
+    if (a.numel <= kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 1>(mode, a, world, stream);
+    if constexpr (HAS_R) {
+        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 2>(mode, a, world, stream);
+    } else {
+        if constexpr (sizeof(T) == 2) {
+            if (a.numel <= 2 * kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 2>(mode, a, world, stream);
+        }
+        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 4>(mode, a, world, stream);
+    }
 }
 
 template <typename T, int G, int BIT>
@@ -268,9 +253,16 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
         else return acc + code * step;
     };
 
-    if (block_first + BLOCK_ELEMS <= a.numel) {
+    // One pass over the block's tiles, every load issued before the arithmetic.  WHOLE: all of the block's outputs exist;
+    // otherwise a lane's vector is cut short at the end (the payload holds whole groups, so a lane with one live output
+    // may read all of its codes).  Element by element the last block was the longest chain of a
+    // mid-sized launch: 10,048 outputs of eight payloads, interleaved bf16 4.2 us then, 2.4 now, fp32 with error feedback
+    // 3.7 and 2.2, 2 Mi of two bf16 payloads with error feedback 5.1 and 4.9; decode of 10,048 2.9 and 1.9.
+    auto tiles = [&](auto whole) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole)::value;
         uint32_t words[UNROLL][WORLD][W::WORDS];
         T stored[UNROLL][WORLD];
+        T pv[UNROLL][VEC];
         int64_t e0[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -279,25 +271,31 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
             const int k0 = static_cast<int>(e0[u] - group * G);
             const int64_t code_at = at.codes(group) + k0;
             const int64_t scale_at = at.scale(group);
-            if constexpr (WINDOWS) {   // 16-bit compact payloads below 2 GiB: aligned windows, scales out of them
+            if constexpr (WINDOWS) {   // 16-bit compact payloads below 2 GiB: aligned windows, scales out of them;
                 static_assert(COMPACT && sizeof(T) == 2 && G == 64 && W::WORDS == 2, "66-byte groups of 8 lanes");
-                const uint32_t payload_bytes = static_cast<uint32_t>(groups * (G + 2));
+                const uint32_t payload_bytes = static_cast<uint32_t>(groups * (G + 2));   // past the payload: zeros
 #pragma unroll
                 for (int r = 0; r < WORLD; ++r) {
                     const uint32_t lead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(a.payloads[r]) & 3u);
                     uint32_t after;
                     load_piece16<window_policy<NT, WORLD>()>(buffer_over(a.payloads[r] - lead, window_span(payload_bytes + lead)),
-                                          static_cast<uint32_t>(code_at) + lead, words[u][r], after);
+                                          static_cast<uint32_t>(WHOLE || e0[u] < groups * G ? code_at : 0) + lead, words[u][r], after);
                     const uint32_t raw = from_last_lane_of_8(after, (lane & 8) != 0);
                     stored[u][r] = __builtin_bit_cast(T, static_cast<uint16_t>(raw));
                 }
             } else {
 #pragma unroll
                 for (int r = 0; r < WORLD; ++r) {
-                    load_words<W::WORDS, sizeof(T), PNT>(a.payloads[r] + code_at, words[u][r]);
-                    stored[u][r] = *reinterpret_cast<const T *>(a.payloads[r] + scale_at);
+#pragma unroll
+                    for (int k = 0; k < W::WORDS; ++k) words[u][r][k] = 0;
+                    stored[u][r] = narrow<T>(0.0f);
+                    if (WHOLE || e0[u] < a.numel) {
+                        load_words<W::WORDS, sizeof(T), PNT>(a.payloads[r] + code_at, words[u][r]);
+                        stored[u][r] = *reinterpret_cast<const T *>(a.payloads[r] + scale_at);
+                    }
                 }
             }
+            if (!WHOLE && new_r != nullptr) load_live<T, VEC, NT == kNonTemporal>(prepared + e0[u], a.numel - e0[u], pv[u]);
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -313,41 +311,24 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
             }
             T o[VEC];
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-                acc[i] = acc[i] * a.inv_divisor;
-                o[i] = narrow<T>(acc[i]);
-            }
-            store_elems<T, VEC, NT>(out + e0[u], o);
+            for (int i = 0; i < VEC; ++i) acc[i] = acc[i] * a.inv_divisor;
+            narrow_all<T, VEC>(acc, o);
+            if constexpr (WHOLE) store_elems<T, VEC, NT>(out + e0[u], o);
+            else store_live<T, VEC, NT == kNonTemporal>(out + e0[u], a.numel - e0[u], o);
             if (new_r != nullptr) {
-                T pv[VEC], d[VEC];
-                load_elems<T, VEC, NT>(prepared + e0[u], pv);
+                T d[VEC];
+                float left[VEC];
+                if constexpr (WHOLE) load_elems<T, VEC, NT>(prepared + e0[u], pv[u]);
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) d[i] = narrow<T>(widen(pv[i]) - acc[i]);
-                store_elems<T, VEC, NT>(new_r + e0[u], d);
+                for (int i = 0; i < VEC; ++i) left[i] = widen(pv[u][i]) - acc[i];
+                narrow_all<T, VEC>(left, d);
+                if constexpr (WHOLE) store_elems<T, VEC, NT>(new_r + e0[u], d);
+                else store_live<T, VEC, NT == kNonTemporal>(new_r + e0[u], a.numel - e0[u], d);
             }
         }
-        return;
-    }
-
-    for (int u = 0; u < UNROLL; ++u) {
-        const int64_t e0 = block_first + static_cast<int64_t>(tile_in_block<UNROLL>(u, wave)) * W::TILE + lane * VEC;
-        for (int i = 0; i < VEC; ++i) {
-            const int64_t e = e0 + i;
-            if (e >= a.numel) break;
-            const int64_t group = e / G;
-            const int k = static_cast<int>(e - group * G);
-            float acc = 0.0f;
-#pragma unroll
-            for (int r = 0; r < WORLD; ++r) {
-                const float step = div127(widen(*reinterpret_cast<const T *>(a.payloads[r] + at.scale(group))));
-                const float code = static_cast<float>(static_cast<int8_t>(a.payloads[r][at.codes(group) + byte_in_group<T>(k)]));
-                acc = accumulate(acc, code, step);
-            }
-            acc = acc * a.inv_divisor;
-            out[e] = narrow<T>(acc);
-            if (new_r != nullptr) new_r[e] = narrow<T>(widen(prepared[e]) - acc);
-        }
-    }
+    };
+    if (block_first + BLOCK_ELEMS <= a.numel) tiles(std::true_type{});
+    else tiles(std::false_type{});
 }
 
 template <typename T, int G, int WORLD, bool FMA, bool COMPACT>
@@ -427,47 +408,45 @@ __global__ __launch_bounds__(kBlock) void wire_decode_kernel(const WireDecodeArg
     const int64_t block_first = static_cast<int64_t>(xcd_contiguous_block(BLOCK_ELEMS)) * BLOCK_ELEMS;
     if (block_first >= valid) return;
 
-    if (block_first + BLOCK_ELEMS <= valid) {
+    auto tiles = [&](auto whole) __attribute__((always_inline)) {   // WHOLE as in the reduce
+        constexpr bool WHOLE = decltype(whole)::value;
         uint32_t words[UNROLL][W::WORDS];
         T stored[UNROLL];
+        T o[UNROLL][VEC];
         int64_t e0[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             e0[u] = block_first + static_cast<int64_t>(tile_in_block<UNROLL>(u, wave)) * W::TILE + lane * VEC;
             const int64_t group = e0[u] / G;
             const int k0 = static_cast<int>(e0[u] - group * G);
-            load_piece<T, BIT, PNT, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words[u]);
-            stored[u] = *reinterpret_cast<const T *>(payload + at.scale(group));
+#pragma unroll
+            for (int k = 0; k < W::WORDS; ++k) words[u][k] = 0;
+            stored[u] = narrow<T>(0.0f);
+            if (WHOLE || e0[u] < valid) {
+                load_piece<T, BIT, PNT, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words[u]);
+                stored[u] = *reinterpret_cast<const T *>(payload + at.scale(group));
+            }
+            if constexpr (OP != 0 && !WHOLE) load_live<T, VEC, NT == kNonTemporal>(out + e0[u], valid - e0[u], o[u]);
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            T o[VEC];
-            if constexpr (OP != 0) load_elems<T, VEC, NT>(out + e0[u], o);
+            if constexpr (OP != 0 && WHOLE) load_elems<T, VEC, NT>(out + e0[u], o[u]);
             const float step = step_of<BIT>(widen(stored[u]));
+            float v[VEC];
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-                float v = round_through<T>(unpack_code<T, BIT, W::WORDS>(words[u], i) * step);
-                if constexpr (OP != 0) v = combine_in<T, OP>(widen(o[i]), v);
-                o[i] = narrow<T>(v);
+            for (int i = 0; i < VEC; ++i) v[i] = unpack_code<T, BIT, W::WORDS>(words[u], i) * step;
+            if constexpr (OP != 0) {
+                round_through_all<T, VEC>(v);
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) v[i] = combine_in<T, OP>(widen(o[u][i]), v[i]);
             }
-            store_elems<T, VEC, NT>(out + e0[u], o);
+            narrow_all<T, VEC>(v, o[u]);
+            if constexpr (WHOLE) store_elems<T, VEC, NT>(out + e0[u], o[u]);
+            else store_live<T, VEC, NT == kNonTemporal>(out + e0[u], valid - e0[u], o[u]);
         }
-        return;
-    }
-
-    for (int u = 0; u < UNROLL; ++u) {
-        const int64_t e0 = block_first + static_cast<int64_t>(tile_in_block<UNROLL>(u, wave)) * W::TILE + lane * VEC;
-        for (int i = 0; i < VEC; ++i) {
-            const int64_t e = e0 + i;
-            if (e >= valid) break;
-            const int64_t group = e / G;
-            const int k = static_cast<int>(e - group * G);
-            const float step = step_of<BIT>(widen(*reinterpret_cast<const T *>(payload + at.scale(group))));
-            float v = round_through<T>(code_at<T, BIT>(payload + at.codes(group), k) * step);
-            if constexpr (OP != 0) v = combine_in<T, OP>(widen(out[e]), v);
-            out[e] = narrow<T>(v);
-        }
-    }
+    };
+    if (block_first + BLOCK_ELEMS <= valid) tiles(std::true_type{});
+    else tiles(std::false_type{});
 }
 
 template <typename T, int G, int BIT, int OP, bool COMPACT>

@@ -134,12 +134,6 @@ template <typename T, int BIT = 8> struct wire {
 template <typename T> __device__ __forceinline__ constexpr int byte_in_word(int k) {
     return sizeof(T) == 4 ? 3 - k : (k ^ 1);
 }
-// Byte position of element k of a group inside the group's code bytes.
-template <typename T> __device__ __forceinline__ int byte_in_group(int k) {
-    constexpr int ITEM = sizeof(T);
-    return (k / ITEM) * ITEM + (ITEM - 1 - k % ITEM);
-}
-
 // COMPACT payloads interleave [G code bytes][scale] per group, so a 128-byte line is shared by
 // neighbouring wavefront instructions and payload accesses must stay cacheable even when the tensors
 // stream with the non-temporal hint (the hint would drop the line between its two uses).  Otherwise
@@ -204,19 +198,6 @@ __device__ __forceinline__ float unpack_code(const uint32_t (&words)[WORDS], int
     } else {
         const int top = 16 - 16 * (i / 4) + 4 * (i % 4);   // left shift that puts the nibble on top
         return static_cast<float>(static_cast<int32_t>(words[0] << top) >> 28);
-    }
-}
-
-// Code of element k of a group read from the group's code bytes (ragged-edge path).
-template <typename T, int BIT> __device__ __forceinline__ float code_at(const uint8_t *group_codes, int k) {
-    if constexpr (BIT == 8) {
-        return static_cast<float>(static_cast<int8_t>(group_codes[byte_in_group<T>(k)]));
-    } else {
-        constexpr int ITEM = sizeof(T), PER_WORD = 2 * ITEM;
-        const int in_word = k % PER_WORD;
-        const uint32_t byte = group_codes[(k / PER_WORD) * ITEM + (ITEM - 1 - in_word / 2)];
-        const uint32_t nibble = (in_word & 1) ? (byte & 0xFu) : (byte >> 4);
-        return static_cast<float>(static_cast<int32_t>(nibble << 28) >> 28);
     }
 }
 

@@ -158,3 +158,57 @@ def test_ring_step_and_feedback_update_at_block_ends_and_start_offsets(hip_devic
     assert ops.ef_update_into(Guarded(n, t, offset, hip_device, prepared).inside,
                               Guarded(n, t, offset, hip_device, restored).inside, residual.inside)
     residual.check((prepared.float() - restored.float()).to(t), "feedback update")
+
+
+# The CUDA byte format: a workgroup spans 1024 elements (fp32) or 2048 (16-bit) of a tensor that the chip holds at once,
+# the reduce of up to two payloads and the decode twice that; a group's scale sits with its last lane
+@pytest.mark.parametrize("n", [1, 60, 67, 131, 1023, 1025, 2047, 2049 + 64, 4095, 4097, 8192 + 3])
+@pytest.mark.parametrize("compact", [True, False])
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_cuda_byte_format_at_block_ends(hip_device, dtype, compact, n):
+    from lowbit_comm_amd.hip import cuda_wire
+    from oracle import cuda_wire_np as wire
+    from tests.test_cuda_wire_parity import from_numpy, to_numpy
+
+    t = DTYPES[dtype]
+    xs = [values(n, t, 10 * n + r) for r in range(3)]
+    r = values(n, t, n + 7, 1e-5)
+    payloads = []
+    for x in xs:
+        out = Guarded(cuda_wire.payload_nbytes(n, t), torch.uint8, 4, hip_device)
+        assert cuda_wire.quant_pack_into(x.to(hip_device), out.inside, compact=compact)
+        out.check(torch.from_numpy(wire.quantize(to_numpy(x), dtype, 64, compact)), "payload")
+        payloads.append(out.inside.clone())
+    out = Guarded(cuda_wire.payload_nbytes(n, t), torch.uint8, 4, hip_device)
+    assert cuda_wire.quant_pack_into(xs[0].to(hip_device), out.inside, compact=compact, residual=r.to(hip_device))
+    out.check(torch.from_numpy(wire.quantize(to_numpy(xs[0]), dtype, 64, compact, residual=to_numpy(r))), "payload with residual")
+    host = [to_numpy(p) for p in payloads]
+    old = values(n, t, n + 1)
+    for op in ("none", "sum"):
+        decoded = Guarded(n, t, 1, hip_device, old)
+        assert cuda_wire.dequant_into(payloads[0], decoded.inside, compact=compact, reduce_op=op)
+        decoded.check(from_numpy(wire.dequantize(host[0], n, dtype, 64, compact, op, to_numpy(old)), dtype, "cpu"), f"decode {op}")
+    for world in (1, 2, 3):
+        p = values(n, t, n + 2)
+        reduced, fresh = Guarded(n, t, 1, hip_device), Guarded(n, t, 1, hip_device)
+        assert cuda_wire.dequant_reduce_into(payloads[:world], reduced.inside, compact=compact, inv_divisor=1.0 / world,
+                                             prepared=Guarded(n, t, 1, hip_device, p).inside, new_residual=fresh.inside)
+        want, left = wire.reduce_mean_error_feedback(host[:world], to_numpy(p), n, dtype, divisor=world, compact=compact)
+        reduced.check(from_numpy(want, dtype, "cpu"), f"reduce of {world}")
+        fresh.check(from_numpy(left, dtype, "cpu"), f"residual of {world}")
+
+
+# the tile count changes with the chip's wavefront slots: 2 Mi fp32 elements, 4 Mi and 8 Mi 16-bit ones
+@pytest.mark.parametrize("dtype, with_residual, n", [("fp32", False, (1 << 21) + 5), ("fp32", True, (1 << 21) + 64),
+                                                     ("bf16", False, (1 << 22) + 5), ("bf16", False, (1 << 23) + 64),
+                                                     ("bf16", True, (1 << 22) + 64)])
+def test_cuda_byte_format_beyond_the_tile_rule(hip_device, dtype, with_residual, n):
+    from lowbit_comm_amd.hip import cuda_wire
+    from oracle import cuda_wire_np as wire
+    from tests.test_cuda_wire_parity import to_numpy
+
+    t = DTYPES[dtype]
+    x, r = values(n, t, n), values(n, t, n + 7, 1e-5) if with_residual else None
+    out = Guarded(cuda_wire.payload_nbytes(n, t), torch.uint8, 4, hip_device)
+    assert cuda_wire.quant_pack_into(x.to(hip_device), out.inside, residual=None if r is None else r.to(hip_device))
+    out.check(torch.from_numpy(wire.quantize(to_numpy(x), dtype, 64, True, residual=None if r is None else to_numpy(r))), "payload")
