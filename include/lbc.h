@@ -329,6 +329,15 @@ int64_t lbc_wire_payload_nbytes(int64_t numel, int group_size, int dtype, int bi
 int lbc_wire_quant_pack(const void *x, const void *residual, int dtype, int64_t numel, int group_size,
                         int bit, int compact, uint8_t *payload, int access, void *stream);
 
+/*
+ * The compensate step and the quantize of its result in one pass: prepared = x + residual (added in fp32 and
+ * rounded to dtype; numel elements that overlap neither), and the payload lbc_wire_quant_pack writes for `prepared`
+ * zero padded to whole groups, without a residual - NaN elements included.  Stands for
+ * ccdl_comm/communication/ddp_hook.py:196 followed by the quantize call of that hook.
+ */
+int lbc_wire_compensate_quant_pack(const void *x, const void *residual, void *prepared, int dtype, int64_t numel,
+                                   int group_size, int bit, int compact, uint8_t *payload, int access, void *stream);
+
 /* As lbc_quant_pack_chunks, in this format: chunk d of ceil(numel/world) elements becomes the
  * payload at payloads + d*payload_stride (ccdl_comm/cuda/transports/compressed_reduce_scatter.py:72-94). */
 int lbc_wire_quant_pack_chunks(const void *x, const void *residual, int dtype, int64_t numel, int world,

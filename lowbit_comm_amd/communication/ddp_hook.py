@@ -29,6 +29,7 @@ from lowbit_comm_amd.exceptions import UnsupportedCollective
 from lowbit_comm_amd.quantization.codec import (
     allocate_dequantized_buffer,
     allocate_quantized_buffer,
+    compensate_and_quantize as compensate_and_quantize_in_one_launch,
     dequantize_reduce_tensors,
     dequantize_reduce_update_error_feedback,
     dequantize_tensor,
@@ -263,6 +264,16 @@ def create_ddp_comm_hook(
             return None
         return prepared, buffer
 
+    # The CUDA extension's format has the same fusion with both outputs freshly allocated, as the sum and the payload of
+    # the two separate calls are.  A feedback state with a compensate step of its own keeps that step.
+    plain_compensate = quantize is None and getattr(type(feedback), "compensate", None) is ErrorFeedbackState.compensate
+
+    def fresh_sum_and_payload(key: Any, original: Any) -> tuple[Any, Any] | None:
+        residual = feedback.get(key) if plain_compensate else None
+        if residual is None:
+            return None
+        return compensate_and_quantize_in_one_launch(original, residual, config, extension_status=extension_status)
+
     def small(tensor: Any) -> bool:
         return min_compress_numel > 0 and _numel(tensor) < min_compress_numel
 
@@ -362,7 +373,9 @@ def create_ddp_comm_hook(
                 return uncompressed(clone(original), reduce)
             decision = policy.decide(key, numel=_numel(original))
             facade = dequantize is None and reduce in ("mean", "sum")
-            fused = compensate_and_quantize(key, original) if decision.apply and facade and fuse_compensate else None
+            fused = None
+            if decision.apply and facade:
+                fused = compensate_and_quantize(key, original) if fuse_compensate else fresh_sum_and_payload(key, original)
             if fused is not None:
                 prepared = fused[0]
             else:

@@ -123,6 +123,7 @@ constexpr Entry kEntries[] = {
     {"lbc_ring_step", make_call<&lbc_ring_step>},
     {"lbc_ef_update", make_call<&lbc_ef_update>},
     {"lbc_wire_quant_pack", make_call<&lbc_wire_quant_pack>},
+    {"lbc_wire_compensate_quant_pack", make_call<&lbc_wire_compensate_quant_pack>},
     {"lbc_wire_quant_pack_chunks", make_call<&lbc_wire_quant_pack_chunks>},
     {"lbc_wire_dequant", make_call<&lbc_wire_dequant>},
     {"lbc_wire_dequant_chunks", make_call<&lbc_wire_dequant_chunks>},
@@ -449,6 +450,41 @@ PyObject *wire_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// wire_compensate_quantize(x, residual, group_size, topk, stochastic, bit, quant_type, compact, access) -> (x + residual, its
+// payload), both from one launch.  Plain codes; operands of one type, one shape and one device that autograd does not watch.
+PyObject *wire_compensate_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Policy p;
+    long compact, access;
+    if (n != 9 || !integer(a[2], p.group) || !integer(a[3], p.topk) || !integer(a[4], p.stochastic) || !integer(a[5], p.bit) ||
+        !integer(a[6], p.quant_type) || !integer(a[7], compact) || !integer(a[8], access))
+        return elsewhere();
+    if (!THPVariable_CheckExact(a[0]) || !THPVariable_CheckExact(a[1])) return elsewhere();
+    const at::Tensor *x = gpu_tensor(a[0]), *r = gpu_tensor(a[1]);
+    if (x == nullptr || r == nullptr || x->numel() == 0 || !cuda_policy(p) || !plain(p)) return elsewhere();
+    const int type = code_of(x->scalar_type());
+    if (type == LBC_NONE || r->scalar_type() != x->scalar_type() || !x->sizes().equals(r->sizes()) || !with(*r, *x) ||
+        x->requires_grad() || r->requires_grad())
+        return elsewhere();
+    const int64_t numel = x->numel();
+    at::Tensor prepared = fresh(x->sizes(), x->scalar_type(), *x);
+    at::Tensor payload = fresh({groups_of(numel, p.group) * cuda_group_bytes(p, type)}, at::kByte, *x);
+    const void *data = x->data_ptr(), *residual = r->data_ptr();
+    void *sum = prepared.data_ptr();
+    uint8_t *base = static_cast<uint8_t *>(payload.data_ptr());
+    const int rc = enqueue(x->get_device(), [&](void *stream) {
+        return lbc_wire_compensate_quant_pack(data, residual, sum, type, numel, static_cast<int>(p.group), static_cast<int>(p.bit),
+                                              compact != 0, base, static_cast<int>(access), stream);
+    });
+    if (rc != LBC_OK) return answer(rc);
+    PyObject *pair = PyTuple_New(2);
+    if (pair == nullptr) return nullptr;
+    PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(std::move(prepared)));
+    PyTuple_SET_ITEM(pair, 1, THPVariable_Wrap(std::move(payload)));
+    return pair;
+    END_HANDLE_TH_ERRORS
+}
+
 // wire_dequantize(payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact, access) -> tensor of that
 // shape (None: flat, every element the payload holds)
 PyObject *wire_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
@@ -572,6 +608,7 @@ PyMethodDef kMethods[] = {
     {"quantize", reinterpret_cast<PyCFunction>(quantize), METH_FASTCALL, "Quantize into a fresh portable payload."},
     {"dequantize", reinterpret_cast<PyCFunction>(dequantize), METH_FASTCALL, "Decode a portable payload into a fresh tensor."},
     {"dequantize_reduce", reinterpret_cast<PyCFunction>(dequantize_reduce), METH_FASTCALL, "Decode and reduce portable payloads into a fresh tensor."},
+    {"wire_compensate_quantize", reinterpret_cast<PyCFunction>(wire_compensate_quantize), METH_FASTCALL, "x + residual and its payload in the CUDA extension's format."},
     {"wire_quantize", reinterpret_cast<PyCFunction>(wire_quantize), METH_FASTCALL, "Quantize into a payload of the CUDA extension's format."},
     {"wire_dequantize", reinterpret_cast<PyCFunction>(wire_dequantize), METH_FASTCALL, "Decode a payload of that format into a fresh tensor."},
     {"wire_reduce", reinterpret_cast<PyCFunction>(wire_reduce), METH_FASTCALL, "Fused reduce of payloads of that format, optionally with the residual update."},

@@ -74,13 +74,14 @@ struct RingStepArgs {
 struct WireQuantArgs {
     const void *x;
     const void *residual;    // may be null; same dtype as x
+    void *prepared;          // may be null; receives x + residual, in the dtype of both (needs residual and one chunk)
     uint8_t *payloads;       // chunk d starts at payloads + d * payload_stride
     int64_t numel;           // valid elements in the whole tensor
     int64_t shard_numel;     // elements per chunk (== numel for a single payload)
     int64_t payload_stride;  // bytes
     int compact;             // scales interleaved after each group's codes
-    int nan_resets;          // group maximum as the reference's general kernels take it (a NaN resets it); needs
-                             // residual == null and whole groups
+    int nan_resets;          // group maximum as the reference's general kernels take it (a NaN resets it): without a
+                             // residual on chunks of whole groups, with `prepared` always
 };
 
 struct WireReduceArgs {

@@ -580,8 +580,9 @@ int64_t lbc_wire_payload_nbytes(int64_t numel, int group_size, int dtype, int bi
     return groups * (group_size * bit / 8 + dtype_size(dtype));
 }
 
-int lbc_wire_quant_pack_chunks(const void *x, const void *residual, int dtype, int64_t numel, int world,
-                               int group_size, int bit, int compact, uint8_t *payloads, int64_t payload_stride, int access, void *stream) {
+namespace {
+int wire_quant(const char *name, const void *x, const void *residual, void *prepared, int dtype, int64_t numel, int world,
+               int group_size, int bit, int compact, uint8_t *payloads, int64_t payload_stride, int access, void *stream) {
     if (!valid_access(access)) return fail(LBC_EINVAL, "unknown access mode %d", access);
     if (numel < 0) return fail(LBC_EINVAL, "numel must be >= 0");
     if (world <= 0) return fail(LBC_EINVAL, "world must be > 0");
@@ -597,18 +598,34 @@ int lbc_wire_quant_pack_chunks(const void *x, const void *residual, int dtype, i
     if (!aligned_to(payloads, item)) return fail(LBC_EINVAL, "payloads must be aligned to the element size");
     if (!aligned_to(x, item) || !aligned_to(residual, item))
         return fail(LBC_EINVAL, "input/residual are not aligned to their element size");
+    if (!aligned_to(prepared, item)) return fail(LBC_EINVAL, "prepared is not aligned to its element size");
     lbc::WireQuantArgs a{};
     a.x = x;
     a.residual = residual;
+    a.prepared = prepared;
     a.payloads = payloads;
     a.numel = numel;
     a.shard_numel = shard;
     a.payload_stride = world > 1 ? payload_stride : 0;
     a.compact = compact != 0;
-    a.nan_resets = residual == nullptr;
+    a.nan_resets = residual == nullptr || prepared != nullptr;
     return finish(lbc::launch_wire_quant(dtype, group_size, bit, pick_mode(true, access), a, world,
                                          static_cast<hipStream_t>(stream)),
-                  "lbc_wire_quant_pack");
+                  name);
+}
+}  // namespace
+
+int lbc_wire_quant_pack_chunks(const void *x, const void *residual, int dtype, int64_t numel, int world,
+                               int group_size, int bit, int compact, uint8_t *payloads, int64_t payload_stride, int access, void *stream) {
+    return wire_quant("lbc_wire_quant_pack", x, residual, nullptr, dtype, numel, world, group_size, bit, compact, payloads,
+                      payload_stride, access, stream);
+}
+
+int lbc_wire_compensate_quant_pack(const void *x, const void *residual, void *prepared, int dtype, int64_t numel, int group_size,
+                                   int bit, int compact, uint8_t *payload, int access, void *stream) {
+    if (numel > 0 && (residual == nullptr || prepared == nullptr)) return fail(LBC_EINVAL, "residual and prepared must not be null");
+    return wire_quant("lbc_wire_compensate_quant_pack", x, residual, prepared, dtype, numel, 1, group_size, bit, compact, payload, 0,
+                      access, stream);
 }
 
 int lbc_wire_quant_pack(const void *x, const void *residual, int dtype, int64_t numel, int group_size, int bit,

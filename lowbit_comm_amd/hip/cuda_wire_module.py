@@ -104,6 +104,13 @@ class HipCudaWireModule:
         if not done:
             raise RuntimeError(f"no HIP quantize kernel for input dtype {input.dtype}")
 
+    def _compensate_quantize(self, input, residual, group_size, topk, stochastic, bit, quant_type, compact):
+        """``(input + residual, the payload quantize() makes of it)`` from one launch, both freshly allocated, or ``None``
+        when there is no such launch (another policy, operands of different types or shapes)."""
+        pair = _host.wire_compensate_quantize(input, residual, group_size, topk, stochastic, bit, quant_type, compact,
+                                              ops.access_code(None))
+        return pair if isinstance(pair, tuple) else None
+
     @staticmethod
     def philox_engine_inputs(device: torch.device, increment: int) -> tuple[int, int]:
         """(seed, offset) of the device's default generator, advanced past ``increment`` draws rounded up to a

@@ -43,6 +43,7 @@ SIGNATURES = {
     "lbc_ef_update": (_c_int, [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_i64, _c_int, _c_ptr]),
     "lbc_wire_payload_nbytes": (_c_i64, [_c_i64, _c_int, _c_int, _c_int]),
     "lbc_wire_quant_pack": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_ptr]),
+    "lbc_wire_compensate_quant_pack": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_ptr]),
     "lbc_wire_quant_pack_chunks": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_ptr,
                                             _c_i64, _c_int, _c_ptr]),
     "lbc_wire_ring_step": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_i64, _c_int, _c_int, _c_int, ctypes.c_float, _c_ptr, _c_int, _c_ptr]),

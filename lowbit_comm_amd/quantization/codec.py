@@ -141,6 +141,17 @@ def writes_prepared(extension_status: Any | None) -> bool:
     return bool(getattr(extension_status, "available", False) and getattr(module, "QUANTIZE_PACK_WRITES_PREPARED", False))
 
 
+def compensate_and_quantize(tensor: Any, residual: Any, config: CompressionConfig, *,
+                            extension_status: Any | None = None) -> tuple[Any, Any] | None:
+    """``(tensor + residual, the payload quantize_tensor makes of it)`` as two fresh tensors from one launch; ``None`` when
+    the native module has none for these operands."""
+    fused = getattr(getattr(extension_status, "module", None), "_compensate_quantize", None)
+    if fused is None or not getattr(extension_status, "available", False):
+        return None
+    return fused(tensor, residual, config.group_size, config.topk, config.stochastic, config.bit,
+                 _quant_type(extension_status.module, config), config.compact)
+
+
 def _try_quantize_pack(module: object, tensor: Any, output: Any, residual: Any | None, config: CompressionConfig,
                        metadata: dict[str, Any] | None, quant_type: Any, prepared_out: Any | None = None) -> bool:
     fused = False

@@ -212,3 +212,85 @@ def test_cuda_byte_format_beyond_the_tile_rule(hip_device, dtype, with_residual,
     out = Guarded(cuda_wire.payload_nbytes(n, t), torch.uint8, 4, hip_device)
     assert cuda_wire.quant_pack_into(x.to(hip_device), out.inside, residual=None if r is None else r.to(hip_device))
     out.check(torch.from_numpy(wire.quantize(to_numpy(x), dtype, 64, True, residual=None if r is None else to_numpy(r))), "payload")
+
+
+# the sum of bucket and residual with its payload, against torch's add and the quantize of the padded sum: workgroup and
+# lane ends, both sides of the tile rule (2 Mi fp32 elements, 4 Mi 16-bit ones), NaN and infinite elements
+@pytest.mark.parametrize("n", [1, 5, 63, 64, 66, 1023, 1025, 2047, 2049, 8193, (1 << 21) + 5, (1 << 22) + 67])
+@pytest.mark.parametrize("specials", [False, True])
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_compensated_quantize_of_the_cuda_byte_format(hip_device, dtype, specials, n):
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.codec import compensate_and_quantize
+
+    t, status = DTYPES[dtype], load_hip_extension(wire_format="native")
+    x, r = values(n, t, n), values(n, t, n + 7, 1e-5)
+    if specials:
+        for seed, special in enumerate((float("nan"), float("inf"), float("-inf"))):
+            for side, tensor in enumerate((x, r)):
+                g = torch.Generator().manual_seed(100 * n + 10 * seed + side)
+                tensor[torch.randint(0, n, (max(1, n // 300),), generator=g)] = special
+    for offset, group, bit, compact in ((0, 64, 8, True), (1, 64, 8, False), (3, 64, 4, False), (0, 32, 4, True), (1, 16, 8, True)):
+        config = CompressionConfig(bit=bit, group_size=group, compact=compact, allow_experimental=bit != 8)
+        x_in, r_in = Guarded(n, t, offset, hip_device, x).inside, Guarded(n, t, offset, hip_device, r).inside
+        want = x_in + r_in
+        prepared, payload = compensate_and_quantize(x_in, r_in, config, extension_status=status)
+        assert torch.equal(prepared.view(torch.uint8), want.view(torch.uint8)), "sum"
+        assert torch.equal(payload, quantize_tensor(want, config, extension_status=status)), (group, bit, compact)
+
+
+def test_compensated_quantize_leaves_other_operands_to_the_separate_calls(hip_device):
+    from lowbit_comm_amd import CompressionConfig
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.codec import compensate_and_quantize
+
+    status, config = load_hip_extension(wire_format="native"), CompressionConfig()
+    x = torch.zeros(256, dtype=torch.bfloat16, device=hip_device)
+    others = [x.float(), x[:128], x.view(4, 64), x.cpu(), torch.zeros(512, dtype=x.dtype, device=hip_device)[::2],
+              x.clone().requires_grad_(True)]
+    for other in others:
+        assert compensate_and_quantize(x, other, config, extension_status=status) is None
+        assert compensate_and_quantize(other, x, config, extension_status=status) is None
+    assert compensate_and_quantize(x, x, CompressionConfig(topk=1), extension_status=status) is None
+    assert compensate_and_quantize(x[:0], x[:0], config, extension_status=status) is None
+    assert compensate_and_quantize(x, x, config, extension_status=load_hip_extension()) is None
+
+
+@pytest.mark.parametrize("dtype, n", [("fp32", 100_001), ("bf16", 64 * 999)])
+def test_hook_iterations_in_the_cuda_byte_format_match_the_separate_calls(hip_device, dtype, n):
+    """A feedback state with a compensate step of its own takes the add and the quantize as two calls; both hooks keep the
+    same residuals, payloads and results over several iterations."""
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+    from lowbit_comm_amd.communication.ddp_hook import create_ddp_comm_hook
+    from lowbit_comm_amd.communication.gather_reduce import GatheredPayloads
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.error_feedback import ErrorFeedbackState
+
+    class OwnStep(ErrorFeedbackState):
+        def compensate(self, key, tensor):
+            return super().compensate(key, tensor)
+
+    class Bucket:
+        def __init__(self, tensor):
+            self.tensor = tensor
+
+        def index(self):
+            return 0
+
+        def buffer(self):
+            return self.tensor
+
+    t, status = DTYPES[dtype], load_hip_extension(wire_format="native")
+    config = CompressionConfig(error_feedback=True)
+    peer = quantize_tensor(values(n, t, 5).to(hip_device), config, extension_status=status)
+    grads = [values(n, t, 20 + i).to(hip_device) for i in range(3)]
+    seen = []
+    for feedback in (ErrorFeedbackState(), OwnStep()):
+        sent = []
+        hook = create_ddp_comm_hook(config, strategy="all_gather", reduce="mean", error_feedback=feedback, extension_status=status,
+                                    all_gather=lambda local: (sent.append(local.buffer), GatheredPayloads([local.buffer, peer], 2))[1])
+        out = [hook(None, Bucket(g)).wait().clone() for g in grads]
+        seen.append([*sent, *out, feedback.get(0)])
+    for a, b in zip(*seen):
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
