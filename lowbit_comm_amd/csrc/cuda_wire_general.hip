@@ -152,7 +152,8 @@ template <int LANES> __device__ __forceinline__ void merge_top3(uint32_t &first,
 // FIXED names what the launch knows about the policy at compile time, so that the code of the other policies
 // is not part of the kernel: bit 0 "no outlier channel", bit 1 "round to nearest", bit 2 "linear codes", bit 3
 // "stochastic rounding" (13: plain linear codes rounded stochastically, 12: the same with outliers, 9: a code book
-// with stochastic rounding).  0 is the kernel for every policy.
+// with stochastic rounding; 6: linear codes rounded to nearest, always with outliers - without them lbc_wire_quant_pack
+// serves the call).  0 is the kernel for every policy.
 // EL: elements per lane, a multiple of 8 that divides G.  TILES: tiles of 64 * EL elements a wavefront owns, all of
 // them asked for before the first is encoded.
 template <typename T, int G, int BIT, int FIXED, int EL, int TILES>
@@ -255,7 +256,8 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         uint32_t scale_raw;
         Raw meta[4] = {0, 0, 0, 0};   // [scale][indices][top1][top2]
         bool any_nan = true;   // "not known": the outlier path does not look
-        if (topk == 0) {
+        uint32_t outlier[2] = {~0u, ~0u};   // place among the lane's elements, beyond them when another lane's
+        if (FIXED != 6 && topk == 0) {
             scale_raw = running_max_raw<T, G, VEC>(mag, k0, start, &any_nan);
         } else {
             // The three largest candidates of the group, a candidate's key being its magnitude and a tie-break rank
@@ -289,27 +291,28 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
                     for (int i = 0; i < VEC; ++i) key[i] = rank[i] == r ? 0 : key[i];   // taken (r = 0 matches nobody)
                 }
             } else {
-                // A 16-bit magnitude and its rank share one 32-bit key, (magnitude << 7) + rank, unique inside the
-                // group.  A lane keeps the three largest of its own keys in order (three instructions an element), and
-                // the group's lanes merge their triples over the DPP butterfly (eight instructions a step): no rounds
-                // over the elements.  Zeros are no candidates: their keys are below 128, under every candidate's, and
-                // are dropped from the result.  NaNs are no candidates either and their keys are above every
+                // A 16-bit magnitude and its rank less one share one 32-bit key, the magnitude in the upper half, unique
+                // inside the group: the element's bits with the sign masked out (in place for the upper half of a loaded
+                // dword) and the rank or-ed in, the quad's part and the constant part apart.  A lane keeps the three
+                // largest of its own keys in order (three instructions an element), and the group's lanes merge their
+                // triples over the DPP butterfly (eight instructions a step): no rounds over the elements.  Zeros are no
+                // candidates: their keys are below 2^16, under every candidate's, and are dropped from the result.  NaNs are no candidates either and their keys are above every
                 // candidate's: the first pass does not look for them, and when one tops any group of the wavefront
                 // (rare) the pass is repeated with every element checked.  Scan positions do not wrap inside four
                 // adjacent elements (a lane's first element and the scan's start are multiples of four).
-                constexpr uint32_t kBelow = 128, kAbove = (RB::INF << 7) + G;
+                constexpr uint32_t kBelow = 1u << 16, kAbove = (RB::INF << 16) | 0xFFFFu;
                 uint32_t largest, runner_up, bronze;
                 auto search = [&](const bool checked) __attribute__((always_inline)) {
                     largest = runner_up = bronze = 0;
                     const uint32_t p0 = static_cast<uint32_t>(k0 - start) & (G - 1);
 #pragma unroll
                     for (int q = 0; q < VEC / 4; ++q) {
-                        const uint32_t rank0 = G - ((p0 + 4 * q) & (G - 1));      // rank = G - scan position
+                        const uint32_t rank0 = (G - 4) ^ ((p0 + 4 * q) & (G - 1));   // rank - 1 = G - 1 - scan position
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const int i = 4 * q + j;
-                            uint32_t key = (mag[i] << 7) + (rank0 - j);
-                            if (checked) key = (mag[i] - 1u) < RB::INF ? key : 0;
+                            uint32_t key = (static_cast<uint32_t>(raw[i]) << 16 & 0x7FFF0000u) | rank0 | (3 - j);
+                            if (checked) key = (key >> 16) - 1u < RB::INF ? key : 0;
                             bronze = umed3(runner_up, bronze, key);
                             runner_up = umed3(largest, runner_up, key);
                             largest = key > largest ? key : largest;
@@ -324,9 +327,9 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
                 bronze = bronze < kBelow ? 0 : bronze;
                 const uint32_t found[3] = {largest, runner_up, bronze};
 #pragma unroll
-                for (int round = 0; round < 3; ++round) {   // rank 1..G <= 64 never carries into the magnitude
-                    best_key[round] = found[round] == 0 ? 0 : ((found[round] - 1) >> 7) + 1;
-                    if (round < 2) best_rank[round] = found[round] == 0 ? 0 : ((found[round] - 1) & 0x7Fu) + 1;
+                for (int round = 0; round < 3; ++round) {
+                    best_key[round] = found[round] == 0 ? 0 : (found[round] >> 16) + 1;
+                    if (round < 2) best_rank[round] = found[round] == 0 ? 0 : (found[round] & 0xFFFFu) + 1;
                 }
             }
             auto index_of = [&](uint32_t r) {
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             int index2 = -1;
             if (topk == 1) {
                 // nothing comparable: the reference falls back to element 1 (as stored for fp32, its magnitude otherwise)
-                const uint32_t element1 = WIDE ? static_cast<uint32_t>(raw[1]) : mag[1];
+                const uint32_t element1 = WIDE ? static_cast<uint32_t>(raw[1]) : raw[1] & RB::ABS;
                 const uint32_t fallback = static_cast<uint32_t>(__shfl(static_cast<int>(element1), lane & ~(LPG - 1)));
                 scale_raw = none ? fallback : (best_key[1] == 0 ? 0u : best_key[1] - 1);
             } else {
@@ -345,9 +348,17 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
                 index2 = none ? 1 : (lonely ? ((index1 + 1) & (G - 1)) : index_of(best_rank[1]));
                 scale_raw = (none || lonely || best_key[2] == 0) ? 0u : best_key[2] - 1;
             }
+            // Outliers encode as 0.  A code book needs the elements gone (they lie above the scale); linear codes, which a
+            // zero element always turns into 0 (the noise stays within +-1/2, which rounds to 0), are cleared in the
+            // packed words: five instructions a word instead of three an element.
+            if constexpr (FIXED & 4) {
+                outlier[0] = static_cast<uint32_t>(index1 - k0);
+                outlier[1] = static_cast<uint32_t>(index2 - k0);
+            } else {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i)
-                if (k0 + i == index1 || k0 + i == index2) v[i] = 0.0f;
+                for (int i = 0; i < VEC; ++i)
+                    if (k0 + i == index1 || k0 + i == index2) v[i] = 0.0f;
+            }
             // The outliers travel as they are stored.  The group's first lane fetches them from the tensor once more
             // (its wavefront has just read those lines) instead of every lane selecting among its elements; the
             // metadata words leave together at the end of the tile, when the values have long arrived.
@@ -367,8 +378,16 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         if (kind == 0) {
             const float multiplier = W::LEVELS / scale;
             constexpr int L = static_cast<int>(W::LEVELS);
+            // Beside outliers and NaNs no magnitude exceeds the scale, so the product stays within the levels and adding
+            // 1.5 * 2^23 leaves its rounding, half to even, in the low bits: two instructions an element instead of four
+            // with conversion and clamp.  An outlier's code is cleared below; a NaN of a 16-bit type has zeros there.
+            // With the search's keys and the clearing of words this took the kernel, bound by instructions, from 20.2 to
+            // 17 us on 26.2 M bf16 elements with two outliers (the round trip 31.9 to 28.6).
+            constexpr bool kByAddition = FIXED == 6 && !WIDE;
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) {
+            for (int i = 0; kByAddition && i < VEC; ++i) c[i] = static_cast<int>(as_u32(v[i] * multiplier + 0x1.8p23f));
+#pragma unroll
+            for (int i = 0; !kByAddition && i < VEC; ++i) {
                 // nvcc contracts v * m + noise into one FMA; without noise the product is rounded alone
                 const float t = stochastic ? __builtin_fmaf(v[i], multiplier, uniform[i] - 0.5f) : v[i] * multiplier;
                 const int r = cvt_i32(__builtin_rintf(t));
@@ -453,6 +472,15 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             uint32_t words[WORDS];
             if constexpr (BIT == 8) pack_codes<T, 8, VEC, WORDS>(c, words);
             else pack_nibbles<T, EL>(c, words);
+            if constexpr ((FIXED & 5) == 4) {
+                constexpr uint32_t PER_WORD = 32 / BIT, ORDER = BIT == 8 ? (WIDE ? 3 : 1) : (WIDE ? 7 : 3);   // place in a word
+                uint32_t code[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) code[k] = ((1u << BIT) - 1) << (((outlier[k] ^ ORDER) * BIT) & 31u);
+#pragma unroll
+                for (uint32_t w = 0; w < WORDS; ++w)
+                    words[w] &= ~((outlier[0] / PER_WORD == w ? code[0] : 0u) | (outlier[1] / PER_WORD == w ? code[1] : 0u));
+            }
             store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
         }
         if (live && k0 == 0) {
