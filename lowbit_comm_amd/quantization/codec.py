@@ -192,7 +192,9 @@ def quantize_tensor(tensor: object, config: CompressionConfig, *, extension_stat
     if output is not None and _try_quantize_pack(module, tensor, output, residual, config, metadata, quant_type):
         return output
     prepared = tensor if residual is None else tensor + residual
-    if output is not None or not getattr(module, "_PADS_THE_LAST_GROUP", False):
+    # A strided tensor is flattened by the padding: modules take contiguous operands only.
+    contiguous = getattr(prepared, "is_contiguous", None)
+    if output is not None or not getattr(module, "_PADS_THE_LAST_GROUP", False) or contiguous is None or not contiguous():
         prepared = _zero_padded(prepared, config.group_size)
     policy = (config.group_size, config.topk, config.stochastic, config.bit, quant_type, config.compact)
     if output is not None:

@@ -330,6 +330,18 @@ def test_quantize_tensor_pads_and_forwards_the_policy_tuple():
     assert policy == [64, 0, False, 8, "<Linear>", False]
 
 
+@pytest.mark.parametrize("strided", [False, True])
+def test_a_module_that_pads_itself_still_receives_contiguous_operands(strided):
+    m = RecordingModule()
+    m._PADS_THE_LAST_GROUP = True
+    x = torch.arange(70.0).view(7, 10)
+    x = x.t() if strided else x
+    assert codec.quantize_tensor(x, CFG, extension_status=status(m)) == "Q"
+    handed = m.calls[0][1]
+    assert handed.is_contiguous() and (handed is x) != strided
+    assert torch.equal(handed.reshape(-1)[:70], x.reshape(-1))
+
+
 def test_quantize_with_output_prefers_the_fused_pack_call_and_reports_metadata():
     m = RecordingModule(pack_result=True)
     x, out, res, meta = torch.ones(100), torch.empty(136, dtype=torch.uint8), torch.zeros(100), {}

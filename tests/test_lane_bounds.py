@@ -294,3 +294,18 @@ def test_hook_iterations_in_the_cuda_byte_format_match_the_separate_calls(hip_de
         seen.append([*sent, *out, feedback.get(0)])
     for a, b in zip(*seen):
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+# a strided tensor that does not fill its last group is flattened on the way in; one of whole groups is refused
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("wire", ["portable", "native"])
+def test_strided_ragged_tensors_quantize_like_their_flat_copies(hip_device, wire, dtype):
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+
+    status, config = load_hip_extension(wire_format=wire), CompressionConfig()
+    x = values(70, DTYPES[dtype], 3).to(hip_device).view(7, 10).t()
+    flat = torch.cat([x.reshape(-1), x.new_zeros(58)])
+    assert torch.equal(quantize_tensor(x, config, extension_status=status), quantize_tensor(flat, config, extension_status=status))
+    with pytest.raises(RuntimeError, match="contiguous"):
+        quantize_tensor(flat.view(2, 64).t(), config, extension_status=status)
