@@ -527,9 +527,10 @@ PyObject *wire_reduce(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 12 || !integer(a[4], p.group) || !integer(a[5], p.topk) || !integer(a[6], p.bit) || !integer(a[7], p.quant_type) ||
         !integer(a[8], compact) || !integer(a[10], fma) || !integer(a[11], access))
         return elsewhere();
-    const double divisor = PyFloat_AsDouble(a[9]);
+    const double divisor = PyFloat_AsDouble(a[9]);   // the library refuses one whose reciprocal is not positive
+    if (divisor == -1.0 && PyErr_Occurred()) return nullptr;
     const at::Tensor *out = gpu_tensor(a[1]);
-    if (out == nullptr || !plain(p) || p.group != 64 || p.bit != 8 || !(divisor > 0.0)) return elsewhere();
+    if (out == nullptr || !plain(p) || p.group != 64 || p.bit != 8) return elsewhere();
     const int type = code_of(out->scalar_type());
     if (type == LBC_NONE || out->numel() == 0 || out->numel() % 64 != 0) return elsewhere();
     int64_t nbytes = out->numel() / 64 * cuda_group_bytes(p, type), numel = out->numel();

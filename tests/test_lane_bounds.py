@@ -309,3 +309,19 @@ def test_strided_ragged_tensors_quantize_like_their_flat_copies(hip_device, wire
     assert torch.equal(quantize_tensor(x, config, extension_status=status), quantize_tensor(flat, config, extension_status=status))
     with pytest.raises(RuntimeError, match="contiguous"):
         quantize_tensor(flat.view(2, 64).t(), config, extension_status=status)
+
+
+@pytest.mark.parametrize("divisor", [float("nan"), float("inf")])
+def test_fused_reduce_of_the_cuda_byte_format_refuses_divisors_without_a_positive_reciprocal(hip_device, divisor):
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+
+    status = load_hip_extension(wire_format="native")
+    module = status.module
+    x = values(128, torch.float32, 5).to(hip_device)
+    payload, out = quantize_tensor(x, CompressionConfig(), extension_status=status), torch.empty_like(x)
+    policy = (64, 0, 8, module.QuantType.Linear, False)
+    assert module.inplace_dequantize_reduce_mean([payload], out, *policy, 2.0)
+    with pytest.raises(RuntimeError, match="divisor must be > 0"):
+        module.inplace_dequantize_reduce_mean([payload], out, *policy, divisor)
+    assert not module.inplace_dequantize_reduce_mean([payload], out[:100], *policy, divisor)   # not the fused reduce's
