@@ -1,3 +1,4 @@
+import gc
 import sys
 from pathlib import Path
 
@@ -22,6 +23,21 @@ def hip_device():
     if not torch.cuda.is_available():
         pytest.skip("no GPU visible")
     return torch.device("cuda:0")
+
+
+@pytest.fixture(autouse=True)
+def steady_allocator_counter(request):
+    """A test that compares readings of the allocator's counter starts without garbage of earlier tests and holds the cycle
+    collector off: tensors of theirs that it frees between two readings are not what the test is about."""
+    if "memory_allocated" not in request.function.__code__.co_names:
+        yield
+        return
+    gc.collect()
+    gc.disable()
+    try:
+        yield
+    finally:
+        gc.enable()
 
 
 @pytest.fixture(scope="session")
