@@ -220,11 +220,11 @@ int code_of(at::ScalarType type) {
 }
 at::ScalarType type_of(long code) { return code == LBC_F32 ? at::kFloat : (code == LBC_F16 ? at::kHalf : at::kBFloat16); }
 
-// The tensor behind `o` when it is a contiguous GPU tensor, else null.
+// The tensor behind `o` when it is a contiguous GPU tensor that holds its values as they are (no lazy negation), else null.
 const at::Tensor *gpu_tensor(PyObject *o) {
     if (!THPVariable_Check(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
-    return t.is_cuda() && t.layout() == at::kStrided && t.is_contiguous() ? &t : nullptr;
+    return t.is_cuda() && t.layout() == at::kStrided && t.is_contiguous() && !t.is_neg() ? &t : nullptr;
 }
 const at::Tensor *payload_tensor(PyObject *o) {
     const at::Tensor *t = gpu_tensor(o);

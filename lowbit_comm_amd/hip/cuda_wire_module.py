@@ -138,7 +138,7 @@ class HipCudaWireModule:
         if input.numel() == 0:
             return True
         seeds = self.philox_engine_inputs(input.device, input.numel()) if stochastic else None
-        return cuda_wire.quant_general_into(input.reshape(-1), output.reshape(-1), group_size=group_size, bit=bit,
+        return cuda_wire.quant_general_into(input.resolve_neg().reshape(-1), output.reshape(-1), group_size=group_size, bit=bit,
                                             quant_type=_KIND[int(quant_type)], topk=topk, stochastic=seeds,
                                             compact=bool(compact))
 
@@ -168,8 +168,8 @@ class HipCudaWireModule:
             raise RuntimeError("output has an invalid quantized payload size")
         if input.numel() == 0:
             return True
-        flat_residual = None if residual is None else residual.reshape(-1)
-        return cuda_wire.quant_pack_into(input.reshape(-1), output.reshape(-1), group_size=group_size,
+        flat_residual = None if residual is None else residual.resolve_neg().reshape(-1)
+        return cuda_wire.quant_pack_into(input.resolve_neg().reshape(-1), output.reshape(-1), group_size=group_size,
                                          compact=bool(compact), residual=flat_residual, bit=bit)
 
     # ---- dequantize -----------------------------------------------------------------------------

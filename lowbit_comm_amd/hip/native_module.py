@@ -197,9 +197,10 @@ class HipNativeModule:
             if output.numel() != 0:
                 raise RuntimeError("output has an invalid quantized payload size")
             return True
-        # payload dtype / contiguity / size are checked where the addresses are taken
-        bind = lambda: ops.bind_quant_pack_payload(input.reshape(-1), output, group_size=group_size,  # noqa: E731
-                                                   residual=None if residual is None else residual.reshape(-1),
+        # payload dtype / contiguity / size are checked where the addresses are taken; a lazily negated view has no key
+        # and is read as the values it stands for
+        bind = lambda: ops.bind_quant_pack_payload(input.resolve_neg().reshape(-1), output, group_size=group_size,  # noqa: E731
+                                                   residual=None if residual is None else residual.resolve_neg().reshape(-1),
                                                    prepared_out=None if prepared_out is None else prepared_out.reshape(-1))
         return (bind() if key is None else self._memoized(key, bind))()
 

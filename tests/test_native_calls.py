@@ -1,0 +1,36 @@
+"""The native host side (``lowbit_comm_amd._host``) in front of the public entry points: what it takes, what it leaves to the
+validating path, and what it must not by-pass."""
+import pytest
+import torch
+
+DTYPES = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
+
+
+def values(n, dtype, seed, sigma=1e-3):
+    return (torch.randn(n, generator=torch.Generator().manual_seed(seed)) * sigma).to(dtype)
+
+
+# a lazily negated view is contiguous and has an address, but the memory there holds the negatives of its values
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [70, 128])
+@pytest.mark.parametrize("wire, policy", [("portable", {}), ("native", {}), ("native", {"topk": 1})])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_negated_views_quantize_as_the_values_they_stand_for(hip_device, dtype, wire, policy, n):
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.codec import compensate_and_quantize
+
+    status, config = load_hip_extension(wire_format=wire), CompressionConfig(**policy)
+    x, r = (torch._neg_view(values(n, DTYPES[dtype], seed).to(hip_device)) for seed in (1, 2))
+    assert x.is_neg() and x.is_contiguous()
+    want = quantize_tensor(x.resolve_neg(), config, extension_status=status)
+    assert torch.equal(quantize_tensor(x, config, extension_status=status), want)
+    if n % 64 == 0:
+        into = torch.zeros_like(want)
+        assert torch.equal(quantize_tensor(x, config, extension_status=status, output=into), want)
+    if not policy:
+        into, sums = torch.zeros_like(want), quantize_tensor(x.resolve_neg() + r.resolve_neg(), config, extension_status=status)
+        quantize_tensor(x, config, extension_status=status, output=into, residual=r)
+        assert torch.equal(into, sums)
+        assert compensate_and_quantize(x, x.resolve_neg(), config, extension_status=status) is None
+        assert compensate_and_quantize(x.resolve_neg(), x, config, extension_status=status) is None
