@@ -230,6 +230,8 @@ const at::Tensor *payload_tensor(PyObject *o) {
     const at::Tensor *t = gpu_tensor(o);
     return t != nullptr && t->scalar_type() == at::kByte ? t : nullptr;
 }
+// Does autograd follow what is computed from `t`, backward or forward?
+bool watched(const at::Tensor &t) { return t.requires_grad() || t._fw_grad(/*level=*/0).defined(); }
 bool with(const at::Tensor &t, const at::Tensor &like) { return t.get_device() == like.get_device(); }
 
 at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor &like) {
@@ -464,7 +466,7 @@ PyObject *wire_compensate_quantize(PyObject *, PyObject *const *a, Py_ssize_t n)
     if (x == nullptr || r == nullptr || x->numel() == 0 || !cuda_policy(p) || !plain(p)) return elsewhere();
     const int type = code_of(x->scalar_type());
     if (type == LBC_NONE || r->scalar_type() != x->scalar_type() || !x->sizes().equals(r->sizes()) || !with(*r, *x) ||
-        x->requires_grad() || r->requires_grad())
+        watched(*x) || watched(*r))
         return elsewhere();
     const int64_t numel = x->numel();
     at::Tensor prepared = fresh(x->sizes(), x->scalar_type(), *x);

@@ -34,3 +34,19 @@ def test_negated_views_quantize_as_the_values_they_stand_for(hip_device, dtype, 
         assert torch.equal(into, sums)
         assert compensate_and_quantize(x, x.resolve_neg(), config, extension_status=status) is None
         assert compensate_and_quantize(x.resolve_neg(), x, config, extension_status=status) is None
+
+
+# the sum that the one launch writes has no history: operands that autograd follows keep torch's own add
+@pytest.mark.gpu
+def test_compensated_quantize_leaves_tangents_to_torch(hip_device):
+    from lowbit_comm_amd import CompressionConfig
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.codec import compensate_and_quantize
+
+    status, config = load_hip_extension(wire_format="native"), CompressionConfig()
+    x, r, tangent = (values(128, torch.float32, seed).to(hip_device) for seed in (1, 2, 3))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, tangent)
+        assert compensate_and_quantize(dual, r, config, extension_status=status) is None
+        assert compensate_and_quantize(r, dual, config, extension_status=status) is None
+    assert compensate_and_quantize(x, r, config, extension_status=status) is not None
