@@ -614,9 +614,11 @@ hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStr
     if (bit != 8 && bit != 4) return hipErrorNotSupported;
     if (bit == 8 && a.kind != 0) return hipErrorNotSupported;   // eight bits: linear codes only
     if (bit == 8) {
+        // the kernel below has no code for a group without outliers: lbc_wire_quant_pack serves those calls
+        if (fixed == 7) return hipErrorNotSupported;
         if (a.stochastic && a.topk == 0) return launch_general_quant_as<T, G, 8, 13, WIDE>(a, stream);
         if (a.stochastic) return launch_general_quant_as<T, G, 8, 12, WIDE>(a, stream);
-        return launch_general_quant_as<T, G, 8, 6, WIDE>(a, stream);   // round to nearest, outliers or none
+        return launch_general_quant_as<T, G, 8, 6, WIDE>(a, stream);   // round to nearest, with outliers
     }
     if (fixed == 6) return launch_general_quant_as<T, G, 4, 6, WIDE>(a, stream);
     if (fixed == 2) return launch_general_quant_as<T, G, 4, 2, WIDE>(a, stream);

@@ -30,6 +30,23 @@ def test_library_loads_on_the_cpu_and_exports_every_declared_symbol():
     assert lib.lbc_abi_version() == library.ABI_VERSION
 
 
+def test_outlier_kernels_launcher_refuses_calls_without_outliers():
+    """The 8-bit kernel for linear codes rounded to nearest has the outlier channel compiled in; the entry point sends calls
+    without outliers elsewhere, and the launcher behind it must not take them either.  No elements: nothing is launched."""
+    class Args(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_void_p), ("payload", ctypes.c_void_p), ("numel", ctypes.c_int64), ("kind", ctypes.c_int),
+                    ("topk", ctypes.c_int), ("stochastic", ctypes.c_int), ("compact", ctypes.c_int),
+                    ("seed", ctypes.c_uint64), ("offset", ctypes.c_uint64)]
+
+    launch = library.load_library()["_ZN3lbc25launch_wire_general_quantEiiiRKNS_20WireGeneralQuantArgsEP12ihipStream_t"]
+    ok, not_supported = 0, 801
+    for dtype in (0, 1, 2):
+        for group in (16, 32, 64):
+            for topk, want in ((0, not_supported), (1, ok), (2, ok)):
+                assert launch(dtype, group, 8, ctypes.byref(Args(topk=topk)), None) == want, (dtype, group, topk)
+            assert launch(dtype, group, 8, ctypes.byref(Args(stochastic=1)), None) == ok
+
+
 def test_argument_validation_happens_before_any_device_work():
     lib = library.load_library()
     none = ctypes.c_void_p(None)
