@@ -184,14 +184,21 @@ int launch_init(PyObject *self, PyObject *args, PyObject *) {
 PyObject *launch_call(PyObject *self, PyObject *args, PyObject *kwargs) {
     HANDLE_TH_ERRORS
     Launch *launch = reinterpret_cast<Launch *>(self);
-    PyObject *given = PyTuple_GET_SIZE(args) > 0 ? PyTuple_GET_ITEM(args, 0) : nullptr;
-    if (given == nullptr && kwargs != nullptr) given = PyDict_GetItemString(kwargs, "stream");
+    PyObject *given = nullptr;
+    if (PyTuple_GET_SIZE(args) != 0 || kwargs != nullptr) {   // the usual call has none
+        static const char *const kNames[] = {"stream", nullptr};
+        if (!PyArg_ParseTupleAndKeywords(args, kwargs, "|O:Launch", const_cast<char **>(kNames), &given)) return nullptr;
+    }
     if (launch->call == nullptr) {
         PyErr_SetString(PyExc_RuntimeError, "the launch was not bound");
         return nullptr;
     }
     if (given == nullptr || given == Py_None)
         return answer(enqueue(static_cast<c10::DeviceIndex>(launch->device), [&](void *stream) { return launch->call->run(stream); }));
+    if (!PyLong_Check(given)) {
+        PyErr_Format(PyExc_TypeError, "stream must be a stream handle or None, not %s", Py_TYPE(given)->tp_name);
+        return nullptr;
+    }
     void *stream = PyLong_AsVoidPtr(given);
     if (PyErr_Occurred()) return nullptr;
     int rc;

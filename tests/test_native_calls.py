@@ -50,3 +50,15 @@ def test_compensated_quantize_leaves_tangents_to_torch(hip_device):
         assert compensate_and_quantize(dual, r, config, extension_status=status) is None
         assert compensate_and_quantize(r, dual, config, extension_status=status) is None
     assert compensate_and_quantize(x, r, config, extension_status=status) is not None
+
+
+# no elements: the call succeeds without a device
+def test_bound_launch_takes_a_stream_and_nothing_else():
+    from lowbit_comm_amd.hip import ops
+
+    nothing = (None, 0, None, -1, 0, 64, None, None, None, -1, None, 0, None, -1, 0)
+    launch = ops.BoundLaunch("lbc_quant_pack", nothing, torch.device("cuda:0"), ())
+    assert launch(0) is True and launch(stream=0) is True
+    for args, kwargs in (((0, 0), {}), ((), {"streams": 0}), ((0,), {"stream": 0}), (("0",), {})):
+        with pytest.raises(TypeError):
+            launch(*args, **kwargs)
