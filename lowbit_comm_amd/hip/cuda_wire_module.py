@@ -80,11 +80,23 @@ class HipCudaWireModule:
         self.fused_multiply_add = bool(fused_multiply_add)
 
     # ---- quantize ------------------------------------------------------------------------------
+    # The native calls stand for the public methods that the same request went through: a subclass, a class or an instance
+    # that puts another method in the place of one of them is asked as before.
+    def _encodes_natively(self, stochastic) -> bool:
+        cls, held = type(self), self.__dict__
+        return (cls.inplace_quantize is _INPLACE_QUANTIZE and "inplace_quantize" not in held
+                and (not stochastic or self._draws_natively()))
+
+    def _draws_natively(self) -> bool:
+        return (type(self).philox_engine_inputs is _PHILOX_ENGINE_INPUTS
+                and "philox_engine_inputs" not in self.__dict__)
+
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
-        payload = _host.wire_quantize(input, None, group_size, topk, stochastic, bit, quant_type, compact,
-                                      ops.access_code(None))
-        if isinstance(payload, torch.Tensor):
-            return payload
+        if self._encodes_natively(stochastic):
+            payload = _host.wire_quantize(input, None, group_size, topk, stochastic, bit, quant_type, compact,
+                                          ops.access_code(None))
+            if isinstance(payload, torch.Tensor):
+                return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         nbytes = cuda_wire.general_payload_nbytes(input.numel(), input.dtype, group_size, bit, topk)
         output = torch.empty(nbytes, dtype=torch.uint8, device=input.device)
@@ -92,7 +104,7 @@ class HipCudaWireModule:
         return output
 
     def inplace_quantize(self, input, output, group_size, topk, stochastic, bit, quant_type, compact) -> None:
-        if output is not None and isinstance(
+        if output is not None and (not stochastic or self._draws_natively()) and isinstance(
                 _host.wire_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact,
                                     ops.access_code(None)), torch.Tensor):
             return
@@ -107,6 +119,8 @@ class HipCudaWireModule:
     def _compensate_quantize(self, input, residual, group_size, topk, stochastic, bit, quant_type, compact):
         """``(input + residual, the payload quantize() makes of it)`` from one launch, both freshly allocated, or ``None``
         when there is no such launch (another policy, operands of different types or shapes)."""
+        if type(self).quantize is not _QUANTIZE or "quantize" in self.__dict__ or not self._encodes_natively(stochastic):
+            return None
         pair = _host.wire_compensate_quantize(input, residual, group_size, topk, stochastic, bit, quant_type, compact,
                                               ops.access_code(None))
         return pair if isinstance(pair, tuple) else None
@@ -176,12 +190,19 @@ class HipCudaWireModule:
     def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
         """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
         all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
+        if type(self).dequantize is not _DEQUANTIZE or "dequantize" in self.__dict__:
+            return None
+        return self._decode(input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
+
+    def _decode(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
+        if type(self).inplace_dequantize is not _INPLACE_DEQUANTIZE or "inplace_dequantize" in self.__dict__:
+            return None
         decoded = _host.wire_dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact,
                                         ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
+        decoded = self._decode(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
         if decoded is not None:
             return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
@@ -311,3 +332,10 @@ class HipCudaWireModule:
             restored = restored / divisor                        # pybind.cpp:126-128: torch's own scalar division
         self.inplace_error_feedback_update(prepared, restored, residual)
         return restored
+
+
+_QUANTIZE = HipCudaWireModule.quantize
+_INPLACE_QUANTIZE = HipCudaWireModule.inplace_quantize
+_PHILOX_ENGINE_INPUTS = HipCudaWireModule.philox_engine_inputs
+_DEQUANTIZE = HipCudaWireModule.dequantize
+_INPLACE_DEQUANTIZE = HipCudaWireModule.inplace_dequantize

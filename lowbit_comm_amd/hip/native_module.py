@@ -149,14 +149,25 @@ class HipNativeModule:
         specs = _host.specs(*operands)
         return None if specs is None else (tag, specs, policy)
 
-    # The portable format pads the last group with zeros while it encodes: the facade need not hand over whole groups.
-    _PADS_THE_LAST_GROUP = True
+    # The native calls stand for the public methods that the same request went through: a subclass, a class or an instance
+    # that puts another method in the place of one of them is asked as before.
 
     # ---- quantize ------------------------------------------------------------------------------
+    @property
+    def _PADS_THE_LAST_GROUP(self) -> bool:
+        """The portable format pads the last group with zeros while it encodes: the facade need not hand over whole groups."""
+        return type(self).quantize is _QUANTIZE and "quantize" not in self.__dict__ and self._encodes_natively()
+
+    def _encodes_natively(self) -> bool:
+        cls, held = type(self), self.__dict__
+        return (cls.inplace_quantize is _INPLACE_QUANTIZE and cls.inplace_quantize_pack is _INPLACE_QUANTIZE_PACK
+                and "inplace_quantize" not in held and "inplace_quantize_pack" not in held)
+
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
-        payload = _host.quantize(input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
-        if isinstance(payload, torch.Tensor):
-            return payload
+        if self._encodes_natively():
+            payload = _host.quantize(input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
+            if isinstance(payload, torch.Tensor):
+                return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         output = torch.empty(ops.payload_nbytes(input.numel(), group_size), dtype=torch.uint8, device=input.device)
         self.inplace_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact)
@@ -208,11 +219,18 @@ class HipNativeModule:
     def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
         """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
         all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
+        if type(self).dequantize is not _DEQUANTIZE or "dequantize" in self.__dict__:
+            return None
+        return self._decode(input, shape, group_size, topk, bit, reduce_op, quant_type, dtype)
+
+    def _decode(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype):
+        if type(self).inplace_dequantize is not _INPLACE_DEQUANTIZE or "inplace_dequantize" in self.__dict__:
+            return None
         decoded = _host.dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = self._dequantize_shaped(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
+        decoded = self._decode(input, None, group_size, topk, bit, reduce_op, quant_type, dtype)
         if decoded is not None:
             return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
@@ -254,6 +272,9 @@ class HipNativeModule:
 
     def _dequantize_reduce_shaped(self, inputs, shape, group_size, topk, bit, quant_type, dtype, divisor):
         """Decode and reduce into a fresh tensor of ``shape`` in one native call; ``None`` as in the decode."""
+        cls = type(self)
+        if any(getattr(cls, name) is not own or name in self.__dict__ for name, own in _REDUCES):
+            return None
         reduced = _host.dequantize_reduce(inputs, shape, dtype, group_size, topk, bit, quant_type, divisor,
                                           ops.access_code(None))
         return reduced if isinstance(reduced, torch.Tensor) else None
@@ -405,3 +426,12 @@ class HipNativeModule:
                                                group_size=group_size, divisor=float(divisor),
                                                prepared=prepared.reshape(-1), new_residual=residual.reshape(-1))
         return (self._memoized(key, bind) if key is not None else bind())()
+
+
+_QUANTIZE = HipNativeModule.quantize
+_INPLACE_QUANTIZE = HipNativeModule.inplace_quantize
+_INPLACE_QUANTIZE_PACK = HipNativeModule.inplace_quantize_pack
+_DEQUANTIZE = HipNativeModule.dequantize
+_INPLACE_DEQUANTIZE = HipNativeModule.inplace_dequantize
+_REDUCES = tuple((name, getattr(HipNativeModule, name)) for name in (
+    "dequantize_reduce", "dequantize_reduce_mean", "inplace_dequantize_reduce", "inplace_dequantize_reduce_mean"))

@@ -62,3 +62,65 @@ def test_bound_launch_takes_a_stream_and_nothing_else():
     for args, kwargs in (((0, 0), {}), ((), {"streams": 0}), ((0,), {"stream": 0}), (("0",), {})):
         with pytest.raises(TypeError):
             launch(*args, **kwargs)
+
+
+def modules():
+    from lowbit_comm_amd.hip.cuda_wire_module import HipCudaWireModule
+    from lowbit_comm_amd.hip.native_module import HipNativeModule
+
+    return {"portable": HipNativeModule, "native": HipCudaWireModule}
+
+
+# what the facade's allocating calls go through, method by method
+CHAINS = [("portable", name, call) for call, names in {
+    "quantize": ("quantize", "inplace_quantize", "inplace_quantize_pack"),
+    "dequantize": ("dequantize", "inplace_dequantize"),
+    "sum": ("dequantize_reduce", "inplace_dequantize_reduce"),
+    "mean": ("dequantize_reduce_mean", "inplace_dequantize_reduce_mean")}.items() for name in names] + [
+    ("native", name, call) for call, names in {
+        "quantize": ("quantize", "inplace_quantize"), "compensate": ("quantize", "inplace_quantize"),
+        "stochastic": ("philox_engine_inputs",), "dequantize": ("dequantize", "inplace_dequantize")}.items() for name in names]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("way", ["subclass", "class", "instance"])
+@pytest.mark.parametrize("wire, name, call", CHAINS)
+def test_a_replaced_method_is_asked(hip_device, monkeypatch, wire, name, call, way):
+    from lowbit_comm_amd import CompressionConfig
+    from lowbit_comm_amd.hip.loader import HipExtensionStatus, load_hip_extension
+    from lowbit_comm_amd.quantization.codec import (compensate_and_quantize, dequantize_reduce_tensors, dequantize_tensor,
+                                                    quantize_tensor)
+
+    config = CompressionConfig(stochastic=call == "stochastic", allow_experimental=call == "stochastic")
+    x = values(100 if wire == "portable" else 128, torch.float32, 1).to(hip_device)
+    payload = quantize_tensor(x, CompressionConfig(), extension_status=load_hip_extension(wire_format=wire))
+    cls, asked = modules()[wire], []
+    before = cls.__dict__[name]
+    own = before.__func__ if isinstance(before, staticmethod) else before
+
+    def spy(*args, **kwargs):
+        asked.append(args[1] if isinstance(args[0], cls) else args[0])
+        return own(*args, **kwargs)
+
+    spy_of_class = staticmethod(spy) if isinstance(before, staticmethod) else spy
+    if way == "subclass":
+        module = type("Sub", (cls,), {name: spy_of_class})()
+    else:
+        module = cls()
+        if way == "class":
+            monkeypatch.setattr(cls, name, spy_of_class)
+        else:
+            monkeypatch.setattr(module, name, spy if isinstance(before, staticmethod) else spy.__get__(module))
+    status = HipExtensionStatus(available=True, module=module)
+    if call in ("quantize", "stochastic"):
+        quantize_tensor(x, config, extension_status=status)
+    elif call == "compensate":
+        assert compensate_and_quantize(x, x, config, extension_status=status) is None
+        asked.append(None)
+    elif call == "dequantize":
+        dequantize_tensor(payload, tuple(x.shape), config, dtype="fp32", extension_status=status)
+    else:
+        dequantize_reduce_tensors([payload, payload], tuple(x.shape), config, dtype="fp32", extension_status=status, reduce=call)
+    assert len(asked) == 1
+    if call == "quantize":
+        assert asked[0].numel() == 128          # whole groups, as every module but the one that pads by itself gets them
