@@ -149,6 +149,12 @@ class HipNativeModule:
         specs = _host.specs(*operands)
         return None if specs is None else (tag, specs, policy)
 
+    @classmethod
+    def _reduce_key(cls, tag, policy, inputs, *operands):
+        """:meth:`_key` of a call on several payloads.  The rows of one tensor are payloads too, but its address and
+        element count do not say how many: such a call has no key."""
+        return cls._key(tag, policy, inputs, *operands) if isinstance(inputs, (list, tuple)) else None
+
     # The native calls stand for the public methods that the same request went through: a subclass, a class or an instance
     # that puts another method in the place of one of them is asked as before.
 
@@ -311,7 +317,7 @@ class HipNativeModule:
         _check_payload(inputs[0], "input")
         flat = output.reshape(-1)
         numel = min(flat.numel(), _padded_numel_of(inputs[0], group_size))
-        key = self._key("reduce", (group_size, topk, bit, int(quant_type), numel), inputs, flat)
+        key = self._reduce_key("reduce", (group_size, topk, bit, int(quant_type), numel), inputs, flat)
         bound = self._recall(key)
         if bound is not None:
             if not bound():
@@ -351,7 +357,7 @@ class HipNativeModule:
                                        divisor) -> bool:
         if divisor <= 0:
             raise RuntimeError("divisor must be > 0")
-        key = self._key("reduce_mean", (group_size, topk, bit, int(quant_type), float(divisor)), inputs, output)
+        key = self._reduce_key("reduce_mean", (group_size, topk, bit, int(quant_type), float(divisor)), inputs, output)
         bound = self._recall(key)
         if bound is None:
             if not self._fused_eligible(inputs, output, group_size, topk, bit, quant_type):
@@ -392,8 +398,8 @@ class HipNativeModule:
         """One launch: ``restored = mean/sum of payloads``, ``residual = prepared - restored``."""
         if divisor <= 0:
             raise RuntimeError("divisor must be > 0")
-        key = self._key("reduce_mean_feedback", (group_size, topk, bit, int(quant_type), float(divisor)),
-                        inputs, prepared, restored, residual)
+        key = self._reduce_key("reduce_mean_feedback", (group_size, topk, bit, int(quant_type), float(divisor)),
+                               inputs, prepared, restored, residual)
         bound = self._recall(key)
         if bound is not None:
             return bound()

@@ -124,3 +124,26 @@ def test_a_replaced_method_is_asked(hip_device, monkeypatch, wire, name, call, w
     assert len(asked) == 1
     if call == "quantize":
         assert asked[0].numel() == 128          # whole groups, as every module but the one that pads by itself gets them
+
+
+# the payloads of a reduce may be the rows of one tensor; another number of rows over the same bytes is another call
+@pytest.mark.gpu
+def test_rows_of_one_tensor_are_counted_on_every_call(hip_device):
+    from lowbit_comm_amd import CompressionConfig, quantize_tensor
+
+    module = modules()["portable"]()
+    n, config = 256, CompressionConfig()
+    rows = torch.stack([quantize_tensor(values(n, torch.float32, seed).to(hip_device), config) for seed in range(4)])
+    policy = (64, 0, 8, module.QuantType.Linear)
+    listed, out = torch.empty(64, device=hip_device), torch.empty(64, device=hip_device)
+    for view in (rows.view(2, -1), rows, rows.view(2, -1), rows.view(8, -1)):
+        module.inplace_dequantize_reduce(list(view), listed, *policy, False)
+        module.inplace_dequantize_reduce(view, out, *policy, False)
+        assert torch.equal(out, listed), tuple(view.shape)
+    whole, feedback = torch.empty(n, device=hip_device), torch.empty(n, device=hip_device)
+    for _ in range(2):
+        assert module.inplace_dequantize_reduce_mean(rows, whole, *policy, False, 4)
+        assert not module.inplace_dequantize_reduce_mean(rows.view(2, -1), whole, *policy, False, 4)
+        fused = module.inplace_dequantize_reduce_mean_update_error_feedback
+        assert fused(rows, whole, whole, feedback, *policy, False, 4)
+        assert not fused(rows.view(2, -1), whole, whole, feedback, *policy, False, 4)
