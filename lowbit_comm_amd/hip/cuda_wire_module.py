@@ -76,7 +76,9 @@ class HipCudaWireModule:
     def __init__(self, fused_multiply_add: bool = True) -> None:
         """``fused_multiply_add``: accumulate the fused reduce as ``fma(code, step, sum)`` (what nvcc's default
         contraction makes of the reference source) or with a separately rounded product."""
+        global _host
         self._lib = load_library()
+        _host = native_host()       # built after this module was imported, it may be
         self.fused_multiply_add = bool(fused_multiply_add)
 
     # ---- quantize ------------------------------------------------------------------------------

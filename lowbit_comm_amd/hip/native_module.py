@@ -96,7 +96,9 @@ class HipNativeModule:
     NATIVE_WIRE_FORMAT = "portable"
 
     def __init__(self) -> None:
+        global _host
         self._lib = load_library()
+        _host = native_host()       # built after this module was imported, it may be
         # Launches of the allocation-free entry points, bound to the addresses they were last called with.  A DDP
         # hook presents the same bucket, payload and workspace addresses every step, so from the second step on a
         # call is one key lookup and one ABI call.  The key holds everything a binding depends on (addresses,

@@ -148,10 +148,22 @@ def current_stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+class _LaunchOfLaterBuild:
+    """``_host.Launch`` for a process that imported this package before the native parts were built."""
+
+    __slots__ = ("_launch",)
+
+    def __init__(self, entry: str, args: tuple, device: int) -> None:
+        self._launch = native_host().Launch(entry, args, device)
+
+    def __call__(self, stream: int | None = None) -> bool:
+        return self._launch(stream)
+
+
 _host = native_host()
 
 
-class BoundLaunch(_host.Launch if _host is not None else object):
+class BoundLaunch(_LaunchOfLaterBuild if _host is None else _host.Launch):
     """One ABI call with every argument validated and marshalled ahead of time.
 
     Calling it enqueues the kernel on torch's current stream of the tensors' device and returns

@@ -147,3 +147,40 @@ def test_rows_of_one_tensor_are_counted_on_every_call(hip_device):
         fused = module.inplace_dequantize_reduce_mean_update_error_feedback
         assert fused(rows, whole, whole, feedback, *policy, False, 4)
         assert not fused(rows.view(2, -1), whole, whole, feedback, *policy, False, 4)
+
+
+# the package may be imported first and built afterwards, in one process
+def test_a_build_after_the_import_is_picked_up():
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    script = """
+import sys, torch
+class NotBuilt:
+    def find_spec(self, name, path=None, target=None):
+        if name == "lowbit_comm_amd._host":
+            raise ImportError("not built")
+sys.meta_path.insert(0, NotBuilt())
+import lowbit_comm_amd
+from lowbit_comm_amd.exceptions import CCDLUnavailableError
+from lowbit_comm_amd.hip import cuda_wire_module, library, native_module, ops
+nothing = ("lbc_quant_pack", (None, 0, None, -1, 0, 64, None, None, None, -1, None, 0, None, -1, 0), torch.device("cuda:0"), ())
+for make in (native_module.HipNativeModule, cuda_wire_module.HipCudaWireModule, lambda: ops.BoundLaunch(*nothing)):
+    try:
+        make()
+        raise SystemExit("made without its native part")
+    except CCDLUnavailableError as exc:
+        assert "not built" in str(exc)
+del sys.meta_path[0]
+assert ops.BoundLaunch(*nothing)(0) is True
+for module in (native_module.HipNativeModule(), cuda_wire_module.HipCudaWireModule()):
+    try:
+        module.quantize(torch.zeros(64), 64, 0, False, 8, module.QuantType.Linear, False)
+        raise SystemExit("a CPU tensor was taken")
+    except RuntimeError as exc:
+        assert "GPU tensor" in str(exc), exc
+"""
+    done = subprocess.run([sys.executable, "-c", script], cwd=Path(__file__).resolve().parent.parent, capture_output=True, text=True,
+                          timeout=100)
+    assert done.returncode == 0, done.stderr
