@@ -154,6 +154,9 @@ def _annotate(hook: Callable[[Any, Any], Any], provider: Callable[[], dict[str, 
         pass
 
 
+_COMPENSATE, _RESIDUAL_OF = ErrorFeedbackState.compensate, ErrorFeedbackState.get
+
+
 def create_ddp_comm_hook(
     config: CompressionConfig,
     *,
@@ -265,11 +268,15 @@ def create_ddp_comm_hook(
         return prepared, buffer
 
     # The CUDA extension's format has the same fusion with both outputs freshly allocated, as the sum and the payload of
-    # the two separate calls are.  A feedback state with a compensate step of its own keeps that step.
-    plain_compensate = quantize is None and getattr(type(feedback), "compensate", None) is ErrorFeedbackState.compensate
+    # the two separate calls are.  A feedback state whose compensate step, or the look-up of a residual, is its own keeps
+    # that step.
+    def plain_compensate() -> bool:
+        cls, held = type(feedback), getattr(feedback, "__dict__", {})
+        return (getattr(cls, "compensate", None) is _COMPENSATE and getattr(cls, "get", None) is _RESIDUAL_OF
+                and "compensate" not in held and "get" not in held)
 
     def fresh_sum_and_payload(key: Any, original: Any) -> tuple[Any, Any] | None:
-        residual = feedback.get(key) if plain_compensate else None
+        residual = feedback.get(key) if quantize is None and plain_compensate() else None
         if residual is None:
             return None
         return compensate_and_quantize_in_one_launch(original, residual, config, extension_status=extension_status)

@@ -184,3 +184,42 @@ for module in (native_module.HipNativeModule(), cuda_wire_module.HipCudaWireModu
     done = subprocess.run([sys.executable, "-c", script], cwd=Path(__file__).resolve().parent.parent, capture_output=True, text=True,
                           timeout=100)
     assert done.returncode == 0, done.stderr
+
+
+# the hook's one launch for bucket + residual stands for ErrorFeedbackState.compensate, which looks the residual up itself
+@pytest.mark.parametrize("way", ["plain", "subclass", "class", "instance"])
+@pytest.mark.parametrize("name", ["compensate", "get"])
+def test_a_feedback_state_of_its_own_keeps_its_compensate_step(monkeypatch, name, way):
+    from lowbit_comm_amd import CompressionConfig
+    from lowbit_comm_amd.communication import ddp_hook
+    from lowbit_comm_amd.communication.gather_reduce import GatheredPayloads
+    from lowbit_comm_amd.hip.loader import HipExtensionStatus
+    from lowbit_comm_amd.quantization.error_feedback import ErrorFeedbackState
+
+    launched = []
+    monkeypatch.setattr(ddp_hook, "compensate_and_quantize_in_one_launch", lambda *a, **k: launched.append(a))
+    monkeypatch.setattr(ddp_hook, "quantize_tensor", lambda tensor, *a, **k: torch.zeros(68, dtype=torch.uint8))
+    monkeypatch.setattr(ddp_hook, "dequantize_reduce_tensors", lambda *a, **k: torch.zeros(64))
+    own = {"compensate": ErrorFeedbackState.compensate, "get": ErrorFeedbackState.get}[name]
+    replacement = lambda self, *args: own(self, *args)  # noqa: E731
+    feedback = (type("Own", (ErrorFeedbackState,), {name: replacement}) if way == "subclass" else ErrorFeedbackState)()
+    if way == "instance":
+        monkeypatch.setattr(feedback, name, replacement.__get__(feedback))
+    elif way == "class":
+        monkeypatch.setattr(ErrorFeedbackState, name, replacement)
+    feedback.put(0, torch.ones(64))
+
+    class Bucket:
+        def index(self):
+            return 0
+
+        def buffer(self):
+            return torch.ones(64)
+
+    hook = ddp_hook.create_ddp_comm_hook(
+        CompressionConfig(error_feedback=True), strategy="all_gather", error_feedback=feedback,
+        extension_status=HipExtensionStatus(available=True, module=object()),
+        native_inplace_dequantize_reduce_update_feedback=lambda *a, **k: False,
+        all_gather=lambda local: GatheredPayloads([local.buffer], 1))
+    hook(None, Bucket())
+    assert len(launched) == (way == "plain")
