@@ -281,7 +281,9 @@ class HipNativeModule:
     def _dequantize_reduce_shaped(self, inputs, shape, group_size, topk, bit, quant_type, dtype, divisor):
         """Decode and reduce into a fresh tensor of ``shape`` in one native call; ``None`` as in the decode."""
         cls = type(self)
-        if any(getattr(cls, name) is not own or name in self.__dict__ for name, own in _REDUCES):
+        if (cls.dequantize_reduce is not _REDUCE or cls.dequantize_reduce_mean is not _REDUCE_MEAN
+                or cls.inplace_dequantize_reduce is not _INPLACE_REDUCE
+                or cls.inplace_dequantize_reduce_mean is not _INPLACE_REDUCE_MEAN or not _REDUCES.isdisjoint(self.__dict__)):
             return None
         reduced = _host.dequantize_reduce(inputs, shape, dtype, group_size, topk, bit, quant_type, divisor,
                                           ops.access_code(None))
@@ -441,5 +443,7 @@ _INPLACE_QUANTIZE = HipNativeModule.inplace_quantize
 _INPLACE_QUANTIZE_PACK = HipNativeModule.inplace_quantize_pack
 _DEQUANTIZE = HipNativeModule.dequantize
 _INPLACE_DEQUANTIZE = HipNativeModule.inplace_dequantize
-_REDUCES = tuple((name, getattr(HipNativeModule, name)) for name in (
-    "dequantize_reduce", "dequantize_reduce_mean", "inplace_dequantize_reduce", "inplace_dequantize_reduce_mean"))
+_REDUCE, _REDUCE_MEAN = HipNativeModule.dequantize_reduce, HipNativeModule.dequantize_reduce_mean
+_INPLACE_REDUCE = HipNativeModule.inplace_dequantize_reduce
+_INPLACE_REDUCE_MEAN = HipNativeModule.inplace_dequantize_reduce_mean
+_REDUCES = frozenset(("dequantize_reduce", "dequantize_reduce_mean", "inplace_dequantize_reduce", "inplace_dequantize_reduce_mean"))
