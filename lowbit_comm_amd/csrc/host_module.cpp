@@ -263,10 +263,28 @@ PyObject *elsewhere() {
     Py_RETURN_NONE;
 }
 
+// The calls below stand for public methods of a codec module, which a subclass, a patched class or an instance may have
+// replaced.  Their first two arguments are the module and a table (name, attribute, name, attribute, ...) of the methods
+// that the call by-passes: it is made only when the module's class has exactly these attributes and the module itself holds
+// none of them.  (Here, because the same test in Python costs a small call 0.1 us.)
+bool owns(PyObject *module, PyObject *table) {
+    if (!PyTuple_Check(table)) return false;
+    PyObject **held = _PyObject_GetDictPtr(module);
+    for (Py_ssize_t i = 0; i + 1 < PyTuple_GET_SIZE(table); i += 2) {
+        PyObject *name = PyTuple_GET_ITEM(table, i);
+        if (_PyType_Lookup(Py_TYPE(module), name) != PyTuple_GET_ITEM(table, i + 1)) return false;
+        if (held != nullptr && *held != nullptr && PyDict_GetItemWithError(*held, name) != nullptr) return false;
+    }
+    return !PyErr_Occurred();
+}
+
 // ---- the portable format ---------------------------------------------------------------------------------------
-// quantize(input, group_size, topk, stochastic, bit, quant_type, access) -> payload
+// quantize(module, table, input, group_size, topk, stochastic, bit, quant_type, access) -> payload
 PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p;
     long access;
     if (n != 7 || !integer(a[1], p.group) || !integer(a[2], p.topk) || !integer(a[3], p.stochastic) || !integer(a[4], p.bit) ||
@@ -308,10 +326,13 @@ bool sizes_of(PyObject *o, int64_t all, c10::SmallVector<int64_t, 5> &sizes, int
     return true;
 }
 
-// dequantize(payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, access) -> tensor of that shape (None:
+// dequantize(module, table, payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, access) -> tensor of that shape (None:
 // flat, every element the payload holds)
 PyObject *dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p{};
     long dtype, op, access;
     if (n != 9 || !integer(a[2], dtype) || !integer(a[3], p.group) || !integer(a[4], p.topk) || !integer(a[5], p.bit) ||
@@ -365,9 +386,12 @@ int payloads_of(PyObject *list, int64_t &nbytes, const uint8_t **pointers, const
     return static_cast<int>(count);
 }
 
-// dequantize_reduce(payloads, shape, dtype, group_size, topk, bit, quant_type, divisor, access) -> tensor, as dequantize
+// dequantize_reduce(module, table, payloads, shape, dtype, group_size, topk, bit, quant_type, divisor, access) -> tensor, as dequantize
 PyObject *dequantize_reduce(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p{};
     long dtype, access;
     if (n != 9 || !integer(a[2], dtype) || !integer(a[3], p.group) || !integer(a[4], p.topk) || !integer(a[5], p.bit) ||
@@ -422,9 +446,12 @@ std::pair<uint64_t, uint64_t> philox_inputs(const at::Tensor &x, uint64_t increm
     return {generator.current_seed(), offset};
 }
 
-// wire_quantize(input, output or None, group_size, topk, stochastic, bit, quant_type, compact, access) -> payload
+// wire_quantize(module, table, input, output or None, group_size, topk, stochastic, bit, quant_type, compact, access) -> payload
 PyObject *wire_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p;
     long compact, access;
     if (n != 9 || !integer(a[2], p.group) || !integer(a[3], p.topk) || !integer(a[4], p.stochastic) || !integer(a[5], p.bit) ||
@@ -459,10 +486,13 @@ PyObject *wire_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// wire_compensate_quantize(x, residual, group_size, topk, stochastic, bit, quant_type, compact, access) -> (x + residual, its
+// wire_compensate_quantize(module, table, x, residual, group_size, topk, stochastic, bit, quant_type, compact, access) -> (x + residual, its
 // payload), both from one launch.  Plain codes; operands of one type, one shape and one device that autograd does not watch.
 PyObject *wire_compensate_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p;
     long compact, access;
     if (n != 9 || !integer(a[2], p.group) || !integer(a[3], p.topk) || !integer(a[4], p.stochastic) || !integer(a[5], p.bit) ||
@@ -494,10 +524,13 @@ PyObject *wire_compensate_quantize(PyObject *, PyObject *const *a, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
-// wire_dequantize(payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact, access) -> tensor of that
+// wire_dequantize(module, table, payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact, access) -> tensor of that
 // shape (None: flat, every element the payload holds)
 PyObject *wire_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
+    if (n < 2 || !owns(a[0], a[1])) return elsewhere();
+    a += 2;
+    n -= 2;
     Policy p{};
     long dtype, op, compact, access;
     if (n != 10 || !integer(a[2], dtype) || !integer(a[3], p.group) || !integer(a[4], p.topk) || !integer(a[5], p.bit) ||
@@ -611,6 +644,13 @@ PyObject *specs(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// own(object, table) -> whether a native call may stand for the object's methods in the table.
+PyObject *own(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n == 2 && owns(a[0], a[1])) Py_RETURN_TRUE;
+    PyErr_Clear();
+    Py_RETURN_FALSE;
+}
+
 PyObject *abi_version(PyObject *, PyObject *) { return PyLong_FromLong(lbc_abi_version() == LBC_ABI_VERSION ? LBC_ABI_VERSION : -1); }
 
 PyMethodDef kMethods[] = {
@@ -622,6 +662,7 @@ PyMethodDef kMethods[] = {
     {"wire_quantize", reinterpret_cast<PyCFunction>(wire_quantize), METH_FASTCALL, "Quantize into a payload of the CUDA extension's format."},
     {"wire_dequantize", reinterpret_cast<PyCFunction>(wire_dequantize), METH_FASTCALL, "Decode a payload of that format into a fresh tensor."},
     {"wire_reduce", reinterpret_cast<PyCFunction>(wire_reduce), METH_FASTCALL, "Fused reduce of payloads of that format, optionally with the residual update."},
+    {"own", reinterpret_cast<PyCFunction>(own), METH_FASTCALL, "Are the methods in a table the module's own?"},
     {"specs", reinterpret_cast<PyCFunction>(specs), METH_FASTCALL, "Addresses, types and element counts of contiguous GPU tensors."},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -25,7 +25,8 @@ import torch
 
 from lowbit_comm_amd.hip import cuda_wire, ops
 from lowbit_comm_amd.hip.library import load_library, native_host
-from lowbit_comm_amd.hip.native_module import DType, QuantType, ReduceOP, _OP_NAME, _TORCH_OF, _check_payload
+from lowbit_comm_amd.hip.native_module import (DType, QuantType, ReduceOP, _OP_NAME, _TORCH_OF, _check_payload,
+                                               own_methods)
 
 _host = native_host()
 
@@ -82,23 +83,13 @@ class HipCudaWireModule:
         self.fused_multiply_add = bool(fused_multiply_add)
 
     # ---- quantize ------------------------------------------------------------------------------
-    # The native calls stand for the public methods that the same request went through: a subclass, a class or an instance
-    # that puts another method in the place of one of them is asked as before.
-    def _encodes_natively(self, stochastic) -> bool:
-        cls, held = type(self), self.__dict__
-        return (cls.inplace_quantize is _INPLACE_QUANTIZE and "inplace_quantize" not in held
-                and (not stochastic or self._draws_natively()))
-
-    def _draws_natively(self) -> bool:
-        return (type(self).philox_engine_inputs is _PHILOX_ENGINE_INPUTS
-                and "philox_engine_inputs" not in self.__dict__)
-
+    # The native calls stand for the public methods that the same request would go through, which they are told: where a
+    # subclass, a patched class or an instance puts another method in the place of one of them, that one is asked.
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
-        if self._encodes_natively(stochastic):
-            payload = _host.wire_quantize(input, None, group_size, topk, stochastic, bit, quant_type, compact,
-                                          ops.access_code(None))
-            if isinstance(payload, torch.Tensor):
-                return payload
+        payload = _host.wire_quantize(self, _ENCODES_WITH_NOISE if stochastic else _ENCODES, input, None, group_size, topk,
+                                      stochastic, bit, quant_type, compact, ops.access_code(None))
+        if isinstance(payload, torch.Tensor):
+            return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         nbytes = cuda_wire.general_payload_nbytes(input.numel(), input.dtype, group_size, bit, topk)
         output = torch.empty(nbytes, dtype=torch.uint8, device=input.device)
@@ -106,9 +97,9 @@ class HipCudaWireModule:
         return output
 
     def inplace_quantize(self, input, output, group_size, topk, stochastic, bit, quant_type, compact) -> None:
-        if output is not None and (not stochastic or self._draws_natively()) and isinstance(
-                _host.wire_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact,
-                                    ops.access_code(None)), torch.Tensor):
+        if output is not None and isinstance(
+                _host.wire_quantize(self, _DRAWS if stochastic else (), input, output, group_size, topk, stochastic, bit,
+                                    quant_type, compact, ops.access_code(None)), torch.Tensor):
             return
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         if _plain(topk, stochastic, quant_type):
@@ -121,10 +112,8 @@ class HipCudaWireModule:
     def _compensate_quantize(self, input, residual, group_size, topk, stochastic, bit, quant_type, compact):
         """``(input + residual, the payload quantize() makes of it)`` from one launch, both freshly allocated, or ``None``
         when there is no such launch (another policy, operands of different types or shapes)."""
-        if type(self).quantize is not _QUANTIZE or "quantize" in self.__dict__ or not self._encodes_natively(stochastic):
-            return None
-        pair = _host.wire_compensate_quantize(input, residual, group_size, topk, stochastic, bit, quant_type, compact,
-                                              ops.access_code(None))
+        pair = _host.wire_compensate_quantize(self, _QUANTIZES, input, residual, group_size, topk, stochastic, bit,
+                                              quant_type, compact, ops.access_code(None))
         return pair if isinstance(pair, tuple) else None
 
     @staticmethod
@@ -192,20 +181,14 @@ class HipCudaWireModule:
     def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
         """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
         all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
-        if type(self).dequantize is not _DEQUANTIZE or "dequantize" in self.__dict__:
-            return None
-        return self._decode(input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
-
-    def _decode(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        if type(self).inplace_dequantize is not _INPLACE_DEQUANTIZE or "inplace_dequantize" in self.__dict__:
-            return None
-        decoded = _host.wire_dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact,
-                                        ops.access_code(None))
+        decoded = _host.wire_dequantize(self, _DEQUANTIZES, input, shape, dtype, group_size, topk, bit, reduce_op,
+                                        quant_type, compact, ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = self._decode(input, None, group_size, topk, bit, reduce_op, quant_type, dtype, compact)
-        if decoded is not None:
+        decoded = _host.wire_dequantize(self, _DECODES, input, None, dtype, group_size, topk, bit, reduce_op, quant_type,
+                                        compact, ops.access_code(None))
+        if isinstance(decoded, torch.Tensor):
             return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
         _check_payload(input, "input")
@@ -336,8 +319,8 @@ class HipCudaWireModule:
         return restored
 
 
-_QUANTIZE = HipCudaWireModule.quantize
-_INPLACE_QUANTIZE = HipCudaWireModule.inplace_quantize
-_PHILOX_ENGINE_INPUTS = HipCudaWireModule.philox_engine_inputs
-_DEQUANTIZE = HipCudaWireModule.dequantize
-_INPLACE_DEQUANTIZE = HipCudaWireModule.inplace_dequantize
+_QUANTIZES = own_methods(HipCudaWireModule, "quantize", "inplace_quantize")
+_DEQUANTIZES = own_methods(HipCudaWireModule, "dequantize", "inplace_dequantize")
+_DRAWS = own_methods(HipCudaWireModule, "philox_engine_inputs")
+_ENCODES, _DECODES = _QUANTIZES[2:], _DEQUANTIZES[2:]
+_ENCODES_WITH_NOISE = _ENCODES + _DRAWS

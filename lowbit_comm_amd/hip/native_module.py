@@ -87,6 +87,11 @@ def _views(buffer: torch.Tensor, group_size: int):
     return flat[:padded].view(torch.int8), flat[padded:].view(torch.float32)
 
 
+def own_methods(cls: type, *names: str) -> tuple:
+    """``(name, attribute, ...)`` of a module class as the native calls take them."""
+    return tuple(part for name in names for part in (name, cls.__dict__[name]))
+
+
 class HipNativeModule:
     """Instance with the reference extension's symbols; constructing it loads (and type-checks) the library."""
 
@@ -157,25 +162,24 @@ class HipNativeModule:
         element count do not say how many: such a call has no key."""
         return cls._key(tag, policy, inputs, *operands) if isinstance(inputs, (list, tuple)) else None
 
-    # The native calls stand for the public methods that the same request went through: a subclass, a class or an instance
-    # that puts another method in the place of one of them is asked as before.
+    # The native calls stand for the public methods that the same request would go through, which they are told: where a
+    # subclass, a patched class or an instance puts another method in the place of one of them, that one is asked.
 
     # ---- quantize ------------------------------------------------------------------------------
     @property
     def _PADS_THE_LAST_GROUP(self) -> bool:
         """The portable format pads the last group with zeros while it encodes: the facade need not hand over whole groups."""
-        return type(self).quantize is _QUANTIZE and "quantize" not in self.__dict__ and self._encodes_natively()
+        return _host.own(self, _QUANTIZES)
 
-    def _encodes_natively(self) -> bool:
-        cls, held = type(self), self.__dict__
-        return (cls.inplace_quantize is _INPLACE_QUANTIZE and cls.inplace_quantize_pack is _INPLACE_QUANTIZE_PACK
-                and "inplace_quantize" not in held and "inplace_quantize_pack" not in held)
+    def _quantize_directly(self, input, group_size, topk, stochastic, bit, quant_type, compact):
+        """The payload of a contiguous GPU tensor of any length in one native call, or ``None`` for any other request."""
+        payload = _host.quantize(self, _QUANTIZES, input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
+        return payload if isinstance(payload, torch.Tensor) else None
 
     def quantize(self, input, group_size, topk, stochastic, bit, quant_type, compact):
-        if self._encodes_natively():
-            payload = _host.quantize(input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
-            if isinstance(payload, torch.Tensor):
-                return payload
+        payload = _host.quantize(self, _ENCODES, input, group_size, topk, stochastic, bit, quant_type, ops.access_code(None))
+        if isinstance(payload, torch.Tensor):
+            return payload
         _require_policy(group_size, topk, stochastic, bit, quant_type)
         output = torch.empty(ops.payload_nbytes(input.numel(), group_size), dtype=torch.uint8, device=input.device)
         self.inplace_quantize(input, output, group_size, topk, stochastic, bit, quant_type, compact)
@@ -227,19 +231,14 @@ class HipNativeModule:
     def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
         """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
         all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
-        if type(self).dequantize is not _DEQUANTIZE or "dequantize" in self.__dict__:
-            return None
-        return self._decode(input, shape, group_size, topk, bit, reduce_op, quant_type, dtype)
-
-    def _decode(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype):
-        if type(self).inplace_dequantize is not _INPLACE_DEQUANTIZE or "inplace_dequantize" in self.__dict__:
-            return None
-        decoded = _host.dequantize(input, shape, dtype, group_size, topk, bit, reduce_op, quant_type, ops.access_code(None))
+        decoded = _host.dequantize(self, _DEQUANTIZES, input, shape, dtype, group_size, topk, bit, reduce_op, quant_type,
+                                   ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = self._decode(input, None, group_size, topk, bit, reduce_op, quant_type, dtype)
-        if decoded is not None:
+        decoded = _host.dequantize(self, _DECODES, input, None, dtype, group_size, topk, bit, reduce_op, quant_type,
+                                   ops.access_code(None))
+        if isinstance(decoded, torch.Tensor):
             return decoded
         _require_policy(group_size, topk, False, bit, quant_type)
         _check_payload(input, "input")
@@ -280,12 +279,7 @@ class HipNativeModule:
 
     def _dequantize_reduce_shaped(self, inputs, shape, group_size, topk, bit, quant_type, dtype, divisor):
         """Decode and reduce into a fresh tensor of ``shape`` in one native call; ``None`` as in the decode."""
-        cls = type(self)
-        if (cls.dequantize_reduce is not _REDUCE or cls.dequantize_reduce_mean is not _REDUCE_MEAN
-                or cls.inplace_dequantize_reduce is not _INPLACE_REDUCE
-                or cls.inplace_dequantize_reduce_mean is not _INPLACE_REDUCE_MEAN or not _REDUCES.isdisjoint(self.__dict__)):
-            return None
-        reduced = _host.dequantize_reduce(inputs, shape, dtype, group_size, topk, bit, quant_type, divisor,
+        reduced = _host.dequantize_reduce(self, _REDUCES, inputs, shape, dtype, group_size, topk, bit, quant_type, divisor,
                                           ops.access_code(None))
         return reduced if isinstance(reduced, torch.Tensor) else None
 
@@ -438,12 +432,7 @@ class HipNativeModule:
         return (self._memoized(key, bind) if key is not None else bind())()
 
 
-_QUANTIZE = HipNativeModule.quantize
-_INPLACE_QUANTIZE = HipNativeModule.inplace_quantize
-_INPLACE_QUANTIZE_PACK = HipNativeModule.inplace_quantize_pack
-_DEQUANTIZE = HipNativeModule.dequantize
-_INPLACE_DEQUANTIZE = HipNativeModule.inplace_dequantize
-_REDUCE, _REDUCE_MEAN = HipNativeModule.dequantize_reduce, HipNativeModule.dequantize_reduce_mean
-_INPLACE_REDUCE = HipNativeModule.inplace_dequantize_reduce
-_INPLACE_REDUCE_MEAN = HipNativeModule.inplace_dequantize_reduce_mean
-_REDUCES = frozenset(("dequantize_reduce", "dequantize_reduce_mean", "inplace_dequantize_reduce", "inplace_dequantize_reduce_mean"))
+_QUANTIZES, _DEQUANTIZES, _REDUCES = (own_methods(HipNativeModule, *names) for names in (
+    ("quantize", "inplace_quantize", "inplace_quantize_pack"), ("dequantize", "inplace_dequantize"),
+    ("dequantize_reduce", "dequantize_reduce_mean", "inplace_dequantize_reduce", "inplace_dequantize_reduce_mean")))
+_ENCODES, _DECODES = _QUANTIZES[2:], _DEQUANTIZES[2:]

@@ -72,10 +72,9 @@ def _padded_numel(numel: int, group_size: int) -> int:
 
 def _zero_padded(tensor: Any, group_size: int) -> Any:
     """Flat copy padded with zeros to a whole number of groups; the tensor itself when already whole."""
-    if not (hasattr(tensor, "numel") and hasattr(tensor, "reshape")):
-        return tensor
-    missing = -tensor.numel() % group_size
-    if missing == 0:
+    numel = getattr(tensor, "numel", None)
+    missing = -numel() % group_size if numel is not None else 0
+    if missing == 0 or not hasattr(tensor, "reshape"):
         return tensor
     import torch
 
@@ -192,11 +191,16 @@ def quantize_tensor(tensor: object, config: CompressionConfig, *, extension_stat
     if output is not None and _try_quantize_pack(module, tensor, output, residual, config, metadata, quant_type):
         return output
     prepared = tensor if residual is None else tensor + residual
+    policy = (config.group_size, config.topk, config.stochastic, config.bit, quant_type, config.compact)
+    direct = getattr(module, "_quantize_directly", None)
+    if direct is not None and output is None:      # a module that takes any length as it is: nothing to pad first
+        payload = direct(prepared, *policy)
+        if payload is not None:
+            return payload
     # A strided tensor is flattened by the padding: modules take contiguous operands only.
     contiguous = getattr(prepared, "is_contiguous", None)
     if output is not None or not getattr(module, "_PADS_THE_LAST_GROUP", False) or contiguous is None or not contiguous():
         prepared = _zero_padded(prepared, config.group_size)
-    policy = (config.group_size, config.topk, config.stochastic, config.bit, quant_type, config.compact)
     if output is not None:
         _symbol(module, "inplace_quantize")(prepared, output, *policy)
         return output
