@@ -25,13 +25,10 @@ def hip_device():
     return torch.device("cuda:0")
 
 
-@pytest.fixture(autouse=True)
-def steady_allocator_counter(request):
-    """A test that compares readings of the allocator's counter starts without garbage of earlier tests and holds the cycle
-    collector off: tensors of theirs that it frees between two readings are not what the test is about."""
-    if "memory_allocated" not in request.function.__code__.co_names:
-        yield
-        return
+@pytest.fixture
+def steady_allocator_counter():
+    """For a test that compares readings of the allocator's counter: it starts without garbage of earlier tests and holds the
+    cycle collector off, because tensors of theirs that it frees between two readings are not what the test is about."""
     gc.collect()
     gc.disable()
     try:

@@ -73,6 +73,12 @@ static uint16_t to_bf16(float f) {   // round to nearest even; the inputs here a
     memcpy(&bits, &f, 4);
     return static_cast<uint16_t>((bits + 0x7FFFu + ((bits >> 16) & 1u)) >> 16);
 }
+static float from_bf16(uint16_t h) {
+    const uint32_t bits = static_cast<uint32_t>(h) << 16;
+    float f;
+    memcpy(&f, &bits, sizeof f);
+    return f;
+}
 
 // Every entry point of the CUDA extension's byte format, on whole groups, against its scalar C restatement.
 static int wire_format_checks(hipStream_t stream, long &checks) {
@@ -118,6 +124,39 @@ static int wire_format_checks(hipStream_t stream, long &checks) {
             }
         }
     }
+
+    // bucket + residual and the payload of that sum in one launch, against the sum on the host and its quantize
+    void *d_residual = nullptr, *d_sum = nullptr;
+    HIP_OK(hipMalloc(&d_residual, n * sizeof(float)));
+    HIP_OK(hipMalloc(&d_sum, n * sizeof(float)));
+    for (int dtype : {LBC_F32, LBC_BF16}) {
+        const size_t item = dtype == LBC_F32 ? 4 : 2;
+        std::vector<uint16_t> half_residual(n), half_sum(n);
+        std::vector<float> sum(n);
+        for (int64_t i = 0; i < n; ++i) {
+            sum[i] = x[0][i] + x[1][i];
+            half_residual[i] = to_bf16(x[1][i]);
+            half_sum[i] = to_bf16(from_bf16(half[i]) + from_bf16(half_residual[i]));
+        }
+        const void *first = dtype == LBC_F32 ? static_cast<const void *>(x[0].data()) : static_cast<const void *>(half.data());
+        const void *second = dtype == LBC_F32 ? static_cast<const void *>(x[1].data()) : static_cast<const void *>(half_residual.data());
+        const void *both = dtype == LBC_F32 ? static_cast<const void *>(sum.data()) : static_cast<const void *>(half_sum.data());
+        HIP_OK(hipMemcpyAsync(d_x, first, n * item, hipMemcpyHostToDevice, stream));
+        HIP_OK(hipMemcpyAsync(d_residual, second, n * item, hipMemcpyHostToDevice, stream));
+        LBC_OK_OR_FAIL(lbc_wire_compensate_quant_pack(d_x, d_residual, d_sum, dtype, n, g, 8, 1, d_payload[0], LBC_ACCESS_AUTO, stream));
+        const int64_t nbytes = lbc_wire_payload_nbytes(n, g, dtype, 8);
+        HIP_OK(hipMemcpyAsync(got.data(), d_payload[0], nbytes, hipMemcpyDeviceToHost, stream));
+        HIP_OK(hipMemcpyAsync(out.data(), d_sum, n * item, hipMemcpyDeviceToHost, stream));
+        HIP_OK(hipStreamSynchronize(stream));
+        lbw_quantize(both, nullptr, dtype, n, g, 1, 8, want.data());
+        if (memcmp(got.data(), want.data(), nbytes) != 0 || memcmp(out.data(), both, n * item) != 0) {
+            printf("FAIL wire format: compensated quantize of dtype %d differs from the oracle\n", dtype);
+            return 27;
+        }
+        checks += 2;
+    }
+    HIP_OK(hipFree(d_residual));
+    HIP_OK(hipFree(d_sum));
 
     // the payloads of four ranks (fp32, interleaved scales), their fused mean, and one ring step on them
     const int64_t bytes = lbc_wire_payload_nbytes(n, g, LBC_F32, 8);

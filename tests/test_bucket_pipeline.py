@@ -156,6 +156,7 @@ def test_one_launch_per_bucket_counted_on_the_device(hip_device):
     assert sum(c for name, c in plain_counts.items() if "lbc" in name) == 3 * buckets
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_second_iteration_allocates_nothing_and_binds_nothing(hip_device):
     from lowbit_comm_amd.hip import ops
 

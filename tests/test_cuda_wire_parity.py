@@ -354,6 +354,35 @@ def test_module_reduce_paths(wire_status, hip_device, name):
     same(got, want)
 
 
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("compact", (True, False))
+@pytest.mark.parametrize("world", (1, 2, 3, 8))
+@pytest.mark.parametrize("fma", (True, False))
+def test_fused_reduce_and_error_feedback_through_the_module(hip, hip_device, access, name, compact, world, fma):
+    """The native call behind the module's in-place reduces, which hands the payloads' addresses to the library itself."""
+    from lowbit_comm_amd.hip.cuda_wire_module import HipCudaWireModule
+
+    module = HipCudaWireModule(fused_multiply_add=fma)
+    policy = (64, 0, 8, module.QuantType.Linear, compact)
+    for n in (64, 64 * 129, 100_003):
+        padded = -(-n // 64) * 64
+        payloads = [hip.quant_pack(make(n, name, 700 + 10 * world + r, hip_device, sigma=10.0 ** (r % 3 - 2)), compact=compact)
+                    for r in range(world)]
+        host = [to_numpy(p) for p in payloads]
+        inv = float(np.float32(1.0) / np.float32(world))
+        out = torch.empty(padded, dtype=NAMES[name], device=hip_device)
+        module.inplace_dequantize_reduce(payloads, out, *policy)
+        same(out, wire.reduce_payloads(host, padded, name, 64, compact, 1.0, fma), f"sum n={n}")
+        assert module.inplace_dequantize_reduce_mean(payloads, out, *policy, world) is True
+        same(out, wire.reduce_payloads(host, padded, name, 64, compact, inv, fma), f"mean n={n}")
+        prepared = make(n, name, 750 + world, hip_device)
+        residual = torch.empty_like(prepared)
+        assert module.inplace_dequantize_reduce_mean_update_error_feedback(payloads, prepared, out, residual, *policy, world) is True
+        want_restored, want_residual = wire.reduce_mean_error_feedback(host, to_numpy(prepared), n, name, 64, compact, world, fma)
+        same(out[:n], want_restored, f"restored n={n}")
+        same(residual, want_residual, f"residual n={n}")
+
+
 def test_module_error_feedback_paths(wire_status, hip_device):
     """tests/test_cuda_extension_smoke.py:37-100 upstream: residual update, fused mean + feedback, ragged prepared."""
     module = wire_status.module

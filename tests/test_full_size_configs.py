@@ -119,6 +119,7 @@ def test_config4_reduce_scatter_all_gather_plan_of_a_200_mib_bucket(ops, hip_dev
                            out[d * shard:(d + 1) * shard].view(torch.int32)), f"idempotence, shard {d}"
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_config5_llama_3_8b_shaped_stream_through_the_workspace_pool(ops, hip_device):
     from lowbit_comm_amd import CompressionConfig
     from lowbit_comm_amd.hip import ShardWorkspaceProvider, StreamOrderedCompletion, WorkspaceKey, create_torch_workspace_pool

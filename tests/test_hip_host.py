@@ -80,6 +80,7 @@ def test_facade_quantize_dequantize_round_trip(status, dev, dtype, name, n):
     assert same_bits(q.dequantize(buffer, (n,)), want)
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_inplace_calls_do_not_allocate_or_touch_inputs(status, dev):
     n = 1 << 20
     x = grad(n, torch.float32, 1, dev)
@@ -311,6 +312,7 @@ def test_all_gather_hook_facade_path_uses_the_fused_kernels(status, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_all_gather_hook_takes_bucket_plus_residual_from_the_quantize_launch(status, dev, dtype):
     """With error feedback the reference's hook first forms ``prepared = bucket + residual`` in a kernel of its own
     (ccdl_comm/communication/ddp_hook.py:196; error_feedback.py:27-36) and needs it again after the gather.  Here
@@ -408,6 +410,7 @@ def test_fused_bucket_processor_equals_the_unfused_reference_sequence(dev, dtype
         assert same_bits(unfused.error_feedback.get(0), cpu_residual), f"unfused residual step {step}"
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_fused_codec_steady_state_allocates_nothing(dev):
     from lowbit_comm_amd.hip.codec import FusedErrorFeedbackCodec
 
@@ -710,6 +713,7 @@ def test_asynchronous_plan_runs_on_the_communication_stream_and_completes_by_str
     assert work.resources == () and work.wait() is result
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_hook_over_the_reduce_scatter_transport_reuses_one_plan_per_bucket_shape(hip_device):
     """``create_ddp_comm_hook(strategy="reduce_scatter", reduce_scatter_all_gather=make_reduce_scatter_transport(...))``:
     every bucket runs the pre-bound plan, results equal the plan called directly, the bucket is reduced in place
@@ -838,6 +842,7 @@ def test_reduce_scatter_plan_beyond_eight_ranks_chains_exactly(dev):
 # --------------------------------------------------------------------------- #
 # workspace pool with real streams and events
 # --------------------------------------------------------------------------- #
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_pool_reuses_buffers_across_streams_without_host_sync(dev):
     from lowbit_comm_amd.hip import EventCompletion, WorkspaceKey, create_torch_workspace_pool
 
@@ -1006,6 +1011,7 @@ def test_stream_ordered_completion_records_nothing_while_a_buffer_stays_on_one_s
     assert done.query() is True and done.peek() is True
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_llama_shaped_bucket_stream_through_the_pool(dev):
     """Config 5 structure at 1/64 scale: bf16 parameter tensors of a Llama-3-8B-shaped layer stack, flattened in
     reverse registration order into fixed-size buckets with a ragged tail; per bucket EF quant-pack and a W=8

@@ -1046,7 +1046,7 @@ def test_shared_launch_reports_what_it_has_no_grid_for(ops, hip_device):
     peers32 = [ops.quant_pack(gradient_like(4096, torch.float32, 3310 + r, hip_device), group_size=32) for r in range(8)]
     assert ops.bind_quant_chunks_and_reduce(ops.bind_quant_pack_chunks(fp32, rows32, world, group_size=32),
                                             ops.bind_dequant_reduce(peers32, out, group_size=32))() is False
-    # an unaligned view: element-wise kernels only
+    # an unaligned view: the kernels at element alignment only
     odd = gradient_like(n + 1, torch.float32, 3303, hip_device)[1:]
     assert ops.bind_quant_chunks_and_reduce(ops.bind_quant_pack_chunks(odd, rows, world), reduce8)() is False
     # one side empty: the other runs alone

@@ -37,10 +37,11 @@ class Guarded:
 @pytest.mark.parametrize("n", [1, 5, 66, 1023, 1025, 2047, 2049, 4097, 8193, 2 * 8192 + 3])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
-def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
+@pytest.mark.parametrize("g", [64, 32, 16])
+def test_quantize_at_block_ends_and_start_offsets(hip_device, g, dtype, offset, n):
     from lowbit_comm_amd.hip import ops
 
-    t, world, g = DTYPES[dtype], 3, 64
+    t, world = DTYPES[dtype], 3
     for residual_type in (None, torch.float32):
         x = values(n, t, n + offset)
         r = None if residual_type is None else values(n, residual_type, n + 7, 1e-5)
@@ -52,7 +53,7 @@ def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
         fresh = Guarded(n, torch.float32, offset, hip_device)
         prepared = Guarded(n, p.dtype, offset, hip_device)
         rows = torch.full((world, ops.payload_nbytes(shard, g) + 12), 0x5A, dtype=torch.uint8, device=hip_device)
-        assert ops.quant_pack_chunks_into(x_in.inside, rows, world, residual=None if r is None else r_in.inside,
+        assert ops.quant_pack_chunks_into(x_in.inside, rows, world, group_size=g, residual=None if r is None else r_in.inside,
                                           new_residual=fresh.inside, restored=restored.inside, prepared_out=prepared.inside)
         padded = torch.zeros(world * shard, dtype=p.dtype)
         padded[:n] = p
@@ -62,7 +63,7 @@ def test_quantize_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
             row, nbytes = rows[d].cpu(), ops.payload_nbytes(shard, g)
             assert torch.equal(row[:nbytes], codec_torch.pack(codes, scales)), (d, residual_type)
             assert bool((row[nbytes:] == 0x5A).all()), d
-            decoded.append(codec_torch.dequantize(codes, scales, shard))
+            decoded.append(codec_torch.dequantize(codes, scales, shard, g))
         want = torch.cat(decoded)[:n]
         restored.check(want, "restored")
         fresh.check(p.float() - want, "new residual")
@@ -131,33 +132,55 @@ def test_decode_and_reduce_at_block_ends_and_start_offsets(hip_device, dtype, of
 
 
 # a workgroup of the ring step spans 1024 (fp32) or 2048 (16-bit) elements, 4096 of a 16-bit chunk above 4 Mi elements
-@pytest.mark.parametrize("n", [1, 7, 66, 1023, 1025, 2047, 2049, 4097, 8193, (1 << 22) + 4095, (1 << 22) + 4097])
+@pytest.mark.parametrize("g, n", [(64, n) for n in (1, 7, 66, 1023, 1025, 2047, 2049, 4097, 8193, (1 << 22) + 4095, (1 << 22) + 4097)] +
+                         [(g, n) for g in (32, 16) for n in (1, 7, 33, 66, 1023, 1025, 2049, 4097)])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
-def test_ring_step_and_feedback_update_at_block_ends_and_start_offsets(hip_device, dtype, offset, n):
+def test_ring_step_and_feedback_update_at_block_ends_and_start_offsets(hip_device, dtype, offset, g, n):
     from lowbit_comm_amd.hip import ops
 
     t = DTYPES[dtype]
-    (pair,), (received,) = payloads_of(1, n, 300 + n, hip_device)
+    (pair,), (received,) = payloads_of(1, n, 300 + n, hip_device, g)
     start = values(n, t, n + 3)
     for op in ("sum", "none"):
         chunk = Guarded(n, t, offset, hip_device, start)
         send = Guarded(received.numel(), torch.uint8, 3 * offset, hip_device)
-        scales_at = -(-n // 64) * 64
+        scales_at = -(-n // g) * g
         if (send.inside.data_ptr() + scales_at) % 4 == 0:        # the payload's scales must lie on 4 bytes
-            assert ops.ring_step_into(received, chunk.inside, send.inside, reduce_op=op, divisor=2.0)
+            assert ops.ring_step_into(received, chunk.inside, send.inside, group_size=g, reduce_op=op, divisor=2.0)
         else:
             send = Guarded(received.numel(), torch.uint8, 0, hip_device)
-            assert ops.ring_step_into(received, chunk.inside, send.inside, reduce_op=op, divisor=2.0)
-        decoded = codec_torch.dequantize(*pair, n, dtype=dtype)
+            assert ops.ring_step_into(received, chunk.inside, send.inside, group_size=g, reduce_op=op, divisor=2.0)
+        decoded = codec_torch.dequantize(*pair, n, g, dtype=dtype)
         want = (start + decoded if op == "sum" else decoded) / 2
         chunk.check(want, f"chunk {op}")
-        send.check(codec_torch.pack(*codec_torch.quantize(want)), f"payload {op}")
+        send.check(codec_torch.pack(*codec_torch.quantize(want, g)), f"payload {op}")
     prepared, restored = values(n, t, n + 4), values(n, t, n + 5)
     residual = Guarded(n, t, offset, hip_device)
     assert ops.ef_update_into(Guarded(n, t, offset, hip_device, prepared).inside,
                               Guarded(n, t, offset, hip_device, restored).inside, residual.inside)
     residual.check((prepared.float() - restored.float()).to(t), "feedback update")
+
+
+# codes of the reduce + requantize at byte addresses of every class, in and out; scales stay on 4 bytes
+@pytest.mark.parametrize("g, n", [(g, n) for g in (64, 32, 16) for n in (1, 66, 1023, 1025, 2047, 2049, 8193)])
+@pytest.mark.parametrize("offset", [1, 2, 3, 4])
+@pytest.mark.parametrize("mid", ["fp32", "bf16"])
+def test_reduce_requantize_of_codes_at_odd_addresses(hip_device, mid, offset, g, n):
+    from lowbit_comm_amd.hip import ops
+
+    for world in (1, 3, 8):
+        pairs, _ = payloads_of(world, n, 400 + n, hip_device, g)
+        held = [(Guarded(codes.numel(), torch.int8, offset + r % 2, hip_device, codes), scales.to(hip_device))
+                for r, (codes, scales) in enumerate(pairs)]
+        codes = Guarded(pairs[0][0].numel(), torch.int8, offset, hip_device)
+        scales = Guarded(pairs[0][1].numel(), torch.float32, 1, hip_device)
+        assert ops.dequant_reduce_quant_into([(c.inside, s) for c, s in held], codes.inside, scales.inside, n, group_size=g,
+                                             divisor=float(world), mid_dtype=DTYPES[mid])
+        reduced = codec_torch.reduce_payloads(pairs, n, g, mid, "mean")
+        want_codes, want_scales = codec_torch.quantize(reduced, g)
+        codes.check(want_codes, f"codes of {world}")
+        scales.check(want_scales, f"scales of {world}")
 
 
 # The CUDA byte format: a workgroup spans 1024 elements (fp32) or 2048 (16-bit) of a tensor that the chip holds at once,

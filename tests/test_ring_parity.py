@@ -262,6 +262,7 @@ def test_ring_reuses_pooled_workspaces_and_launches_one_kernel_per_hop(ops, hip_
 
 
 @pytest.mark.parametrize("fuse_steps", [True, False])
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_ring_replays_a_buckets_plan_without_allocating(ops, hip_device, fuse_steps):
     world, n, g = 4, 64 * 777 + 5, 64
     ring = build_ring(hip_device, world, n, "bf16", g, fuse_steps)

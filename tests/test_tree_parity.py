@@ -81,6 +81,7 @@ def test_tree_all_reduce_matches_the_oracle_on_every_rank(hip_device, mode, dtyp
         assert np.array_equal(raw(to_np(buckets[rank], dtype)), raw(want[rank])), (rank, mode, dtype, world, n, g, root)
 
 
+@pytest.mark.usefixtures("steady_allocator_counter")
 def test_tree_replays_its_plan_without_allocating_and_launches_once_per_changing_step(hip_device):
     world, n, g = 5, 64 * 500 + 7, 64
     executors = build_tree(hip_device, world, n, "fp32", g)

@@ -35,9 +35,12 @@ def kernel_names(run):
 
 @pytest.mark.gpu
 def test_every_entry_point_is_exactly_one_kernel_launch(hip_device):
+    from lowbit_comm_amd import CompressionConfig
     from lowbit_comm_amd.hip import cuda_wire, ops
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization import codec
 
-    dev = hip_device
+    dev, native = hip_device, load_hip_extension(wire_format="native")
     n, world, g = 64 * 8 * 100 + 24, 8, 64                     # ragged: interior and edge blocks in one launch
     shard = -(-n // world)
     x = torch.randn(n, device=dev) * 1e-3
@@ -84,6 +87,8 @@ def test_every_entry_point_is_exactly_one_kernel_launch(hip_device):
         "lbc_ring_step": lambda: ops.ring_step_into(packed, out, send, reduce_op="sum", divisor=8.0),
         "lbc_ef_update": lambda: ops.ef_update_into(x, out, residual),
         "lbc_wire_quant_pack": lambda: cuda_wire.quant_pack_into(x, wire, residual=residual),
+        "lbc_wire_compensate_quant_pack": lambda: isinstance(codec.compensate_and_quantize(
+            whole, whole, CompressionConfig(), extension_status=native), tuple),
         "lbc_wire_quant_pack_chunks": lambda: cuda_wire.bind_quant_pack_chunks(x, wire_rows, world)(),
         "lbc_wire_dequant": lambda: cuda_wire.dequant_into(wire, out),
         "lbc_wire_dequant_chunks": lambda: cuda_wire.bind_dequant_chunks(wire_rows, gathered, shard)(),
