@@ -62,9 +62,10 @@ const char *lbc_last_error(void);
  *                      faster than streaming then, 10-25 % slower when they do not).
  *   LBC_ACCESS_STREAM  non-temporal loads (each operand is read once); stores plain, non-temporal or
  *                      written through, as measured best per kernel and output size.
- * Operands without the alignment the vector kernels need (16 bytes for tensors, the lane's code
- * width for codes) are processed element by element under every mode.  Any other value:
- * LBC_EINVAL.
+ * The argument does not apply to a call of the portable format with an operand that does not start
+ * on 16 bytes (codes: on a lane's share of them, 4 or 8 bytes): such a call runs kernels of its own,
+ * with vector instructions at element alignment and non-temporal loads, under every mode.
+ * Any other value: LBC_EINVAL.
  */
 enum { LBC_ACCESS_AUTO = 0, LBC_ACCESS_CACHED = 1, LBC_ACCESS_STREAM = 2 };
 

@@ -274,9 +274,10 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
         else return acc + code * step;
     };
 
-    // One pass over the block's tiles, every load issued before the arithmetic.  WHOLE: all of the block's outputs exist;
-    // otherwise a lane's vector is cut short at the end (the payload holds whole groups, so a lane with one live output
-    // may read all of its codes).  Element by element the last block was the longest chain of a
+    // One pass over the block's tiles, the codes and scales of all of them issued before the arithmetic (`prepared` with
+    // them in the last block; whole blocks load it tile by tile, after the decode).  WHOLE: all of the block's outputs
+    // exist; otherwise a lane's vector is cut short at the end (the payload holds whole groups, so a lane with one live
+    // output may read all of its codes).  Element by element the last block was the longest chain of a
     // mid-sized launch: 10,048 outputs of eight payloads, interleaved bf16 4.2 us then, 2.4 now, fp32 with error feedback
     // 3.7 and 2.2, 2 Mi of two bf16 payloads with error feedback 5.1 and 4.9; decode of 10,048 2.9 and 1.9.
     auto tiles = [&](auto whole) __attribute__((always_inline)) {

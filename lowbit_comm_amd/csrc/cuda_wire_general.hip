@@ -597,17 +597,19 @@ hipError_t launch_general_quant_as(const WireGeneralQuantArgs &a, hipStream_t st
 
 template <typename T, int G>
 hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStream_t stream) {
-    // Each common policy runs a kernel without the code of the others (26.2 M fp32 elements: top-2 30.8 instead of
-    // 32.3 us, a code book 30.0 instead of 31.7 us).  Stochastic rounding of plain linear codes gains most: in the
-    // kernel for every policy it holds 126 vector registers for sixteen 16-bit elements a lane (four wavefronts a
-    // SIMD), on its own 65 (seven): 26.2 M bf16 elements 17.0 instead of 20.4 us, fp32 23.7 instead of 24.2 us.
-    // With outliers 32.4 / 26.8 instead of 35.3 / 28.5 us (fp32 / bf16), with a code book 36.5 / 34.5 instead of
-    // 40.8 / 38.8 us.
+    // Each common policy runs a kernel without the code of the others: its own against the kernel for every policy, us for
+    // 26.2 M elements in groups of 64, fp32 and bf16 (8 and 16 buffer sets in turn): top-2 28.5 / 28.5 and 19.3 / 24.2,
+    // stochastic 23.8 / 24.0 and 18.0 / 21.8, the two together 32.2 / 33.9 and 23.6 / 27.0, 4-bit top-2 26.4 / 27.3 and
+    // 17.5 / 23.8, a code book 24.6 / 26.2 and 19.9 / 23.7, rounded stochastically 37.9 / 40.6 and 34.7 / 38.2, with outliers
+    // 32.3 / 32.6 and 30.1 / 30.2.  What they save is registers: for sixteen 16-bit elements a lane the kernel for every
+    // policy holds four wavefronts a SIMD, the one for plain stochastic codes seven.
     //
-    // 32 bytes a lane against 16 (26.2 M elements, group 64, us): fp32 top-2 27.4 / 30.5, stochastic 24.3 / 26.6,
-    // a code book 25.5 / 27.9; bf16 top-2 22.1 / 23.3, stochastic 21.5 / 22.6, a code book through the cell table
-    // 19.8 / 19.3 - the one case that keeps 16 bytes, and the one case that gains from two such tiles a wavefront,
-    // both asked for before either is encoded (18.2 against 19.4 us; the others lose 8-20 % with two tiles).
+    // 32 bytes a lane against 16, bf16 as above: top-2 19.3 / 22.8, stochastic 18.0 / 19.8, the two together 23.6 / 27.3,
+    // 4-bit top-2 17.5 / 21.7, a code book rounded stochastically 34.7 / 34.5, with outliers 30.1 / 29.9.  (fp32, with 16
+    // bytes a lane still a form of this kernel: top-2 27.4 / 30.5, stochastic 24.3 / 26.6, a code book 25.5 / 27.9.)  A
+    // code book through the cell table is the one case that keeps 16 bytes (19.3 against 19.8), and the one that gains
+    // from two such tiles a wavefront, both asked for before either is encoded (18.2 against 19.4 us; the others lost
+    // 8-20 % with two tiles).
     constexpr int WIDE = general_quant_elems<T>() <= G ? general_quant_elems<T>() : G;
     constexpr int CELLS = sizeof(T) == 4 ? WIDE : 8, CELL_TILES = sizeof(T) == 4 ? 1 : 2;
     const int fixed = a.stochastic ? 0 : ((a.topk == 0 ? 1 : 0) | 2 | (a.kind == 0 ? 4 : 0));

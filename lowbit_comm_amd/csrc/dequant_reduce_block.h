@@ -84,8 +84,9 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
     OT *new_r = static_cast<OT *>(a.new_residual);
     const bool mean = a.divisor != 1.0f;
 
-    // One pass over the block's tiles with every load issued before the arithmetic.  WHOLE: all of the block's outputs
-    // exist.  Whole blocks of aligned tensors use one descriptor per stream over the block's span and 32-bit offsets
+    // One pass over the block's tiles with the codes and scales of all of them issued before the arithmetic (`prepared`
+    // with them in the last block; whole blocks load it tile by tile, after the tile's outputs are on their way).  WHOLE:
+    // all of the block's outputs exist.  Whole blocks of aligned tensors use one descriptor per stream over the block's span and 32-bit offsets
     // per lane; the block at the end and tensors at element alignment use 64-bit addresses, a lane's vector cut short
     // at the end.  (A payload holds whole groups, so a lane with one live output may read all of its codes.)  Walked
     // element by element, that last block was the longest chain of the kernel: 3,186,579 bf16 outputs of two payloads
@@ -283,7 +284,9 @@ __device__ __forceinline__ void decode_block(const DecodeArgs &a, unsigned block
     const int64_t block_first = static_cast<int64_t>(xcd_contiguous_block(block_x, grid_x, T::BLOCK_ELEMS)) * T::BLOCK_ELEMS;
     if (block_first >= valid) return;
 
-    // WHOLE: all of the block's outputs exist; otherwise a lane's vector is cut short at the end of the shard.  At
+    // WHOLE: all of the block's outputs exist; otherwise a lane's vector is cut short at the end of the shard.  The codes and
+    // scales of all tiles are issued first; what a combining decode adds to is loaded with them in the last block, and tile
+    // by tile in whole ones.  At
     // element alignment the stores keep the non-temporal hint (52.4 M fp32 outputs in eight odd shards: 44.8 us with it,
     // 48.7 us without, 112.7 us element by element; 9.8 M bf16 6.4, 8.9 and 23.2 us).  A 100,001-element tensor whose
     // last block walked its elements one dependent load at a time took 4.1 us, now 2.0 us.

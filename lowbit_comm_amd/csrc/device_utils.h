@@ -362,8 +362,8 @@ template <typename T, int N> __device__ __forceinline__ void divide_all(float (&
 // all 2^23 scale mantissas x 256 half-integers x 13 neighbouring dividends at three exponents (8*10^10 pairs, every
 // such case) and 2.6*10^10 sampled pairs over the whole exponent range 2^-23 .. 2^120, among them dividends with 8
 // or 11 significant bits: no code and no quotient differs.  The one case outside, a remainder that underflows,
-// needs |p/scale| < 2^-64, where the code is 0 whatever the last bit of the quotient is.  The ragged edge uses
-// the same operations (encode below), so an element's code does not depend on the block it falls into.
+// needs |p/scale| < 2^-64, where the code is 0 whatever the last bit of the quotient is.  Whole blocks and
+// the block at a chunk's end run the same code, so an element's code does not depend on the block it falls into.
 // (A reciprocal-multiply fast path with a fallback
 // for quotients next to a tie, which this replaces, took the fallback in most wavefronts of a 16-bit tensor -
 // 127*x/absmax hits exact ties all the time when x and absmax have 8-bit mantissas - and ran it 25 % slower.)
@@ -403,15 +403,6 @@ __device__ __forceinline__ void encode_group(const float (&p)[N], float scale, f
 template <int N>
 __device__ __forceinline__ void encode_group(const float (&p)[N], float scale, int (&codes)[N]) {
     encode_group<N>(p, scale, 1.0f / scale, codes);
-}
-
-// Single-element form for the ragged edge: the same operations as encode_group, so that an element gets the same
-// code whether it falls into an interior block or into the tail.
-__device__ __forceinline__ int encode(float p, float scale) {
-    const float one[1] = {p};
-    int bits[1];
-    encode_group<1>(one, scale, bits);
-    return static_cast<int>(code_value(bits[0]));   // an integer in [-127, 127]: the conversion is exact
 }
 
 // Low bytes of four ints -> one little-endian word (three v_perm_b32).

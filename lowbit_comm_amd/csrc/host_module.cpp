@@ -7,7 +7,7 @@
 //
 //   Launch       one call of the C ABI (include/lbc.h) with its arguments converted once; calling it looks up torch's
 //                current stream and enqueues the kernel, 1.4 us less than the same call through ctypes (four 1 MiB bf16
-//                buckets through the pipelined hook 74.6 -> 66.6 us, a ring of fourteen hops 142 -> 134 us)
+//                buckets through the pipelined hook 74.6 -> 66.6 us; a ring of fourteen hops gains less than its runs differ)
 //   functions    the codec facade's allocating calls, from tensors to the launch (quantize and decode of a 10,007-element tensor
 //                38.1 -> 11.2 us together, of 25 MiB fp32 23.2 -> 15.3, which is what the two kernels take)
 //

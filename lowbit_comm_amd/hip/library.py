@@ -1,7 +1,8 @@
-"""ctypes binding of ``liblbc_hip.so`` (the C ABI declared in ``include/lbc.h``).
+"""Loading of the two native parts: ``liblbc_hip.so`` (the C ABI declared in ``include/lbc.h``, checked and bound through ctypes
+for its queries) and ``_host.so``, the extension module in front of it that issues the launches.
 
-The library is built in-tree by ``lowbit_comm_amd/csrc/Makefile``.  Loading never falls back to
-anything else: if the shared object is missing or a symbol is absent, :func:`load_library` raises.
+Both are built in-tree by ``lowbit_comm_amd/csrc/Makefile``.  Loading never falls back to anything else: if a shared object
+is missing or a symbol is absent, :func:`load_library` raises.
 """
 from __future__ import annotations
 
@@ -12,9 +13,6 @@ from lowbit_comm_amd.exceptions import CCDLUnavailableError
 
 LIBRARY_PATH = Path(__file__).resolve().parent.parent / "liblbc_hip.so"
 ABI_VERSION = 8
-
-LBC_OK = 0
-LBC_UNSUPPORTED = 1
 
 _c_ptr = ctypes.c_void_p
 _c_i64 = ctypes.c_int64
