@@ -308,10 +308,14 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// The sizes of the tensor to make: `o` is a tuple of them, or None for one dimension of `all` elements.  False: neither.
+// _host.FLAT: the shape of everything that a payload holds, in one dimension.  An object of its own, because None and the
+// like are shapes that a caller may get wrong.
+PyObject *flat = nullptr;
+
+// The sizes of the tensor to make: `o` is a tuple of them, or FLAT for one dimension of `all` elements.  False: neither.
 bool sizes_of(PyObject *o, int64_t all, c10::SmallVector<int64_t, 5> &sizes, int64_t &numel) {
     numel = 1;
-    if (o == Py_None) {
+    if (o == flat) {
         sizes.push_back(all);
         numel = all;
         return true;
@@ -319,15 +323,15 @@ bool sizes_of(PyObject *o, int64_t all, c10::SmallVector<int64_t, 5> &sizes, int
     if (!PyTuple_Check(o)) return false;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(o); ++i) {
         long v;
-        if (!integer(PyTuple_GET_ITEM(o, i), v) || v < 0) return false;
+        if (PyBool_Check(PyTuple_GET_ITEM(o, i)) || !integer(PyTuple_GET_ITEM(o, i), v) || v < 0) return false;
         sizes.push_back(v);
-        numel *= v;
+        if (__builtin_mul_overflow(numel, v, &numel)) return false;
     }
     return true;
 }
 
-// dequantize(module, table, payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, access) -> tensor of that shape (None:
-// flat, every element the payload holds)
+// dequantize(module, table, payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, access) -> tensor of that
+// shape (FLAT: every element the payload holds)
 PyObject *dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n < 2 || !owns(a[0], a[1])) return elsewhere();
@@ -525,7 +529,7 @@ PyObject *wire_compensate_quantize(PyObject *, PyObject *const *a, Py_ssize_t n)
 }
 
 // wire_dequantize(module, table, payload, shape, dtype, group_size, topk, bit, reduce_op, quant_type, compact, access) -> tensor of that
-// shape (None: flat, every element the payload holds)
+// shape (FLAT: every element the payload holds)
 PyObject *wire_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n < 2 || !owns(a[0], a[1])) return elsewhere();
@@ -683,6 +687,13 @@ PyMODINIT_FUNC PyInit__host(void) {
     if (PyType_Ready(&LaunchType) < 0) return nullptr;
     PyObject *module = PyModule_Create(&kModule);
     if (module == nullptr) return nullptr;
+    if (flat == nullptr) flat = PyUnicode_FromString("FLAT");
+    Py_XINCREF(flat);
+    if (flat == nullptr || PyModule_AddObject(module, "FLAT", flat) < 0) {
+        Py_XDECREF(flat);
+        Py_DECREF(module);
+        return nullptr;
+    }
     Py_INCREF(&LaunchType);
     if (PyModule_AddObject(module, "Launch", reinterpret_cast<PyObject *>(&LaunchType)) < 0) {
         Py_DECREF(&LaunchType);

@@ -229,14 +229,14 @@ class HipNativeModule:
 
     # ---- dequantize -----------------------------------------------------------------------------
     def _dequantize_shaped(self, input, shape, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call (``None``:
-        all of them, flat), or ``None`` when the request is anything but a plain decode of a payload of that size."""
+        """The payload's first ``prod(shape)`` elements as a fresh tensor of that shape in one native call, or ``None`` when
+        the request is anything but a plain decode of a payload of that size."""
         decoded = _host.dequantize(self, _DEQUANTIZES, input, shape, dtype, group_size, topk, bit, reduce_op, quant_type,
                                    ops.access_code(None))
         return decoded if isinstance(decoded, torch.Tensor) else None
 
     def dequantize(self, input, group_size, topk, bit, reduce_op, quant_type, dtype, compact):
-        decoded = _host.dequantize(self, _DECODES, input, None, dtype, group_size, topk, bit, reduce_op, quant_type,
+        decoded = _host.dequantize(self, _DECODES, input, _host.FLAT, dtype, group_size, topk, bit, reduce_op, quant_type,
                                    ops.access_code(None))
         if isinstance(decoded, torch.Tensor):
             return decoded

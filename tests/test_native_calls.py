@@ -223,3 +223,23 @@ def test_a_feedback_state_of_its_own_keeps_its_compensate_step(monkeypatch, name
         all_gather=lambda local: GatheredPayloads([local.buffer], 1))
     hook(None, Bucket())
     assert len(launched) == (way == "plain")
+
+
+# what a shape may be is torch's to say, also where the decode writes straight into it
+@pytest.mark.gpu
+@pytest.mark.parametrize("wire", ["portable", "native"])
+@pytest.mark.parametrize("shape", [None, (True, 128), (1 << 62, 4), (1 << 33, 1 << 33), ..., (128.0,), (-1,)])
+def test_shapes_that_torch_refuses_are_refused(hip_device, wire, shape):
+    from lowbit_comm_amd import CompressionConfig
+    from lowbit_comm_amd.hip.loader import load_hip_extension
+    from lowbit_comm_amd.quantization.codec import dequantize_reduce_tensors, dequantize_tensor, quantize_tensor
+
+    status, config = load_hip_extension(wire_format=wire), CompressionConfig()
+    payload = quantize_tensor(values(128, torch.float32, 1).to(hip_device), config, extension_status=status)
+    if shape == (-1,):       # torch's "as many as there are": accepted, with the last element trimmed away by the facade
+        assert dequantize_tensor(payload, shape, config, dtype="fp32", extension_status=status).numel() == 127
+        return
+    for call in (lambda: dequantize_tensor(payload, shape, config, dtype="fp32", extension_status=status),
+                 lambda: dequantize_reduce_tensors([payload] * 2, shape, config, dtype="fp32", extension_status=status, reduce="mean")):
+        with pytest.raises((TypeError, RuntimeError)):
+            call()
