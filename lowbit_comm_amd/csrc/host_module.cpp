@@ -185,7 +185,9 @@ PyObject *launch_call(PyObject *self, PyObject *args, PyObject *kwargs) {
     HANDLE_TH_ERRORS
     Launch *launch = reinterpret_cast<Launch *>(self);
     PyObject *given = nullptr;
-    if (PyTuple_GET_SIZE(args) != 0 || kwargs != nullptr) {   // the usual call has none
+    if (kwargs == nullptr && PyTuple_GET_SIZE(args) == 1) {   // the usual calls: a stream, or nothing
+        given = PyTuple_GET_ITEM(args, 0);
+    } else if (kwargs != nullptr || PyTuple_GET_SIZE(args) != 0) {
         static const char *const kNames[] = {"stream", nullptr};
         if (!PyArg_ParseTupleAndKeywords(args, kwargs, "|O:Launch", const_cast<char **>(kNames), &given)) return nullptr;
     }
