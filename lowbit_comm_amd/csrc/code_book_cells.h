@@ -5,10 +5,15 @@
 // `entry + (t - book[entry] > (book[entry + 1] - book[entry]) * 0.5f)` (inner.cuh:74-118).  For one book that is a
 // non-decreasing step function of t with fourteen steps.  The places of the steps (the smallest float at which the
 // code becomes k + 1) are found here by bisection over the float line with the reference's own arithmetic, and
-// [-1, 1] is cut into 256 cells of width 1/128, none of which holds two steps.  A cell stores the code at its left
-// end and the step inside it, if any, so that on the device
+// [-1, 1] is cut into 256 cells of width 1/128.  A cell stores the code at its left end and the next step from there
+// on, inside the cell or beyond it, so that
 //     code(t) = cell.base + (t >= cell.threshold),   cell = cells[(unsigned)fma(t, 128, 128)]
 // for every finite t in [-1, 1].  tests/native/check_book_cells.cpp compares the two forms on every such float.
+//
+// The quantize kernel does not form t.  Steps lie at least two cells apart, so a cell answers for every t from its left
+// end to one and a half cells behind it: the cell one below the rounded place of an approximate quotient (`nearest_place`)
+// is right for any error up to a quarter of a cell.  Whether the quotient, rounded to a float, reaches
+// the step is then decided without a division (`reaches`).
 // Plain C++17 (host and device): no HIP types.
 #pragma once
 #include <cstdint>
@@ -35,7 +40,7 @@ constexpr Books kBookSet = {{
 }};
 
 struct Cell {
-    float threshold;   // the code rises by one at this value; +inf when the cell holds no step
+    float threshold;   // the code rises by one at this value, the next step at or behind the left end; +inf behind the last
     uint32_t base;     // the code at the cell's left end
 };
 struct Table {
@@ -87,35 +92,82 @@ constexpr Table make_table(const float (&book)[16]) {
         float threshold = __builtin_inff();
         for (int k = 0; k < 14; ++k) {
             if (cell_of(step[k]) < i) ++base;
-            else if (cell_of(step[k]) == i) threshold = step[k];
+            else if (step[k] < threshold) threshold = step[k];
         }
         table.cell[i] = Cell{threshold, base};
     }
     return table;
 }
 
-// One step per cell at most, or the lookup would miss a step.
-constexpr bool steps_in_separate_cells(const float (&book)[16]) {
-    int previous = -1;
+// Steps at least two cells apart (up to a unit in the last place): see nearest_place.  None is a positive power of two,
+// which would be closer to the float before it than its exponent says: see reaches.
+constexpr bool steps_far_apart(const float (&book)[16]) {
     for (int k = 0; k < 14; ++k) {
-        const int cell = cell_of(step_after(book, k));
-        if (cell <= previous) return false;
-        previous = cell;
+        const float step = step_after(book, k);
+        if (k > 0 && (step - step_after(book, k - 1)) * 128.0f < 1.999f) return false;
+        if (step > 0.0f && (__builtin_bit_cast(uint32_t, step) & 0x007FFFFFu) == 0) return false;
     }
     return true;
 }
 
 constexpr Tables kTables = {{make_table(kBookSet.value[0]), make_table(kBookSet.value[1]), make_table(kBookSet.value[2]),
                                make_table(kBookSet.value[3])}};
-static_assert(steps_in_separate_cells(kBookSet.value[0]) && steps_in_separate_cells(kBookSet.value[1]) &&
-                  steps_in_separate_cells(kBookSet.value[2]) && steps_in_separate_cells(kBookSet.value[3]),
-              "a cell of width 1/128 holds two steps of a code book");
+static_assert(steps_far_apart(kBookSet.value[0]) && steps_far_apart(kBookSet.value[1]) &&
+                  steps_far_apart(kBookSet.value[2]) && steps_far_apart(kBookSet.value[3]),
+              "two steps of a code book lie too close for one lookup");
 
-// The lookup, as the device does it.
+// The lookup of a quotient t.
 constexpr int cell_code(const Table &table, float t) {
     const Cell &cell = table.cell[cell_of(t)];
     return static_cast<int>(cell.base) + (t >= cell.threshold ? 1 : 0);
 }
 
+// ---- the lookup of v / scale without the quotient ----
+#if defined(__HIPCC__)
+#define LBC_CELLS_HOST_DEVICE __attribute__((host)) __attribute__((device)) __attribute__((always_inline)) inline
+#else
+#define LBC_CELLS_HOST_DEVICE inline
+#endif
+
+constexpr float kBeyond = 3.0f;   // no quotient of at most 1 reaches it
+
+// The cells as the quantize kernel reads them, by place: entry p is the cell one below p, kBeyond stands behind the last
+// step, and the code plus one lies in the top four bits, from where a funnel shift pushes it into a word of codes.
+struct Places {
+    Cell entry[kBooks][kCells];
+};
+constexpr Places make_places() {
+    Places places{};
+    for (int b = 0; b < kBooks; ++b)
+        for (int p = 0; p < kCells; ++p) {
+            const Cell &cell = kTables.book[b].cell[p == 0 ? 0 : p - 1];
+            places.entry[b][p] = Cell{cell.threshold < kBeyond ? cell.threshold : kBeyond, (cell.base + 1) << 28};
+        }
+    return places;
+}
+constexpr Places kPlaces = make_places();
+
+// The place of v / scale, round(128 * v / scale) + 128, in the low bits of a float: adding 1.5 * 2^23 + 128 rounds to an
+// integer.  `reciprocal128` is 128 / scale with a few ulps of error.
+constexpr float kPlaceMagic = 12582912.0f + 128.0f;
+constexpr uint32_t kPlaceBits = 0x4B400000u;   // bits of 1.5 * 2^23: place 0
+LBC_CELLS_HOST_DEVICE uint32_t nearest_place(float v, float reciprocal128) {
+    return __builtin_bit_cast(uint32_t, __builtin_fmaf(v, reciprocal128, kPlaceMagic));
+}
+
+// A number whose sign bit is clear when RN(v / scale) >= threshold and set when it is below, for a scale of at least
+// 2^-20.  The quotient rounds up to the threshold when it lies above m, the middle between the threshold and the float
+// before it: m = threshold - h, with h half a unit in the threshold's last place (no threshold is a positive power of two, so the
+// float before it has the same exponent).  It never equals m: m has 25 significant bits, so m * scale has at least 25 and
+// is no float.  With b = v - threshold * scale, exactly, what counts is the sign of b + h * scale.  The inner operation
+// gives b exactly while |b| <= 2 h scale (b is then a multiple of 2^-24 of its bound: v, being near threshold * scale,
+// is a coarser multiple than the product), otherwise a rounded b on the same side of -h * scale; the outer one adds
+// h * scale, whose power of two is threshold's exponent times 2^-24 (`scale24` is scale * 2^-24, exact).  (An infinite threshold
+// would meet itself here: kBeyond.)
+LBC_CELLS_HOST_DEVICE float reaches(float threshold, float v, float scale, float scale24) {
+    const float b = __builtin_fmaf(-threshold, scale, v);
+    const float exponent = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, threshold) & 0xFF800000u);
+    return __builtin_fmaf(__builtin_fabsf(exponent), scale24, b);
+}
 }  // namespace book_cells
 }  // namespace lbc

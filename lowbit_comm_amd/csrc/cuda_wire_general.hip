@@ -31,7 +31,7 @@ namespace {
 
 // inner.cuh:9-35, and the one-lookup form of the encoder built from them at compile time
 __constant__ book_cells::Books kCodeBooks = book_cells::kBookSet;
-__constant__ book_cells::Tables kBookCells = book_cells::kTables;
+__constant__ book_cells::Places kBookPlaces = book_cells::kPlaces;
 
 // Philox4x32-10: one block of four 32-bit words.  A round is two 32x32->64 multiplies and two three-way
 // exclusive-ors; gfx950 has the latter as one instruction (v_bitop3_b32 with the truth table 0x96), which the
@@ -75,17 +75,34 @@ __device__ __forceinline__ const float *wave_code_book(int kind, int lane) {
     return book;
 }
 
-// The workgroup's copy of a book's cell table (code_book_cells.h) in LDS.  Every wavefront of the workgroup must
-// come here: the copy ends in a workgroup barrier.
-__device__ __forceinline__ const book_cells::Cell *block_book_cells(int kind) {
-    __shared__ book_cells::Cell cells[book_cells::kCells];
-    static_assert(book_cells::kCells <= kBlock + 1, "one table entry per thread, and one more");
-    const book_cells::Cell *table = kBookCells.book[kind - 1].cell;
-    cells[threadIdx.x] = table[threadIdx.x];
-    if (threadIdx.x == 0) cells[kBlock] = table[kBlock];
-    __syncthreads();
-    return cells;
-}
+// The workgroup's copy of a book's cell table (code_book_cells.h) in LDS.  The loads of the table are issued by `fetch`,
+// ahead of the tensor's own, so that `publish` need not wait for those; every wavefront of the workgroup must come to
+// `publish`, which ends in a workgroup barrier that orders LDS only.
+struct BlockCells {
+    static constexpr int PER_THREAD = (book_cells::kCells + kBlock - 1) / kBlock;
+    u32x2 held[PER_THREAD];
+
+    __device__ __forceinline__ void fetch(int kind) {
+        const u32x2 *table = reinterpret_cast<const u32x2 *>(kBookPlaces.entry[kind - 1]);
+#pragma unroll
+        for (int k = 0; k < PER_THREAD; ++k) {
+            const int place = k * kBlock + threadIdx.x;
+            if (place < book_cells::kCells) held[k] = table[place];
+        }
+    }
+    __device__ __forceinline__ const book_cells::Cell *publish() {
+        __shared__ u32x2 cells[book_cells::kCells];
+#pragma unroll
+        for (int k = 0; k < PER_THREAD; ++k) {
+            const int place = k * kBlock + threadIdx.x;
+            if (place < book_cells::kCells) cells[place] = held[k];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        return reinterpret_cast<const book_cells::Cell *>(cells);
+    }
+};
 
 __device__ __forceinline__ int meta_words_of(int topk) { return topk == 0 ? 1 : topk + 2; }
 
@@ -174,6 +191,9 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     constexpr int TILE = kWave * EL;
     const int64_t first = (static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6)) * (TILES * TILE);
 
+    constexpr bool BY_CELLS = (FIXED & 2) != 0 && (FIXED & 4) == 0;
+    BlockCells block_cells;
+    if constexpr (BY_CELLS) block_cells.fetch(kind);
     // all of the wavefront's elements are asked for before anything else
     Raw raws[TILES][VEC];
 #pragma unroll
@@ -192,12 +212,10 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             }
         }
     }
-    // After the loads were issued: the waits of the tables cover theirs.  The cell table pays for its copy and its
-    // barrier from eight elements a lane on.
-    const bool by_cells = kind != 0 && !stochastic;   // uniform over the grid
-    const book_cells::Cell *cells = by_cells ? block_book_cells(kind) : nullptr;
+    const book_cells::Cell *cells = nullptr;
+    if constexpr (BY_CELLS) cells = block_cells.publish();
     if (first >= a.numel) return;   // wavefront-uniform, behind the workgroup's barrier
-    const float *book = wave_code_book(kind, lane);
+    const float *book = BY_CELLS ? nullptr : wave_code_book(kind, lane);
 
     auto encode_tile = [&](const int64_t tile_first, const Raw (&raw)[VEC]) __attribute__((always_inline)) {
         const int64_t e0 = tile_first + lane * VEC;
@@ -370,9 +388,71 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             }
         }
         meta[0] = static_cast<Raw>(scale_raw);
+        auto store_meta = [&]() __attribute__((always_inline)) {
+            if (live && k0 == 0) {
+                Raw *words = reinterpret_cast<Raw *>(group_meta);
+                if (topk == 2) {
+                    store_elems<Raw, 4, kPlain>(words, meta);
+                } else if (topk == 1) {
+                    const Raw pair[2] = {meta[0], meta[1]};
+                    store_elems<Raw, 2, kPlain>(words, pair);
+                    words[2] = meta[2];
+                } else {
+                    words[0] = meta[0];
+                }
+            }
+        };
 
         float scale = value_of<T>(scale_raw);
         scale = scale < 1.0e-6f ? 1.0e-6f : scale;   // a NaN scale stays NaN and encodes every element as 0
+
+        if constexpr (BY_CELLS) {
+            // A code book, rounded to nearest (uniform: kind is not 0).  The cell lookup answers v / scale without forming
+            // the quotient: per element a fused multiply-add and an address, one LDS read, and four operations that leave
+            // the comparison with the step in a sign bit and push it and the cell's code into a word of eight.  It
+            // holds for a scale within 2^60 of 1 either way and |v| <= scale; the scale is at least 1e-6 here, and beside
+            // outliers or a NaN an element may lie above it.  A wavefront with any other operand divides, and looks the
+            // quotient up with scale 1; what lies outside [-1, 1] takes the first or last code, a NaN the last, as the search
+            // does.  9 instead of 21 instructions an element: 26.2 M elements of the normal book 24.5 -> 21.3 us (fp32, 119
+            // MB, 5.6 TB/s) and 19.9 -> 14.2 us (bf16), with two outliers 32.5 -> 27.5 and 30.0 -> 21.0; what is left of the
+            // difference to the linear 4-bit pack kernel (19.6 and 13.0) is the table, 2 KiB copied per 2048 or 4096
+            // elements (by workgroups half and a quarter as large: 25.8 and 29.4 us, fp32).
+            const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
+            bool unusual = scale_exponent > 127u + 60u;
+            if (any_nan) {   // wavefront-uniform
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
+            }
+            float divisor = scale;
+            if (__ballot(unusual) != 0) {   // wavefront-uniform
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) {
+                    const float t = v[i] / scale;
+                    v[i] = t < 1.0f ? (t > -1.0f ? t : -1.0f) : 1.0f;
+                }
+                divisor = 1.0f;
+            }
+            const float reciprocal128 = __builtin_amdgcn_rcpf(divisor) * 128.0f, divisor24 = divisor * 0x1p-24f;
+            if (live) {
+                uint32_t words[WORDS];
+#pragma unroll
+                for (int k = 0; k < WORDS; ++k) {
+                    uint32_t codes = 0, below = 0;
+#pragma unroll
+                    for (int i = 8 * k; i < 8 * k + 8; ++i) {
+                        const book_cells::Cell cell = cells[book_cells::nearest_place(v[i], reciprocal128) - book_cells::kPlaceBits];
+                        const float sign = book_cells::reaches(cell.threshold, v[i], divisor, divisor24);
+                        codes = __builtin_amdgcn_alignbit(codes, cell.base, 28);          // (codes << 4) | code + 1
+                        below = __builtin_amdgcn_alignbit(below, as_u32(sign), 28);
+                    }
+                    codes -= (below >> 3) & 0x11111111u;
+                    words[k] = WIDE ? codes : __builtin_amdgcn_alignbit(codes, codes, 16);
+                }
+                store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
+            }
+            store_meta();
+            return;
+        }
 
         int c[VEC];
         if (kind == 0) {
@@ -427,14 +507,6 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) t[i] = v[i] / scale;
             }
-            if (usual && by_cells) {
-                // Every t is a number in [-1, 1]: search and rounding are one table lookup (code_book_cells.h).
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    const book_cells::Cell cell = cells[static_cast<uint32_t>(__builtin_fmaf(t[i], 128.0f, 128.0f))];
-                    c[i] = static_cast<int>(cell.base) + (t[i] >= cell.threshold ? 1 : 0);
-                }
-            } else {
             // The largest entry in [0, 14] with not (t < book[entry]); a NaN ends at 14.  Four halving steps, each
             // over all of the lane's elements so that their LDS reads are in flight together; positions are kept as
             // byte offsets into the book.
@@ -466,7 +538,6 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) c[i] += excess[i] > gap[i] * 0.5f ? 1 : 0;
             }
-            }
         }
         if (live) {
             uint32_t words[WORDS];
@@ -483,18 +554,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             }
             store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
         }
-        if (live && k0 == 0) {
-            Raw *words = reinterpret_cast<Raw *>(group_meta);
-            if (topk == 2) {
-                store_elems<Raw, 4, kPlain>(words, meta);
-            } else if (topk == 1) {
-                const Raw pair[2] = {meta[0], meta[1]};
-                store_elems<Raw, 2, kPlain>(words, pair);
-                words[2] = meta[2];
-            } else {
-                words[0] = meta[0];
-            }
-        }
+        store_meta();
     };
 #pragma unroll
     for (int tile = 0; tile < TILES; ++tile) {
@@ -600,18 +660,15 @@ hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStr
     // Each common policy runs a kernel without the code of the others: its own against the kernel for every policy, us for
     // 26.2 M elements in groups of 64, fp32 and bf16 (8 and 16 buffer sets in turn): top-2 28.5 / 28.5 and 19.3 / 24.2,
     // stochastic 23.8 / 24.0 and 18.0 / 21.8, the two together 32.2 / 33.9 and 23.6 / 27.0, 4-bit top-2 26.4 / 27.3 and
-    // 17.5 / 23.8, a code book 24.6 / 26.2 and 19.9 / 23.7, rounded stochastically 37.9 / 40.6 and 34.7 / 38.2, with outliers
-    // 32.3 / 32.6 and 30.1 / 30.2.  What they save is registers: for sixteen 16-bit elements a lane the kernel for every
-    // policy holds four wavefronts a SIMD, the one for plain stochastic codes seven.
+    // 17.5 / 23.8, a code book rounded stochastically 37.9 / 40.6 and 34.7 / 38.2.  What they save is registers: for
+    // sixteen 16-bit elements a lane the kernel for every policy holds four wavefronts a SIMD, the one for plain
+    // stochastic codes seven.
     //
     // 32 bytes a lane against 16, bf16 as above: top-2 19.3 / 22.8, stochastic 18.0 / 19.8, the two together 23.6 / 27.3,
-    // 4-bit top-2 17.5 / 21.7, a code book rounded stochastically 34.7 / 34.5, with outliers 30.1 / 29.9.  (fp32, with 16
-    // bytes a lane still a form of this kernel: top-2 27.4 / 30.5, stochastic 24.3 / 26.6, a code book 25.5 / 27.9.)  A
-    // code book through the cell table is the one case that keeps 16 bytes (19.3 against 19.8), and the one that gains
-    // from two such tiles a wavefront, both asked for before either is encoded (18.2 against 19.4 us; the others lost
-    // 8-20 % with two tiles).
+    // 4-bit top-2 17.5 / 21.7, a code book 14.2 / 15.7, rounded stochastically 34.7 / 34.5.  (fp32, with 16 bytes a lane
+    // still a form of this kernel: top-2 27.4 / 30.5, stochastic 24.3 / 26.6.)  Two such tiles a wavefront are slower for
+    // all of them, a code book 22.0 against 21.3 us (fp32) and 14.7 against 14.2 (bf16).
     constexpr int WIDE = general_quant_elems<T>() <= G ? general_quant_elems<T>() : G;
-    constexpr int CELLS = sizeof(T) == 4 ? WIDE : 8, CELL_TILES = sizeof(T) == 4 ? 1 : 2;
     const int fixed = a.stochastic ? 0 : ((a.topk == 0 ? 1 : 0) | 2 | (a.kind == 0 ? 4 : 0));
     if (bit != 8 && bit != 4) return hipErrorNotSupported;
     if (bit == 8 && a.kind != 0) return hipErrorNotSupported;   // eight bits: linear codes only
@@ -626,7 +683,7 @@ hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStr
     if (fixed == 2) return launch_general_quant_as<T, G, 4, 2, WIDE>(a, stream);
     if (a.stochastic && a.topk == 0 && a.kind == 0) return launch_general_quant_as<T, G, 4, 13, WIDE>(a, stream);
     if (a.stochastic && a.topk == 0) return launch_general_quant_as<T, G, 4, 9, WIDE>(a, stream);
-    if (fixed == 3) return launch_general_quant_as<T, G, 4, 3, CELLS, CELL_TILES>(a, stream);
+    if (fixed == 3) return launch_general_quant_as<T, G, 4, 3, WIDE>(a, stream);
     return launch_general_quant_as<T, G, 4, 0, WIDE>(a, stream);
 }
 
