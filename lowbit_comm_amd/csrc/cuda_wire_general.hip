@@ -171,9 +171,11 @@ template <int LANES> __device__ __forceinline__ void merge_top3(uint32_t &first,
 // "stochastic rounding" (13: plain linear codes rounded stochastically, 12: the same with outliers, 9: a code book
 // with stochastic rounding; 6: linear codes rounded to nearest, always with outliers - without them lbc_wire_quant_pack
 // serves the call).  0 is the kernel for every policy.
-// EL: elements per lane, a multiple of 8 that divides G.  TILES: tiles of 64 * EL elements a wavefront owns, all of
-// them asked for before the first is encoded.
-template <typename T, int G, int BIT, int FIXED, int EL, int TILES>
+// EL: elements per lane, a multiple of 8 that divides G; a wavefront owns one tile of 64 * EL elements.
+// Codes leave in plain stores: with the non-temporal hint a launch alone is up to 6 % faster, and what reads the payload
+// next pays for it (quantize and decode of 26.2 M elements with two outliers: fp32 44.9 plain against 52.0 us, bf16 28.6
+// against 31.4).
+template <typename T, int G, int BIT, int FIXED, int EL>
 __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGeneralQuantArgs a) {
     const int topk = (FIXED & 1) ? 0 : a.topk;
     const bool stochastic = (FIXED & 2) ? false : ((FIXED & 8) ? true : a.stochastic != 0);
@@ -189,379 +191,379 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     const int meta_bytes = meta_words_of(topk) * ITEM;
     const int64_t groups = a.numel / G;
     constexpr int TILE = kWave * EL;
-    const int64_t first = (static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6)) * (TILES * TILE);
+    const int64_t tile_first = (static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6)) * TILE;
+    const int64_t e0 = tile_first + lane * VEC;
+    const bool live = e0 < a.numel;      // numel is a multiple of G: dead lanes form whole dead groups
 
     constexpr bool BY_CELLS = (FIXED & 2) != 0 && (FIXED & 4) == 0;
     BlockCells block_cells;
     if constexpr (BY_CELLS) block_cells.fetch(kind);
-    // all of the wavefront's elements are asked for before anything else
-    Raw raws[TILES][VEC];
+    // All of the wavefront's elements are asked for before anything else, and kept as whole dwords: 16-bit elements taken
+    // apart inside the branch would be waited for there, ahead of the tables and of the draws (26.2 M bf16 elements with
+    // two outliers, rounded stochastically, 23.7 against 22.4 us, 3.3 M 6.4 against 5.4).
+    constexpr int PARTS = EL / W::VEC, DWORDS = W::VEC * ITEM / 4;
+    uint32_t held[PARTS][DWORDS];
 #pragma unroll
-    for (int tile = 0; tile < TILES; ++tile) {
+    for (int part = 0; part < PARTS; ++part)
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) raws[tile][i] = 0;
-        const int64_t e0 = first + tile * TILE + lane * VEC;
-        // numel is a multiple of G: dead lanes form whole dead groups.  Instruction-bound: a cache hint only costs.
-        if (e0 < a.numel) {
+        for (int i = 0; i < DWORDS; ++i) held[part][i] = 0;
+    if (live) {   // instruction-bound: a cache hint only costs
 #pragma unroll
-            for (int part = 0; part < EL / W::VEC; ++part) {
-                Raw piece[W::VEC];
-                load_elems<Raw, W::VEC, kPlain>(static_cast<const Raw *>(a.x) + e0 + part * W::VEC, piece);
-#pragma unroll
-                for (int i = 0; i < W::VEC; ++i) raws[tile][part * W::VEC + i] = piece[i];
-            }
-        }
+        for (int part = 0; part < PARTS; ++part)
+            load_words<DWORDS, ITEM, kPlain>(reinterpret_cast<const uint8_t *>(static_cast<const Raw *>(a.x) + e0 + part * W::VEC), held[part]);
     }
     const book_cells::Cell *cells = nullptr;
     if constexpr (BY_CELLS) cells = block_cells.publish();
-    if (first >= a.numel) return;   // wavefront-uniform, behind the workgroup's barrier
+    if (tile_first >= a.numel) return;   // wavefront-uniform, behind the workgroup's barrier
     const float *book = BY_CELLS ? nullptr : wave_code_book(kind, lane);
 
-    auto encode_tile = [&](const int64_t tile_first, const Raw (&raw)[VEC]) __attribute__((always_inline)) {
-        const int64_t e0 = tile_first + lane * VEC;
-        const bool live = e0 < a.numel;
-        const int64_t group = e0 / G;
-        const int k0 = static_cast<int>(e0 - group * G);
-        const int start = scan_start<T, G>(group);
-        // The draws depend on the element's place only: they are computed while its value is still on its way.
-        float uniform[VEC];
+    const int64_t group = e0 / G;
+    const int k0 = static_cast<int>(e0 - group * G);
+    const int start = scan_start<T, G>(group);
+    // The draws depend on the element's place only: they are computed while its value is still on its way.
+    float uniform[VEC];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) uniform[i] = 0.0f;
-        if (stochastic) {
-            const uint32_t key0 = static_cast<uint32_t>(a.seed), key1 = static_cast<uint32_t>(a.seed >> 32);
-            const uint32_t sub0 = static_cast<uint32_t>(group), sub1 = static_cast<uint32_t>(static_cast<uint64_t>(group) >> 32);
-            const int phase = static_cast<int>(a.offset & 3);
-            // curand_uniform, (0, 1]: x * 2^-32 + 2^-33.  The product is exact, so the fused form rounds as the two steps do.
-            auto to_uniform = [](uint32_t x) { return __builtin_fmaf(static_cast<float>(x), 0x1p-32f, 0x1p-33f); };
-            uint64_t block[VEC / 4];
+    for (int i = 0; i < VEC; ++i) uniform[i] = 0.0f;
+    if (stochastic) {
+        const uint32_t key0 = static_cast<uint32_t>(a.seed), key1 = static_cast<uint32_t>(a.seed >> 32);
+        const uint32_t sub0 = static_cast<uint32_t>(group), sub1 = static_cast<uint32_t>(static_cast<uint64_t>(group) >> 32);
+        const int phase = static_cast<int>(a.offset & 3);
+        // curand_uniform, (0, 1]: x * 2^-32 + 2^-33.  The product is exact, so the fused form rounds as the two steps do.
+        auto to_uniform = [](uint32_t x) { return __builtin_fmaf(static_cast<float>(x), 0x1p-32f, 0x1p-33f); };
+        uint64_t block[VEC / 4];
+#pragma unroll
+        for (int q = 0; q < VEC / 4; ++q)
+            block[q] = (a.offset + static_cast<uint64_t>((k0 + 4 * q - start) & (G - 1))) >> 2;   // positions are multiples of 4
+        uint32_t lo[VEC / 4][4];
+#pragma unroll
+        for (int q = 0; q < VEC / 4; ++q)
+            philox_block(static_cast<uint32_t>(block[q]), static_cast<uint32_t>(block[q] >> 32), sub0, sub1, key0, key1, lo[q]);
+        if (phase == 0) {   // uniform; the offsets torch hands out are multiples of four: one block a quad
 #pragma unroll
             for (int q = 0; q < VEC / 4; ++q)
-                block[q] = (a.offset + static_cast<uint64_t>((k0 + 4 * q - start) & (G - 1))) >> 2;   // positions are multiples of 4
-            uint32_t lo[VEC / 4][4];
 #pragma unroll
-            for (int q = 0; q < VEC / 4; ++q)
-                philox_block(static_cast<uint32_t>(block[q]), static_cast<uint32_t>(block[q] >> 32), sub0, sub1, key0, key1, lo[q]);
-            if (phase == 0) {   // uniform; the offsets torch hands out are multiples of four: one block a quad
+                for (int e = 0; e < 4; ++e) uniform[4 * q + e] = to_uniform(lo[q][e]);
+        } else {            // a quad's draws lie across two blocks
 #pragma unroll
-                for (int q = 0; q < VEC / 4; ++q)
+            for (int q = 0; q < VEC / 4; ++q) {
+                uint32_t hi[4];
+                philox_block(static_cast<uint32_t>(block[q] + 1), static_cast<uint32_t>((block[q] + 1) >> 32), sub0, sub1,
+                             key0, key1, hi);
+                const uint32_t w[8] = {lo[q][0], lo[q][1], lo[q][2], lo[q][3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) uniform[4 * q + e] = to_uniform(lo[q][e]);
-            } else {            // a quad's draws lie across two blocks
-#pragma unroll
-                for (int q = 0; q < VEC / 4; ++q) {
-                    uint32_t hi[4];
-                    philox_block(static_cast<uint32_t>(block[q] + 1), static_cast<uint32_t>((block[q] + 1) >> 32), sub0, sub1,
-                                 key0, key1, hi);
-                    const uint32_t w[8] = {lo[q][0], lo[q][1], lo[q][2], lo[q][3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        uniform[4 * q + e] = to_uniform(phase == 1 ? w[e + 1] : (phase == 2 ? w[e + 2] : w[e + 3]));
-                }
+                for (int e = 0; e < 4; ++e)
+                    uniform[4 * q + e] = to_uniform(phase == 1 ? w[e + 1] : (phase == 2 ? w[e + 2] : w[e + 3]));
             }
         }
+    }
 
-        float v[VEC];
-        uint32_t mag[VEC];
+    Raw raw[VEC];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-            v[i] = value_of<T>(raw[i]);
-            mag[i] = raw[i] & RB::ABS;
-        }
+    for (int i = 0; i < VEC; ++i)
+        raw[i] = static_cast<Raw>(held[i / W::VEC][i % W::VEC * ITEM / 4] >> (ITEM == 2 && (i & 1) ? 16 : 0));
+    float v[VEC];
+    uint32_t mag[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        v[i] = value_of<T>(raw[i]);
+        mag[i] = raw[i] & RB::ABS;
+    }
 
-        uint8_t *group_codes = a.payload + (a.compact ? group * (CB + meta_bytes) : group * CB);
-        uint8_t *group_meta = a.compact ? group_codes + CB : a.payload + groups * CB + group * meta_bytes;
+    uint8_t *group_codes = a.payload + (a.compact ? group * (CB + meta_bytes) : group * CB);
+    uint8_t *group_meta = a.compact ? group_codes + CB : a.payload + groups * CB + group * meta_bytes;
 
-        uint32_t scale_raw;
-        Raw meta[4] = {0, 0, 0, 0};   // [scale][indices][top1][top2]
-        bool any_nan = true;   // "not known": the outlier path does not look
-        uint32_t outlier[2] = {~0u, ~0u};   // place among the lane's elements, beyond them when another lane's
-        if (FIXED != 6 && topk == 0) {
-            scale_raw = running_max_raw<T, G, VEC>(mag, k0, start, &any_nan);
-        } else {
-            // The three largest candidates of the group, a candidate's key being its magnitude and a tie-break rank
-            // (1..G, unique inside a group; the larger rank wins).
-            uint32_t best_key[3] = {0, 0, 0}, best_rank[2] = {0, 0};              // magnitude + 1, rank
-            if constexpr (WIDE) {
-                // Three rounds of "largest remaining candidate": the group maximum of the magnitude keys, then, among
-                // the elements that hold it, the maximum of the ranks.
-                uint32_t key[VEC], rank[VEC];
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    rank[i] = static_cast<uint32_t>(k0 + i + 1);
-                    key[i] = mag[i] <= RB::INF ? mag[i] + 1 : 0;                  // 0 stands for "none"
-                }
-#pragma unroll
-                for (int round = 0; round < 3; ++round) {
-                    if (round == 2 && topk == 1) break;                         // uniform
-                    uint32_t m = 0;
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) m = key[i] > m ? key[i] : m;
-                    m = group_max_bits<LPG>(m);
-                    best_key[round] = m;
-                    if (round == 2) break;
-                    uint32_t r = 0;
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) r = (key[i] == m && rank[i] > r) ? rank[i] : r;
-                    r = group_max_bits<LPG>(r);
-                    r = m == 0 ? 0 : r;
-                    best_rank[round] = r;
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) key[i] = rank[i] == r ? 0 : key[i];   // taken (r = 0 matches nobody)
-                }
-            } else {
-                // A 16-bit magnitude and its rank less one share one 32-bit key, the magnitude in the upper half, unique
-                // inside the group: the element's bits with the sign masked out (in place for the upper half of a loaded
-                // dword) and the rank or-ed in, the quad's part and the constant part apart.  A lane keeps the three
-                // largest of its own keys in order (three instructions an element), and the group's lanes merge their
-                // triples over the DPP butterfly (eight instructions a step): no rounds over the elements.  Zeros are no
-                // candidates: their keys are below 2^16, under every candidate's, and are dropped from the result.  NaNs are no candidates either and their keys are above every
-                // candidate's: the first pass does not look for them, and when one tops any group of the wavefront
-                // (rare) the pass is repeated with every element checked.  Scan positions do not wrap inside four
-                // adjacent elements (a lane's first element and the scan's start are multiples of four).
-                constexpr uint32_t kBelow = 1u << 16, kAbove = (RB::INF << 16) | 0xFFFFu;
-                uint32_t largest, runner_up, bronze;
-                auto search = [&](const bool checked) __attribute__((always_inline)) {
-                    largest = runner_up = bronze = 0;
-                    const uint32_t p0 = static_cast<uint32_t>(k0 - start) & (G - 1);
-#pragma unroll
-                    for (int q = 0; q < VEC / 4; ++q) {
-                        const uint32_t rank0 = (G - 4) ^ ((p0 + 4 * q) & (G - 1));   // rank - 1 = G - 1 - scan position
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int i = 4 * q + j;
-                            uint32_t key = (static_cast<uint32_t>(raw[i]) << 16 & 0x7FFF0000u) | rank0 | (3 - j);
-                            if (checked) key = (key >> 16) - 1u < RB::INF ? key : 0;
-                            bronze = umed3(runner_up, bronze, key);
-                            runner_up = umed3(largest, runner_up, key);
-                            largest = key > largest ? key : largest;
-                        }
-                    }
-                    merge_top3<LPG>(largest, runner_up, bronze);
-                };
-                search(false);
-                if (__ballot(largest > kAbove) != 0) search(true);   // wavefront-uniform
-                largest = largest < kBelow ? 0 : largest;
-                runner_up = runner_up < kBelow ? 0 : runner_up;
-                bronze = bronze < kBelow ? 0 : bronze;
-                const uint32_t found[3] = {largest, runner_up, bronze};
-#pragma unroll
-                for (int round = 0; round < 3; ++round) {
-                    best_key[round] = found[round] == 0 ? 0 : (found[round] >> 16) + 1;
-                    if (round < 2) best_rank[round] = found[round] == 0 ? 0 : (found[round] & 0xFFFFu) + 1;
-                }
-            }
-            auto index_of = [&](uint32_t r) {
-                return WIDE ? static_cast<int>(r) - 1 : ((G - static_cast<int>(r)) + start) & (G - 1);
-            };
-            const bool none = best_key[0] == 0;
-            const int index1 = none ? 0 : index_of(best_rank[0]);
-            int index2 = -1;
-            if (topk == 1) {
-                // nothing comparable: the reference falls back to element 1 (as stored for fp32, its magnitude otherwise)
-                const uint32_t element1 = WIDE ? static_cast<uint32_t>(raw[1]) : raw[1] & RB::ABS;
-                const uint32_t fallback = static_cast<uint32_t>(__shfl(static_cast<int>(element1), lane & ~(LPG - 1)));
-                scale_raw = none ? fallback : (best_key[1] == 0 ? 0u : best_key[1] - 1);
-            } else {
-                const bool lonely = !none && best_key[1] == 0;
-                index2 = none ? 1 : (lonely ? ((index1 + 1) & (G - 1)) : index_of(best_rank[1]));
-                scale_raw = (none || lonely || best_key[2] == 0) ? 0u : best_key[2] - 1;
-            }
-            // Outliers encode as 0.  A code book needs the elements gone (they lie above the scale); linear codes, which a
-            // zero element always turns into 0 (the noise stays within +-1/2, which rounds to 0), are cleared in the
-            // packed words: five instructions a word instead of three an element.
-            if constexpr (FIXED & 4) {
-                outlier[0] = static_cast<uint32_t>(index1 - k0);
-                outlier[1] = static_cast<uint32_t>(index2 - k0);
-            } else {
-#pragma unroll
-                for (int i = 0; i < VEC; ++i)
-                    if (k0 + i == index1 || k0 + i == index2) v[i] = 0.0f;
-            }
-            // The outliers travel as they are stored.  The group's first lane fetches them from the tensor once more
-            // (its wavefront has just read those lines) instead of every lane selecting among its elements; the
-            // metadata words leave together at the end of the tile, when the values have long arrived.
-            meta[1] = static_cast<Raw>(topk == 1 ? index1 : (index1 | (index2 << 8)));
-            if (live && k0 == 0) {
-                const Raw *members = static_cast<const Raw *>(a.x) + group * G;
-                meta[2] = members[index1];
-                if (topk == 2) meta[3] = members[index2];
-            }
-        }
-        meta[0] = static_cast<Raw>(scale_raw);
-        auto store_meta = [&]() __attribute__((always_inline)) {
-            if (live && k0 == 0) {
-                Raw *words = reinterpret_cast<Raw *>(group_meta);
-                if (topk == 2) {
-                    store_elems<Raw, 4, kPlain>(words, meta);
-                } else if (topk == 1) {
-                    const Raw pair[2] = {meta[0], meta[1]};
-                    store_elems<Raw, 2, kPlain>(words, pair);
-                    words[2] = meta[2];
-                } else {
-                    words[0] = meta[0];
-                }
-            }
-        };
-
-        float scale = value_of<T>(scale_raw);
-        scale = scale < 1.0e-6f ? 1.0e-6f : scale;   // a NaN scale stays NaN and encodes every element as 0
-
-        if constexpr (BY_CELLS) {
-            // A code book, rounded to nearest (uniform: kind is not 0).  The cell lookup answers v / scale without forming
-            // the quotient: per element a fused multiply-add and an address, one LDS read, and four operations that leave
-            // the comparison with the step in a sign bit and push it and the cell's code into a word of eight.  It
-            // holds for a scale within 2^60 of 1 either way and |v| <= scale; the scale is at least 1e-6 here, and beside
-            // outliers or a NaN an element may lie above it.  A wavefront with any other operand divides, and looks the
-            // quotient up with scale 1; what lies outside [-1, 1] takes the first or last code, a NaN the last, as the search
-            // does.  9 instead of 21 instructions an element: 26.2 M elements of the normal book 24.5 -> 21.3 us (fp32, 119
-            // MB, 5.6 TB/s) and 19.9 -> 14.2 us (bf16), with two outliers 32.5 -> 27.5 and 30.0 -> 21.0; what is left of the
-            // difference to the linear 4-bit pack kernel (19.6 and 13.0) is the table, 2 KiB copied per 2048 or 4096
-            // elements (by workgroups half and a quarter as large: 25.8 and 29.4 us, fp32).
-            const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
-            bool unusual = scale_exponent > 127u + 60u;
-            if (any_nan) {   // wavefront-uniform
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
-            }
-            float divisor = scale;
-            if (__ballot(unusual) != 0) {   // wavefront-uniform
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    const float t = v[i] / scale;
-                    v[i] = t < 1.0f ? (t > -1.0f ? t : -1.0f) : 1.0f;
-                }
-                divisor = 1.0f;
-            }
-            const float reciprocal128 = __builtin_amdgcn_rcpf(divisor) * 128.0f, divisor24 = divisor * 0x1p-24f;
-            if (live) {
-                uint32_t words[WORDS];
-#pragma unroll
-                for (int k = 0; k < WORDS; ++k) {
-                    uint32_t codes = 0, below = 0;
-#pragma unroll
-                    for (int i = 8 * k; i < 8 * k + 8; ++i) {
-                        const book_cells::Cell cell = cells[book_cells::nearest_place(v[i], reciprocal128) - book_cells::kPlaceBits];
-                        const float sign = book_cells::reaches(cell.threshold, v[i], divisor, divisor24);
-                        codes = __builtin_amdgcn_alignbit(codes, cell.base, 28);          // (codes << 4) | code + 1
-                        below = __builtin_amdgcn_alignbit(below, as_u32(sign), 28);
-                    }
-                    codes -= (below >> 3) & 0x11111111u;
-                    words[k] = WIDE ? codes : __builtin_amdgcn_alignbit(codes, codes, 16);
-                }
-                store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
-            }
-            store_meta();
-            return;
-        }
-
-        int c[VEC];
-        if (kind == 0) {
-            const float multiplier = W::LEVELS / scale;
-            constexpr int L = static_cast<int>(W::LEVELS);
-            // Beside outliers and NaNs no magnitude exceeds the scale, so the product stays within the levels and adding
-            // 1.5 * 2^23 leaves its rounding, half to even, in the low bits: two instructions an element instead of four
-            // with conversion and clamp.  An outlier's code is cleared below; a NaN of a 16-bit type has zeros there.
-            // With the search's keys and the clearing of words this took the kernel, bound by instructions, from 20.2 to
-            // 17 us on 26.2 M bf16 elements with two outliers (the round trip 31.9 to 28.6).
-            constexpr bool kByAddition = FIXED == 6 && !WIDE;
-#pragma unroll
-            for (int i = 0; kByAddition && i < VEC; ++i) c[i] = static_cast<int>(as_u32(v[i] * multiplier + 0x1.8p23f));
-#pragma unroll
-            for (int i = 0; !kByAddition && i < VEC; ++i) {
-                // nvcc contracts v * m + noise into one FMA; without noise the product is rounded alone
-                const float t = stochastic ? __builtin_fmaf(v[i], multiplier, uniform[i] - 0.5f) : v[i] * multiplier;
-                const int r = cvt_i32(__builtin_rintf(t));
-                c[i] = r < -L ? -L : (r > L ? L : r);
-            }
-        } else {
-            // t = v / scale, the IEEE quotient.  A lane's elements share the divisor, so the reciprocal part of the
-            // division is done once: v_rcp_f32 and one Newton step, then per element the product and two corrections.
-            // These are the very operations the compiler emits for `v / scale`, minus its operand scaling and
-            // special-case fix-up (v_div_scale / v_div_fmas / v_div_fixup), which change nothing while the divisor
-            // lies in [2^-60, 2^60], |v| <= scale, and the dividend is not so small (below 2^-103) that the division
-            // would rescale it.  The scale is at least 1e-6 here, so such a dividend means a quotient below 2^-80, and a
-            // quotient below 2^-30 encodes as the book's zero whatever its last bits are: it is closer to that entry
-            // than the rounding error of the comparisons with its neighbours.  A wavefront with any other divisor,
-            // or with an element above its scale (only a group that holds a NaN has one) or not a number, takes the
-            // division.  tests/native/quotient_check.hip compares the two forms on the device.
-            float t[VEC];
-            const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
-            bool unusual = scale_exponent < 127u - 60u || scale_exponent > 127u + 60u;
-            // Without outliers the scale is the group's largest magnitude unless a NaN reset the running maximum, and
-            // the wavefront is known to hold no NaN: no element needs to be looked at.
-            if (any_nan) {   // wavefront-uniform
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
-            }
-            const bool usual = __ballot(unusual) == 0;   // wavefront-uniform
-            if (usual) {
-                float reciprocal = __builtin_amdgcn_rcpf(scale);
-                reciprocal = __builtin_fmaf(__builtin_fmaf(-scale, reciprocal, 1.0f), reciprocal, reciprocal);
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    float q = v[i] * reciprocal;
-                    q = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
-                    t[i] = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) t[i] = v[i] / scale;
-            }
-            // The largest entry in [0, 14] with not (t < book[entry]); a NaN ends at 14.  Four halving steps, each
-            // over all of the lane's elements so that their LDS reads are in flight together; positions are kept as
-            // byte offsets into the book.
-            const char *book_bytes = reinterpret_cast<const char *>(book);
-            int at[VEC];
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) at[i] = 0;
-#pragma unroll
-            for (int step = 8 * 4; step >= 4; step >>= 1) {
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    const int mid = at[i] + step;
-                    const float entry = *reinterpret_cast<const float *>(book_bytes + mid);
-                    at[i] = (mid < 15 * 4 && !(t[i] < entry)) ? mid : at[i];
-                }
-            }
-            float excess[VEC], gap[VEC];
+    uint32_t scale_raw;
+    Raw meta[4] = {0, 0, 0, 0};   // [scale][indices][top1][top2]
+    bool any_nan = true;   // "not known": the outlier path does not look
+    uint32_t outlier[2] = {~0u, ~0u};   // place among the lane's elements, beyond them when another lane's
+    if (FIXED != 6 && topk == 0) {
+        scale_raw = running_max_raw<T, G, VEC>(mag, k0, start, &any_nan);
+    } else {
+        // The three largest candidates of the group, a candidate's key being its magnitude and a tie-break rank
+        // (1..G, unique inside a group; the larger rank wins).  The sign travels below the rank, so that what the search
+        // finds is the element itself: fetched from the tensor once more, at the end of a wavefront's chain, the two
+        // outliers of a group made the 16-bit kernel 14 % slower (26.2 M bf16 elements 19.5 against 17.1 us).
+        uint32_t best_key[3] = {0, 0, 0}, best_rank[2] = {0, 0};              // magnitude + 1, rank
+        uint32_t best_raw[2] = {0, 0};                                        // the element as stored
+        if constexpr (WIDE) {
+            // Three rounds of "largest remaining candidate": the group maximum of the magnitude keys, then, among
+            // the elements that hold it, the maximum of the ranks.
+            uint32_t key[VEC], rank[VEC];
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
-                const float low = *reinterpret_cast<const float *>(book_bytes + at[i]);
-                gap[i] = *reinterpret_cast<const float *>(book_bytes + at[i] + 4) - low;
-                excess[i] = t[i] - low;
-                c[i] = at[i] >> 2;
+                rank[i] = __builtin_amdgcn_alignbit(static_cast<uint32_t>(k0 + i + 1), raw[i], 31);   // sign below it
+                key[i] = mag[i] <= RB::INF ? mag[i] + 1 : 0;                  // 0 stands for "none"
             }
-            if (stochastic) {   // uniform: the second division only runs when it is needed
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) c[i] += uniform[i] < excess[i] / gap[i] ? 1 : 0;
-            } else {
+            for (int round = 0; round < 3; ++round) {
+                if (round == 2 && topk == 1) break;                         // uniform
+                uint32_t m = 0;
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) c[i] += excess[i] > gap[i] * 0.5f ? 1 : 0;
+                for (int i = 0; i < VEC; ++i) m = key[i] > m ? key[i] : m;
+                m = group_max_bits<LPG>(m);
+                best_key[round] = m;
+                if (round == 2) break;
+                uint32_t r = 0;
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) r = (key[i] == m && rank[i] > r) ? rank[i] : r;
+                r = group_max_bits<LPG>(r);
+                r = m == 0 ? 0 : r;
+                best_rank[round] = r >> 1;
+                best_raw[round] = (m - 1) | (r << 31);
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) key[i] = rank[i] == r ? 0 : key[i];   // taken (r = 0 matches nobody)
+            }
+        } else {
+            // A 16-bit magnitude, its rank less one and its sign share one 32-bit key, unique inside the group: the
+            // loaded dword rotated so that the magnitude lies on top and the sign at the bottom, the rest masked out
+            // and the rank or-ed in, the quad's part and the constant part apart.  A lane keeps the three
+            // largest of its own keys in order (three instructions an element), and the group's lanes merge their
+            // triples over the DPP butterfly (eight instructions a step): no rounds over the elements.  Zeros are no
+            // candidates: their keys are below 2^17, under every candidate's, and are dropped from the result.  NaNs are no candidates either and their keys are above every
+            // candidate's: the first pass does not look for them, and when one tops any group of the wavefront
+            // (rare) the pass is repeated with every element checked.  Scan positions do not wrap inside four
+            // adjacent elements (a lane's first element and the scan's start are multiples of four).
+            constexpr uint32_t kBelow = 1u << 17, kAbove = (RB::INF << 17) | 0x1FFFFu;
+            uint32_t largest, runner_up, bronze;
+            auto search = [&](const bool checked) __attribute__((always_inline)) {
+                largest = runner_up = bronze = 0;
+                const uint32_t p0 = static_cast<uint32_t>(k0 - start) & (G - 1);
+#pragma unroll
+                for (int q = 0; q < VEC / 4; ++q) {
+                    const uint32_t rank0 = (G - 4) ^ ((p0 + 4 * q) & (G - 1));   // rank - 1 = G - 1 - scan position
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int i = 4 * q + j;
+                        const uint32_t pair = static_cast<uint32_t>(raw[i & ~1]) | static_cast<uint32_t>(raw[i | 1]) << 16;
+                        const uint32_t turned = __builtin_amdgcn_alignbit(pair, pair, (i & 1) ? 31 : 15);
+                        uint32_t key = (turned & 0xFFFE0001u) | (rank0 << 1) | (2 * (3 - j));
+                        if (checked) key = (key >> 17) - 1u < RB::INF ? key : 0;
+                        bronze = umed3(runner_up, bronze, key);
+                        runner_up = umed3(largest, runner_up, key);
+                        largest = key > largest ? key : largest;
+                    }
+                }
+                merge_top3<LPG>(largest, runner_up, bronze);
+            };
+            search(false);
+            if (__ballot(largest > kAbove) != 0) search(true);   // wavefront-uniform
+            largest = largest < kBelow ? 0 : largest;
+            runner_up = runner_up < kBelow ? 0 : runner_up;
+            bronze = bronze < kBelow ? 0 : bronze;
+            const uint32_t found[3] = {largest, runner_up, bronze};
+#pragma unroll
+            for (int round = 0; round < 3; ++round) {
+                best_key[round] = found[round] == 0 ? 0 : (found[round] >> 17) + 1;
+                if (round < 2) {
+                    best_rank[round] = found[round] == 0 ? 0 : ((found[round] & 0x1FFFFu) >> 1) + 1;
+                    best_raw[round] = (found[round] >> 17) | (found[round] << 15);
+                }
             }
         }
+        auto index_of = [&](uint32_t r) {
+            return WIDE ? static_cast<int>(r) - 1 : ((G - static_cast<int>(r)) + start) & (G - 1);
+        };
+        const bool none = best_key[0] == 0, second_missing = best_key[1] == 0;
+        const int index1 = none ? 0 : index_of(best_rank[0]);
+        int index2 = -1;
+        if (topk == 1) {
+            // nothing comparable: the reference falls back to element 1 (as stored for fp32, its magnitude otherwise)
+            const uint32_t element1 = WIDE ? static_cast<uint32_t>(raw[1]) : raw[1] & RB::ABS;
+            const uint32_t fallback = static_cast<uint32_t>(__shfl(static_cast<int>(element1), lane & ~(LPG - 1)));
+            scale_raw = none ? fallback : (best_key[1] == 0 ? 0u : best_key[1] - 1);
+        } else {
+            const bool lonely = !none && best_key[1] == 0;
+            index2 = none ? 1 : (lonely ? ((index1 + 1) & (G - 1)) : index_of(best_rank[1]));
+            scale_raw = (none || lonely || best_key[2] == 0) ? 0u : best_key[2] - 1;
+        }
+        // Outliers encode as 0.  A code book needs the elements gone (they lie above the scale); linear codes, which a
+        // zero element always turns into 0 (the noise stays within +-1/2, which rounds to 0), are cleared in the
+        // packed words: five instructions a word instead of three an element.
+        if constexpr (FIXED & 4) {
+            outlier[0] = static_cast<uint32_t>(index1 - k0);
+            outlier[1] = static_cast<uint32_t>(index2 - k0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i)
+                if (k0 + i == index1 || k0 + i == index2) v[i] = 0.0f;
+        }
+        meta[1] = static_cast<Raw>(topk == 1 ? index1 : (index1 | (index2 << 8)));
+        meta[2] = static_cast<Raw>(best_raw[0]);
+        meta[3] = static_cast<Raw>(best_raw[1]);
+        if (live && k0 == 0 && (none || second_missing)) {   // rare: an index that the search did not give
+            const Raw *members = static_cast<const Raw *>(a.x) + group * G;
+            meta[2] = members[index1];
+            if (topk == 2) meta[3] = members[index2];
+        }
+    }
+    meta[0] = static_cast<Raw>(scale_raw);
+    auto store_meta = [&]() __attribute__((always_inline)) {
+        if (live && k0 == 0) {
+            Raw *words = reinterpret_cast<Raw *>(group_meta);
+            if (topk == 2) {
+                store_elems<Raw, 4, kPlain>(words, meta);
+            } else if (topk == 1) {
+                const Raw pair[2] = {meta[0], meta[1]};
+                store_elems<Raw, 2, kPlain>(words, pair);
+                words[2] = meta[2];
+            } else {
+                words[0] = meta[0];
+            }
+        }
+    };
+
+    float scale = value_of<T>(scale_raw);
+    scale = scale < 1.0e-6f ? 1.0e-6f : scale;   // a NaN scale stays NaN and encodes every element as 0
+
+    if constexpr (BY_CELLS) {
+        // A code book, rounded to nearest (uniform: kind is not 0).  The cell lookup answers v / scale without forming
+        // the quotient: per element a fused multiply-add and an address, one LDS read, and four operations that leave
+        // the comparison with the step in a sign bit and push it and the cell's code into a word of eight.  It
+        // holds for a scale within 2^60 of 1 either way and |v| <= scale; the scale is at least 1e-6 here, and beside
+        // outliers or a NaN an element may lie above it.  A wavefront with any other operand divides, and looks the
+        // quotient up with scale 1; what lies outside [-1, 1] takes the first or last code, a NaN the last, as the search
+        // does.  9 instead of 21 instructions an element: 26.2 M elements of the normal book 24.5 -> 21.3 us (fp32, 119
+        // MB, 5.6 TB/s) and 19.9 -> 14.2 us (bf16), with two outliers 32.5 -> 27.5 and 30.0 -> 21.0; what is left of the
+        // difference to the linear 4-bit pack kernel (19.6 and 13.0) is the table, 2 KiB copied per 2048 or 4096
+        // elements (by workgroups half and a quarter as large: 25.8 and 29.4 us, fp32).
+        const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
+        bool unusual = scale_exponent > 127u + 60u;
+        if (any_nan) {   // wavefront-uniform
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
+        }
+        float divisor = scale;
+        if (__ballot(unusual) != 0) {   // wavefront-uniform
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                const float t = v[i] / scale;
+                v[i] = t < 1.0f ? (t > -1.0f ? t : -1.0f) : 1.0f;
+            }
+            divisor = 1.0f;
+        }
+        const float reciprocal128 = __builtin_amdgcn_rcpf(divisor) * 128.0f, divisor24 = divisor * 0x1p-24f;
         if (live) {
             uint32_t words[WORDS];
-            if constexpr (BIT == 8) pack_codes<T, 8, VEC, WORDS>(c, words);
-            else pack_nibbles<T, EL>(c, words);
-            if constexpr ((FIXED & 5) == 4) {
-                constexpr uint32_t PER_WORD = 32 / BIT, ORDER = BIT == 8 ? (WIDE ? 3 : 1) : (WIDE ? 7 : 3);   // place in a word
-                uint32_t code[2];
 #pragma unroll
-                for (int k = 0; k < 2; ++k) code[k] = ((1u << BIT) - 1) << (((outlier[k] ^ ORDER) * BIT) & 31u);
+            for (int k = 0; k < WORDS; ++k) {
+                uint32_t codes = 0, below = 0;
 #pragma unroll
-                for (uint32_t w = 0; w < WORDS; ++w)
-                    words[w] &= ~((outlier[0] / PER_WORD == w ? code[0] : 0u) | (outlier[1] / PER_WORD == w ? code[1] : 0u));
+                for (int i = 8 * k; i < 8 * k + 8; ++i) {
+                    const book_cells::Cell cell = cells[book_cells::nearest_place(v[i], reciprocal128) - book_cells::kPlaceBits];
+                    const float sign = book_cells::reaches(cell.threshold, v[i], divisor, divisor24);
+                    codes = __builtin_amdgcn_alignbit(codes, cell.base, 28);          // (codes << 4) | code + 1
+                    below = __builtin_amdgcn_alignbit(below, as_u32(sign), 28);
+                }
+                codes -= (below >> 3) & 0x11111111u;
+                words[k] = WIDE ? codes : __builtin_amdgcn_alignbit(codes, codes, 16);
             }
             store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
         }
         store_meta();
-    };
-#pragma unroll
-    for (int tile = 0; tile < TILES; ++tile) {
-        const int64_t tile_first = first + tile * TILE;
-        if (tile_first >= a.numel) return;   // wavefront-uniform
-        encode_tile(tile_first, raws[tile]);
+        return;
     }
+
+    int c[VEC];
+    if (kind == 0) {
+        const float multiplier = W::LEVELS / scale;
+        constexpr int L = static_cast<int>(W::LEVELS);
+        // Beside outliers and NaNs no magnitude exceeds the scale, so the product stays within the levels and adding
+        // 1.5 * 2^23 leaves its rounding, half to even, in the low bits: two instructions an element instead of four
+        // with conversion and clamp.  An outlier's code is cleared below; a NaN of a 16-bit type has zeros there.
+        // With the search's keys and the clearing of words this took the kernel, bound by instructions, from 20.2 to
+        // 17 us on 26.2 M bf16 elements with two outliers (the round trip 31.9 to 28.6).
+        constexpr bool kByAddition = FIXED == 6 && !WIDE;
+#pragma unroll
+        for (int i = 0; kByAddition && i < VEC; ++i) c[i] = static_cast<int>(as_u32(v[i] * multiplier + 0x1.8p23f));
+#pragma unroll
+        for (int i = 0; !kByAddition && i < VEC; ++i) {
+            // nvcc contracts v * m + noise into one FMA; without noise the product is rounded alone
+            const float t = stochastic ? __builtin_fmaf(v[i], multiplier, uniform[i] - 0.5f) : v[i] * multiplier;
+            const int r = cvt_i32(__builtin_rintf(t));
+            c[i] = r < -L ? -L : (r > L ? L : r);
+        }
+    } else {
+        // t = v / scale, the IEEE quotient.  A lane's elements share the divisor, so the reciprocal part of the
+        // division is done once: v_rcp_f32 and one Newton step, then per element the product and two corrections.
+        // These are the very operations the compiler emits for `v / scale`, minus its operand scaling and
+        // special-case fix-up (v_div_scale / v_div_fmas / v_div_fixup), which change nothing while the divisor
+        // lies in [2^-60, 2^60], |v| <= scale, and the dividend is not so small (below 2^-103) that the division
+        // would rescale it.  The scale is at least 1e-6 here, so such a dividend means a quotient below 2^-80, and a
+        // quotient below 2^-30 encodes as the book's zero whatever its last bits are: it is closer to that entry
+        // than the rounding error of the comparisons with its neighbours.  A wavefront with any other divisor,
+        // or with an element above its scale (only a group that holds a NaN has one) or not a number, takes the
+        // division.  tests/native/quotient_check.hip compares the two forms on the device.
+        float t[VEC];
+        const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
+        bool unusual = scale_exponent < 127u - 60u || scale_exponent > 127u + 60u;
+        // Without outliers the scale is the group's largest magnitude unless a NaN reset the running maximum, and
+        // the wavefront is known to hold no NaN: no element needs to be looked at.
+        if (any_nan) {   // wavefront-uniform
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
+        }
+        const bool usual = __ballot(unusual) == 0;   // wavefront-uniform
+        if (usual) {
+            float reciprocal = __builtin_amdgcn_rcpf(scale);
+            reciprocal = __builtin_fmaf(__builtin_fmaf(-scale, reciprocal, 1.0f), reciprocal, reciprocal);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                float q = v[i] * reciprocal;
+                q = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
+                t[i] = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) t[i] = v[i] / scale;
+        }
+        // The largest entry in [0, 14] with not (t < book[entry]); a NaN ends at 14.  Four halving steps, each
+        // over all of the lane's elements so that their LDS reads are in flight together; positions are kept as
+        // byte offsets into the book.
+        const char *book_bytes = reinterpret_cast<const char *>(book);
+        int at[VEC];
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) at[i] = 0;
+#pragma unroll
+        for (int step = 8 * 4; step >= 4; step >>= 1) {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                const int mid = at[i] + step;
+                const float entry = *reinterpret_cast<const float *>(book_bytes + mid);
+                at[i] = (mid < 15 * 4 && !(t[i] < entry)) ? mid : at[i];
+            }
+        }
+        float excess[VEC], gap[VEC];
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+            const float low = *reinterpret_cast<const float *>(book_bytes + at[i]);
+            gap[i] = *reinterpret_cast<const float *>(book_bytes + at[i] + 4) - low;
+            excess[i] = t[i] - low;
+            c[i] = at[i] >> 2;
+        }
+        if (stochastic) {   // uniform: the second division only runs when it is needed
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) c[i] += uniform[i] < excess[i] / gap[i] ? 1 : 0;
+        } else {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) c[i] += excess[i] > gap[i] * 0.5f ? 1 : 0;
+        }
+    }
+    if (live) {
+        uint32_t words[WORDS];
+        if constexpr (BIT == 8) pack_codes<T, 8, VEC, WORDS>(c, words);
+        else pack_nibbles<T, EL>(c, words);
+        if constexpr ((FIXED & 5) == 4) {
+            constexpr uint32_t PER_WORD = 32 / BIT, ORDER = BIT == 8 ? (WIDE ? 3 : 1) : (WIDE ? 7 : 3);   // place in a word
+            uint32_t code[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) code[k] = ((1u << BIT) - 1) << (((outlier[k] ^ ORDER) * BIT) & 31u);
+#pragma unroll
+            for (uint32_t w = 0; w < WORDS; ++w)
+                words[w] &= ~((outlier[0] / PER_WORD == w ? code[0] : 0u) | (outlier[1] / PER_WORD == w ? code[1] : 0u));
+        }
+        store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
+    }
+    store_meta();
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -644,30 +646,29 @@ __global__ __launch_bounds__(kBlock) void wire_general_decode_kernel(const WireG
     store_elems<Raw, VEC, kNonTemporal>(out, decoded);
 }
 
-template <typename T, int G, int BIT, int FIXED, int EL, int TILES = 1>
+template <typename T, int G, int BIT, int FIXED, int EL>
 hipError_t launch_general_quant_as(const WireGeneralQuantArgs &a, hipStream_t stream) {
-    const int64_t tile = static_cast<int64_t>(kWave) * EL * kWavesPerBlock * TILES;
+    const int64_t tile = static_cast<int64_t>(kWave) * EL * kWavesPerBlock;
     const int64_t blocks = (a.numel + tile - 1) / tile;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((wire_general_quant_kernel<T, G, BIT, FIXED, EL, TILES>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
-                       stream, a);
+    const dim3 grid(static_cast<unsigned>(blocks));
+    hipLaunchKernelGGL((wire_general_quant_kernel<T, G, BIT, FIXED, EL>), grid, dim3(kBlock), 0, stream, a);
     return hipGetLastError();
 }
 
 template <typename T, int G>
 hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStream_t stream) {
-    // Each common policy runs a kernel without the code of the others: its own against the kernel for every policy, us for
-    // 26.2 M elements in groups of 64, fp32 and bf16 (8 and 16 buffer sets in turn): top-2 28.5 / 28.5 and 19.3 / 24.2,
-    // stochastic 23.8 / 24.0 and 18.0 / 21.8, the two together 32.2 / 33.9 and 23.6 / 27.0, 4-bit top-2 26.4 / 27.3 and
-    // 17.5 / 23.8, a code book rounded stochastically 37.9 / 40.6 and 34.7 / 38.2.  What they save is registers: for
-    // sixteen 16-bit elements a lane the kernel for every policy holds four wavefronts a SIMD, the one for plain
-    // stochastic codes seven.
+    // Each common policy runs a kernel without the code of the others: its own, us for 26.2 M elements in groups of 64 with
+    // the codes apart, fp32 and bf16 (in rotation over 1 GB), and the kernel for every policy as it was when they were split
+    // off: top-2 25.5 and 16.2 (28.5 and 24.2), stochastic 23.2 and 17.3 (24.0 and 21.8), the two together 31.3 and 22.4
+    // (33.9 and 27.0), 4-bit top-2 24.5 and 15.0 (27.3 and 23.8), a code book 20.9 and 13.5, with outliers 26.9 and 20.3,
+    // rounded stochastically 38.0 and 34.5 (40.6 and 38.2).  What they save is registers: for sixteen 16-bit elements a
+    // lane the kernel for every policy holds four wavefronts a SIMD, the one for plain stochastic codes eight.
     //
-    // 32 bytes a lane against 16, bf16 as above: top-2 19.3 / 22.8, stochastic 18.0 / 19.8, the two together 23.6 / 27.3,
-    // 4-bit top-2 17.5 / 21.7, a code book 14.2 / 15.7, rounded stochastically 34.7 / 34.5.  (fp32, with 16 bytes a lane
-    // still a form of this kernel: top-2 27.4 / 30.5, stochastic 24.3 / 26.6.)  Two such tiles a wavefront are slower for
-    // all of them, a code book 22.0 against 21.3 us (fp32) and 14.7 against 14.2 (bf16).
+    // One tile of 32 bytes a lane a wavefront.  Two such tiles, both asked for before either is encoded: top-2 29.9 against
+    // 26.7 us (fp32) and 21.0 against 17.4 (bf16), a code book 22.0 against 21.3 and 14.7 against 14.2.  16 bytes a lane
+    // for 16-bit types: a code book 15.7, two tiles of top-2 22.0; 64 bytes: top-2 17.7, and 26.9 (fp32).
     constexpr int WIDE = general_quant_elems<T>() <= G ? general_quant_elems<T>() : G;
     const int fixed = a.stochastic ? 0 : ((a.topk == 0 ? 1 : 0) | 2 | (a.kind == 0 ? 4 : 0));
     if (bit != 8 && bit != 4) return hipErrorNotSupported;
