@@ -62,8 +62,9 @@ constexpr uint32_t kEpsBits = 0x34000000u;  // 2^-23, torch.finfo(float32).eps
 // 16 MB to 600 MB of traffic (with it the time no longer depends on what the
 // 256 MiB memory-side cache holds; cached loads are ~5 % faster only when
 // everything is resident).  Stores under kStream are chosen per kernel.
-// kStreamThrough (fused reduce only): kStream with write-through stores.
-enum AccessMode { kUnaligned = 0, kVector = 1, kStream = 2, kStreamThrough = 3 };
+// kStreamThrough (fused reduce; codes of a quantize): kStream with write-through stores.  kStreamKept (codes of a
+// quantize): kStream with plain stores.
+enum AccessMode { kUnaligned = 0, kVector = 1, kStream = 2, kStreamThrough = 3, kStreamKept = 4 };
 
 template <typename T, int N>
 using vec_t = T __attribute__((ext_vector_type(N)));
