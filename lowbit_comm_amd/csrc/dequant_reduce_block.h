@@ -186,10 +186,13 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
 constexpr int kReduceQuantVec = 4;
 constexpr int kReduceQuantBlockElems = kWave * kReduceQuantVec * kWavesPerBlock;
 
-// One workgroup's share: block `block_x` of a grid of `grid_x` workgroups.
+// One workgroup's share: block `block_x` of a grid of `grid_x` workgroups.  W payloads; 0: as many as the call says, the
+// absent ones skipped by uniform branches.
 template <typename MT, int G, int W, int MODE>
 __device__ __forceinline__ void dequant_reduce_quant_block(const ReduceQuantArgs &a, unsigned block_x, unsigned grid_x) {
     constexpr int VEC = kReduceQuantVec;
+    constexpr int MAX = W == 0 ? kMaxPayloads : W;
+    const int world = W == 0 ? a.world : W;
     constexpr int LPG = G / VEC;
     constexpr int TILE = kWave * VEC;
     constexpr int BLOCK_ELEMS = TILE * kWavesPerBlock;
@@ -206,19 +209,21 @@ __device__ __forceinline__ void dequant_reduce_quant_block(const ReduceQuantArgs
 #pragma unroll
     for (int i = 0; i < VEC; ++i) p[i] = 0.0f;
     if (live) {
-        uint32_t words[W][VEC / 4];
-        float scale[W];
+        uint32_t words[MAX][VEC / 4];
+        float scale[MAX];
         const int64_t g = e0 / G;
 #pragma unroll
-        for (int r = 0; r < W; ++r) {
-            load_codes<VEC, code_load_mode<W>(MODE)>(a.codes[r] + e0, words[r]);
+        for (int r = 0; r < MAX; ++r) {
+            if (r >= world) break;
+            load_codes<VEC, code_load_mode<MAX>(MODE)>(a.codes[r] + e0, words[r]);
             scale[r] = a.scales[r][g];
         }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) p[i] = code_to_float(words[0][i / 4], i % 4) * scale[0];
         round_through_all<MT, VEC>(p);
 #pragma unroll
-        for (int r = 1; r < W; ++r) {
+        for (int r = 1; r < MAX; ++r) {
+            if (r >= world) break;
             float t[VEC];
 #pragma unroll
             for (int i = 0; i < VEC; ++i) t[i] = code_to_float(words[r][i / 4], i % 4) * scale[r];

@@ -120,6 +120,7 @@ constexpr Entry kEntries[] = {
     {"lbc_quant_pack_chunks_and_dequant_reduce", make_call<&lbc_quant_pack_chunks_and_dequant_reduce>},
     {"lbc_dequant_reduce_quant", make_call<&lbc_dequant_reduce_quant>},
     {"lbc_bucket_pipeline_step", make_call<&lbc_bucket_pipeline_step>},
+    {"lbc_bucket_pipeline_step_any", make_call<&lbc_bucket_pipeline_step_any>},
     {"lbc_ring_step", make_call<&lbc_ring_step>},
     {"lbc_ef_update", make_call<&lbc_ef_update>},
     {"lbc_wire_quant_pack", make_call<&lbc_wire_quant_pack>},

@@ -269,6 +269,7 @@ ReduceQuantCall prepare_reduce_quant(const int8_t *const *codes, const float *co
     c.args.out_scales = out_scales;
     c.args.numel = numel;
     c.args.divisor = divisor;
+    c.args.world = world;
     c.mid_dtype = mid_dtype;
     c.world = world;
     c.aligned = aligned;
@@ -441,8 +442,8 @@ int lbc_dequant_reduce_quant(const int8_t *const *codes, const float *const *sca
                   "lbc_dequant_reduce_quant");
 }
 
-int lbc_bucket_pipeline_step(const lbc_quant_chunks_stage *quant, const lbc_reduce_quant_stage *reduce,
-                             const lbc_dequant_chunks_stage *decode, int group_size, int access, void *stream) {
+static int pipeline_step(const char *what, bool any, const lbc_quant_chunks_stage *quant, const lbc_reduce_quant_stage *reduce,
+                         const lbc_dequant_chunks_stage *decode, int group_size, int access, void *stream) {
     if (!valid_access(access)) return fail(LBC_EINVAL, "unknown access mode %d", access);
     QuantCall q;
     q.empty = true;
@@ -505,25 +506,39 @@ int lbc_bucket_pipeline_step(const lbc_quant_chunks_stage *quant, const lbc_redu
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (stages == 1) {          // one stage with work: its own kernel
-        if (!q.empty) return launch_quant(q, "lbc_bucket_pipeline_step", access, stream);
+        if (!q.empty) return launch_quant(q, what, access, stream);
         if (!r.empty)
             return finish(lbc::launch_dequant_reduce_quant(r.mid_dtype, group_size, r.world, pick_mode(r.aligned, access), r.args, s),
-                          "lbc_bucket_pipeline_step");
+                          what);
         return finish(lbc::launch_decode(d.out_dtype, group_size, LBC_REDUCE_NONE, pick_mode(d.aligned, access), d.args, d.world, s),
-                      "lbc_bucket_pipeline_step");
+                      what);
     }
-    // one grid exists for group 64, operands aligned for the vector kernels, a residual that is absent or fp32,
-    // and one element type for the bucket, the reduce and the decoded output
-    if (group_size != 64 || (!q.empty && !q.aligned) || (!r.empty && !r.aligned) || (!d.empty && !d.aligned))
-        return LBC_UNSUPPORTED;
+    // one grid exists for a residual that is absent or fp32 and one element type for the bucket, the reduce and the decoded
+    // output; group 64 and operands aligned for the vector kernels have kernels of their own, the rest only where `any`
+    const bool aligned = (q.empty || q.aligned) && (r.empty || r.aligned) && (d.empty || d.aligned);
+    if ((group_size != 64 || !aligned) && !any) return LBC_UNSUPPORTED;
     if (!q.empty && q.r_dtype != LBC_NONE && q.r_dtype != LBC_F32) return LBC_UNSUPPORTED;
     const int dtype = !q.empty ? q.x_dtype : (!r.empty ? r.mid_dtype : d.out_dtype);
     if ((!r.empty && r.mid_dtype != dtype) || (!d.empty && d.out_dtype != dtype)) return LBC_UNSUPPORTED;
     const int vec = q.empty ? 4 : lbc::quant_pack_vec(q.x_dtype, q.r_dtype, q.d_dtype, q.outputs);
-    return finish(lbc::launch_pipeline_step(dtype, q.empty ? LBC_NONE : q.r_dtype, vec, pick_mode(true, access),
-                                            q.empty ? nullptr : &q.args, q.world, r.empty ? nullptr : &r.args, r.world,
-                                            d.empty ? nullptr : &d.args, d.world, s),
-                  "lbc_bucket_pipeline_step");
+    const int r_dtype = q.empty ? LBC_NONE : q.r_dtype;
+    const lbc::QuantArgs *qa = q.empty ? nullptr : &q.args;
+    const lbc::ReduceQuantArgs *ra = r.empty ? nullptr : &r.args;
+    const lbc::DecodeArgs *da = d.empty ? nullptr : &d.args;
+    if (group_size == 64 && aligned)
+        return finish(lbc::launch_pipeline_step(dtype, r_dtype, vec, pick_mode(true, access), qa, q.world, ra, r.world, da, d.world, s), what);
+    return finish(lbc::launch_pipeline_step_any(dtype, r_dtype, vec, group_size, pick_mode(aligned, LBC_ACCESS_AUTO), qa, q.world, ra,
+                                                da, d.world, s), what);
+}
+
+int lbc_bucket_pipeline_step(const lbc_quant_chunks_stage *quant, const lbc_reduce_quant_stage *reduce,
+                             const lbc_dequant_chunks_stage *decode, int group_size, int access, void *stream) {
+    return pipeline_step("lbc_bucket_pipeline_step", false, quant, reduce, decode, group_size, access, stream);
+}
+
+int lbc_bucket_pipeline_step_any(const lbc_quant_chunks_stage *quant, const lbc_reduce_quant_stage *reduce,
+                                 const lbc_dequant_chunks_stage *decode, int group_size, int access, void *stream) {
+    return pipeline_step("lbc_bucket_pipeline_step_any", true, quant, reduce, decode, group_size, access, stream);
 }
 
 int lbc_ring_step(const int8_t *recv_codes, const float *recv_scales, void *chunk, int dtype, int64_t numel,

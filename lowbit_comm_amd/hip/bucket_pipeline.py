@@ -14,8 +14,8 @@ independent of each other, so at any moment three compute stages of three differ
 ``lbc_quant_pack_chunks_and_dequant_reduce`` for the reduce-scatter leg alone): on this part the shard-sized stages
 are mostly launch ramp on their own, and behind a quantize that fills the chip that ramp is hidden (25 MiB bf16 buckets
 with error feedback, W = 8: 31 us per bucket in one grid against 37 us as three launches).  When a combination has no
-shared grid (unaligned tensors, a group size other than 64, more than eight ranks) the same stages go out as separate launches,
-in the same order, with the same results.
+shared grid (more than eight ranks; for the reduce-scatter leg alone also unaligned tensors and a group size other than 64)
+the same stages go out as separate launches, in the same order, with the same results.
 
 Ordering.  Everything is enqueued on the caller's current stream (or on the pipeline's lanes, see ``lanes``), so a
 stage is ordered after the exchange it depends on by the stream itself when the exchange callables enqueue on that
@@ -233,7 +233,7 @@ class BucketPipeline:
 
     def _bind_merged(self, quant, reduce, decode):
         if self.all_gather is not None:
-            return ops.bind_bucket_pipeline_step(quant, reduce, decode)
+            return ops.bind_bucket_pipeline_step(quant, reduce, decode, any_layout=True)
         return ops.bind_quant_chunks_and_reduce(quant, reduce)
 
     def _launch(self, lane: _Lane, quant, reduce, decode) -> None:

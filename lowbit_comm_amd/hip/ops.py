@@ -511,13 +511,14 @@ def bind_dequant_reduce_quant(payloads: Sequence[tuple[torch.Tensor, torch.Tenso
 
 
 def bind_bucket_pipeline_step(quant: BoundLaunch | None = None, reduce: BoundLaunch | None = None,
-                              decode: BoundLaunch | None = None) -> BoundLaunch:
+                              decode: BoundLaunch | None = None, *, any_layout: bool = False) -> BoundLaunch:
     """One launch for up to three stages of a bucket stream (``lbc_bucket_pipeline_step``): ``quant`` from
     :func:`bind_quant_pack_chunks` (bucket k, without ``restored`` / ``prepared_out``), ``reduce`` from
     :func:`bind_dequant_reduce_quant` (bucket k-1) and ``decode`` from :func:`bind_dequant_chunks` (bucket k-2); any
     may be ``None``.  The stages must not touch each other's outputs.  The access mode is that of the first stage
     given.  Calling the result returns ``False`` when the combination has no shared grid (then call the stages
-    themselves); the results are bit-identical either way."""
+    themselves); the results are bit-identical either way.  ``any_layout``: also for operands at element alignment and
+    groups of 32 and 16 (``lbc_bucket_pipeline_step_any``)."""
     from lowbit_comm_amd.hip.library import DequantChunksStage, QuantChunksStage, ReduceQuantStage
 
     given = [stage for stage in (quant, reduce, decode) if stage is not None]
@@ -556,7 +557,7 @@ def bind_bucket_pipeline_step(quant: BoundLaunch | None = None, reduce: BoundLau
         hold.append(d_stage)
         d_ref = ctypes.addressof(d_stage)
     args = (q_ref, r_ref, d_ref, group_size, given[0]._args[-1])
-    return BoundLaunch("lbc_bucket_pipeline_step", args, given[0]._device, tuple(stage._keep for stage in given),
+    return BoundLaunch("lbc_bucket_pipeline_step_any" if any_layout else "lbc_bucket_pipeline_step", args, given[0]._device, tuple(stage._keep for stage in given),
                        kind="bucket_pipeline_step", hold=tuple(hold))
 
 
