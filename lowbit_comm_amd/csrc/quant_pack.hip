@@ -35,7 +35,9 @@ hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t str
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    // A single payload without a residual keeps its codes within reach of the launch that reads them next.  us of quantize +
+    // A single payload without a residual keeps its codes within reach of the launch that reads them next (16-bit tensors
+    // beyond 8 Mi elements: up to there the round trip gains little, and the all_gather hook's reduce of eight payloads loses,
+    // 18.5 against 18.8 us on 6.6 M bf16 elements).  us of quantize +
     // decode, codes non-temporal / plain / written through, three tensors in rotation and (in brackets) enough of them to
     // outrun the last-level cache: fp32 4.0 M 8.6 / 8.7 / 9.2 (10.7 / 9.5 / 10.0), 5.3 M 13.1 / 12.2 / 11.7 (12.9 / 11.4 /
     // 11.9), 6.6 M 15.0 / 14.3 / 13.7 (14.7 / 13.3 / 13.6), 12 M 24.3 / 23.8 / 22.1 (23.4 / 21.0 / 21.1), 32 M 54.9 / 49.8 /
@@ -49,8 +51,10 @@ hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t str
                     return hipGetLastError();
                 }
             }
-            hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamKept, TILES>), grid, dim3(kBlock), 0, stream, a);
-            return hipGetLastError();
+            if (VEC == 4 || a.numel > (int64_t{8} << 20)) {
+                hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamKept, TILES>), grid, dim3(kBlock), 0, stream, a);
+                return hipGetLastError();
+            }
         }
     }
     switch (mode) {
