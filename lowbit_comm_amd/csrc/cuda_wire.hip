@@ -38,9 +38,16 @@ namespace {
 // ---------------------------------------------------------------------------
 // quantize + pack (optionally x + residual), `world` chunks via blockIdx.y
 // ---------------------------------------------------------------------------
-template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int NT, int TILES>
+// Code stores beside kPlain and kNonTemporal: written through the L2 (fp32 tensors, 8-bit codes apart from the scales).
+constexpr int kWrittenThrough = 2;
+
+// NT: hint of the tensors' loads; CODES: how the codes leave (launch_wire_quant_c).  The sum is read again by the reduce that
+// follows: plain stores, 6.6 M elements of two payloads through the all_gather hook with error feedback 31.4 -> 29.0 us (fp32)
+// and 19.9 -> 17.3 (bf16), 20 M of eight 109 -> 104 and 75.7 -> 73.0; interleaved 16-bit payloads, which gain nothing,
+// keep the hint (6.6 M of four 22.8 against 23.2 us).
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int NT, int CODES, int TILES>
 __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs a) {
-    constexpr int PNT = COMPACT ? kPlain : NT;
+    constexpr int SUM_NT = COMPACT && sizeof(T) == 2 ? NT : kPlain;
     using W = wire<T, BIT>;
     constexpr int VEC = W::VEC;
     constexpr int LPG = G / VEC;
@@ -139,8 +146,8 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
                         if (p[i] != p[i]) held[i] = __builtin_bit_cast(T, static_cast<Raw>(raw_bits<T>::INF | (raw_bits<T>::INF >> 1)));
                 }
                 if (prepared != nullptr) {
-                    if constexpr (WHOLE) store_elems<T, VEC, NT>(prepared + e0[u], held);
-                    else store_live<T, VEC, NT == kNonTemporal>(prepared + e0[u], valid - e0[u], held);
+                    if constexpr (WHOLE) store_elems<T, VEC, SUM_NT>(prepared + e0[u], held);
+                    else store_live<T, VEC, SUM_NT == kNonTemporal>(prepared + e0[u], valid - e0[u], held);
                 }
             } else {
 #pragma unroll
@@ -183,7 +190,12 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
             // it pay to stage a wavefront's run of eight groups (528 bytes, 16-byte aligned) in LDS and carry it out
             // as 33 aligned 16-byte stores: 16.2 us (16.4 us non-temporal) against 15.6 us on 26.2 M elements, no
             // workgroup barrier involved.  The misaligned stores are not what this layout costs.
-            store_piece<T, BIT, PNT, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words);
+            if constexpr (CODES == kWrittenThrough && WHOLE) {
+                static_assert(CODES != kWrittenThrough || (!COMPACT && BIT == 8), "codes in the elements' order, a byte each");
+                buffer_store<uint32_t, W::WORDS, kSc1Bit>(buffer_over(payload + block_first, BLOCK_ELEMS), static_cast<uint32_t>(e0[u] - block_first), words);
+            } else {
+                store_piece<T, BIT, CODES == kNonTemporal ? kNonTemporal : kPlain, W::WORDS>(payload + at.codes(group) + piece_offset<T, BIT>(k0), words);
+            }
             if ((lane & (LPG - 1)) == 0) *reinterpret_cast<Raw *>(payload + at.scale(group)) = stored;
         }
     };
@@ -191,7 +203,7 @@ __global__ __launch_bounds__(kBlock) void wire_quant_kernel(const WireQuantArgs 
     else tiles(std::false_type{});
 }
 
-template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int TILES>
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int CODES, int TILES>
 hipError_t launch_wire_quant_tiles(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
     constexpr int BLOCK_ELEMS = wire<T, BIT>::TILE * kWavesPerBlock * TILES;
     const int64_t groups = (a.shard_numel + G - 1) / G;
@@ -199,8 +211,8 @@ hipError_t launch_wire_quant_tiles(int mode, const WireQuantArgs &a, int world, 
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    if (mode == kStream) hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kNonTemporal, TILES>), grid, dim3(kBlock), 0, stream, a);
-    else hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kPlain, TILES>), grid, dim3(kBlock), 0, stream, a);
+    if (mode == kStream) hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kNonTemporal, CODES, TILES>), grid, dim3(kBlock), 0, stream, a);
+    else hipLaunchKernelGGL((wire_quant_kernel<T, G, BIT, HAS_R, COMPACT, kPlain, kPlain, TILES>), grid, dim3(kBlock), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -209,18 +221,37 @@ hipError_t launch_wire_quant_tiles(int mode, const WireQuantArgs &a, int world, 
 // where a residual is read as well (13.1 M fp32 19.9 us, 20.7 with four; bf16 12.6 / 13.1), and without one four - for a
 // 16-bit tensor two until there are twice the slots (6.6 M bf16 5.3 us with two, 6.0 with four; 13.1 M 9.3 / 9.1; fp32
 // 6.6 M 7.8 / 7.6, 26.2 M 23.3 / 22.1).
-template <typename T, int G, int BIT, bool HAS_R, bool COMPACT>
-hipError_t launch_wire_quant_c(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT, int CODES>
+hipError_t launch_wire_quant_s(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
     constexpr int64_t kOneEach = kResidentWaves * wire<T, BIT>::TILE;
-    if (a.numel <= kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 1>(mode, a, world, stream);
+    if (a.numel <= kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, CODES, 1>(mode, a, world, stream);
     if constexpr (HAS_R) {
-        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 2>(mode, a, world, stream);
+        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, CODES, 2>(mode, a, world, stream);
     } else {
         if constexpr (sizeof(T) == 2) {
-            if (a.numel <= 2 * kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 2>(mode, a, world, stream);
+            if (a.numel <= 2 * kOneEach) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, CODES, 2>(mode, a, world, stream);
         }
-        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, 4>(mode, a, world, stream);
+        return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, CODES, 4>(mode, a, world, stream);
     }
+}
+
+// How the codes leave.  Interleaved with the scales in plain stores (a line is shared by neighbouring wavefronts).  Apart
+// from them with the non-temporal hint where they leave for other ranks (chunks), and for small tensors; the one payload of a large
+// tensor is read by its decode, or by a reduce, next.  us of quantize + decode of 26.2 M elements, non-temporal
+// against plain: fp32 46.5 / 41.5, bf16 31.1 / 29.1 (4-bit codes 41.5 / 41.5 and 27.3 / 28.0, which keep the hint); of 6.6 M
+// fp32 15.3, plain 16.4, written through 13.9; bf16 8.7 / 8.7, but the all_gather hook without error feedback 18.2 / 18.7.
+// Beside a residual plain at every size (SUM_NT above; 1.6 M fp32 of two payloads 10.9 -> 8.3 us).
+template <typename T, int G, int BIT, bool HAS_R, bool COMPACT>
+hipError_t launch_wire_quant_c(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
+    if constexpr (COMPACT) return launch_wire_quant_s<T, G, BIT, HAS_R, COMPACT, kPlain>(mode, a, world, stream);
+    if constexpr (HAS_R && !COMPACT) {
+        if (world == 1) return launch_wire_quant_s<T, G, BIT, HAS_R, COMPACT, kPlain>(mode, a, world, stream);
+    } else if constexpr (BIT == 8 && !COMPACT) {
+        constexpr int64_t kLarge = (sizeof(T) == 4 ? int64_t{4} : int64_t{8}) << 20;
+        constexpr int KEPT = sizeof(T) == 4 ? kWrittenThrough : kPlain;
+        if (world == 1 && a.numel > kLarge) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, KEPT, 4>(mode, a, world, stream);
+    }
+    return launch_wire_quant_s<T, G, BIT, HAS_R, COMPACT, kNonTemporal>(mode, a, world, stream);
 }
 
 template <typename T, int G, int BIT>
