@@ -651,6 +651,133 @@ PyObject *specs(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the stages of the pipelined reduce-scatter ------------------------------------------------------------------
+// What one step of the bucket pipeline launches, from the plans of its buckets: the arguments of the three stages come out of
+// a plan's buffers and the step's tensors here, where binding them per tensor address and looking the bound launches and
+// their merged launch up again took the interpreter 5 us a step (four 1 MiB bf16 buckets through the hook 66 -> 48 us).
+struct Stages {   // a plan's buffers, as the stages address them
+    PyObject_HEAD
+    at::Tensor *rows;   // send, received, gathered; null until initialised
+    int64_t numel, shard, stride, code_bytes;
+    int world, rank, group, dtype;
+};
+
+int stages_init(PyObject *self, PyObject *args, PyObject *) {
+    long long numel;
+    int world, rank, group, dtype;
+    PyObject *tensors[3];
+    if (!PyArg_ParseTuple(args, "LiiiiOOO", &numel, &world, &rank, &group, &dtype, &tensors[0], &tensors[1], &tensors[2])) return -1;
+    const bool sane = numel > 0 && world >= 1 && world <= LBC_MAX_PAYLOADS && rank >= 0 && rank < world && valid_group(group) &&
+                      dtype >= LBC_F32 && dtype <= LBC_BF16;
+    const int64_t shard = sane ? (numel + world - 1) / world : 0, groups = sane ? groups_of(shard, group) : 0;
+    const at::Tensor *rows[3];
+    bool fit = sane;
+    for (int i = 0; fit && i < 3; ++i) {
+        rows[i] = payload_tensor(tensors[i]);
+        fit = rows[i] != nullptr && rows[i]->dim() == 2 && rows[i]->size(0) == world && rows[i]->size(1) >= groups * (group + 4) &&
+              rows[i]->size(1) == rows[0]->size(1) && with(*rows[i], *rows[0]);
+    }
+    if (!fit) {
+        PyErr_SetString(PyExc_ValueError, "the buffers do not belong to such a plan");
+        return -1;
+    }
+    Stages *s = reinterpret_cast<Stages *>(self);
+    delete[] s->rows;
+    s->rows = new at::Tensor[3]{*rows[0], *rows[1], *rows[2]};
+    s->numel = numel;
+    s->shard = shard;
+    s->stride = rows[0]->size(1);
+    s->code_bytes = groups * group;
+    s->world = world;
+    s->rank = rank;
+    s->group = group;
+    s->dtype = dtype;
+    return 0;
+}
+
+void stages_dealloc(PyObject *self) {
+    delete[] reinterpret_cast<Stages *>(self)->rows;
+    Py_TYPE(self)->tp_free(self);
+}
+
+PyTypeObject StagesType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+const Stages *stages_of(PyObject *o) {
+    const Stages *s = Py_TYPE(o) == &StagesType ? reinterpret_cast<const Stages *>(o) : nullptr;
+    return s != nullptr && s->rows != nullptr ? s : nullptr;
+}
+uint8_t *row_of(const Stages &s, int which, int64_t row) { return static_cast<uint8_t *>(s.rows[which].data_ptr()) + row * s.stride; }
+
+// pipeline_step(table, plan, stages, tensor, residual, plan, stages, mean, plan, stages, out, stream): quantize of `tensor` (with
+// `residual`, updated in place, or None), reduce + requantize, decode into `out`; a stage whose plan is None is absent.  `table`
+// names the plan methods the call stands for.  One launch: True; no grid for this combination: False, nothing was launched.
+PyObject *pipeline_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 12) return elsewhere();
+    PyObject *const table = a[0];
+    lbc_quant_chunks_stage quant{};
+    lbc_reduce_quant_stage reduce{};
+    lbc_dequant_chunks_stage decode{};
+    const int8_t *codes[LBC_MAX_PAYLOADS];
+    const float *scales[LBC_MAX_PAYLOADS];
+    const Stages *first = nullptr;
+    auto belongs = [&](PyObject *plan, const Stages *s) {
+        if (s == nullptr || !owns(plan, table)) return false;
+        if (first == nullptr) first = s;
+        return s->group == first->group && s->dtype == first->dtype && with(s->rows[0], first->rows[0]);
+    };
+    const bool has_quant = a[1] != Py_None, has_reduce = a[5] != Py_None, has_decode = a[8] != Py_None;
+    if (has_quant) {
+        const Stages *s = stages_of(a[2]);
+        const at::Tensor *x = gpu_tensor(a[3]);
+        if (!belongs(a[1], s) || x == nullptr || x->numel() != s->numel || code_of(x->scalar_type()) != s->dtype || !with(*x, s->rows[0]))
+            return elsewhere();
+        quant = {x->data_ptr(), nullptr, row_of(*s, 0, 0), nullptr, s->numel, s->stride, s->dtype, LBC_NONE, LBC_NONE, s->world};
+        if (a[4] != Py_None) {
+            const at::Tensor *residual = gpu_tensor(a[4]);
+            if (residual == nullptr || residual->numel() != s->numel || residual->scalar_type() != at::kFloat || !with(*residual, *x))
+                return elsewhere();
+            quant.residual = quant.new_residual = residual->data_ptr();
+            quant.residual_dtype = quant.new_residual_dtype = LBC_F32;
+        }
+    }
+    if (has_reduce) {
+        const Stages *s = stages_of(a[6]);
+        if (!belongs(a[5], s) || !PyBool_Check(a[7])) return elsewhere();
+        for (int r = 0; r < s->world; ++r) {
+            const uint8_t *row = row_of(*s, 1, r);
+            codes[r] = reinterpret_cast<const int8_t *>(row);
+            scales[r] = reinterpret_cast<const float *>(row + s->code_bytes);
+        }
+        uint8_t *mine = row_of(*s, 2, s->rank);
+        reduce = {codes, scales, reinterpret_cast<int8_t *>(mine), reinterpret_cast<float *>(mine + s->code_bytes), s->shard,
+                  a[7] == Py_True ? static_cast<float>(s->world) : 1.0f, s->world, s->dtype};
+    }
+    if (has_decode) {
+        const Stages *s = stages_of(a[9]);
+        const at::Tensor *out = gpu_tensor(a[10]);
+        if (!belongs(a[8], s) || out == nullptr || out->numel() != s->numel || code_of(out->scalar_type()) != s->dtype ||
+            !with(*out, s->rows[0]))
+            return elsewhere();
+        decode = {row_of(*s, 2, 0), out->data_ptr(), s->stride, s->shard, s->numel, s->world, s->dtype};
+    }
+    if (first == nullptr) return elsewhere();
+    auto call = [&](void *stream) {
+        return lbc_bucket_pipeline_step_any(has_quant ? &quant : nullptr, has_reduce ? &reduce : nullptr, has_decode ? &decode : nullptr,
+                                            first->group, LBC_ACCESS_AUTO, stream);
+    };
+    if (a[11] == Py_None) return answer(enqueue(first->rows[0].get_device(), call));
+    if (!PyLong_Check(a[11])) return elsewhere();
+    void *stream = PyLong_AsVoidPtr(a[11]);
+    if (PyErr_Occurred()) return elsewhere();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = call(stream);
+    Py_END_ALLOW_THREADS
+    return answer(rc);
+    END_HANDLE_TH_ERRORS
+}
+
 // own(object, table) -> whether a native call may stand for the object's methods in the table.
 PyObject *own(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n == 2 && owns(a[0], a[1])) Py_RETURN_TRUE;
@@ -669,6 +796,7 @@ PyMethodDef kMethods[] = {
     {"wire_quantize", reinterpret_cast<PyCFunction>(wire_quantize), METH_FASTCALL, "Quantize into a payload of the CUDA extension's format."},
     {"wire_dequantize", reinterpret_cast<PyCFunction>(wire_dequantize), METH_FASTCALL, "Decode a payload of that format into a fresh tensor."},
     {"wire_reduce", reinterpret_cast<PyCFunction>(wire_reduce), METH_FASTCALL, "Fused reduce of payloads of that format, optionally with the residual update."},
+    {"pipeline_step", reinterpret_cast<PyCFunction>(pipeline_step), METH_FASTCALL, "One launch for the ready stages of a bucket pipeline."},
     {"own", reinterpret_cast<PyCFunction>(own), METH_FASTCALL, "Are the methods in a table the module's own?"},
     {"specs", reinterpret_cast<PyCFunction>(specs), METH_FASTCALL, "Addresses, types and element counts of contiguous GPU tensors."},
     {nullptr, nullptr, 0, nullptr},
@@ -688,6 +816,14 @@ PyMODINIT_FUNC PyInit__host(void) {
     LaunchType.tp_call = launch_call;
     LaunchType.tp_dealloc = launch_dealloc;
     if (PyType_Ready(&LaunchType) < 0) return nullptr;
+    StagesType.tp_name = "lowbit_comm_amd._host.Stages";
+    StagesType.tp_basicsize = sizeof(Stages);
+    StagesType.tp_flags = Py_TPFLAGS_DEFAULT;
+    StagesType.tp_doc = "Stages(numel, world, rank, group, dtype code, send, received, gathered): a plan's buffers for pipeline_step.";
+    StagesType.tp_new = PyType_GenericNew;
+    StagesType.tp_init = stages_init;
+    StagesType.tp_dealloc = stages_dealloc;
+    if (PyType_Ready(&StagesType) < 0) return nullptr;
     PyObject *module = PyModule_Create(&kModule);
     if (module == nullptr) return nullptr;
     if (flat == nullptr) flat = PyUnicode_FromString("FLAT");
@@ -697,11 +833,13 @@ PyMODINIT_FUNC PyInit__host(void) {
         Py_DECREF(module);
         return nullptr;
     }
-    Py_INCREF(&LaunchType);
-    if (PyModule_AddObject(module, "Launch", reinterpret_cast<PyObject *>(&LaunchType)) < 0) {
-        Py_DECREF(&LaunchType);
-        Py_DECREF(module);
-        return nullptr;
+    for (auto [name, type] : {std::make_pair("Launch", &LaunchType), std::make_pair("Stages", &StagesType)}) {
+        Py_INCREF(type);
+        if (PyModule_AddObject(module, name, reinterpret_cast<PyObject *>(type)) < 0) {
+            Py_DECREF(type);
+            Py_DECREF(module);
+            return nullptr;
+        }
     }
     return module;
 }

@@ -39,7 +39,7 @@ import torch
 
 from lowbit_comm_amd.config import CompressionConfig
 from lowbit_comm_amd.hip import ops
-from lowbit_comm_amd.hip.reduce_scatter import AllGatherPlan, ReduceScatterPlan, ResidualStore
+from lowbit_comm_amd.hip.reduce_scatter import STAGE_METHODS, AllGatherPlan, ReduceScatterPlan, ResidualStore
 
 
 class _Bucket:
@@ -145,6 +145,8 @@ class BucketPipeline:
         # replaceable: the scheduling is testable without a GPU
         self._plan_factory = plan_factory or (AllGatherPlan if whole_gather is not None else ReduceScatterPlan)
         self._merge_stages = merge_stages or self._bind_merged
+        # the whole step is one native call when nothing of it has been replaced
+        self._own_merge = self._merge_stages if merge_stages is None and all_gather is not None else None
         self._dirty = False                                        # something was submitted since the last flush
         self._lock = threading.RLock()
         self._plans: OrderedDict[Any, list[ReduceScatterPlan]] = OrderedDict()   # shape key -> `depth` plans per lane
@@ -253,6 +255,37 @@ class BucketPipeline:
                 raise ValueError("no HIP kernel for this stage")
             self.stats["separate_launches"] += 1
 
+    def _step_natively(self, lane: _Lane, arriving: _Bucket | None, residual: torch.Tensor | None, reducing: _Bucket | None,
+                       decoding: _Bucket | None) -> bool:
+        """The ready stages as one native call; ``False``: nothing was launched, bind and launch them instead."""
+        if self._merge_stages is not self._own_merge or type(self) is not BucketPipeline:
+            return False
+        args: list = [STAGE_METHODS, None, None, None, None, None, None, None, None, None, None, lane.handle]
+        count = 0
+        if arriving is not None:
+            plan = arriving.plan
+            stages = plan.stages()
+            if stages is None or plan.exchange_in_flight is not None:
+                return False
+            args[1:5] = plan, stages, arriving.tensor, residual
+            count += 1
+        if reducing is not None:
+            stages = reducing.plan.stages()
+            if stages is None:
+                return False
+            args[5:8] = reducing.plan, stages, reducing.op == "mean"
+            count += 1
+        if decoding is not None:
+            stages = decoding.plan.stages()
+            if stages is None:
+                return False
+            args[8:11] = decoding.plan, stages, decoding.out
+            count += 1
+        if not count or not ops._host.pipeline_step(*args):
+            return False
+        self.stats["merged_launches" if count > 1 else "separate_launches"] += 1
+        return True
+
     def _advance(self, lane: _Lane, arriving: _Bucket | None, residual: torch.Tensor | None) -> None:
         """One pipeline step on ``lane``: the stages that are ready, their exchanges, the completion of the oldest."""
         reducing, decoding = lane.reduce_next, lane.decode_next
@@ -260,19 +293,23 @@ class BucketPipeline:
         quant = reduce = decode = None
         if arriving is not None:
             arriving.plan._order_after_previous_use()
-            quant = arriving.plan.bound_quantize(arriving.tensor, residual=residual, new_residual=residual)
-        if reducing is not None:
+        if reducing is not None and reducing.exchange is not None:
             _wait_for(reducing.exchange)
             reducing.exchange = None
-            if full:
-                reduce = reducing.plan.bound_reduce_requantize(op=reducing.op)
-            else:
-                reduce = reducing.plan.bound_reduce(op=reducing.op, out=reducing.out)
-        if decoding is not None:
+        if decoding is not None and decoding.gather is not None:
             _wait_for(decoding.gather)
             decoding.gather = None
-            decode = decoding.plan.bound_decode(decoding.out, remember=decoding.lasting_out)
-        self._launch(lane, quant, reduce, decode)
+        if not self._step_natively(lane, arriving, residual, reducing, decoding):
+            if arriving is not None:
+                quant = arriving.plan.bound_quantize(arriving.tensor, residual=residual, new_residual=residual)
+            if reducing is not None:
+                if full:
+                    reduce = reducing.plan.bound_reduce_requantize(op=reducing.op)
+                else:
+                    reduce = reducing.plan.bound_reduce(op=reducing.op, out=reducing.out)
+            if decoding is not None:
+                decode = decoding.plan.bound_decode(decoding.out, remember=decoding.lasting_out)
+            self._launch(lane, quant, reduce, decode)
         if arriving is not None:
             if self.whole_gather is not None:
                 arriving.exchange = self.whole_gather(arriving.plan.received, arriving.plan.my_payload)
@@ -286,7 +323,8 @@ class BucketPipeline:
             else:
                 self._complete(reducing, reducing.plan.reduced_shard(reducing.out, op=reducing.op, caller_owned=True))
         if decoding is not None:
-            self._complete(decoding, decoding.out.reshape(decoding.plan.shape))
+            out, shape = decoding.out, decoding.plan.shape
+            self._complete(decoding, out if out.shape == shape else out.reshape(shape))
         lane.decode_next = reducing if full else None
         lane.reduce_next = arriving
 
@@ -324,7 +362,7 @@ class BucketPipeline:
             if whole:
                 if out is None:
                     lasting_out = self.inplace and tensor.is_contiguous()
-                    out = tensor.reshape(-1) if lasting_out else torch.empty(
+                    out = tensor if lasting_out else torch.empty(
                         tensor.numel(), dtype=plan.reduced_dtype, device=tensor.device)
                 elif out.numel() != tensor.numel() or out.dtype != plan.reduced_dtype:
                     raise ValueError("out does not match the bucket")
@@ -334,7 +372,8 @@ class BucketPipeline:
                 elif out.numel() != plan.chunks.shard_numel or out.dtype != plan.reduced_dtype:
                     raise ValueError("out does not match this rank's shard")
             spans = (_span(tensor),)
-            if out.data_ptr() != spans[0][0] or out.numel() * out.element_size() != spans[0][1] - spans[0][0]:
+            if out is not tensor and (out.data_ptr() != spans[0][0] or
+                                      out.numel() * out.element_size() != spans[0][1] - spans[0][0]):
                 spans += (_span(out),)            # not the bucket itself: a second range
             if self._touches_a_bucket_in_flight(spans):
                 # The same memory again before its earlier bucket has been decoded (not a DDP iteration, where every

@@ -71,6 +71,7 @@ class ReduceScatterPlan:
         self._bound_lock = threading.Lock()   # DDP calls its hook from the autograd thread, a user may call from another
         self._last_stream: Any | None = None
         self._last_stream_handle: int | None = None
+        self._stages: tuple | None = None
         self.exchange_in_flight: Any | None = None     # work object of an exchange that nobody has waited for yet
 
     # Every bucket of one shape shares the plan, and every bucket has its own addresses: a transformer's stream of
@@ -107,6 +108,19 @@ class ReduceScatterPlan:
             event.record(self._last_stream)                   # the stream object is kept, so its handle stays valid
             stream.wait_event(event)
         self._last_stream, self._last_stream_handle = stream, handle
+
+    def stages(self) -> Any | None:
+        """This plan's buffers as the native pipeline step addresses them, or ``None`` for a plan it does not serve."""
+        held = self._stages
+        if held is not None and held[0] is self.send and held[1] is self.received and held[2] is self.gathered:
+            return held[3]
+        if (type(self) is not ReduceScatterPlan or ops._host is None or self.reduced_dtype != self.dtype or not self.numel
+                or self.world_size > ops.MAX_PAYLOADS or self.device.type != "cuda"):
+            return None
+        made = ops._host.Stages(self.numel, self.world_size, self.rank, self.config.group_size, ops.DTYPE_CODES[self.dtype],
+                                self.send, self.received, self.gathered)
+        self._stages = (self.send, self.received, self.gathered, made)
+        return made
 
     # ---- payload views ---------------------------------------------------------------------------
     def payload(self, rows: torch.Tensor, index: int) -> torch.Tensor:
@@ -269,6 +283,12 @@ class ReduceScatterPlan:
         if not remember:
             return make()
         return self._remember(("d", rows.data_ptr(), rows.numel(), target.data_ptr(), target.dtype, target.numel()), make)
+
+
+# The methods that a native pipeline step stands for: it is made only for a plan that has these as its own.
+STAGE_METHODS = ("bound_quantize", ReduceScatterPlan.bound_quantize,
+                 "bound_reduce_requantize", ReduceScatterPlan.bound_reduce_requantize,
+                 "bound_decode", ReduceScatterPlan.bound_decode)
 
 
 class AllGatherPlan(ReduceScatterPlan):

@@ -108,3 +108,66 @@ def test_any_layout_still_says_what_has_no_shared_grid(ops, hip_device):
     assert ops.bind_bucket_pipeline_step(plain, reduce(torch.float32), any_layout=True)() is False
     assert ops.bind_bucket_pipeline_step(ops.bind_quant_pack_chunks(x, send, world, residual=half), reduce(torch.bfloat16),
                                          any_layout=True)() is False
+
+
+def test_native_step_stands_back_for_replaced_parts(hip_device, monkeypatch):
+    """A plan whose method has been replaced (its class or the instance), a subclass of the pipeline and a merge step of its own
+    are asked as before the native call; every way gives the same bucket."""
+    from lowbit_comm_amd.hip import bucket_pipeline
+    from lowbit_comm_amd.hip.reduce_scatter import ReduceScatterPlan
+
+    def run(make=bucket_pipeline.BucketPipeline, prepare=None, **kwargs):
+        pipe = make(world_size=4, rank=0, all_to_all=lambda received, send: received.copy_(send),
+                    all_gather=lambda gathered, mine: gathered[1:, :mine.numel()].copy_(mine), **kwargs)
+        tensors = [gradient(n, torch.bfloat16, n, hip_device) for n in (10_001, 10_001, 4096, 10_001)]
+        for _ in range(2):
+            if prepare is not None and pipe._plans:
+                prepare(pipe)
+            futures = [pipe.submit(t, config=CompressionConfig()) for t in tensors]
+            pipe.flush()
+        return [f.wait().clone() for f in futures]
+
+    want = run()
+    seen = []
+    quantize, decode, requantize = (getattr(ReduceScatterPlan, "bound_" + n) for n in ("quantize", "decode", "reduce_requantize"))
+
+    def on_instances(pipe):
+        for plan in next(iter(pipe._plans.values())):
+            plan.bound_decode = lambda *a, plan=plan, **k: seen.append("instance") or decode(plan, *a, **k)
+
+    class Sub(bucket_pipeline.BucketPipeline):
+        def _launch(self, *args):
+            seen.append("subclass")
+            return super()._launch(*args)
+
+    outcomes = [run(prepare=on_instances), run(make=Sub),
+                run(merge_stages=lambda q, r, d: seen.append("merge") or (lambda stream=None: False))]
+    with monkeypatch.context() as patched:
+        patched.setattr(ReduceScatterPlan, "bound_quantize", lambda self, *a, **k: seen.append("class") or quantize(self, *a, **k))
+        outcomes.append(run())
+    assert set(seen) == {"instance", "subclass", "merge", "class"}
+    for outcome in outcomes:
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(outcome, want))
+
+
+def test_native_step_leaves_other_operands_to_the_bound_launches(hip_device):
+    """A strided bucket is refused as it was, an output of its own is taken; buffers that are no plan's are refused."""
+    from lowbit_comm_amd import _host
+    from lowbit_comm_amd.hip.bucket_pipeline import BucketPipeline
+
+    def make():
+        return BucketPipeline(world_size=2, rank=0, all_to_all=lambda received, send: received.copy_(send),
+                              all_gather=lambda gathered, mine: gathered[1:, :mine.numel()].copy_(mine))
+
+    base = gradient(2 * 6400, torch.float32, 5, hip_device)
+    with pytest.raises(RuntimeError, match="contiguous"):
+        make().submit(base[::2], config=CompressionConfig())
+    pipe, out = make(), torch.empty(6400, device=hip_device)
+    futures = [pipe.submit(base[:6400].clone(), config=CompressionConfig()),
+               pipe.submit(base[:6400].clone(), config=CompressionConfig(), out=out)]
+    pipe.flush()
+    first, second = (f.wait() for f in futures)
+    assert second.data_ptr() == out.data_ptr() and torch.equal(first, second)
+    rows = torch.zeros(2, 64, dtype=torch.uint8, device=hip_device)
+    with pytest.raises(ValueError, match="do not belong"):
+        _host.Stages(6400, 2, 0, 64, 0, rows, rows, rows)
