@@ -147,6 +147,54 @@ constexpr Places make_places() {
 }
 constexpr Places kPlaces = make_places();
 
+// ---- stochastic rounding: the largest entry not above t, its gap to the next one and that gap's reciprocal ----
+// The same cells over the entries 1 .. 14 instead of the steps (they lie two cells apart or more as well): by place, `base` the
+// count of entries passed.
+constexpr Places make_floors() {
+    Places places{};
+    for (int b = 0; b < kBooks; ++b)
+        for (int p = 0; p < kCells; ++p) {
+            const int cell = p == 0 ? 0 : p - 1;
+            uint32_t base = 0;
+            float threshold = kBeyond;
+            for (int k = 1; k <= 14; ++k) {
+                const float entry = kBookSet.value[b][k];
+                if (entry * 128.0f + 128.0f < static_cast<float>(cell)) ++base;
+                else if (entry < threshold) threshold = entry;
+            }
+            places.entry[b][p] = Cell{threshold, base};
+        }
+    return places;
+}
+constexpr Places kFloors = make_floors();
+constexpr bool entries_far_apart(const float (&book)[16]) {
+    for (int k = 1; k < 14; ++k)
+        if ((book[k + 1] - book[k]) * 128.0f < 1.999f) return false;
+    return true;
+}
+static_assert(entries_far_apart(kBookSet.value[0]) && entries_far_apart(kBookSet.value[1]) &&
+                  entries_far_apart(kBookSet.value[2]) && entries_far_apart(kBookSet.value[3]),
+              "two entries of a code book lie too close for one lookup");
+
+// Entry 14 is the last that the search gives and 1 the largest t: its gap, infinite in the book, only has to keep the
+// fraction (t - 1) / gap from being positive.
+struct Gap {
+    float low, gap, reciprocal, unused;
+};
+struct Gaps {
+    Gap entry[kBooks][16];
+};
+constexpr Gaps make_gaps() {
+    Gaps gaps{};
+    for (int b = 0; b < kBooks; ++b)
+        for (int k = 0; k < 16; ++k) {
+            const float low = kBookSet.value[b][k < 15 ? k : 14], gap = k < 14 ? kBookSet.value[b][k + 1] - low : 1.0f;
+            gaps.entry[b][k] = Gap{low, gap, 1.0f / gap, 0.0f};
+        }
+    return gaps;
+}
+constexpr Gaps kGaps = make_gaps();
+
 // The place of v / scale, round(128 * v / scale) + 128, in the low bits of a float: adding 1.5 * 2^23 + 128 rounds to an
 // integer.  `reciprocal128` is 128 / scale with a few ulps of error.
 constexpr float kPlaceMagic = 12582912.0f + 128.0f;
@@ -168,6 +216,14 @@ LBC_CELLS_HOST_DEVICE float reaches(float threshold, float v, float scale, float
     const float b = __builtin_fmaf(-threshold, scale, v);
     const float exponent = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, threshold) & 0xFF800000u);
     return __builtin_fmaf(__builtin_fabsf(exponent), scale24, b);
+}
+
+// excess / gap for a gap of the books, as the division rounds it: the product with the reciprocal and one correction
+// (Markstein).  tests/native/check_book_quotients.cpp compares the two for every significand of the dividend and every gap; a
+// quotient that underflows on the way is below 2^-100, and no draw is.
+LBC_CELLS_HOST_DEVICE float fraction_of_gap(float excess, float gap, float reciprocal) {
+    const float q = excess * reciprocal;
+    return __builtin_fmaf(__builtin_fmaf(-q, gap, excess), reciprocal, q);
 }
 }  // namespace book_cells
 }  // namespace lbc

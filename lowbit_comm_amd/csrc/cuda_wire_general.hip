@@ -31,7 +31,8 @@ namespace {
 
 // inner.cuh:9-35, and the one-lookup form of the encoder built from them at compile time
 __constant__ book_cells::Books kCodeBooks = book_cells::kBookSet;
-__constant__ book_cells::Places kBookPlaces = book_cells::kPlaces;
+__constant__ book_cells::Places kBookPlaces = book_cells::kPlaces, kBookFloors = book_cells::kFloors;
+__constant__ book_cells::Gaps kBookGaps = book_cells::kGaps;
 
 // Philox4x32-10: one block of four 32-bit words.  A round is two 32x32->64 multiplies and two three-way
 // exclusive-ors; gfx950 has the latter as one instruction (v_bitop3_b32 with the truth table 0x96), which the
@@ -75,32 +76,39 @@ __device__ __forceinline__ const float *wave_code_book(int kind, int lane) {
     return book;
 }
 
-// The workgroup's copy of a book's cell table (code_book_cells.h) in LDS.  The loads of the table are issued by `fetch`,
-// ahead of the tensor's own, so that `publish` need not wait for those; every wavefront of the workgroup must come to
-// `publish`, which ends in a workgroup barrier that orders LDS only.
-struct BlockCells {
+// The workgroup's copy of a book's cell table (code_book_cells.h) in LDS, and for stochastic rounding (GAPS) of its entries
+// with their gaps.  The loads are issued by `fetch`, ahead of the tensor's own, so that `publish` need not wait for those; every
+// wavefront of the workgroup must come to `publish`, which ends in a workgroup barrier that orders LDS only.
+template <bool GAPS> struct BlockCells {
     static constexpr int PER_THREAD = (book_cells::kCells + kBlock - 1) / kBlock;
     u32x2 held[PER_THREAD];
+    u32x4 held_gap;
+    const book_cells::Cell *cells;
+    const book_cells::Gap *gaps;
 
     __device__ __forceinline__ void fetch(int kind) {
-        const u32x2 *table = reinterpret_cast<const u32x2 *>(kBookPlaces.entry[kind - 1]);
+        const u32x2 *table = reinterpret_cast<const u32x2 *>((GAPS ? kBookFloors : kBookPlaces).entry[kind - 1]);
 #pragma unroll
         for (int k = 0; k < PER_THREAD; ++k) {
             const int place = k * kBlock + threadIdx.x;
             if (place < book_cells::kCells) held[k] = table[place];
         }
+        if (GAPS && threadIdx.x < 16) held_gap = reinterpret_cast<const u32x4 *>(kBookGaps.entry[kind - 1])[threadIdx.x];
     }
-    __device__ __forceinline__ const book_cells::Cell *publish() {
-        __shared__ u32x2 cells[book_cells::kCells];
+    __device__ __forceinline__ void publish() {
+        __shared__ u32x2 cell_table[book_cells::kCells];
+        __shared__ u32x4 gap_table[GAPS ? 16 : 1];
 #pragma unroll
         for (int k = 0; k < PER_THREAD; ++k) {
             const int place = k * kBlock + threadIdx.x;
-            if (place < book_cells::kCells) cells[place] = held[k];
+            if (place < book_cells::kCells) cell_table[place] = held[k];
         }
+        if (GAPS && threadIdx.x < 16) gap_table[threadIdx.x] = held_gap;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        return reinterpret_cast<const book_cells::Cell *>(cells);
+        cells = reinterpret_cast<const book_cells::Cell *>(cell_table);
+        gaps = reinterpret_cast<const book_cells::Gap *>(gap_table);
     }
 };
 
@@ -166,11 +174,10 @@ template <int LANES> __device__ __forceinline__ void merge_top3(uint32_t &first,
     if constexpr (LANES >= 16) merge_top3_step<0x140>(first, second, third);  // row_mirror
 }
 
-// FIXED names what the launch knows about the policy at compile time, so that the code of the other policies
-// is not part of the kernel: bit 0 "no outlier channel", bit 1 "round to nearest", bit 2 "linear codes", bit 3
-// "stochastic rounding" (13: plain linear codes rounded stochastically, 12: the same with outliers, 9: a code book
-// with stochastic rounding; 6: linear codes rounded to nearest, always with outliers - without them lbc_wire_quant_pack
-// serves the call).  0 is the kernel for every policy.
+// FIXED names the policy, so that the code of the others is not part of the kernel: bit 0 "no outlier channel", bit 1 "round
+// to nearest", bit 2 "linear codes" (else a code book), bit 3 "stochastic rounding".  13 and 12: linear codes rounded
+// stochastically, without and with outliers; 9 and 8: a code book likewise; 6: linear codes rounded to nearest with
+// outliers (without them lbc_wire_quant_pack serves the call); 3 and 2: a code book rounded to nearest, without and with.
 // EL: elements per lane, a multiple of 8 that divides G; a wavefront owns one tile of 64 * EL elements.
 // Codes leave in plain stores: with the non-temporal hint a launch alone is up to 6 % faster, and what reads the payload
 // next pays for it (quantize and decode of 26.2 M elements with two outliers: fp32 44.9 plain against 52.0 us, bf16 28.6
@@ -178,8 +185,7 @@ template <int LANES> __device__ __forceinline__ void merge_top3(uint32_t &first,
 template <typename T, int G, int BIT, int FIXED, int EL>
 __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGeneralQuantArgs a) {
     const int topk = (FIXED & 1) ? 0 : a.topk;
-    const bool stochastic = (FIXED & 2) ? false : ((FIXED & 8) ? true : a.stochastic != 0);
-    const int kind = (FIXED & 4) ? 0 : a.kind;
+    constexpr bool STOCHASTIC = (FIXED & 8) != 0;
     using W = wire<T, BIT>;
     using RB = raw_bits<T>;
     using Raw = typename RB::type;
@@ -195,9 +201,9 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     const int64_t e0 = tile_first + lane * VEC;
     const bool live = e0 < a.numel;      // numel is a multiple of G: dead lanes form whole dead groups
 
-    constexpr bool BY_CELLS = (FIXED & 2) != 0 && (FIXED & 4) == 0;
-    BlockCells block_cells;
-    if constexpr (BY_CELLS) block_cells.fetch(kind);
+    constexpr bool BOOK = (FIXED & 4) == 0, STOCHASTIC_BOOK = BOOK && (FIXED & 8) != 0;
+    BlockCells<STOCHASTIC_BOOK> table;
+    if constexpr (BOOK) table.fetch(a.kind);
     // All of the wavefront's elements are asked for before anything else, and kept as whole dwords: 16-bit elements taken
     // apart inside the branch would be waited for there, ahead of the tables and of the draws (26.2 M bf16 elements with
     // two outliers, rounded stochastically, 23.7 against 22.4 us, 3.3 M 6.4 against 5.4).
@@ -212,10 +218,8 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         for (int part = 0; part < PARTS; ++part)
             load_words<DWORDS, ITEM, kPlain>(reinterpret_cast<const uint8_t *>(static_cast<const Raw *>(a.x) + e0 + part * W::VEC), held[part]);
     }
-    const book_cells::Cell *cells = nullptr;
-    if constexpr (BY_CELLS) cells = block_cells.publish();
+    if constexpr (BOOK) table.publish();
     if (tile_first >= a.numel) return;   // wavefront-uniform, behind the workgroup's barrier
-    const float *book = BY_CELLS ? nullptr : wave_code_book(kind, lane);
 
     const int64_t group = e0 / G;
     const int k0 = static_cast<int>(e0 - group * G);
@@ -224,7 +228,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     float uniform[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; ++i) uniform[i] = 0.0f;
-    if (stochastic) {
+    if constexpr (STOCHASTIC) {
         const uint32_t key0 = static_cast<uint32_t>(a.seed), key1 = static_cast<uint32_t>(a.seed >> 32);
         const uint32_t sub0 = static_cast<uint32_t>(group), sub1 = static_cast<uint32_t>(static_cast<uint64_t>(group) >> 32);
         const int phase = static_cast<int>(a.offset & 3);
@@ -274,9 +278,9 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
 
     uint32_t scale_raw;
     Raw meta[4] = {0, 0, 0, 0};   // [scale][indices][top1][top2]
-    bool any_nan = true;   // "not known": the outlier path does not look
+    bool any_nan = true;   // does the wavefront hold one?
     uint32_t outlier[2] = {~0u, ~0u};   // place among the lane's elements, beyond them when another lane's
-    if (FIXED != 6 && topk == 0) {
+    if constexpr ((FIXED & 1) != 0) {
         scale_raw = running_max_raw<T, G, VEC>(mag, k0, start, &any_nan);
     } else {
         // The three largest candidates of the group, a candidate's key being its magnitude and a tie-break rank
@@ -288,11 +292,18 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         if constexpr (WIDE) {
             // Three rounds of "largest remaining candidate": the group maximum of the magnitude keys, then, among
             // the elements that hold it, the maximum of the ranks.
-            uint32_t key[VEC], rank[VEC];
+            uint32_t key[VEC], rank[VEC], top = 0;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) top = mag[i] > top ? mag[i] : top;
+            any_nan = __ballot(top > RB::INF) != 0;   // wavefront-uniform
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
                 rank[i] = __builtin_amdgcn_alignbit(static_cast<uint32_t>(k0 + i + 1), raw[i], 31);   // sign below it
-                key[i] = mag[i] <= RB::INF ? mag[i] + 1 : 0;                  // 0 stands for "none"
+                key[i] = mag[i] + 1;                                          // 0 stands for "none"
+            }
+            if (any_nan) {
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) key[i] = mag[i] <= RB::INF ? key[i] : 0;
             }
 #pragma unroll
             for (int round = 0; round < 3; ++round) {
@@ -346,7 +357,8 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
                 merge_top3<LPG>(largest, runner_up, bronze);
             };
             search(false);
-            if (__ballot(largest > kAbove) != 0) search(true);   // wavefront-uniform
+            any_nan = __ballot(largest > kAbove) != 0;   // wavefront-uniform
+            if (any_nan) search(true);
             largest = largest < kBelow ? 0 : largest;
             runner_up = runner_up < kBelow ? 0 : runner_up;
             bronze = bronze < kBelow ? 0 : bronze;
@@ -415,8 +427,8 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     float scale = value_of<T>(scale_raw);
     scale = scale < 1.0e-6f ? 1.0e-6f : scale;   // a NaN scale stays NaN and encodes every element as 0
 
-    if constexpr (BY_CELLS) {
-        // A code book, rounded to nearest (uniform: kind is not 0).  The cell lookup answers v / scale without forming
+    if constexpr (BOOK) {
+        // A code book.  Rounded to nearest, the cell lookup answers v / scale without forming
         // the quotient: per element a fused multiply-add and an address, one LDS read, and four operations that leave
         // the comparison with the step in a sign bit and push it and the cell's code into a word of eight.  It
         // holds for a scale within 2^60 of 1 either way and |v| <= scale; the scale is at least 1e-6 here, and beside
@@ -441,6 +453,39 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
             }
             divisor = 1.0f;
         }
+        if constexpr (STOCHASTIC_BOOK) {
+            // The quotient itself is wanted: how far it lies between two entries decides against the draw.  t = v / scale, the
+            // IEEE quotient: a lane's elements share the divisor, so the reciprocal part of the division is done once
+            // (v_rcp_f32 and one Newton step), then per element the product and two corrections.  These are the very
+            // operations the compiler emits for `v / scale`, minus its operand scaling and special-case fix-up
+            // (v_div_scale / v_div_fmas / v_div_fixup), which change nothing while the divisor lies in [2^-60, 2^60],
+            // |v| <= scale, and the dividend is not so small (below 2^-103) that the division would rescale it; the
+            // quotient is then below 2^-80, and no draw is below 2^-33.  tests/native/quotient_check.hip compares the
+            // two forms on the device.  The entry below t is one table lookup and the fraction of the gap three operations: 26.2 M elements
+            // of the normal book 27.1 us (fp32) and 23.2 (bf16), with a search in four halving steps and a division 37.6 and 34.7.
+            float reciprocal = __builtin_amdgcn_rcpf(divisor);
+            reciprocal = __builtin_fmaf(__builtin_fmaf(-divisor, reciprocal, 1.0f), reciprocal, reciprocal);
+            uint32_t words[WORDS];
+#pragma unroll
+            for (int k = 0; k < WORDS; ++k) {
+                uint32_t codes = 0;
+#pragma unroll
+                for (int i = 8 * k; i < 8 * k + 8; ++i) {
+                    float t = v[i] * reciprocal;
+                    t = __builtin_fmaf(__builtin_fmaf(-divisor, t, v[i]), reciprocal, t);
+                    t = __builtin_fmaf(__builtin_fmaf(-divisor, t, v[i]), reciprocal, t);
+                    const book_cells::Cell cell = table.cells[book_cells::nearest_place(t, 128.0f) - book_cells::kPlaceBits];
+                    const uint32_t entry = cell.base + (t >= cell.threshold ? 1u : 0u);
+                    const book_cells::Gap gap = table.gaps[entry];
+                    const float fraction = book_cells::fraction_of_gap(t - gap.low, gap.gap, gap.reciprocal);
+                    codes = (codes << 4) | (entry + (uniform[i] < fraction ? 1u : 0u));
+                }
+                words[k] = WIDE ? codes : __builtin_amdgcn_alignbit(codes, codes, 16);
+            }
+            if (live) store_words<WORDS, ITEM, kPlain>(group_codes + k0 * BIT / 8, words);
+            store_meta();
+            return;
+        }
         const float reciprocal128 = __builtin_amdgcn_rcpf(divisor) * 128.0f, divisor24 = divisor * 0x1p-24f;
         if (live) {
             uint32_t words[WORDS];
@@ -449,7 +494,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
                 uint32_t codes = 0, below = 0;
 #pragma unroll
                 for (int i = 8 * k; i < 8 * k + 8; ++i) {
-                    const book_cells::Cell cell = cells[book_cells::nearest_place(v[i], reciprocal128) - book_cells::kPlaceBits];
+                    const book_cells::Cell cell = table.cells[book_cells::nearest_place(v[i], reciprocal128) - book_cells::kPlaceBits];
                     const float sign = book_cells::reaches(cell.threshold, v[i], divisor, divisor24);
                     codes = __builtin_amdgcn_alignbit(codes, cell.base, 28);          // (codes << 4) | code + 1
                     below = __builtin_amdgcn_alignbit(below, as_u32(sign), 28);
@@ -464,7 +509,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
     }
 
     int c[VEC];
-    if (kind == 0) {
+    {
         const float multiplier = W::LEVELS / scale;
         constexpr int L = static_cast<int>(W::LEVELS);
         // Beside outliers and NaNs no magnitude exceeds the scale, so the product stays within the levels and adding
@@ -472,87 +517,30 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         // with conversion and clamp.  An outlier's code is cleared below; a NaN of a 16-bit type has zeros there.
         // With the search's keys and the clearing of words this took the kernel, bound by instructions, from 20.2 to
         // 17 us on 26.2 M bf16 elements with two outliers (the round trip 31.9 to 28.6).
-        constexpr bool kByAddition = FIXED == 6 && !WIDE;
+        // With noise the product is clamped first, which a NaN would not survive as the 0 it encodes as: a wavefront that
+        // holds one, or an infinite scale (infinity times the multiplier 0), rounds, converts and clamps.
+        // nvcc contracts v * m + noise into one FMA; without noise the product is rounded alone
+        auto scaled = [&](int i) { return STOCHASTIC ? __builtin_fmaf(v[i], multiplier, uniform[i] - 0.5f) : v[i] * multiplier; };
+        if (!STOCHASTIC && (!WIDE || !any_nan)) {
 #pragma unroll
-        for (int i = 0; kByAddition && i < VEC; ++i) c[i] = static_cast<int>(as_u32(v[i] * multiplier + 0x1.8p23f));
+            for (int i = 0; i < VEC; ++i) c[i] = static_cast<int>(as_u32(scaled(i) + 0x1.8p23f));
+        } else if (STOCHASTIC && !any_nan && __ballot(scale_not_finite(scale)) == 0) {   // wavefront-uniform
 #pragma unroll
-        for (int i = 0; !kByAddition && i < VEC; ++i) {
-            // nvcc contracts v * m + noise into one FMA; without noise the product is rounded alone
-            const float t = stochastic ? __builtin_fmaf(v[i], multiplier, uniform[i] - 0.5f) : v[i] * multiplier;
-            const int r = cvt_i32(__builtin_rintf(t));
-            c[i] = r < -L ? -L : (r > L ? L : r);
-        }
-    } else {
-        // t = v / scale, the IEEE quotient.  A lane's elements share the divisor, so the reciprocal part of the
-        // division is done once: v_rcp_f32 and one Newton step, then per element the product and two corrections.
-        // These are the very operations the compiler emits for `v / scale`, minus its operand scaling and
-        // special-case fix-up (v_div_scale / v_div_fmas / v_div_fixup), which change nothing while the divisor
-        // lies in [2^-60, 2^60], |v| <= scale, and the dividend is not so small (below 2^-103) that the division
-        // would rescale it.  The scale is at least 1e-6 here, so such a dividend means a quotient below 2^-80, and a
-        // quotient below 2^-30 encodes as the book's zero whatever its last bits are: it is closer to that entry
-        // than the rounding error of the comparisons with its neighbours.  A wavefront with any other divisor,
-        // or with an element above its scale (only a group that holds a NaN has one) or not a number, takes the
-        // division.  tests/native/quotient_check.hip compares the two forms on the device.
-        float t[VEC];
-        const uint32_t scale_exponent = (as_u32(scale) >> 23) & 0xFFu;
-        bool unusual = scale_exponent < 127u - 60u || scale_exponent > 127u + 60u;
-        // Without outliers the scale is the group's largest magnitude unless a NaN reset the running maximum, and
-        // the wavefront is known to hold no NaN: no element needs to be looked at.
-        if (any_nan) {   // wavefront-uniform
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) unusual |= !(__builtin_fabsf(v[i]) <= scale);
-        }
-        const bool usual = __ballot(unusual) == 0;   // wavefront-uniform
-        if (usual) {
-            float reciprocal = __builtin_amdgcn_rcpf(scale);
-            reciprocal = __builtin_fmaf(__builtin_fmaf(-scale, reciprocal, 1.0f), reciprocal, reciprocal);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-                float q = v[i] * reciprocal;
-                q = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
-                t[i] = __builtin_fmaf(__builtin_fmaf(-scale, q, v[i]), reciprocal, q);
-            }
+            for (int i = 0; i < VEC; ++i)
+                c[i] = static_cast<int>(as_u32(__builtin_amdgcn_fmed3f(scaled(i), -W::LEVELS, W::LEVELS) + 0x1.8p23f));
         } else {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) t[i] = v[i] / scale;
-        }
-        // The largest entry in [0, 14] with not (t < book[entry]); a NaN ends at 14.  Four halving steps, each
-        // over all of the lane's elements so that their LDS reads are in flight together; positions are kept as
-        // byte offsets into the book.
-        const char *book_bytes = reinterpret_cast<const char *>(book);
-        int at[VEC];
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) at[i] = 0;
-#pragma unroll
-        for (int step = 8 * 4; step >= 4; step >>= 1) {
-#pragma unroll
             for (int i = 0; i < VEC; ++i) {
-                const int mid = at[i] + step;
-                const float entry = *reinterpret_cast<const float *>(book_bytes + mid);
-                at[i] = (mid < 15 * 4 && !(t[i] < entry)) ? mid : at[i];
+                const int r = cvt_i32(__builtin_rintf(scaled(i)));
+                c[i] = r < -L ? -L : (r > L ? L : r);
             }
-        }
-        float excess[VEC], gap[VEC];
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-            const float low = *reinterpret_cast<const float *>(book_bytes + at[i]);
-            gap[i] = *reinterpret_cast<const float *>(book_bytes + at[i] + 4) - low;
-            excess[i] = t[i] - low;
-            c[i] = at[i] >> 2;
-        }
-        if (stochastic) {   // uniform: the second division only runs when it is needed
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) c[i] += uniform[i] < excess[i] / gap[i] ? 1 : 0;
-        } else {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) c[i] += excess[i] > gap[i] * 0.5f ? 1 : 0;
         }
     }
     if (live) {
         uint32_t words[WORDS];
         if constexpr (BIT == 8) pack_codes<T, 8, VEC, WORDS>(c, words);
         else pack_nibbles<T, EL>(c, words);
-        if constexpr ((FIXED & 5) == 4) {
+        if constexpr (!(FIXED & 1)) {
             constexpr uint32_t PER_WORD = 32 / BIT, ORDER = BIT == 8 ? (WIDE ? 3 : 1) : (WIDE ? 7 : 3);   // place in a word
             uint32_t code[2];
 #pragma unroll
@@ -659,33 +647,35 @@ hipError_t launch_general_quant_as(const WireGeneralQuantArgs &a, hipStream_t st
 
 template <typename T, int G>
 hipError_t launch_general_quant_g(int bit, const WireGeneralQuantArgs &a, hipStream_t stream) {
-    // Each common policy runs a kernel without the code of the others: its own, us for 26.2 M elements in groups of 64 with
-    // the codes apart, fp32 and bf16 (in rotation over 1 GB), and the kernel for every policy as it was when they were split
-    // off: top-2 25.5 and 16.2 (28.5 and 24.2), stochastic 23.2 and 17.3 (24.0 and 21.8), the two together 31.3 and 22.4
-    // (33.9 and 27.0), 4-bit top-2 24.5 and 15.0 (27.3 and 23.8), a code book 20.9 and 13.5, with outliers 26.9 and 20.3,
-    // rounded stochastically 38.0 and 34.5 (40.6 and 38.2).  What they save is registers: for sixteen 16-bit elements a
-    // lane the kernel for every policy holds four wavefronts a SIMD, the one for plain stochastic codes eight.
+    // Every policy runs a kernel without the code of the others.  us for 26.2 M elements in groups of 64 with the codes apart, fp32
+    // and bf16 (launches alone, in rotation over 1 GB): top-2 25.2 and 17.0, stochastic 24.0 and 16.6, the two together 29.3 and
+    // 21.6, 4-bit top-2 23.0 and 15.6, a code book 21.3 and 14.2, with outliers 26.0 and 19.1, rounded stochastically 27.1 and
+    // 23.2, with outliers 36.3 and 29.3.  (As one kernel for every policy top-2 took 28.5 and 24.2, stochastic 24.0 and
+    // 21.8, the two together 33.9 and 27.0: for sixteen 16-bit elements a lane it held four wavefronts a SIMD, the one for
+    // plain stochastic codes holds eight.)
     //
     // One tile of 32 bytes a lane a wavefront.  Two such tiles, both asked for before either is encoded: top-2 29.9 against
     // 26.7 us (fp32) and 21.0 against 17.4 (bf16), a code book 22.0 against 21.3 and 14.7 against 14.2.  16 bytes a lane
     // for 16-bit types: a code book 15.7, two tiles of top-2 22.0; 64 bytes: top-2 17.7, and 26.9 (fp32).
     constexpr int WIDE = general_quant_elems<T>() <= G ? general_quant_elems<T>() : G;
-    const int fixed = a.stochastic ? 0 : ((a.topk == 0 ? 1 : 0) | 2 | (a.kind == 0 ? 4 : 0));
     if (bit != 8 && bit != 4) return hipErrorNotSupported;
     if (bit == 8 && a.kind != 0) return hipErrorNotSupported;   // eight bits: linear codes only
+    // plain linear codes: lbc_wire_quant_pack serves those calls, and no kernel here has their code
+    if (a.kind == 0 && a.topk == 0 && !a.stochastic) return hipErrorNotSupported;
     if (bit == 8) {
-        // the kernel below has no code for a group without outliers: lbc_wire_quant_pack serves those calls
-        if (fixed == 7) return hipErrorNotSupported;
         if (a.stochastic && a.topk == 0) return launch_general_quant_as<T, G, 8, 13, WIDE>(a, stream);
         if (a.stochastic) return launch_general_quant_as<T, G, 8, 12, WIDE>(a, stream);
-        return launch_general_quant_as<T, G, 8, 6, WIDE>(a, stream);   // round to nearest, with outliers
+        return launch_general_quant_as<T, G, 8, 6, WIDE>(a, stream);
     }
-    if (fixed == 6) return launch_general_quant_as<T, G, 4, 6, WIDE>(a, stream);
-    if (fixed == 2) return launch_general_quant_as<T, G, 4, 2, WIDE>(a, stream);
-    if (a.stochastic && a.topk == 0 && a.kind == 0) return launch_general_quant_as<T, G, 4, 13, WIDE>(a, stream);
+    if (a.kind == 0) {
+        if (a.stochastic && a.topk == 0) return launch_general_quant_as<T, G, 4, 13, WIDE>(a, stream);
+        if (a.stochastic) return launch_general_quant_as<T, G, 4, 12, WIDE>(a, stream);
+        return launch_general_quant_as<T, G, 4, 6, WIDE>(a, stream);
+    }
     if (a.stochastic && a.topk == 0) return launch_general_quant_as<T, G, 4, 9, WIDE>(a, stream);
-    if (fixed == 3) return launch_general_quant_as<T, G, 4, 3, WIDE>(a, stream);
-    return launch_general_quant_as<T, G, 4, 0, WIDE>(a, stream);
+    if (a.stochastic) return launch_general_quant_as<T, G, 4, 8, WIDE>(a, stream);
+    if (a.topk == 0) return launch_general_quant_as<T, G, 4, 3, WIDE>(a, stream);
+    return launch_general_quant_as<T, G, 4, 2, WIDE>(a, stream);
 }
 
 template <typename T> hipError_t launch_general_quant_t(int g, int bit, const WireGeneralQuantArgs &a, hipStream_t s) {

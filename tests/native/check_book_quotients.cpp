@@ -47,7 +47,46 @@ static void check(int b, float v, float scale) {
     }
 }
 
+// Stochastic rounding: the entry below t by the cells against the search, on every float of a stride and next to every
+// entry; the fraction of the gap against the division, for every significand of the dividend and every gap.
+static void check_floors() {
+    for (int b = 0; b < bc::kBooks; ++b) {
+        const float *book = bc::kBookSet.value[b];
+        auto floor_of = [&](float t) {
+            int at = 0;
+            for (int step = 8; step >= 1; step >>= 1) {
+                const int mid = at + step;
+                if (mid < 15 && !(t < book[mid])) at = mid;
+            }
+            return at;
+        };
+        auto one = [&](float t) {
+            if (!(std::fabs(t) <= 1.0f)) return;
+            const bc::Cell &cell = bc::kFloors.entry[b][bc::nearest_place(t, 128.0f) - bc::kPlaceBits];
+            mismatches += static_cast<int>(cell.base) + (t >= cell.threshold ? 1 : 0) != floor_of(t);
+            ++checked;
+        };
+        for (uint32_t key = bc::key_of(-1.0f); key <= bc::key_of(1.0f); key += 509) one(bc::float_of(key));
+        for (int k = 0; k < 15; ++k)
+            for (int d = -4; d <= 4; ++d) one(bc::float_of(bc::key_of(book[k]) + d));
+        for (int place = -256; place <= 256; ++place)
+            for (int d = -2; d <= 2; ++d) one(bc::float_of(bc::key_of(place / 256.0f) + d));
+        for (int k = 0; k < 14; ++k) {
+            const bc::Gap &g = bc::kGaps.entry[b][k];
+            if (g.low != book[k] || g.gap != book[k + 1] - book[k]) ++mismatches;
+            unsigned long long bad = 0;
+            for (uint32_t m = 0; m < (1u << 23); ++m) {
+                const float excess = bc::float_of(0x80000000u | (120u << 23) | m);
+                bad += bc::fraction_of_gap(excess, g.gap, g.reciprocal) != excess / g.gap;
+            }
+            mismatches += bad;
+            checked += 1u << 23;
+        }
+    }
+}
+
 int main(int argc, char **argv) {
+    check_floors();
     const int scales = argc > 1 ? std::atoi(argv[1]) : 20000;
     std::mt19937_64 rng(17);
     for (int i = 0; i < scales; ++i) {
