@@ -115,7 +115,7 @@ template <bool GAPS> struct BlockCells {
 __device__ __forceinline__ int meta_words_of(int topk) { return topk == 0 ? 1 : topk + 2; }
 
 // ---------------------------------------------------------------------------------------------
-// quantize: a wavefront works on tiles of 64 * EL elements (64 lanes x 32 bytes of the tensor, 16 for one policy)
+// quantize: a wavefront owns one tile of 64 * EL elements (64 lanes x 32 bytes of the tensor)
 // ---------------------------------------------------------------------------------------------
 // Elements per lane: 32 bytes of the tensor, twice what the other kernels of this format give a lane.  What a
 // policy costs per group - addresses, the NaN rule of the running maximum, the outlier searches, the division behind
