@@ -708,12 +708,13 @@ const Stages *stages_of(PyObject *o) {
 }
 uint8_t *row_of(const Stages &s, int which, int64_t row) { return static_cast<uint8_t *>(s.rows[which].data_ptr()) + row * s.stride; }
 
-// pipeline_step(table, plan, stages, tensor, residual, plan, stages, mean, plan, stages, out, stream): quantize of `tensor` (with
-// `residual`, updated in place, or None), reduce + requantize, decode into `out`; a stage whose plan is None is absent.  `table`
-// names the plan methods the call stands for.  One launch: True; no grid for this combination: False, nothing was launched.
+// pipeline_step(table, plan, stages, tensor, residual, plan, stages, mean, plan, stages, out, access, stream): quantize of `tensor`
+// (with `residual`, updated in place, or None), reduce + requantize, decode into `out`; a stage whose plan is None is absent.
+// `table` names the plan methods the call stands for.  One launch: True; no grid for this combination: False, nothing was launched.
 PyObject *pipeline_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 12) return elsewhere();
+    long access;
+    if (n != 13 || !integer(a[11], access)) return elsewhere();
     PyObject *const table = a[0];
     lbc_quant_chunks_stage quant{};
     lbc_reduce_quant_stage reduce{};
@@ -764,11 +765,11 @@ PyObject *pipeline_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (first == nullptr) return elsewhere();
     auto call = [&](void *stream) {
         return lbc_bucket_pipeline_step_any(has_quant ? &quant : nullptr, has_reduce ? &reduce : nullptr, has_decode ? &decode : nullptr,
-                                            first->group, LBC_ACCESS_AUTO, stream);
+                                            first->group, static_cast<int>(access), stream);
     };
-    if (a[11] == Py_None) return answer(enqueue(first->rows[0].get_device(), call));
-    if (!PyLong_Check(a[11])) return elsewhere();
-    void *stream = PyLong_AsVoidPtr(a[11]);
+    if (a[12] == Py_None) return answer(enqueue(first->rows[0].get_device(), call));
+    if (!PyLong_Check(a[12])) return elsewhere();
+    void *stream = PyLong_AsVoidPtr(a[12]);
     if (PyErr_Occurred()) return elsewhere();
     int rc;
     Py_BEGIN_ALLOW_THREADS

@@ -257,10 +257,11 @@ class BucketPipeline:
 
     def _step_natively(self, lane: _Lane, arriving: _Bucket | None, residual: torch.Tensor | None, reducing: _Bucket | None,
                        decoding: _Bucket | None) -> bool:
-        """The ready stages as one native call; ``False``: nothing was launched, bind and launch them instead."""
+        """The ready stages as one native call, in the access mode that is the default now (:class:`ops.access_mode`); ``False``:
+        nothing was launched, bind and launch them instead."""
         if self._merge_stages is not self._own_merge or type(self) is not BucketPipeline:
             return False
-        args: list = [STAGE_METHODS, None, None, None, None, None, None, None, None, None, None, lane.handle]
+        args: list = [STAGE_METHODS, None, None, None, None, None, None, None, None, None, None, ops.access_code(None), lane.handle]
         count = 0
         if arriving is not None:
             plan = arriving.plan

@@ -38,7 +38,8 @@ class access_mode:
     """``with access_mode("cached"):`` - launches *bound* inside the block without an explicit ``access=`` use
     that mode ("auto": the library's rule, "cached": plain cached accesses for operands that are still in cache,
     "stream": non-temporal loads).  The mode is fixed when a launch is bound; replaying a :class:`BoundLaunch`
-    later does not consult this default again.  Results never depend on the mode."""
+    later does not consult this default again.  The pipelined transport's steps and the codec modules' calls, which are not
+    bound, take the default of the moment they are made in.  Results never depend on the mode."""
 
     def __init__(self, mode: str) -> None:
         if mode not in ACCESS_MODES:

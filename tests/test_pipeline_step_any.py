@@ -171,3 +171,43 @@ def test_native_step_leaves_other_operands_to_the_bound_launches(hip_device):
     rows = torch.zeros(2, 64, dtype=torch.uint8, device=hip_device)
     with pytest.raises(ValueError, match="do not belong"):
         _host.Stages(6400, 2, 0, 64, 0, rows, rows, rows)
+
+
+def step_kernels(run):
+    """The shared-grid kernels that `run` launches, as (access mode, group size); fp32 buckets only."""
+    import re
+
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    found = [re.search(r"bucket_pipeline_step_kernel<float, \w+, \d+, \d+, (\d+), (\d+)>", e.name) for e in prof.events()]
+    return [tuple(int(v) for v in f.groups()) for f in found if f]
+
+
+MODES = {"auto": 2, "stream": 2, "cached": 1}      # kStream, kVector
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("group", (64,))
+def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device, group, mode):
+    from lowbit_comm_amd.hip.reduce_scatter import make_reduce_scatter_transport
+
+    def run(transport, tensors):
+        futures = [transport(t, config=CompressionConfig(group_size=group), op="mean") for t in tensors]
+        transport.flush()
+        return [f.wait() for f in futures]
+
+    def transport():
+        return make_reduce_scatter_transport(world_size=4, rank=0, pipelined=True, all_to_all=lambda received, send: received.copy_(send),
+                                             all_gather=lambda gathered, mine: gathered[1:, :mine.numel()].copy_(mine))
+
+    sources = [gradient(64 * 4 * 40, torch.float32, 400 + k, hip_device) for k in range(4)]
+    want = run(transport(), [t.clone() for t in sources])
+    mine, pipe = [t.clone() for t in sources], transport()
+    with ops.access_mode(mode):
+        kernels = step_kernels(lambda: run(pipe, mine))
+    assert kernels == [(MODES[mode], group)] * 4
+    assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(mine, want))
