@@ -266,8 +266,7 @@ int lbc_bucket_pipeline_step(const lbc_quant_chunks_stage *quant, const lbc_redu
 
 /* The same, in one grid also for groups of 32 and 16 and for operands at element alignment (a bucket whose size is no
  * multiple of anything, a view): LBC_UNSUPPORTED only for another residual than none or fp32 and for stages of different
- * element types.  The access mode counts where lbc_bucket_pipeline_step has a grid; other launches stream.  Results are
- * bit-identical to the separate calls. */
+ * element types.  Results are bit-identical to the separate calls. */
 int lbc_bucket_pipeline_step_any(const lbc_quant_chunks_stage *quant, const lbc_reduce_quant_stage *reduce,
                                  const lbc_dequant_chunks_stage *decode, int group_size, int access, void *stream);
 

@@ -527,7 +527,7 @@ static int pipeline_step(const char *what, bool any, const lbc_quant_chunks_stag
     const lbc::DecodeArgs *da = d.empty ? nullptr : &d.args;
     if (group_size == 64 && aligned)
         return finish(lbc::launch_pipeline_step(dtype, r_dtype, vec, pick_mode(true, access), qa, q.world, ra, r.world, da, d.world, s), what);
-    return finish(lbc::launch_pipeline_step_any(dtype, r_dtype, vec, group_size, pick_mode(aligned, LBC_ACCESS_AUTO), qa, q.world, ra,
+    return finish(lbc::launch_pipeline_step_any(dtype, r_dtype, vec, group_size, pick_mode(aligned, access), qa, q.world, ra,
                                                 da, d.world, s), what);
 }
 

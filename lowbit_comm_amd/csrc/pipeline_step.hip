@@ -113,7 +113,7 @@ hipError_t launch_t(int r_dtype, int quant_vec, int reduce_world, int mode, cons
     return hipErrorNotSupported;
 }
 
-// Buckets whose chunks start anywhere, and groups of 32 and 16: one kernel per group size and alignment, the number of
+// Buckets whose chunks start anywhere, and groups of 32 and 16: one kernel per group size, alignment and access mode, the number of
 // payloads a run-time value (a template over it would be eight times as many kernels).  When one stage's operands are at
 // element alignment all three run that code; the ramps and the launches saved are worth more.  An iteration through the
 // pipelined hook, three launches a bucket against one: eight buckets of 13,107,201 elements, W = 8, bf16 with error feedback
@@ -122,14 +122,16 @@ hipError_t launch_t(int r_dtype, int quant_vec, int reduce_world, int mode, cons
 template <typename T, typename RT, int VEC>
 hipError_t launch_any_v(int g, int mode, const QuantArgs *q, int quant_world, const ReduceQuantArgs *r, const DecodeArgs *d,
                         int decode_world, hipStream_t s) {
-    const bool aligned = mode != kUnaligned;
+    const bool vector = mode == kVector, stream = mode == kStream;
     switch (g) {
-        case 64: return aligned ? launch_step<T, RT, VEC, 0, kStream, 64>(q, quant_world, r, d, decode_world, s)
-                                : launch_step<T, RT, VEC, 0, kUnaligned, 64>(q, quant_world, r, d, decode_world, s);
-        case 32: return aligned ? launch_step<T, RT, VEC, 0, kStream, 32>(q, quant_world, r, d, decode_world, s)
-                                : launch_step<T, RT, VEC, 0, kUnaligned, 32>(q, quant_world, r, d, decode_world, s);
-        case 16: return aligned ? launch_step<T, RT, VEC, 0, kStream, 16>(q, quant_world, r, d, decode_world, s)
-                                : launch_step<T, RT, VEC, 0, kUnaligned, 16>(q, quant_world, r, d, decode_world, s);
+        case 64: return stream ? launch_step<T, RT, VEC, 0, kStream, 64>(q, quant_world, r, d, decode_world, s)
+                               : launch_step<T, RT, VEC, 0, kUnaligned, 64>(q, quant_world, r, d, decode_world, s);
+        case 32: return vector ? launch_step<T, RT, VEC, 0, kVector, 32>(q, quant_world, r, d, decode_world, s)
+                      : stream ? launch_step<T, RT, VEC, 0, kStream, 32>(q, quant_world, r, d, decode_world, s)
+                               : launch_step<T, RT, VEC, 0, kUnaligned, 32>(q, quant_world, r, d, decode_world, s);
+        case 16: return vector ? launch_step<T, RT, VEC, 0, kVector, 16>(q, quant_world, r, d, decode_world, s)
+                      : stream ? launch_step<T, RT, VEC, 0, kStream, 16>(q, quant_world, r, d, decode_world, s)
+                               : launch_step<T, RT, VEC, 0, kUnaligned, 16>(q, quant_world, r, d, decode_world, s);
         default: return hipErrorNotSupported;
     }
 }

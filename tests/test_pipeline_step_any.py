@@ -191,8 +191,10 @@ MODES = {"auto": 2, "stream": 2, "cached": 1}      # kStream, kVector
 
 
 @pytest.mark.parametrize("mode", MODES)
-@pytest.mark.parametrize("group", (64,))
-def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device, group, mode):
+@pytest.mark.parametrize("group", (64, 32, 16))
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("error_feedback", (False, True))
+def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device, dtype, error_feedback, group, mode):
     from lowbit_comm_amd.hip.reduce_scatter import make_reduce_scatter_transport
 
     def run(transport, tensors):
@@ -200,14 +202,17 @@ def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device
         transport.flush()
         return [f.wait() for f in futures]
 
-    def transport():
-        return make_reduce_scatter_transport(world_size=4, rank=0, pipelined=True, all_to_all=lambda received, send: received.copy_(send),
-                                             all_gather=lambda gathered, mine: gathered[1:, :mine.numel()].copy_(mine))
+    def transport(**kwargs):
+        return make_reduce_scatter_transport(world_size=4, rank=0, all_to_all=lambda received, send: received.copy_(send),
+                                             all_gather=lambda gathered, mine: gathered[1:, :mine.numel()].copy_(mine),
+                                             error_feedback=error_feedback, **kwargs)
 
-    sources = [gradient(64 * 4 * 40, torch.float32, 400 + k, hip_device) for k in range(4)]
-    want = run(transport(), [t.clone() for t in sources])
-    mine, pipe = [t.clone() for t in sources], transport()
+    sources = [gradient(64 * 4 * 40, dtype, 400 + k, hip_device) for k in range(4)]
+    plain = transport()
+    want = [plain(t.clone(), config=CompressionConfig(group_size=group), op="mean") for t in sources]
+    mine, pipe = [t.clone() for t in sources], transport(pipelined=True)
     with ops.access_mode(mode):
         kernels = step_kernels(lambda: run(pipe, mine))
-    assert kernels == [(MODES[mode], group)] * 4
-    assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(mine, want))
+    assert dtype != torch.float32 or kernels == [(MODES[mode], group)] * 4
+    assert pipe.pipeline.stats["merged_launches"] == 4
+    assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(mine, want))
