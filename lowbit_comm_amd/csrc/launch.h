@@ -156,7 +156,7 @@ hipError_t launch_bucket_step(int x_dtype, int r_dtype, int quant_vec, int out_d
 hipError_t launch_pipeline_step(int dtype, int r_dtype, int quant_vec, int mode, const QuantArgs *quant, int quant_world,
                                 const ReduceQuantArgs *reduce, int reduce_world, const DecodeArgs *decode, int decode_world,
                                 hipStream_t stream);
-// The same in any group size, at element alignment (mode 0) or aligned (modes 1 and 2).
+// The same for what that has no kernel for: groups of 32 and 16, and any group at element alignment (mode 0).
 hipError_t launch_pipeline_step_any(int dtype, int r_dtype, int quant_vec, int group_size, int mode, const QuantArgs *quant,
                                     int quant_world, const ReduceQuantArgs *reduce, const DecodeArgs *decode, int decode_world,
                                     hipStream_t stream);

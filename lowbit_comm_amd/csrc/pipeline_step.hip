@@ -124,8 +124,8 @@ hipError_t launch_any_v(int g, int mode, const QuantArgs *q, int quant_world, co
                         int decode_world, hipStream_t s) {
     const bool vector = mode == kVector, stream = mode == kStream;
     switch (g) {
-        case 64: return stream ? launch_step<T, RT, VEC, 0, kStream, 64>(q, quant_world, r, d, decode_world, s)
-                               : launch_step<T, RT, VEC, 0, kUnaligned, 64>(q, quant_world, r, d, decode_world, s);
+        case 64: return vector || stream ? hipErrorNotSupported     // aligned groups of 64: launch_pipeline_step
+                                         : launch_step<T, RT, VEC, 0, kUnaligned, 64>(q, quant_world, r, d, decode_world, s);
         case 32: return vector ? launch_step<T, RT, VEC, 0, kVector, 32>(q, quant_world, r, d, decode_world, s)
                       : stream ? launch_step<T, RT, VEC, 0, kStream, 32>(q, quant_world, r, d, decode_world, s)
                                : launch_step<T, RT, VEC, 0, kUnaligned, 32>(q, quant_world, r, d, decode_world, s);
