@@ -117,8 +117,11 @@ class ReduceScatterPlan:
         if (type(self) is not ReduceScatterPlan or ops._host is None or self.reduced_dtype != self.dtype or not self.numel
                 or self.world_size > ops.MAX_PAYLOADS or self.device.type != "cuda"):
             return None
-        made = ops._host.Stages(self.numel, self.world_size, self.rank, self.config.group_size, ops.DTYPE_CODES[self.dtype],
-                                self.send, self.received, self.gathered)
+        try:
+            made = ops._host.Stages(self.numel, self.world_size, self.rank, self.config.group_size, ops.DTYPE_CODES[self.dtype],
+                                    self.send, self.received, self.gathered)
+        except ValueError:      # matrices that have been replaced by others, of another layout: the bound launches take them
+            made = None
         self._stages = (self.send, self.received, self.gathered, made)
         return made
 

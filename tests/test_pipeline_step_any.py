@@ -216,3 +216,32 @@ def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device
     assert dtype != torch.float32 or kernels == [(MODES[mode], group)] * 4
     assert pipe.pipeline.stats["merged_launches"] == 4
     assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(mine, want))
+
+
+@pytest.mark.parametrize("change", ("row stride", "spaced rows"))
+def test_pipelined_transport_takes_plans_with_matrices_of_their_own(hip_device, change):
+    """A plan whose receive matrix has another row stride or rows that are not back to back, and one that requantizes into a row
+    of its own (which is what the gather is handed), give the buckets that the plain plan gives."""
+    from lowbit_comm_amd.hip.bucket_pipeline import BucketPipeline
+    from lowbit_comm_amd.hip.reduce_scatter import ReduceScatterPlan
+
+    def factory(*args, **kwargs):
+        plan = ReduceScatterPlan(*args, **kwargs)
+        world, stride = plan.received.shape
+        if change == "row stride":
+            plan.received = torch.zeros(world, stride + 256, dtype=torch.uint8, device=hip_device)
+        elif change == "spaced rows":
+            plan.received = torch.zeros(world, 2 * stride, dtype=torch.uint8, device=hip_device)[:, :stride]
+        else:
+            plan.my_row = torch.zeros(plan.payload_bytes, dtype=torch.uint8, device=hip_device)
+        return plan
+
+    def run(**kwargs):
+        pipe = BucketPipeline(world_size=4, rank=1, all_to_all=lambda received, send: received[:, :send.shape[1]].copy_(send),
+                              all_gather=lambda gathered, mine: gathered[:, :mine.numel()].copy_(mine.clone()), **kwargs)
+        futures = [pipe.submit(gradient(n, torch.bfloat16, n, hip_device), config=CompressionConfig()) for n in (10_001, 4096, 10_001, 10_001)]
+        pipe.flush()
+        return [f.wait().clone() for f in futures]
+
+    for got, want in zip(run(plan_factory=factory), run()):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
