@@ -112,17 +112,20 @@ class ReduceScatterPlan:
     def stages(self) -> Any | None:
         """This plan's buffers as the native pipeline step addresses them, or ``None`` for a plan it does not serve."""
         held = self._stages
-        if held is not None and held[0] is self.send and held[1] is self.received and held[2] is self.gathered:
-            return held[3]
+        if (held is not None and held[0] is self.send and held[1] is self.received and held[2] is self.gathered
+                and held[3] is self.my_row):
+            return held[4]
         if (type(self) is not ReduceScatterPlan or ops._host is None or self.reduced_dtype != self.dtype or not self.numel
                 or self.world_size > ops.MAX_PAYLOADS or self.device.type != "cuda"):
             return None
-        try:
-            made = ops._host.Stages(self.numel, self.world_size, self.rank, self.config.group_size, ops.DTYPE_CODES[self.dtype],
-                                    self.send, self.received, self.gathered)
-        except ValueError:      # matrices that have been replaced by others, of another layout: the bound launches take them
-            made = None
-        self._stages = (self.send, self.received, self.gathered, made)
+        made = None
+        if self.my_row.data_ptr() == self.gathered[self.rank].data_ptr():      # else the shard goes somewhere else
+            try:
+                made = ops._host.Stages(self.numel, self.world_size, self.rank, self.config.group_size,
+                                        ops.DTYPE_CODES[self.dtype], self.send, self.received, self.gathered)
+            except ValueError:  # matrices that have been replaced by others, of another layout: the bound launches take them
+                pass
+        self._stages = (self.send, self.received, self.gathered, self.my_row, made)
         return made
 
     # ---- payload views ---------------------------------------------------------------------------

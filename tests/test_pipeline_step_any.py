@@ -218,7 +218,7 @@ def test_pipelined_transport_launches_in_the_default_access_mode(ops, hip_device
     assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(mine, want))
 
 
-@pytest.mark.parametrize("change", ("row stride", "spaced rows"))
+@pytest.mark.parametrize("change", ("row stride", "spaced rows", "own row"))
 def test_pipelined_transport_takes_plans_with_matrices_of_their_own(hip_device, change):
     """A plan whose receive matrix has another row stride or rows that are not back to back, and one that requantizes into a row
     of its own (which is what the gather is handed), give the buckets that the plain plan gives."""
