@@ -86,6 +86,11 @@ class _Lane:
         self.ready = None if stream is None else torch.cuda.Event()    # "the caller's stream has got this far", reused
 
 
+def _stages_of(plan: Any) -> Any | None:
+    """A plan's buffers for the native step; ``None`` for a plan of another kind, of which only the bound stages are known."""
+    return plan.stages() if isinstance(plan, ReduceScatterPlan) else None
+
+
 class BucketPipeline:
     """``submit(tensor, config=..., op=...)`` per bucket, in arrival order; ``flush()`` after the last one.
 
@@ -265,19 +270,19 @@ class BucketPipeline:
         count = 0
         if arriving is not None:
             plan = arriving.plan
-            stages = plan.stages()
+            stages = _stages_of(plan)
             if stages is None or plan.exchange_in_flight is not None:
                 return False
             args[1:5] = plan, stages, arriving.tensor, residual
             count += 1
         if reducing is not None:
-            stages = reducing.plan.stages()
+            stages = _stages_of(reducing.plan)
             if stages is None:
                 return False
             args[5:8] = reducing.plan, stages, reducing.op == "mean"
             count += 1
         if decoding is not None:
-            stages = decoding.plan.stages()
+            stages = _stages_of(decoding.plan)
             if stages is None:
                 return False
             args[8:11] = decoding.plan, stages, decoding.out

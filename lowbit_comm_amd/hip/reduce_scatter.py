@@ -111,12 +111,14 @@ class ReduceScatterPlan:
 
     def stages(self) -> Any | None:
         """This plan's buffers as the native pipeline step addresses them, or ``None`` for a plan it does not serve."""
+        if type(self) is not ReduceScatterPlan:      # a subclass need not have been made by this class's constructor either
+            return None
         held = self._stages
         if (held is not None and held[0] is self.send and held[1] is self.received and held[2] is self.gathered
                 and held[3] is self.my_row):
             return held[4]
-        if (type(self) is not ReduceScatterPlan or ops._host is None or self.reduced_dtype != self.dtype or not self.numel
-                or self.world_size > ops.MAX_PAYLOADS or self.device.type != "cuda"):
+        if (ops._host is None or self.reduced_dtype != self.dtype or not self.numel or self.world_size > ops.MAX_PAYLOADS
+                or self.device.type != "cuda"):
             return None
         made = None
         if self.my_row.data_ptr() == self.gathered[self.rank].data_ptr():      # else the shard goes somewhere else

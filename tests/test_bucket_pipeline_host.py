@@ -482,3 +482,22 @@ def test_the_two_forms_exclude_each_other():
         BucketPipeline(world_size=2, rank=0, all_to_all=lambda r, s: None, whole_gather=lambda r, m: None)
     with pytest.raises(ValueError, match="one exchange"):
         BucketPipeline(world_size=2, rank=0, whole_gather=lambda r, m: None, all_gather=lambda g, m: None)
+
+
+def test_plans_of_another_class_need_only_the_bound_stages():
+    """Without a merge step of its own a pipeline still asks a plan for nothing but its buffers and bound stages."""
+    log = []
+    pipe = BucketPipeline(world_size=8, rank=0, all_to_all=lambda received, send: log.append("a2a"),
+                          all_gather=lambda gathered, mine: log.append("ag"), future_factory=torch.futures.Future,
+                          plan_factory=lambda *a, **k: FakePlan(*a, log=log, **k))
+    FakePlan.made = 0
+    tensor = bucket_tensor(0)
+    future = pipe.submit(tensor, config=CFG, op="mean")
+    pipe.flush()
+    assert future.done() and log == [("Q", 0, False), "a2a", ("RQ", 1, "mean"), "ag", ("D", 1)]
+
+
+def test_a_subclass_with_a_constructor_of_its_own_has_no_native_stages():
+    from lowbit_comm_amd.hip.reduce_scatter import AllGatherPlan
+
+    assert AllGatherPlan(640, torch.float32, world_size=2, rank=0, config=CFG, device="cpu").stages() is None
