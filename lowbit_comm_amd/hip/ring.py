@@ -524,11 +524,11 @@ class HipPipelinedRingRuntime:
         if self.stream is None and not self.callers_stream:
             self.stream = torch.cuda.Stream()       # default priority
 
-    def run_stream(self) -> Any:
-        """The stream that a run submitted now goes to."""
+    def run_stream(self, tensor: Any) -> Any:
+        """The stream that a run on ``tensor`` submitted now goes to."""
         import torch
 
-        return torch.cuda.current_stream() if self.callers_stream else self.stream
+        return torch.cuda.current_stream(tensor.device) if self.callers_stream else self.stream
 
     def _plan_of(self, tensor: Any, raw_stream: int) -> dict | None:
         if self.max_plans == 0:
@@ -921,9 +921,8 @@ def make_pipelined_ring_executor(*, config: CompressionConfig, dtype: str, numel
                                       collective="all_reduce", strategy="pipelined_ring", device=device)
 
     def session_for(tensor: Any) -> Any:
-        del tensor
         runtime._ready()
-        return provider.begin(stream=runtime.run_stream())
+        return provider.begin(stream=runtime.run_stream(tensor))
 
     return PipelinedRingExecutor(schedule=schedule, runtime=runtime, workspace_session_factory=session_for,
                                  completion_manager=manager)

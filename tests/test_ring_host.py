@@ -378,3 +378,33 @@ def test_runtime_rejects_policies_the_ring_step_kernel_does_not_serve():
         HipPipelinedRingRuntime(config=CompressionConfig(), **{**ok, "rank": 4})
     with pytest.raises(TypeError, match="exchange must be callable"):
         HipPipelinedRingRuntime(config=CompressionConfig(), **{**ok, "exchange": None})
+
+
+def test_callers_stream_workspaces_are_leased_for_the_stream_of_the_tensors_device(monkeypatch):
+    """The launches of a run go to the stream that is current on the tensor's device, which need not be the current device."""
+    import torch
+
+    from lowbit_comm_amd.config import CompressionConfig
+    from lowbit_comm_amd.hip.ring import make_pipelined_ring_executor
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: ("current stream of", str(device)))
+    executor = make_pipelined_ring_executor(config=CompressionConfig(), dtype="fp32", numel=640, world_size=4, rank=0,
+                                            exchange=lambda *a, **k: None, device="cuda:1", max_plans=0, callers_stream=True)
+    bucket = type("Bucket", (), {"device": torch.device("cuda:1")})()
+    assert executor._sessions(bucket)._stream == ("current stream of", "cuda:1")
+
+
+def test_callers_stream_plans_are_kept_per_stream():
+    import torch
+
+    from lowbit_comm_amd.config import CompressionConfig
+    from lowbit_comm_amd.hip.ring import HipPipelinedRingRuntime
+
+    common = dict(config=CompressionConfig(), dtype="fp32", world_size=4, rank=0, exchange=lambda *a, **k: None)
+    bucket, other = torch.zeros(640), torch.zeros(640)
+    runtime = HipPipelinedRingRuntime(callers_stream=True, **common)
+    first, second = runtime._plan_of(bucket, 0x10), runtime._plan_of(bucket, 0x20)
+    assert first is not second and first is not runtime._plan_of(other, 0x10)
+    assert runtime._plan_of(bucket, 0x10) is first and runtime._plan_of(bucket, 0x20) is second and len(runtime.plans) == 3
+    runtime = HipPipelinedRingRuntime(**common)               # a stream of the ring's own: one plan for a bucket
+    assert runtime._plan_of(bucket, 0x10) is runtime._plan_of(bucket, 0x20)
