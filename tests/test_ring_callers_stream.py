@@ -57,6 +57,12 @@ def test_ring_on_the_callers_stream(hip_device, dtype):
         torch.cuda.synchronize()
         assert set(used) == {stream.cuda_stream}
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    # a plan per stream, with buffers of its own: one plan for both would have two streams write the same buffers
+    (synchronous,) = transport.executors.values()
+    plans = synchronous._runtime.plans
+    assert [key[2] for key in plans] == [default.cuda_stream, side.cuda_stream]
+    buffers = [{value.data_ptr() for key, value in plan.items() if key[0] in ("send", "recv")} for plan in plans.values()]
+    assert all(len(b) >= 2 * (world - 1) for b in buffers) and not buffers[0] & buffers[1]
     bucket.copy_(source)
     work = transport(bucket, config=config, op="mean", async_op=True)
     got = work.wait().clone()
