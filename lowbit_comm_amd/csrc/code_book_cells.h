@@ -39,7 +39,7 @@ constexpr Books kBookSet = {{
      0.125f, 0.16666666666666666f, 0.25f, 0.3333333333333333f, 0.5f, 0.6666666666666666f, 1.0f, __builtin_inff()},
 }};
 
-struct Cell {
+struct alignas(8) Cell {   // the kernel copies it as two dwords
     float threshold;   // the code rises by one at this value, the next step at or behind the left end; +inf behind the last
     uint32_t base;     // the code at the cell's left end
 };
@@ -178,7 +178,7 @@ static_assert(entries_far_apart(kBookSet.value[0]) && entries_far_apart(kBookSet
 
 // Entry 14 is the last that the search gives and 1 the largest t: its gap, infinite in the book, only has to keep the
 // fraction (t - 1) / gap from being positive.
-struct Gap {
+struct alignas(16) Gap {   // the kernel copies it as four dwords
     float low, gap, reciprocal, unused;
 };
 struct Gaps {

@@ -81,6 +81,9 @@ __device__ __forceinline__ const float *wave_code_book(int kind, int lane) {
 // wavefront of the workgroup must come to `publish`, which ends in a workgroup barrier that orders LDS only.
 template <bool GAPS> struct BlockCells {
     static constexpr int PER_THREAD = (book_cells::kCells + kBlock - 1) / kBlock;
+    static_assert(sizeof(book_cells::Cell) == sizeof(u32x2) && alignof(book_cells::Cell) >= alignof(u32x2) &&
+                      sizeof(book_cells::Gap) == sizeof(u32x4) && alignof(book_cells::Gap) >= alignof(u32x4),
+                  "the tables are copied in whole entries");
     u32x2 held[PER_THREAD];
     u32x4 held_gap;
     const book_cells::Cell *cells;
