@@ -8,7 +8,8 @@
 // [-1, 1] is cut into 256 cells of width 1/128.  A cell stores the code at its left end and the next step from there
 // on, inside the cell or beyond it, so that
 //     code(t) = cell.base + (t >= cell.threshold),   cell = cells[(unsigned)fma(t, 128, 128)]
-// for every finite t in [-1, 1].  tests/native/check_book_cells.cpp compares the two forms on every such float.
+// for every finite t in [-1, 1].  tests/native/check_book_cells.cpp compares the two forms on every such float on the host,
+// tests/native/book_cells_check.hip what the quantize kernel makes of them (below) on the device.
 //
 // The quantize kernel does not form t.  Steps lie at least two cells apart, so a cell answers for every t from its left
 // end to one and a half cells behind it: the cell one below the rounded place of an approximate quotient (`nearest_place`)
@@ -116,7 +117,8 @@ static_assert(steps_far_apart(kBookSet.value[0]) && steps_far_apart(kBookSet.val
                   steps_far_apart(kBookSet.value[2]) && steps_far_apart(kBookSet.value[3]),
               "two steps of a code book lie too close for one lookup");
 
-// The lookup of a quotient t.
+// The lookup of a quotient t.  No kernel runs it: the kernel's tables below are made from these cells, and
+// tests/native/check_book_cells.cpp holds them against the search.
 constexpr int cell_code(const Table &table, float t) {
     const Cell &cell = table.cell[cell_of(t)];
     return static_cast<int>(cell.base) + (t >= cell.threshold ? 1 : 0);

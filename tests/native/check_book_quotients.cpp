@@ -90,7 +90,7 @@ int main(int argc, char **argv) {
     const int scales = argc > 1 ? std::atoi(argv[1]) : 20000;
     std::mt19937_64 rng(17);
     for (int i = 0; i < scales; ++i) {
-        int exponent = static_cast<int>(rng() % 80) - 20;            // 2^-20 .. 2^59
+        int exponent = static_cast<int>(rng() % 81) - 20;            // 2^-20 .. 2^60, with the mantissa the kernel's range
         uint32_t mantissa = static_cast<uint32_t>(rng()) & 0x7FFFFFu;
         const int kind = i % 4;                                       // all bits, 8 significant ones, 11, few (exact quotients)
         if (kind == 1) mantissa &= 0x7F0000u;

@@ -6,7 +6,7 @@ ROOT = pathlib.Path(__file__).resolve().parent.parent
 
 
 def test_lookup_without_a_quotient_is_the_search_on_the_ieee_quotient(tmp_path):
-    """For each book and 20,000 scales from 2^-20 to 2^59 (all mantissa bits, 8, 11 and few): dividends next to every step
+    """For each book and 20,000 scales from 1e-6 to 2^61 (all mantissa bits, 8, 11 and few): dividends next to every step
     and cell end, 16-bit dividends around the steps and random ones, with reciprocals two ulps to either side.  For stochastic
     rounding the entry below a quotient against the search, and the fraction of the gap against the division for every
     significand and gap."""
