@@ -348,3 +348,23 @@ def test_fused_reduce_of_the_cuda_byte_format_refuses_divisors_without_a_positiv
     with pytest.raises(RuntimeError, match="divisor must be > 0"):
         module.inplace_dequantize_reduce_mean([payload], out, *policy, divisor)
     assert not module.inplace_dequantize_reduce_mean([payload], out[:100], *policy, divisor)   # not the fused reduce's
+
+
+# whole tensors whose codes stay within reach of the decode: written through above 4 Mi fp32 elements, plain above 8 Mi 16-bit
+# ones; the last workgroup and the last group are cut short
+@pytest.mark.parametrize("g", [64, 32, 16])
+@pytest.mark.parametrize("dtype, n", [("fp32", (1 << 22) + 4096 + 5), ("fp16", (1 << 23) + 4096 + 5), ("bf16", (1 << 23) + 4096 + 5)])
+def test_whole_tensors_whose_codes_are_kept(hip_device, dtype, n, g):
+    from lowbit_comm_amd.hip import cuda_wire, ops
+    from oracle import cuda_wire_np as wire
+    from tests.test_cuda_wire_parity import to_numpy
+
+    t = DTYPES[dtype]
+    x = values(n, t, n + g)
+    x_in = x.to(hip_device)
+    out = Guarded(cuda_wire.payload_nbytes(n, t, g), torch.uint8, 4, hip_device)
+    assert cuda_wire.quant_pack_into(x_in, out.inside, group_size=g, compact=False)
+    out.check(torch.from_numpy(wire.quantize(to_numpy(x), dtype, g, False)), "payload of the CUDA byte format")
+    out = Guarded(ops.payload_nbytes(n, g), torch.uint8, 16, hip_device)
+    assert ops.quant_pack_payload_into(x_in, out.inside, group_size=g)
+    out.check(codec_torch.pack(*codec_torch.quantize(x, g)), "portable payload")
