@@ -35,14 +35,18 @@ hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t str
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    // A single payload without a residual keeps its codes within reach of the launch that reads them next (16-bit tensors
-    // beyond 8 Mi elements: up to there the round trip gains little, and the all_gather hook's reduce of eight payloads loses,
-    // 18.5 against 18.8 us on 6.6 M bf16 elements).  us of quantize +
-    // decode, codes non-temporal / plain / written through, three tensors in rotation and (in brackets) enough of them to
-    // outrun the last-level cache: fp32 4.0 M 8.6 / 8.7 / 9.2 (10.7 / 9.5 / 10.0), 5.3 M 13.1 / 12.2 / 11.7 (12.9 / 11.4 /
-    // 11.9), 6.6 M 15.0 / 14.3 / 13.7 (14.7 / 13.3 / 13.6), 12 M 24.3 / 23.8 / 22.1 (23.4 / 21.0 / 21.1), 32 M 54.9 / 49.8 /
-    // 49.7 (54.6 / 49.6 / 49.3); bf16 6.6 M 9.1 / 9.2 / 9.3 (10.3 / 9.6 / 9.7), 12 M 12.7 / 12.6 / 14.4 (16.7 / 14.5 / 14.5),
-    // 32 M 32.7 / 31.8 / 31.4 (35.8 / 32.0 / 31.4).
+    // A single payload without a residual keeps its codes within reach of the launch that reads them next: plain stores up to
+    // 4 Mi fp32 elements and written through beyond; 16-bit tensors plain beyond 20 Mi elements.  us of quantize + decode, codes
+    // non-temporal / plain / written through, three tensors in rotation and (in brackets) enough of them to outrun the
+    // last-level cache: fp32 4.1 M 8.9 / 9.3 / 8.6 (10.9 / 9.7 / -), 5.2 M 12.7 / 11.8 / 11.2 (12.6 / 11.1 / 11.5), 6.6 M
+    // 14.9 / 16.0 / 14.3 (14.7 / 13.4 / 13.6), 13.1 M 26.5 / 26.2 / 23.9 (25.1 / 22.9 / 22.6), 26.2 M 46.3 / 41.5 / 42.3 (45.5 /
+    // 41.2 / 41.2); with the reduce of two payloads as the reader 13.1 M 28.2 / 27.6 / 26.2 (27.2 / 25.6 / 26.0); of four and eight
+    // within 2 % either way, but 4.3 and 5.2 M 3 % slower (4 payloads in rotation 13.2 / 13.7 / 13.7 and 15.2 / 15.6 / 15.6).
+    // 16-bit, non-temporal / plain, decode and reduce of two, four and eight payloads: 8.4 M 10.0 / 10.0, 14.4 / 16.3, 17.2 /
+    // 16.8, 22.6 / 22.4 (13.5 / 11.9, 15.0 / 14.7, 18.0 / 17.6, 22.7 / 22.5), 13.1 M 13.3 / 13.3, 19.9 / 22.0, 22.9 / 23.1,
+    // 31.6 / 30.8 (17.9 / 15.5, 20.6 / 19.3, 23.9 / 22.9, 32.7 / 31.3), 19.7 M 18.8 / 18.4, 26.7 / 26.7, 32.2 / 31.2, 46.4 / 44.9,
+    // 26.2 M 25.0 / 24.8, 32.7 / 32.2, 39.8 / 39.2, 58.9 / 55.8 (30.5 / 27.0, 34.9 / 32.6, 40.7 / 39.4, 60.3 / 57.1): below the
+    // line few buckets of two ranks lose up to 18 %; written through, the decode loses up to 15 % up to 23 M.
     if constexpr (is_void_t<RT>::value) {
         if (mode == kStream && world == 1) {
             if constexpr (VEC == 4 && TILES > 1) {
@@ -51,7 +55,7 @@ hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t str
                     return hipGetLastError();
                 }
             }
-            if (VEC == 4 || a.numel > (int64_t{8} << 20)) {
+            if (VEC == 4 || a.numel > (int64_t{20} << 20)) {
                 hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamKept, TILES>), grid, dim3(kBlock), 0, stream, a);
                 return hipGetLastError();
             }

@@ -33,7 +33,7 @@ template <> struct or_float<void> { using type = float; };
 // shard reduce) measured 20.17 ms that way against 20.74 ms with both non-temporal, 20.75 both written through,
 // 21.57 both plain and 21.97 the other way round; the 52 M-element bucket alone 89.9 against 93.2 us.
 // That holds for chunks, which leave for other ranks.  The one payload of a whole tensor is read on this GPU next, by its
-// decode or by a reduce that has it among its inputs: kStreamKept and kStreamThrough, chosen at quant_pack.hip's launch_typed.
+// decode or by a reduce that has it among its inputs: kStreamKept and kStreamThrough, chosen in quant_pack.hip's launch_tiles.
 template <bool HAS_RESIDUAL, int MODE> constexpr int quant_code_store_policy() {
     if (MODE < kStream || MODE == kStreamKept) return kCached;
     return HAS_RESIDUAL || MODE == kStreamThrough ? kSc1Bit : kNtBit;

@@ -350,10 +350,10 @@ def test_fused_reduce_of_the_cuda_byte_format_refuses_divisors_without_a_positiv
     assert not module.inplace_dequantize_reduce_mean([payload], out[:100], *policy, divisor)   # not the fused reduce's
 
 
-# whole tensors whose codes stay within reach of the decode: written through above 4 Mi fp32 elements, plain above 8 Mi 16-bit
+# whole tensors whose codes stay within reach of the decode: written through above 4 Mi fp32 elements, plain above 20 Mi 16-bit
 # ones; the last workgroup and the last group are cut short
 @pytest.mark.parametrize("g", [64, 32, 16])
-@pytest.mark.parametrize("dtype, n", [("fp32", (1 << 22) + 4096 + 5), ("fp16", (1 << 23) + 4096 + 5), ("bf16", (1 << 23) + 4096 + 5)])
+@pytest.mark.parametrize("dtype, n", [("fp32", (4 << 20) + 4096 + 5), ("fp16", (20 << 20) + 4096 + 5), ("bf16", (20 << 20) + 4096 + 5)])
 def test_whole_tensors_whose_codes_are_kept(hip_device, dtype, n, g):
     from lowbit_comm_amd.hip import cuda_wire, ops
     from oracle import cuda_wire_np as wire
@@ -368,3 +368,25 @@ def test_whole_tensors_whose_codes_are_kept(hip_device, dtype, n, g):
     out = Guarded(ops.payload_nbytes(n, g), torch.uint8, 16, hip_device)
     assert ops.quant_pack_payload_into(x_in, out.inside, group_size=g)
     out.check(codec_torch.pack(*codec_torch.quantize(x, g)), "portable payload")
+
+
+def template_numbers(name):
+    """The whole numbers among a kernel's template arguments, as the profiler prints them (mangled or not)."""
+    import re
+
+    if name.startswith("_Z"):
+        return [int(v) for v in re.findall(r"Li(\d+)E", name)]
+    return [int(v) for v in re.findall(r"(?<=[ <])\d+(?=[,>])", name)]
+
+
+# which form the codes of a whole tensor are stored in: kStream 2 (non-temporal), kStreamThrough 3, kStreamKept 4
+@pytest.mark.parametrize("dtype, n, mode", [("fp32", 4 << 20, 4), ("fp32", (4 << 20) + 64, 3), ("fp16", 20 << 20, 2),
+                                            ("fp16", (20 << 20) + 64, 4), ("bf16", 20 << 20, 2), ("bf16", (20 << 20) + 64, 4)])
+def test_store_form_of_a_whole_tensors_codes(hip_device, dtype, n, mode):
+    from lowbit_comm_amd.hip import ops
+    from tests.test_zy_perf_gate import kernel_names
+
+    x = torch.zeros(n, dtype=DTYPES[dtype], device=hip_device)
+    payload = torch.empty(ops.payload_nbytes(n), dtype=torch.uint8, device=hip_device)
+    (name,) = kernel_names(lambda: ops.quant_pack_payload_into(x, payload))
+    assert "quant_pack_kernel" in name and template_numbers(name)[:3] == [64, 4 if dtype == "fp32" else 8, mode], name
