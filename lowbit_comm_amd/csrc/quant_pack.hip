@@ -47,15 +47,23 @@ hipError_t launch_tiles(int mode, const QuantArgs &a, int world, hipStream_t str
     // 31.6 / 30.8 (17.9 / 15.5, 20.6 / 19.3, 23.9 / 22.9, 32.7 / 31.3), 19.7 M 18.8 / 18.4, 26.7 / 26.7, 32.2 / 31.2, 46.4 / 44.9,
     // 26.2 M 25.0 / 24.8, 32.7 / 32.2, 39.8 / 39.2, 58.9 / 55.8 (30.5 / 27.0, 34.9 / 32.6, 40.7 / 39.4, 60.3 / 57.1): below the
     // line few buckets of two ranks lose up to 18 %; written through, the decode loses up to 15 % up to 23 M.
+    // A launch with outputs of its own (the first one with error feedback, which has no residual yet) is not what the codes wait
+    // for: it keeps the hint up to 10 Mi elements of four a lane and writes through beyond.  us of the launch with an fp32 new
+    // residual, non-temporal / plain / written through, in rotation (beyond the cache): fp32 3.0 M 5.5 / 5.9 / 6.1 (5.9 / 6.2 /
+    // 6.4), 5.2 M 7.9 / 8.4 / 8.8 (9.0 / 9.2 / 9.6), 9.5 M 15.3 / 15.7 / 15.2 (15.9 / 15.8 / 15.5), 26.2 M 39.2 / 37.3 / 37.0; bf16
+    // 4.3 M 8.0 / 8.9 / 9.1 (8.3 / 9.0 / 8.8), 8.4 M 12.4 / 13.3 / 13.0 (12.8 / 13.4 / 13.1), 11 M 14.7 / 15.0 / 14.6, 26.2 M
+    // 31.5 / 30.1 / 29.7.
     if constexpr (is_void_t<RT>::value) {
-        if (mode == kStream && world == 1) {
-            if constexpr (VEC == 4 && TILES > 1) {
-                if (a.numel > (int64_t{4} << 20)) {
-                    hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamThrough, TILES>), grid, dim3(kBlock), 0, stream, a);
-                    return hipGetLastError();
-                }
+        const bool outputs = a.new_residual != nullptr || a.restored != nullptr || a.prepared != nullptr;
+        const bool whole = mode == kStream && world == 1;
+        if constexpr (VEC == 4 && TILES > 1) {
+            if (whole && a.numel > int64_t{outputs ? 10 : 4} << 20) {
+                hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamThrough, TILES>), grid, dim3(kBlock), 0, stream, a);
+                return hipGetLastError();
             }
-            if (VEC == 4 || a.numel > (int64_t{20} << 20)) {
+        }
+        if constexpr (VEC == 8 ? TILES > 1 : sizeof(XT) == 4) {   // four 16-bit elements a lane: always with outputs
+            if (whole && (VEC == 8 ? a.numel > int64_t{20} << 20 : !outputs)) {
                 hipLaunchKernelGGL((quant_pack_kernel<XT, RT, DT, G, VEC, kStreamKept, TILES>), grid, dim3(kBlock), 0, stream, a);
                 return hipGetLastError();
             }

@@ -380,13 +380,16 @@ def template_numbers(name):
 
 
 # which form the codes of a whole tensor are stored in: kStream 2 (non-temporal), kStreamThrough 3, kStreamKept 4
-@pytest.mark.parametrize("dtype, n, mode", [("fp32", 4 << 20, 4), ("fp32", (4 << 20) + 64, 3), ("fp16", 20 << 20, 2),
-                                            ("fp16", (20 << 20) + 64, 4), ("bf16", 20 << 20, 2), ("bf16", (20 << 20) + 64, 4)])
-def test_store_form_of_a_whole_tensors_codes(hip_device, dtype, n, mode):
+@pytest.mark.parametrize("dtype, new_residual, n, mode", [
+    ("fp32", False, 4 << 20, 4), ("fp32", False, (4 << 20) + 64, 3), ("fp16", False, 20 << 20, 2), ("fp16", False, (20 << 20) + 64, 4),
+    ("bf16", False, 20 << 20, 2), ("bf16", False, (20 << 20) + 64, 4), ("fp32", True, 10 << 20, 2), ("fp32", True, (10 << 20) + 64, 3),
+    ("fp16", True, 10 << 20, 2), ("fp16", True, (10 << 20) + 64, 3)])
+def test_store_form_of_a_whole_tensors_codes(hip_device, dtype, new_residual, n, mode):
     from lowbit_comm_amd.hip import ops
     from tests.test_zy_perf_gate import kernel_names
 
     x = torch.zeros(n, dtype=DTYPES[dtype], device=hip_device)
     payload = torch.empty(ops.payload_nbytes(n), dtype=torch.uint8, device=hip_device)
-    (name,) = kernel_names(lambda: ops.quant_pack_payload_into(x, payload))
-    assert "quant_pack_kernel" in name and template_numbers(name)[:3] == [64, 4 if dtype == "fp32" else 8, mode], name
+    fresh = torch.empty(n, device=hip_device) if new_residual else None
+    (name,) = kernel_names(lambda: ops.quant_pack_payload_into(x, payload, new_residual=fresh))
+    assert "quant_pack_kernel" in name and template_numbers(name)[:3] == [64, 4 if new_residual or dtype == "fp32" else 8, mode], name
