@@ -237,17 +237,24 @@ hipError_t launch_wire_quant_s(int mode, const WireQuantArgs &a, int world, hipS
 
 // How the codes leave.  Interleaved with the scales in plain stores (a line is shared by neighbouring wavefronts).  Apart
 // from them with the non-temporal hint where they leave for other ranks (chunks), and for small tensors; the one payload of a large
-// tensor is read by its decode, or by a reduce, next.  us of quantize + decode of 26.2 M elements, non-temporal
-// against plain: fp32 46.5 / 41.5, bf16 31.1 / 29.1 (4-bit codes 41.5 / 41.5 and 27.3 / 28.0, which keep the hint); of 6.6 M
-// fp32 15.3, plain 16.4, written through 13.9; bf16 8.7 / 8.7, but the all_gather hook without error feedback 18.2 / 18.7.
-// Beside a residual plain at every size (SUM_NT above; 1.6 M fp32 of two payloads 10.9 -> 8.3 us).
+// tensor is read by its decode, or by a reduce, next.  us of quantize + decode, non-temporal / plain / written through, three
+// tensors in rotation and (in brackets) enough of them to outrun the last-level cache: fp32 4.3 M 11.5 / 11.0 / 10.4 (11.6 /
+// 10.5 / 10.8), 6.6 M 15.4 / 14.7 / 14.2 (15.3 / 13.6 / 14.0), 13.1 M 26.8 / 26.1 / 24.0 (25.6 / 23.1 / 23.1), 26.2 M 46.0 / 42.0 /
+// 42.4 (45.3 / 41.3 / 41.1), 52.4 M 85.6 / 79.0 / 77.3 (85.9 / 79.2 / 77.5); with the reduce of two payloads as the reader 6.6 M
+// 16.3 / 15.4 / 15.4, 13.1 M 28.5 / 27.0 / 26.1, 26.2 M 49.5 / 45.3 / 45.1, of four and eight 2 % slower at 6.6 M (18.9 / 19.3 / 19.3,
+// 23.6 / 23.7 / 24.1) and 2 % faster at 26.2 M.  16-bit, non-temporal / plain, decode and reduce of two: 8.4 M 13.8 / 14.2 and
+// 15.0 / 15.6 (14.0 / 12.4 and 16.1 / 15.5), 13.1 M 19.0 / 19.3 and 19.7 / 20.3 (18.5 / 16.1 and 20.0 / 19.2), 14.7 M 22.3 / 21.0 and
+// 20.9 / 21.3, 16.8 M 23.3 / 23.3 and 23.7 / 23.5 (22.9 / 20.0 and 24.9 / 23.8), 26.2 M 31.4 / 29.3 and 33.0 / 31.9: up to 7 %
+// slower in rotation below the line, faster on both sides of the cache from it on.  4-bit codes keep the hint (26.2 M 41.5 / 41.5 and
+// 27.3 / 28.0).  Beside a residual plain at every size (SUM_NT above; the hook's two launches, 2.5 M fp32 of two payloads 14.8 ->
+// 11.6 us, of eight 16.5 -> 15.9, 26.2 M 113.5 -> 104.8 and 140.9 -> 132.4; four payloads of 4.3 and 9.0 M 2 % slower).
 template <typename T, int G, int BIT, bool HAS_R, bool COMPACT>
 hipError_t launch_wire_quant_c(int mode, const WireQuantArgs &a, int world, hipStream_t stream) {
     if constexpr (COMPACT) return launch_wire_quant_s<T, G, BIT, HAS_R, COMPACT, kPlain>(mode, a, world, stream);
     if constexpr (HAS_R && !COMPACT) {
         if (world == 1) return launch_wire_quant_s<T, G, BIT, HAS_R, COMPACT, kPlain>(mode, a, world, stream);
     } else if constexpr (BIT == 8 && !COMPACT) {
-        constexpr int64_t kLarge = (sizeof(T) == 4 ? int64_t{4} : int64_t{8}) << 20;
+        constexpr int64_t kLarge = (sizeof(T) == 4 ? int64_t{4} : int64_t{16}) << 20;
         constexpr int KEPT = sizeof(T) == 4 ? kWrittenThrough : kPlain;
         if (world == 1 && a.numel > kLarge) return launch_wire_quant_tiles<T, G, BIT, HAS_R, COMPACT, KEPT, 4>(mode, a, world, stream);
     }

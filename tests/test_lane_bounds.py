@@ -351,7 +351,7 @@ def test_fused_reduce_of_the_cuda_byte_format_refuses_divisors_without_a_positiv
 
 
 # whole tensors whose codes stay within reach of the decode: written through above 4 Mi fp32 elements, plain above 20 Mi 16-bit
-# ones; the last workgroup and the last group are cut short
+# ones (16 Mi in the CUDA byte format); the last workgroup and the last group are cut short
 @pytest.mark.parametrize("g", [64, 32, 16])
 @pytest.mark.parametrize("dtype, n", [("fp32", (4 << 20) + 4096 + 5), ("fp16", (20 << 20) + 4096 + 5), ("bf16", (20 << 20) + 4096 + 5)])
 def test_whole_tensors_whose_codes_are_kept(hip_device, dtype, n, g):
@@ -393,3 +393,16 @@ def test_store_form_of_a_whole_tensors_codes(hip_device, dtype, new_residual, n,
     fresh = torch.empty(n, device=hip_device) if new_residual else None
     (name,) = kernel_names(lambda: ops.quant_pack_payload_into(x, payload, new_residual=fresh))
     assert "quant_pack_kernel" in name and template_numbers(name)[:3] == [64, 4 if new_residual or dtype == "fp32" else 8, mode], name
+
+
+# the same in the CUDA byte format, scales apart: 1 non-temporal, 0 plain, 2 written through
+@pytest.mark.parametrize("dtype, n, codes", [("fp32", 4 << 20, 1), ("fp32", (4 << 20) + 64, 2), ("fp16", 16 << 20, 1),
+                                             ("fp16", (16 << 20) + 64, 0), ("bf16", 16 << 20, 1), ("bf16", (16 << 20) + 64, 0)])
+def test_store_form_of_a_whole_tensors_codes_in_the_cuda_byte_format(hip_device, dtype, n, codes):
+    from lowbit_comm_amd.hip import cuda_wire
+    from tests.test_zy_perf_gate import kernel_names
+
+    x = torch.zeros(n, dtype=DTYPES[dtype], device=hip_device)
+    payload = torch.empty(cuda_wire.payload_nbytes(n, x.dtype), dtype=torch.uint8, device=hip_device)
+    (name,) = kernel_names(lambda: cuda_wire.quant_pack_into(x, payload, compact=False))
+    assert "wire_quant_kernel" in name and template_numbers(name) == [64, 8, 1, codes, 4], name
