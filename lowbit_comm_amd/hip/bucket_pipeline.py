@@ -42,10 +42,15 @@ from lowbit_comm_amd.hip import ops
 from lowbit_comm_amd.hip.reduce_scatter import STAGE_METHODS, AllGatherPlan, ReduceScatterPlan, ResidualStore
 
 
+def _no_stages() -> None:
+    return None
+
+
 class _Bucket:
     """One bucket in flight: its plan (send / received / gathered rows), tensors, future and pending exchanges."""
 
-    __slots__ = ("plan", "tensor", "out", "op", "future", "exchange", "gather", "result", "lane", "lasting_out", "spans")
+    __slots__ = ("plan", "tensor", "out", "op", "future", "exchange", "gather", "result", "lane", "lasting_out", "spans",
+                 "stages")
 
     def __init__(self, plan: ReduceScatterPlan, tensor: torch.Tensor, out: torch.Tensor | None, op: str, future: Any,
                  lane: int, lasting_out: bool, spans: tuple) -> None:
@@ -60,6 +65,8 @@ class _Bucket:
         self.result: Any | None = None
         self.lane = lane
         self.spans = spans                    # byte ranges this bucket reads and writes while it is in flight
+        # the plan's buffers for the native step; of a plan of another kind only the bound stages are known
+        self.stages = plan.stages if isinstance(plan, ReduceScatterPlan) else _no_stages
 
 
 def _span(tensor: torch.Tensor) -> tuple[int, int]:
@@ -84,11 +91,6 @@ class _Lane:
         self.reduce_next: _Bucket | None = None
         self.decode_next: _Bucket | None = None
         self.ready = None if stream is None else torch.cuda.Event()    # "the caller's stream has got this far", reused
-
-
-def _stages_of(plan: Any) -> Any | None:
-    """A plan's buffers for the native step; ``None`` for a plan of another kind, of which only the bound stages are known."""
-    return plan.stages() if isinstance(plan, ReduceScatterPlan) else None
 
 
 class BucketPipeline:
@@ -266,28 +268,25 @@ class BucketPipeline:
         nothing was launched, bind and launch them instead."""
         if self._merge_stages is not self._own_merge or type(self) is not BucketPipeline:
             return False
-        args: list = [STAGE_METHODS, None, None, None, None, None, None, None, None, None, None, ops.access_code(None), lane.handle]
+        new = new_stages = tensor = middle = middle_stages = mean = old = old_stages = out = None
         count = 0
         if arriving is not None:
-            plan = arriving.plan
-            stages = _stages_of(plan)
-            if stages is None or plan.exchange_in_flight is not None:
+            new, new_stages, tensor = arriving.plan, arriving.stages(), arriving.tensor
+            if new_stages is None or new.exchange_in_flight is not None:
                 return False
-            args[1:5] = plan, stages, arriving.tensor, residual
             count += 1
         if reducing is not None:
-            stages = _stages_of(reducing.plan)
-            if stages is None:
+            middle, middle_stages, mean = reducing.plan, reducing.stages(), reducing.op == "mean"
+            if middle_stages is None:
                 return False
-            args[5:8] = reducing.plan, stages, reducing.op == "mean"
             count += 1
         if decoding is not None:
-            stages = _stages_of(decoding.plan)
-            if stages is None:
+            old, old_stages, out = decoding.plan, decoding.stages(), decoding.out
+            if old_stages is None:
                 return False
-            args[8:11] = decoding.plan, stages, decoding.out
             count += 1
-        if not count or not ops._host.pipeline_step(*args):
+        if not count or not ops._host.pipeline_step(STAGE_METHODS, new, new_stages, tensor, residual, middle, middle_stages, mean,
+                                                    old, old_stages, out, ops.ACCESS_MODES[ops._default_access], lane.handle):
             return False
         self.stats["merged_launches" if count > 1 else "separate_launches"] += 1
         return True

@@ -37,6 +37,9 @@ _ROW_ALIGN = 256
 class ReduceScatterPlan:
     """Pre-bound compute of one bucket shape at world size ``W`` for rank ``rank``."""
 
+    # what stages() answered and for which buffers; here, because a subclass may have a constructor of its own
+    _stages: tuple = (None, None, None, None, None)
+
     def __init__(self, numel: int, dtype: torch.dtype, *, world_size: int, rank: int, config: CompressionConfig,
                  device: torch.device | str, reduced_dtype: torch.dtype | None = None,
                  shape: tuple[int, ...] | None = None) -> None:
@@ -71,7 +74,6 @@ class ReduceScatterPlan:
         self._bound_lock = threading.Lock()   # DDP calls its hook from the autograd thread, a user may call from another
         self._last_stream: Any | None = None
         self._last_stream_handle: int | None = None
-        self._stages: tuple | None = None
         self.exchange_in_flight: Any | None = None     # work object of an exchange that nobody has waited for yet
 
     # Every bucket of one shape shares the plan, and every bucket has its own addresses: a transformer's stream of
@@ -111,14 +113,11 @@ class ReduceScatterPlan:
 
     def stages(self) -> Any | None:
         """This plan's buffers as the native pipeline step addresses them, or ``None`` for a plan it does not serve."""
-        if type(self) is not ReduceScatterPlan:      # a subclass need not have been made by this class's constructor either
-            return None
-        held = self._stages
-        if (held is not None and held[0] is self.send and held[1] is self.received and held[2] is self.gathered
-                and held[3] is self.my_row):
-            return held[4]
-        if (ops._host is None or self.reduced_dtype != self.dtype or not self.numel or self.world_size > ops.MAX_PAYLOADS
-                or self.device.type != "cuda"):
+        send, received, gathered, my_row, made = self._stages
+        if send is self.send and received is self.received and gathered is self.gathered and my_row is self.my_row:
+            return made
+        if (type(self) is not ReduceScatterPlan or ops._host is None or self.reduced_dtype != self.dtype or not self.numel
+                or self.world_size > ops.MAX_PAYLOADS or self.device.type != "cuda"):
             return None
         made = None
         if self.my_row.data_ptr() == self.gathered[self.rank].data_ptr():      # else the shard goes somewhere else
