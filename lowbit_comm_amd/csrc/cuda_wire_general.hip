@@ -437,7 +437,8 @@ __global__ __launch_bounds__(kBlock) void wire_general_quant_kernel(const WireGe
         // holds for a scale within 2^60 of 1 either way and |v| <= scale; the scale is at least 1e-6 here, and beside
         // outliers or a NaN an element may lie above it.  A wavefront with any other operand divides, and looks the
         // quotient up with scale 1; what lies outside [-1, 1] takes the first or last code, a NaN the last, as the search
-        // does.  9 instead of 21 instructions an element: 26.2 M elements of the normal book 24.5 -> 21.3 us (fp32, 119
+        // does.  15.2 instead of 21.1 vector instructions an element over the whole kernel (14.3 instead of 20.5 for 16-bit types):
+        // 26.2 M elements of the normal book 24.5 -> 21.3 us (fp32, 119
         // MB, 5.6 TB/s) and 19.9 -> 14.2 us (bf16), with two outliers 32.5 -> 27.5 and 30.0 -> 21.0; what is left of the
         // difference to the linear 4-bit pack kernel (19.6 and 13.0) is the table, 2 KiB copied per 2048 or 4096
         // elements (by workgroups half and a quarter as large: 25.8 and 29.4 us, fp32).
