@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define LBC_ABI_VERSION 8
+#define LBC_ABI_VERSION 9
 
 enum { LBC_OK = 0, LBC_UNSUPPORTED = 1, LBC_EINVAL = -1, LBC_ELAUNCH = -2 };
 
@@ -289,6 +289,14 @@ int lbc_bucket_pipeline_step_any(const lbc_quant_chunks_stage *quant, const lbc_
 int lbc_ring_step(const int8_t *recv_codes, const float *recv_scales, void *chunk, int dtype,
                   int64_t numel, int group_size, int reduce_op, float divisor, int8_t *send_codes,
                   float *send_scales, int access, void *stream);
+
+/*
+ * A hop of the ring's first phase that does not complete the sum: send = quantize(chunk + decode(received)), the sum
+ * in `dtype` arithmetic, with the chunk left as it is.  Same payload as lbc_ring_step with LBC_REDUCE_SUM and divisor 1
+ * writes; for a schedule that overwrites the chunk before it is read again.
+ */
+int lbc_ring_relay(const int8_t *recv_codes, const float *recv_scales, const void *chunk, int dtype, int64_t numel,
+                   int group_size, int8_t *send_codes, float *send_scales, int access, void *stream);
 
 /*
  * residual = prepared - restored, element-wise, subtraction in fp32, rounded to

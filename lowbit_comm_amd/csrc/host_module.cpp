@@ -122,6 +122,7 @@ constexpr Entry kEntries[] = {
     {"lbc_bucket_pipeline_step", make_call<&lbc_bucket_pipeline_step>},
     {"lbc_bucket_pipeline_step_any", make_call<&lbc_bucket_pipeline_step_any>},
     {"lbc_ring_step", make_call<&lbc_ring_step>},
+    {"lbc_ring_relay", make_call<&lbc_ring_relay>},
     {"lbc_ef_update", make_call<&lbc_ef_update>},
     {"lbc_wire_quant_pack", make_call<&lbc_wire_quant_pack>},
     {"lbc_wire_compensate_quant_pack", make_call<&lbc_wire_compensate_quant_pack>},

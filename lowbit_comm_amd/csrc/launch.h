@@ -69,6 +69,7 @@ struct RingStepArgs {
     float *send_scales;
     int64_t numel;
     float divisor;              // 1 = no division
+    int keep;                   // 0: the updated chunk is quantized but not written back
 };
 
 // ---- payload format of the reference's CUDA extension (cuda_wire.hip) ----------

@@ -541,8 +541,9 @@ int lbc_bucket_pipeline_step_any(const lbc_quant_chunks_stage *quant, const lbc_
     return pipeline_step("lbc_bucket_pipeline_step_any", true, quant, reduce, decode, group_size, access, stream);
 }
 
-int lbc_ring_step(const int8_t *recv_codes, const float *recv_scales, void *chunk, int dtype, int64_t numel,
-                  int group_size, int reduce_op, float divisor, int8_t *send_codes, float *send_scales, int access, void *stream) {
+namespace {
+int ring_step(const char *name, const int8_t *recv_codes, const float *recv_scales, void *chunk, bool keep, int dtype, int64_t numel,
+              int group_size, int reduce_op, float divisor, int8_t *send_codes, float *send_scales, int access, void *stream) {
     if (!valid_access(access)) return fail(LBC_EINVAL, "unknown access mode %d", access);
     if (numel < 0) return fail(LBC_EINVAL, "numel must be >= 0");
     if (!valid_dtype(dtype)) return fail(LBC_EINVAL, "unsupported chunk dtype %d", dtype);
@@ -563,10 +564,24 @@ int lbc_ring_step(const int8_t *recv_codes, const float *recv_scales, void *chun
     const int vec = 16 / dtype_size(dtype);   // elements, and code bytes, one lane owns
     const bool aligned = aligned_to(chunk, 16) && aligned_to(recv_codes, vec) &&
                          (send_codes == nullptr || aligned_to(send_codes, vec));
-    lbc::RingStepArgs a{recv_codes, recv_scales, chunk, send_codes, send_scales, numel, divisor};
+    lbc::RingStepArgs a{recv_codes, recv_scales, chunk, send_codes, send_scales, numel, divisor, keep};
     return finish(lbc::launch_ring_step(dtype, group_size, reduce_op == LBC_REDUCE_SUM, pick_mode(aligned, access), a,
                                         static_cast<hipStream_t>(stream)),
-                  "lbc_ring_step");
+                  name);
+}
+}  // namespace
+
+int lbc_ring_step(const int8_t *recv_codes, const float *recv_scales, void *chunk, int dtype, int64_t numel,
+                  int group_size, int reduce_op, float divisor, int8_t *send_codes, float *send_scales, int access, void *stream) {
+    return ring_step("lbc_ring_step", recv_codes, recv_scales, chunk, true, dtype, numel, group_size, reduce_op, divisor, send_codes,
+                     send_scales, access, stream);
+}
+
+int lbc_ring_relay(const int8_t *recv_codes, const float *recv_scales, const void *chunk, int dtype, int64_t numel,
+                   int group_size, int8_t *send_codes, float *send_scales, int access, void *stream) {
+    if (numel > 0 && send_codes == nullptr) return fail(LBC_EINVAL, "send codes and send scales must not be null");
+    return ring_step("lbc_ring_relay", recv_codes, recv_scales, const_cast<void *>(chunk), false, dtype, numel, group_size,
+                     LBC_REDUCE_SUM, 1.0f, send_codes, send_scales, access, stream);
 }
 
 int lbc_ef_update(const void *prepared, int prepared_dtype, const void *restored, int restored_dtype,

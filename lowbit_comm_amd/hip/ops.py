@@ -594,6 +594,19 @@ def bind_ring_step(received: torch.Tensor, chunk: torch.Tensor, send: torch.Tens
     return BoundLaunch("lbc_ring_step", args + (access_code(access),), device, (received, chunk, send))
 
 
+def bind_ring_relay(received: torch.Tensor, chunk: torch.Tensor, send: torch.Tensor, *, group_size: int = 64,
+                    access: str | None = None) -> BoundLaunch:
+    """:func:`bind_ring_step` with a sum that is only passed on: ``send`` receives the payload of ``chunk +
+    decode(received)`` and ``chunk`` stays as it is."""
+    code = _float_tensor(chunk, "chunk")
+    device, n = chunk.device, chunk.numel()
+    recv_codes, recv_scales = payload_addresses(received, n, group_size, name="received payload", device=device)
+    send_codes, send_scales = payload_addresses(send, n, group_size, name="send payload", device=device)
+    _require(n == 0 or send.data_ptr() != received.data_ptr(), "the payload to send must not alias the received one")
+    args = (recv_codes, recv_scales, _ptr(chunk), code, n, group_size, send_codes, send_scales)
+    return BoundLaunch("lbc_ring_relay", args + (access_code(access),), device, (received, chunk, send))
+
+
 def ring_step_into(received: torch.Tensor, chunk: torch.Tensor, send: torch.Tensor | None = None, *,
                    group_size: int = 64, reduce_op: str = "sum", divisor: float = 1.0,
                    access: str | None = None) -> bool:

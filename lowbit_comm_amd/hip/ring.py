@@ -10,7 +10,8 @@ the mean is handed round (all-gather).  One rule generates the whole schedule: a
 just received into, starting with its predecessor's chunk index, so that after W-1 steps rank r holds the complete
 chunk r.  The reference runs "decode into the chunk" and "quantize the chunk for the next hop" as separate kernels;
 the runtime here issues them as one launch of the ring-step kernel (``lbc_ring_step``), which quantizes the updated
-chunk while it is still in registers, and hands the staged payload to the next ``quant_pack`` call.  The point-to-point
+chunk while it is still in registers, and hands the staged payload to the next ``quant_pack`` call.  A hop whose chunk the
+second phase overwrites unread writes the payload only (``lbc_ring_relay``).  The point-to-point
 exchange itself is injected: ``exchange(payload, received, send_peer=, recv_peer=, stream=) -> handle``.
 """
 from __future__ import annotations
@@ -380,6 +381,9 @@ class PipelinedRingExecutor(TopologyExecutor):
                 for handle in handles:
                     submission.after_p2p(handle)
                 return
+        begin = getattr(runtime, "begin_schedule", None)
+        if callable(begin):
+            begin(context)
         for step in self.schedule.steps:
             received, handle = self._exchange(submission, step)
             submission.after(runtime.fused_reduce(tensor, received, step.recv_chunk, step.received_contributors,
@@ -421,6 +425,7 @@ class RingSubmissionContext:
     plan: dict | None = None           # buffers and bound launches of this tensor, when the runtime keeps plans
     raw_stream: int = 0
     program: list | None = None        # the launches and exchanges of this run in order, while a plan is being made
+    whole_schedule: bool = False       # the steps are those of a ring from its first to its last, in order
 
     def query(self) -> bool:
         return bool(self.producer_completion.query())
@@ -564,6 +569,15 @@ class HipPipelinedRingRuntime:
         recording = plan is not None and "program" not in plan and not self._facade
         return RingSubmissionContext(tensor=tensor, stream=stream, producer_completion=produced,
                                      plan=plan, raw_stream=raw_stream, program=[] if recording else None)
+
+    def begin_schedule(self, context: RingSubmissionContext) -> None:
+        """Every step of the ring follows: the second phase overwrites each chunk but this rank's own, so a hop that does not
+        complete the sum has no use for the updated chunk beyond its payload.  A run that fails in between leaves those
+        chunks as they came."""
+        cls = type(self)
+        context.whole_schedule = self.fuse_steps and not self._wire_direct and all(
+            getattr(cls, name) is getattr(HipPipelinedRingRuntime, name) and name not in self.__dict__
+            for name in ("quant_pack", "send_recv", "fused_reduce", "apply_broadcast", "_step", "_bind_step"))
 
     # ---- replay of a recorded run ------------------------------------------- #
     def finish_program(self, context: RingSubmissionContext) -> None:
@@ -742,14 +756,16 @@ class HipPipelinedRingRuntime:
             return self._facade_step(tensor, received, chunk, context, reduce_op=reduce_op, divisor=divisor)
         if another_hop is None:
             another_hop = context.steps_done < 2 * (self.world_size - 1)
-        plan, key = context.plan, ("step", context.steps_done, chunk.start, chunk.stop, received.data_ptr())
+        relay = context.whole_schedule and context.steps_done < self.world_size - 1
+        plan, key = context.plan, ("step", context.steps_done, chunk.start, chunk.stop, received.data_ptr(), relay)
         bound = None if plan is None else plan.get(key)
         if bound is None:
             view = _view(tensor, chunk)
             g = self.config.group_size
             if self.fuse_steps:
                 send = self._send_buffer(view, workspace, context) if another_hop else None
-                launches = (self._bind_step(received, view, send, reduce_op, divisor),)
+                launches = (ops.bind_ring_relay(received, view, send, group_size=g) if relay else
+                            self._bind_step(received, view, send, reduce_op, divisor),)
             else:
                 send = None
                 launches = (ops.bind_dequant(*ops.split_payload(received, view.numel(), g), view, group_size=g,
