@@ -1,6 +1,6 @@
 // Evidence for the quantizer's division-free exact quotient (csrc/device_utils.h: encode_group): for dividends p
 // and scales s from its domain (|p| <= 127.5 s, 2^-23 <= s <= FLT_MAX / 127), q1 = fma(fma(-q0, s, p), y, q0) with
-// y = 1/s and q0 = p*y is compared on the device with the division p/s, bit for bit, and so are the codes rint()
+// y = 1/s (reciprocal_of_scale there) and q0 = p*y is compared on the device with the division p/s, bit for bit, and so are the codes rint()
 // makes of them.
 //
 // Sampled modes, scale exponents over the whole domain (2^-23 .. 2^120): 0 random, 1 scale mantissa (almost) all
@@ -13,7 +13,8 @@
 // two as long as nothing underflows or overflows, which cannot happen for |p/s| >= 0.5 in the domain.  So mode 6
 // walks every one of the 2^23 mantissas of s (at exponent 0, and again at both ends of the exponent range), all 256
 // half-integers k + 0.5 in (-128, 128) and the 13 dividends within six ulps of RN((k + 0.5) * s): every case in
-// which the refined quotient could change a code.
+// which the refined quotient could change a code.  It also compares y itself, the hardware's reciprocal with one Newton
+// step, with the division 1.0f / s, for every mantissa at every exponent of the scales' range, bit for bit.
 //
 // Mode 7 is the other division-free quotient of the library (csrc/cuda_wire_general.hip, code-book quantizer):
 // the compiler's own expansion of v / s - v_rcp_f32, a Newton step, product, two corrections - with the reciprocal
@@ -34,8 +35,12 @@
 #include <stdlib.h>
 __device__ __forceinline__ uint32_t mix(uint64_t x) { x ^= x >> 33; x *= 0xff51afd7ed558ccdULL; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ULL; x ^= x >> 33; return (uint32_t)x; }
 struct Tally { unsigned long long tiny, quotient, code; };
+__device__ __forceinline__ float reciprocal(float s) {          // device_utils.h: reciprocal_of_scale
+    const float y = __builtin_amdgcn_rcpf(s);
+    return __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
+}
 __device__ __forceinline__ void compare(float p, float s, Tally &t, float *ex) {
-    const float y = 1.0f / s;
+    const float y = reciprocal(s);
     const float q0 = p * y;
     const float rem = __builtin_fmaf(-q0, s, p);
     const float q1 = __builtin_fmaf(rem, y, q0);
@@ -62,6 +67,12 @@ __global__ void check_all_ties(uint32_t sexp, unsigned long long *bad, float *ex
             if (fabsf(p) <= 127.5f * s) compare(p, s, t, ex);
         }
     }
+    publish(t, bad);
+}
+__global__ void check_reciprocals(uint32_t sexp, unsigned long long *bad, float *ex) {
+    const float s = __uint_as_float((sexp << 23) | (blockIdx.x * blockDim.x + threadIdx.x));
+    Tally t = {0, 0, 0};
+    if (__float_as_uint(reciprocal(s)) != __float_as_uint(1.0f / s)) { ++t.quotient; ex[0] = 1.0f; ex[1] = s; }
     publish(t, bad);
 }
 __global__ void check_shared_reciprocal(uint64_t seed, unsigned long long *bad, float *ex) {
@@ -145,7 +156,8 @@ int main(int argc, char **argv) {
         } else {
             const uint32_t exponents[3] = {127, 104, 247};      // 1, the smallest scale, the largest the domain holds
             for (uint32_t sexp : exponents) hipLaunchKernelGGL(check_all_ties, dim3((1u << 23) / 256), dim3(256), 0, 0, sexp, bad, ex);
-            n = 3ULL * (1ULL << 23) * 256ULL * 13ULL;
+            for (uint32_t sexp = 104; sexp <= 247; ++sexp) hipLaunchKernelGGL(check_reciprocals, dim3((1u << 23) / 256), dim3(256), 0, 0, sexp, bad, ex);
+            n = 3ULL * (1ULL << 23) * 256ULL * 13ULL + 144ULL * (1ULL << 23);
         }
         unsigned long long h[3]; float he[2];
         if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(h, bad, 24, hipMemcpyDeviceToHost) != hipSuccess ||
