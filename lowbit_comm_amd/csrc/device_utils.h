@@ -296,15 +296,15 @@ __device__ __forceinline__ float scale_from_absmax(float absmax) {
 }
 
 // Bit pattern of the largest magnitude in the group that the VEC values of LPG adjacent lanes form; every lane gets it.
+// Inside a lane the maximum is IEEE 754-2019's maximum, which keeps a NaN: gfx950 takes three operands and their absolute
+// values in one instruction (v_maximum3_f32), half of what masking the patterns for an integer maximum took: GPU time of the
+// ring of eight ranks on 26.2 M bf16 elements 59.9 -> 59.0 us, on 13.1 M 47.1 -> 46.6, of the plan on 4 M 10.5 -> 10.45.
 template <int VEC, int LPG>
 __device__ __forceinline__ uint32_t group_absmax_bits(const float (&p)[VEC]) {
-    uint32_t m = 0;
+    float m = __builtin_fabsf(p[0]);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        const uint32_t a = as_u32(p[i]) & 0x7FFFFFFFu;
-        m = a > m ? a : m;
-    }
-    return group_max_bits<LPG>(m);
+    for (int i = 1; i < VEC; ++i) m = __builtin_elementwise_maximum(m, __builtin_fabsf(p[i]));
+    return group_max_bits<LPG>(as_u32(m));
 }
 
 // 1 / scale, correctly rounded, for the scales a group can have (2^-23 .. FLT_MAX / 127; any other, an Inf or a NaN, has

@@ -107,12 +107,25 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
         const int64_t live_here = valid - block_first, padded_here = padded - block_first;
         const buffer_t x_b = buffer_over(x + block_first, T::BLOCK_ELEMS * sizeof(XT));
         const buffer_t r_b = buffer_over(HAS_R ? r + block_first : nullptr, T::BLOCK_ELEMS * sizeof(RLoad));
+        // The order in which whole blocks issue the two tensors' loads is worth up to 3 % where a wavefront has four tiles, and
+        // left alone the scheduler changes it with every change to the arithmetic behind: the residual's loads follow two
+        // tiles behind the input's (x0 x1 x2 r0 x3 r1 r2 r3).  us of the local step, input first / tile by tile / residual
+        // first tile by tile / residual first / this: 52.4 M bf16 elements 107.1 / 106.5 / 106.1 / 105.9 / 105.4, 26.2 M fp32
+        // 73.3 / 70.9 / 71.2 / 71.3 / 70.9.
+        constexpr int kLead = UNROLL > 2 ? 2 : 0;
+        auto load_r = [&](int u) __attribute__((always_inline)) {
+            buffer_load<RLoad, VEC, kLoad>(r_b, at[u] * sizeof(RLoad), rv[u]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             at[u] = static_cast<uint32_t>(tile_in_block<UNROLL>(u, wave)) * T::TILE + lane * VEC;
             if constexpr (BUFFERS) {
                 buffer_load<XT, VEC, kLoad>(x_b, at[u] * sizeof(XT), xv[u]);
-                if constexpr (HAS_R) buffer_load<RLoad, VEC, kLoad>(r_b, at[u] * sizeof(RLoad), rv[u]);
+                if constexpr (HAS_R) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (u >= kLead) load_r(u - kLead);
+                }
             } else if constexpr (WHOLE) {
                 load_any<XT, VEC, kLoadNt>(x + block_first + at[u], xv[u]);
                 if constexpr (HAS_R) load_any<RLoad, VEC, kLoadNt>(r + block_first + at[u], rv[u]);
@@ -120,6 +133,10 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
                 load_live<XT, VEC, kLoadNt>(x + block_first + at[u], live_here - at[u], xv[u]);
                 if constexpr (HAS_R) load_live<RLoad, VEC, kLoadNt>(r + block_first + at[u], live_here - at[u], rv[u]);
             }
+        }
+        if constexpr (BUFFERS && HAS_R) {
+#pragma unroll
+            for (int u = UNROLL - kLead; u < UNROLL; ++u) load_r(u);
         }
         const buffer_t codes_b = buffer_over(codes + block_first, T::BLOCK_ELEMS);
         const buffer_t scales_b = buffer_over(scales + block_first / G, T::BLOCK_ELEMS / G * 4);
