@@ -121,9 +121,9 @@ hipError_t launch_reduce_quant_t(int g, int world, int mode, const ReduceQuantAr
 // ---------------------------------------------------------------------------
 // decode of one payload, or of `world` shard payloads into consecutive shards: decode_block
 // ---------------------------------------------------------------------------
-template <typename OT, int G, int OP, int MODE>
+template <typename OT, int G, int OP, int MODE, int STREAM_STORE = kNtBit>
 __global__ __launch_bounds__(kBlock) void decode_kernel(const DecodeArgs a) {
-    decode_block<OT, G, OP, MODE>(a, blockIdx.x, gridDim.x, blockIdx.y);
+    decode_block<OT, G, OP, MODE, STREAM_STORE>(a, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
 template <typename OT, int G, int OP>
@@ -133,6 +133,16 @@ hipError_t launch_decode_op(int mode, const DecodeArgs &a, int world, hipStream_
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
+    // Outputs of 16 MiB and more leave written through as well as non-temporal, but not several fp32 shards.  us of quantize +
+    // decode, nt alone / both, three tensors in rotation (and twelve, beyond the last-level cache): 6.6 M fp32 elements 14.4 / 13.9
+    // (13.6 / 13.7), 13.1 M bf16 13.5 / 13.3 (18.1 / 17.4), 26.2 M fp32 42.9 / 42.2 (42.7 / 42.7), 1 Mi bf16 4.49 / 4.38 (4.85 /
+    // 5.29); of the plan's three launches on fp32, 8.4 M elements in four shards 20.0 / 20.4, 12.6 M 27.7 / 27.9.
+    if constexpr (OP == 0) {
+        if (mode == kStream && (sizeof(OT) == 2 || world == 1) && a.total_numel * static_cast<int64_t>(sizeof(OT)) >= int64_t{16} << 20) {
+            hipLaunchKernelGGL((decode_kernel<OT, G, OP, kStream, kNtBit | kSc1Bit>), grid, dim3(kBlock), 0, stream, a);
+            return hipGetLastError();
+        }
+    }
     switch (mode) {
         case kStream: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kStream>), grid, dim3(kBlock), 0, stream, a); break;
         case kVector: hipLaunchKernelGGL((decode_kernel<OT, G, OP, kVector>), grid, dim3(kBlock), 0, stream, a); break;

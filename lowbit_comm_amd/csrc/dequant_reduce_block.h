@@ -55,7 +55,17 @@ template <typename OT, int W, int MODE> constexpr int reduce_store_policy() {
     if (MODE < kStream) return kCached;
     if (read_write_class<OT, W>() == 0) return kNtBit;
     if (MODE == kStreamThrough) return kSc1Bit;
-    return read_write_class<OT, W>() == 1 ? kNtBit : kCached;
+    return read_write_class<OT, W>() == 1 ? (W <= 2 ? kNtBit | kSc1Bit : kNtBit) : kCached;
+}
+
+// Whether whole blocks issue the load of `prepared` together with the codes' or behind the outputs' stores.  Early it is one
+// round trip to memory less; where reads and writes are about even (class 1) it only pays for outputs within the L2s, of two
+// payloads.  GPU us of the all_gather hook's two launches with error feedback, late / early, three states in rotation (and
+// twelve, beyond the last-level cache): two payloads fp32 4 M 25.3 / 22.7 (25.3 / 23.1), three 1 M 8.8 / 8.4, eight bf16
+// 2 M 11.9 / 11.2 (12.4 / 12.0), 13.1 M 45.2 / 44.9; class 1, two of bf16 1 M 7.7 / 6.8, with the outputs written through as
+// well as non-temporal 6.5 (7.9 / 7.0), 8 M 27.9 / 25.9 (27.3 / 25.0), 13.1 M 34.2 / 34.8; four of fp32 2 M 13.5 / 14.4.
+template <typename OT, int W, int MODE> constexpr bool prepared_early() {
+    return read_write_class<OT, W>() != 1 || (W <= 2 && MODE != kStreamThrough);
 }
 
 // The VEC codes of a lane, from any address under kUnaligned.
@@ -85,7 +95,7 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
     const bool mean = a.divisor != 1.0f;
 
     // One pass over the block's tiles with the codes and scales of all of them issued before the arithmetic (`prepared`
-    // with them in the last block; whole blocks load it tile by tile, after the tile's outputs are on their way).  WHOLE:
+    // with them in the last block; in whole blocks as prepared_early says, else tile by tile after the tile's outputs).  WHOLE:
     // all of the block's outputs exist.  Whole blocks of aligned tensors use one descriptor per stream over the block's span and 32-bit offsets
     // per lane; the block at the end and tensors at element alignment use 64-bit addresses, a lane's vector cut short
     // at the end.  (A payload holds whole groups, so a lane with one live output may read all of its codes.)  Walked
@@ -100,11 +110,13 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
         constexpr int kLoad = policy_of<kLike>();
         constexpr int kStore = reduce_store_policy<OT, W, kLike>();
         constexpr int kCodeAlign = MODE == kUnaligned ? 1 : VEC;
+        constexpr bool kEarly = BUFFERS && prepared_early<OT, W, MODE>();
         uint32_t words[UNROLL][W][VEC / 4];
         float scale[UNROLL][W];
         OT pv[UNROLL][VEC];
         uint32_t at[UNROLL];   // element offset inside the block
         const int64_t live_here = a.numel - block_first;
+        const buffer_t prepared_b = buffer_over(prepared + block_first, T::BLOCK_ELEMS * sizeof(OT));
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) at[u] = static_cast<uint32_t>(tile_in_block<UNROLL>(u, wave)) * T::TILE + lane * VEC;
 #pragma unroll
@@ -130,9 +142,12 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
                 }
             }
         }
-        if (!WHOLE && new_r != nullptr) {   // the end of the tensor: nothing else hides this load
+        if (new_r != nullptr) {
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) load_live<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], live_here - at[u], pv[u]);
+            for (int u = 0; u < UNROLL; ++u) {
+                if constexpr (kEarly) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
+                else if constexpr (!WHOLE) load_live<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], live_here - at[u], pv[u]);
+            }
         }
         const buffer_t out_b = buffer_over(out + block_first, T::BLOCK_ELEMS * sizeof(OT));
 #pragma unroll
@@ -159,8 +174,8 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
             else store_live<OT, VEC, kStore == kNtBit>(out + block_first + at[u], live_here - at[u], o);
             if (new_r != nullptr) {
                 OT d[VEC];
-                if constexpr (BUFFERS) buffer_load<OT, VEC, kLoad>(buffer_over(prepared + block_first, T::BLOCK_ELEMS * sizeof(OT)), at[u] * sizeof(OT), pv[u]);
-                else if constexpr (WHOLE) load_any<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], pv[u]);
+                if constexpr (BUFFERS && !kEarly) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
+                else if constexpr (WHOLE && !BUFFERS) load_any<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], pv[u]);
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) d[i] = narrow<OT>(widen(pv[u][i]) - acc[i]);
                 if constexpr (BUFFERS) buffer_store<OT, VEC, kStore>(buffer_over(new_r + block_first, T::BLOCK_ELEMS * sizeof(OT)), at[u] * sizeof(OT), d);
@@ -270,12 +285,9 @@ template <typename OT> struct decode1_tiling {
     static constexpr int BLOCK_ELEMS = TILE * kWavesPerBlock * UNROLL;
 };
 
-// One workgroup's share: block `block_x` of `grid_x` along shard `chunk_index`.  STREAM_STORE: how whole blocks of aligned
-// outputs leave in the streaming mode.  Non-temporal and written through from the decode's own kernel; us of quantize +
-// decode, nt alone / both / written through alone: 6.6 M fp32 elements 13.85 / 13.45 / 13.4, 13.1 M bf16 13.4 / 13.2 / 13.1,
-// 1 Mi bf16 4.48 / 4.37 / 4.37; the plan on 52.4 M fp32 93.9 / 93.4 / 101.3.  Beside the other stages of a bucket pipeline the hint
-// alone: four 1 MiB bf16 buckets 16.35 us, written through as well 16.8.
-template <typename OT, int G, int OP, int MODE, int STREAM_STORE = kNtBit | kSc1Bit>
+// One workgroup's share: block `block_x` of `grid_x` along shard `chunk_index`.  STREAM_STORE: cache policy of whole blocks of
+// aligned outputs in the streaming mode.
+template <typename OT, int G, int OP, int MODE, int STREAM_STORE = kNtBit>
 __device__ __forceinline__ void decode_block(const DecodeArgs &a, unsigned block_x, unsigned grid_x, unsigned chunk_index) {
     using T = decode1_tiling<OT>;
     constexpr int VEC = T::VEC;

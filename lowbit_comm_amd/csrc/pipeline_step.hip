@@ -37,7 +37,7 @@ __global__ __launch_bounds__(kBlock) void bucket_pipeline_step_kernel(const Quan
     } else if (step_segment_holds(reduce_part, blockIdx.x, block_x, row)) {
         if (block_x < reduce_part.grid_x) reduce::dequant_reduce_quant_block<T, G, W, MODE>(r, block_x, reduce_part.grid_x);
     } else if (step_segment_holds(decode_part, blockIdx.x, block_x, row)) {
-        if (block_x < decode_part.grid_x) reduce::decode_block<T, G, 0, MODE, kNtBit>(d, block_x, decode_part.grid_x, row);
+        if (block_x < decode_part.grid_x) reduce::decode_block<T, G, 0, MODE>(d, block_x, decode_part.grid_x, row);
     }
 }
 
