@@ -290,7 +290,14 @@ hipError_t launch_wire_quant_t(int g, int bit, int mode, const WireQuantArgs &a,
 // ---------------------------------------------------------------------------
 // fused dequant-reduce of up to 8 payloads (+ mean, + error-feedback update)
 // ---------------------------------------------------------------------------
-template <typename T, int G, int WORLD, bool FMA, bool COMPACT, int NT, bool WINDOWS = false>
+// Buffer stores go to 16-byte aligned tensors only; everything else here takes any element.
+bool whole_vectors(const void *a, const void *b = nullptr) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
+}
+
+// KEPT: whole blocks write their outputs through the L2 without the non-temporal hint and load `prepared` with the codes; the
+// launcher says when.
+template <typename T, int G, int WORLD, bool FMA, bool COMPACT, int NT, bool WINDOWS = false, bool KEPT = false>
 __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArgs a) {
     constexpr int PNT = payload_load_hint<COMPACT, NT, WORLD>();
     using W = wire<T>;
@@ -307,6 +314,10 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
     const T *prepared = static_cast<const T *>(a.prepared);  // may alias new_r
     T *new_r = static_cast<T *>(a.new_residual);
 
+    auto store_whole = [&](T *base, int64_t e, const T (&v)[VEC]) __attribute__((always_inline)) {
+        if constexpr (KEPT) buffer_store<T, VEC, kSc1Bit>(buffer_over(base + block_first, BLOCK_ELEMS * sizeof(T)), static_cast<uint32_t>(e - block_first) * sizeof(T), v);
+        else store_elems<T, VEC, NT>(base + e, v);
+    };
     auto accumulate = [](float acc, float code, float step) {
         if constexpr (FMA) return __builtin_fmaf(code, step, acc);
         else return acc + code * step;
@@ -355,7 +366,10 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
                     }
                 }
             }
-            if (!WHOLE && new_r != nullptr) load_live<T, VEC, NT == kNonTemporal>(prepared + e0[u], a.numel - e0[u], pv[u]);
+            if (new_r != nullptr) {
+                if constexpr (WHOLE && KEPT) load_elems<T, VEC, NT>(prepared + e0[u], pv[u]);
+                else if constexpr (!WHOLE) load_live<T, VEC, NT == kNonTemporal>(prepared + e0[u], a.numel - e0[u], pv[u]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -373,16 +387,16 @@ __global__ __launch_bounds__(kBlock) void wire_reduce_kernel(const WireReduceArg
 #pragma unroll
             for (int i = 0; i < VEC; ++i) acc[i] = acc[i] * a.inv_divisor;
             narrow_all<T, VEC>(acc, o);
-            if constexpr (WHOLE) store_elems<T, VEC, NT>(out + e0[u], o);
+            if constexpr (WHOLE) store_whole(out, e0[u], o);
             else store_live<T, VEC, NT == kNonTemporal>(out + e0[u], a.numel - e0[u], o);
             if (new_r != nullptr) {
                 T d[VEC];
                 float left[VEC];
-                if constexpr (WHOLE) load_elems<T, VEC, NT>(prepared + e0[u], pv[u]);
+                if constexpr (WHOLE && !KEPT) load_elems<T, VEC, NT>(prepared + e0[u], pv[u]);
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) left[i] = widen(pv[u][i]) - acc[i];
                 narrow_all<T, VEC>(left, d);
-                if constexpr (WHOLE) store_elems<T, VEC, NT>(new_r + e0[u], d);
+                if constexpr (WHOLE) store_whole(new_r, e0[u], d);
                 else store_live<T, VEC, NT == kNonTemporal>(new_r + e0[u], a.numel - e0[u], d);
             }
         }
@@ -402,6 +416,18 @@ hipError_t launch_wire_reduce_c(int mode, const WireReduceArgs &a, hipStream_t s
         if ((a.numel + G - 1) / G * (G + 2) < (1LL << 31)) {   // a buffer descriptor spans the payload
             if (mode == kStream) hipLaunchKernelGGL((wire_reduce_kernel<T, G, WORLD, FMA, COMPACT, kNonTemporal, true>), grid, dim3(kBlock), 0, stream, a);
             else hipLaunchKernelGGL((wire_reduce_kernel<T, G, WORLD, FMA, COMPACT, kPlain, true>), grid, dim3(kBlock), 0, stream, a);
+            return hipGetLastError();
+        }
+    }
+    // Scales apart, four payloads or more and an output below 48 MiB: KEPT.  GPU us of the hook's two launches with error feedback,
+    // non-temporal / KEPT, three states in rotation (and twelve, beyond the last-level cache): eight payloads fp32 2 M 13.9 / 13.1
+    // (14.2 / 13.2), 6.6 M 38.7 / 37.1 (38.6 / 38.9), 13.1 M 72.2 / 71.8 (71.8 / 74.6), 26.2 M 135.6 / 142.8; bf16 2 M 12.0 / 11.1
+    // (12.6 / 12.2), 13.1 M 48.0 / 45.4 (47.7 / 47.6), 21 M 75.0 / 72.1 (74.2 / 74.8); four fp32 6.6 M 35.0 / 33.3 (34.8 / 34.5), bf16
+    // 300,032 5.4 / 4.9 (5.7 / 5.2), 13.1 M 40.0 / 38.0 (39.9 / 39.1); without feedback eight fp32 6.6 M 33.0 / 31.4.  Two payloads
+    // lose beyond the cache (fp32 6.6 M 29.9 / 34.1), interleaved scales everywhere (eight fp32 6.6 M 35.9 / 38.4).
+    if constexpr (!COMPACT && WORLD >= 4) {
+        if (mode == kStream && whole_vectors(a.out, a.new_residual) && a.numel * static_cast<int64_t>(sizeof(T)) < int64_t{48} << 20) {
+            hipLaunchKernelGGL((wire_reduce_kernel<T, G, WORLD, FMA, COMPACT, kNonTemporal, false, true>), grid, dim3(kBlock), 0, stream, a);
             return hipGetLastError();
         }
     }
@@ -447,7 +473,8 @@ template <typename T, int OP> __device__ __forceinline__ float combine_in(float 
     else return v;
 }
 
-template <typename T, int G, int BIT, int OP, bool COMPACT, int NT>
+// THROUGH: whole blocks write their outputs through the L2 beside the non-temporal hint.
+template <typename T, int G, int BIT, int OP, bool COMPACT, int NT, bool THROUGH = false>
 __global__ __launch_bounds__(kBlock) void wire_decode_kernel(const WireDecodeArgs a) {
     constexpr int PNT = payload_load_hint<COMPACT, NT, 1>();
     using W = wire<T, BIT>;
@@ -501,7 +528,8 @@ __global__ __launch_bounds__(kBlock) void wire_decode_kernel(const WireDecodeArg
                 for (int i = 0; i < VEC; ++i) v[i] = combine_in<T, OP>(widen(o[u][i]), v[i]);
             }
             narrow_all<T, VEC>(v, o[u]);
-            if constexpr (WHOLE) store_elems<T, VEC, NT>(out + e0[u], o[u]);
+            if constexpr (WHOLE && THROUGH) buffer_store<T, VEC, kNtBit | kSc1Bit>(buffer_over(out + block_first, BLOCK_ELEMS * sizeof(T)), static_cast<uint32_t>(e0[u] - block_first) * sizeof(T), o[u]);
+            else if constexpr (WHOLE) store_elems<T, VEC, NT>(out + e0[u], o[u]);
             else store_live<T, VEC, NT == kNonTemporal>(out + e0[u], valid - e0[u], o[u]);
         }
     };
@@ -516,6 +544,15 @@ hipError_t launch_wire_decode_c(int mode, const WireDecodeArgs &a, int world, hi
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
+    // One payload of 16 MiB of outputs and more: THROUGH.  us of quantize + decode, nt alone / both, three tensors in rotation (and
+    // twelve, beyond the last-level cache): fp32 6.6 M 14.5 / 14.0 (14.1 / 14.2), 26.2 M 42.3 / 41.6 (42.9 / 42.5), interleaved 6.6 M 15.4 /
+    // 15.0 (13.8 / 13.8); bf16 13.1 M 19.2 / 18.2 (18.6 / 18.0), 4-bit 26.2 M 27.5 / 26.3 (26.4 / 26.1), 1 Mi 4.50 / 4.40 (4.9 / 5.3).
+    if constexpr (OP == 0) {
+        if (mode == kStream && world == 1 && whole_vectors(a.out) && a.total_numel * static_cast<int64_t>(sizeof(T)) >= int64_t{16} << 20) {
+            hipLaunchKernelGGL((wire_decode_kernel<T, G, BIT, OP, COMPACT, kNonTemporal, true>), grid, dim3(kBlock), 0, stream, a);
+            return hipGetLastError();
+        }
+    }
     if (mode == kStream) hipLaunchKernelGGL((wire_decode_kernel<T, G, BIT, OP, COMPACT, kNonTemporal>), grid, dim3(kBlock), 0, stream, a);
     else hipLaunchKernelGGL((wire_decode_kernel<T, G, BIT, OP, COMPACT, kPlain>), grid, dim3(kBlock), 0, stream, a);
     return hipGetLastError();
