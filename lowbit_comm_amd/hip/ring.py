@@ -396,6 +396,32 @@ class PipelinedRingExecutor(TopologyExecutor):
         if callable(finish):
             finish(context)
 
+    def replay(self, tensor: Any) -> bool:
+        """The schedule on ``tensor`` when the runtime has a record of it for the stream that is current: its launches and
+        exchanges, ordered on that stream and on nothing else, so that there is no work to make, no workspace to lease and no
+        completion to record.  ``False``: nothing was done, :meth:`run` takes the tensor.  A replay that fails is held as a
+        failed run is.
+
+        Bound by the host: a 13.1 M bf16 bucket of eight ranks spent 34 of its 80 us a pass on the bookkeeping of a submission
+        whose buffers belong to the runtime's plan and whose completion is the order of the caller's own stream."""
+        if not self._busy.acquire(blocking=False):
+            raise RuntimeError("concurrent run() on one topology executor is unsupported")
+        try:
+            if self._pending:
+                self._reap()
+            recorded = self._runtime.recorded(tensor)
+            if recorded is None:
+                return False
+            try:
+                self._runtime.replay(tensor, *recorded)
+            except BaseException:
+                context = self._runtime.create_submission_context(tensor)
+                self._fail(_Submission(tensor=tensor, workspace=self._sessions(tensor), context=context))
+                raise
+            return True
+        finally:
+            self._busy.release()
+
     def _exchange(self, submission: _Submission, step: Any) -> tuple[Any, Any]:
         runtime, context, workspace = self._runtime, submission.context, submission.workspace
         payload = runtime.quant_pack(submission.tensor, step.send_chunk, workspace, context=context)
@@ -435,6 +461,16 @@ class RingSubmissionContext:
 
     def wait_stream(self, stream: Any) -> None:
         self.producer_completion.wait_stream(stream)
+
+
+@dataclass(frozen=True)
+class _Replays:
+    """What the look-up of a record needs, at hand: an import inside a function costs the call half a microsecond."""
+
+    own: Callable[..., bool]
+    tensor_type: type
+    dtype: Any
+    current_stream: Callable[[Any], Any]
 
 
 def _view(tensor: Any, chunk: ChunkRange) -> Any:
@@ -514,6 +550,7 @@ class HipPipelinedRingRuntime:
         self._completions = completion_manager
         self.stream = stream
         self.graph_replay = bool(graph_replay)
+        self._replays: _Replays | None = None       # once a run on a caller's stream has been recorded
         self.callers_stream = bool(callers_stream)
         if self.callers_stream and stream is not None:
             raise ValueError("give either a stream or callers_stream=True")
@@ -585,6 +622,13 @@ class HipPipelinedRingRuntime:
         if context.plan is not None and context.program is not None:
             context.plan["program"] = tuple(context.program)
             context.program = None
+            if self._replays is None and self.callers_stream and not self.graph_replay:
+                import torch
+
+                from lowbit_comm_amd.hip import ops
+                from lowbit_comm_amd.hip.library import native_host
+
+                self._replays = _Replays(native_host().own, torch.Tensor, ops.TORCH_DTYPES[self.dtype], torch.cuda.current_stream)
 
     def _run_program(self, program: tuple, stream: Any, raw_stream: int) -> list:
         handles = []
@@ -628,6 +672,29 @@ class HipPipelinedRingRuntime:
         with torch.cuda.stream(context.stream):
             graph.replay()
         return []
+
+    def recorded(self, tensor: Any) -> tuple | None:
+        """``(program, stream, raw stream)`` of a run on ``tensor`` that can be replayed on the caller's stream as it is."""
+        known = self._replays
+        if known is None or not known.own(self, _REPLAYED) or not isinstance(tensor, known.tensor_type):
+            return None
+        if not tensor.is_cuda or not tensor.is_contiguous() or tensor.dtype != known.dtype:
+            return None
+        stream = known.current_stream(tensor.device)
+        raw_stream = stream.cuda_stream
+        key = (tensor.data_ptr(), tensor.numel(), raw_stream)
+        plan = self.plans.get(key)
+        program = None if plan is None else plan.get("program")
+        if program is None:
+            return None
+        self.plans.move_to_end(key)
+        return program, stream, raw_stream
+
+    def replay(self, tensor: Any, program: tuple, stream: Any, raw_stream: int) -> None:
+        tensor.record_stream(stream)
+        for handle in self._run_program(program, stream, raw_stream):
+            if _probe(handle) is None:
+                raise TypeError("P2P dependency must provide nonblocking query() or is_completed()")
 
     def wait_for_producer(self, tensor: Any, *, context: RingSubmissionContext) -> None:
         context.wait_stream(context.stream)
@@ -848,6 +915,12 @@ class HipPipelinedRingRuntime:
         return self._step(tensor, received, chunk, workspace, context, dependency, reduce_op="none", divisor=1.0)
 
 
+# What a replay stands for: a subclass, a patched class or an instance with another method in the place of one of these is asked.
+_REPLAYED = tuple(part for name in ("create_submission_context", "replay_program", "_run_program", "wait_for_producer",
+                                    "record_completion", "_plan_of")
+                  for part in (name, HipPipelinedRingRuntime.__dict__[name]))
+
+
 # --------------------------------------------------------------------------- #
 # every rank of a ring on one device
 # --------------------------------------------------------------------------- #
@@ -962,13 +1035,13 @@ def make_pipelined_ring_transport(*, world_size: int, rank: int, exchange: Calla
 
     from lowbit_comm_amd.exceptions import UnsupportedCollective
 
+    from lowbit_comm_amd.hip import ops
+
     executors: OrderedDict = OrderedDict()
 
     def transport(tensor: Any, *, config: CompressionConfig, op: str = "mean", async_op: bool = False,
                   dtype: str | None = None, extension_status: Any | None = None) -> Any:
         del extension_status                      # the runtime calls the C ABI directly
-        from lowbit_comm_amd.hip import ops
-
         if op != "mean":
             raise UnsupportedCollective(f"pipelined_ring:{op}", reason="the quantized ring computes the mean")
         name = ops.DTYPE_NAMES.get(tensor.dtype)
@@ -985,6 +1058,8 @@ def make_pipelined_ring_transport(*, world_size: int, rank: int, exchange: Calla
                 executors.popitem(last=False)
         else:
             executors.move_to_end(key)
+        if not async_op and completion_manager is None and executor.replay(tensor):
+            return tensor
         work = executor.run(tensor)
         return work if async_op else work.wait()
 
