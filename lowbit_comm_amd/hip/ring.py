@@ -984,6 +984,13 @@ class LoopbackRing:
         return exchange
 
 
+def policy_beside_group_size(config: CompressionConfig) -> tuple:
+    """What of a policy, besides the group size, an executor is made for or refuses: part of the key that a transport keeps its
+    executors under, so that a call is answered by its own policy whatever ran before it.  Empty for the default policy."""
+    policy = (config.bit, config.topk, config.quant_type, config.stochastic, config.compact)
+    return () if policy == (8, 0, "linear", False, False) else policy
+
+
 def make_pipelined_ring_executor(*, config: CompressionConfig, dtype: str, numel: int, world_size: int, rank: int,
                                  exchange: Callable[..., Any], pool: Any | None = None,
                                  completion_manager: Any | None = None, device: str = "cuda:0",
@@ -1026,7 +1033,7 @@ def make_pipelined_ring_transport(*, world_size: int, rank: int, exchange: Calla
     the ring in place and returns it, ordered on the caller's current stream (``async_op``: the executor's work
     object, whose ``wait()`` returns the tensor).  The ring computes the mean, as the reference's executor does
     (the division sits on the hop that completes the sum, ``ccdl_comm/cuda/transports/torch_topology.py:287-289``);
-    any other ``op`` is refused.  One executor is kept per (element count, dtype, device, group size).
+    any other ``op`` is refused.  One executor is kept per (element count, dtype, device, policy).
 
     A call that is waited for at once (``async_op=False``) runs on the caller's stream: on a stream of the ring's own the
     caller's would wait for all of it, with two events and two stream waits a bucket in between (25 MiB bf16 bucket,
@@ -1047,7 +1054,8 @@ def make_pipelined_ring_transport(*, world_size: int, rank: int, exchange: Calla
         name = ops.DTYPE_NAMES.get(tensor.dtype)
         if name is None or (dtype is not None and dtype != name):
             raise ValueError(f"the ring reduces in the bucket's dtype; got dtype={dtype!r} for {tensor.dtype}")
-        key = (tensor.numel(), name, str(tensor.device), config.group_size) + (("async",) if async_op else ())
+        key = ((tensor.numel(), name, str(tensor.device), config.group_size) + policy_beside_group_size(config)
+               + (("async",) if async_op else ()))
         executor = executors.get(key)
         if executor is None:
             executor = executors[key] = make_pipelined_ring_executor(

@@ -332,7 +332,7 @@ def make_topology_transport(*, world_size: int, rank: int, send: Callable[..., A
     from collections import OrderedDict
 
     from lowbit_comm_amd.exceptions import UnsupportedCollective
-    from lowbit_comm_amd.hip.ring import make_pipelined_ring_executor
+    from lowbit_comm_amd.hip.ring import make_pipelined_ring_executor, policy_beside_group_size
 
     executors: OrderedDict = OrderedDict()
 
@@ -350,7 +350,7 @@ def make_topology_transport(*, world_size: int, rank: int, send: Callable[..., A
         if name is None or (dtype is not None and dtype != name):
             raise ValueError(f"the topology schedules reduce in the bucket's dtype; got dtype={dtype!r} for {tensor.dtype}")
         n = tensor.numel()
-        key = (n, name, str(tensor.device), config.group_size)
+        key = (n, name, str(tensor.device), config.group_size) + policy_beside_group_size(config)
         executor = executors.get(key)
         if executor is None:
             aligned = world_size >= 2 and n % world_size == 0 and (n // world_size) % config.group_size == 0
