@@ -262,6 +262,7 @@ class TopologyExecutor:
         self._runtime = runtime
         self._sessions = workspace_session_factory
         self._works = completion_manager
+        self._made_with = (workspace_session_factory, completion_manager)
         self._pending: list[_Submission] = []
         self._busy = threading.Lock()
 
@@ -382,7 +383,7 @@ class PipelinedRingExecutor(TopologyExecutor):
                     submission.after_p2p(handle)
                 return
         begin = getattr(runtime, "begin_schedule", None)
-        if callable(begin):
+        if callable(begin) and type(self)._exchange is PipelinedRingExecutor._exchange and "_exchange" not in self.__dict__:
             begin(context)
         for step in self.schedule.steps:
             received, handle = self._exchange(submission, step)
@@ -399,11 +400,15 @@ class PipelinedRingExecutor(TopologyExecutor):
     def replay(self, tensor: Any) -> bool:
         """The schedule on ``tensor`` when the runtime has a record of it for the stream that is current: its launches and
         exchanges, ordered on that stream and on nothing else, so that there is no work to make, no workspace to lease and no
-        completion to record.  ``False``: nothing was done, :meth:`run` takes the tensor.  A replay that fails is held as a
-        failed run is.
+        completion to record.  ``False``: nothing was done, :meth:`run` takes the tensor - no record, or something else in the place
+        of one of the methods, the session factory or the work factory that a run goes through.  A replay that fails is held as
+        a failed run is.
 
         Bound by the host: a 13.1 M bf16 bucket of eight ranks spent 34 of its 80 us a pass on the bookkeeping of a submission
         whose buffers belong to the runtime's plan and whose completion is the order of the caller's own stream."""
+        known = getattr(self._runtime, "_replays", None)
+        if known is None or not known.own(self, _SUBMITTED) or (self._sessions, self._works) != self._made_with:
+            return False
         if not self._busy.acquire(blocking=False):
             raise RuntimeError("concurrent run() on one topology executor is unsupported")
         try:
@@ -431,6 +436,18 @@ class PipelinedRingExecutor(TopologyExecutor):
         submission.keep(received)
         submission.after_p2p(handle)
         return received, handle
+
+
+def _methods(cls: type, names: tuple[str, ...]) -> tuple:
+    """``(name, attribute, name, attribute, ...)`` as a look-up on the class finds them: the table that ``_host.own`` takes."""
+    return tuple(part for name in names
+                 for part in (name, next(base.__dict__[name] for base in cls.__mro__ if name in base.__dict__)))
+
+
+# What a run goes through and a replay passes by: a subclass, a patched class or an instance with another method in the place of one
+# of these submits.
+_SUBMITTED = _methods(PipelinedRingExecutor, ("run", "_submit", "_enqueue", "_exchange", "_record", "_finish", "_fail", "_hold",
+                                              "_release", "_reap"))
 
 
 # --------------------------------------------------------------------------- #
@@ -916,9 +933,8 @@ class HipPipelinedRingRuntime:
 
 
 # What a replay stands for: a subclass, a patched class or an instance with another method in the place of one of these is asked.
-_REPLAYED = tuple(part for name in ("create_submission_context", "replay_program", "_run_program", "wait_for_producer",
-                                    "record_completion", "_plan_of")
-                  for part in (name, HipPipelinedRingRuntime.__dict__[name]))
+_REPLAYED = _methods(HipPipelinedRingRuntime, ("create_submission_context", "replay_program", "_run_program", "wait_for_producer",
+                                               "record_completion", "_plan_of"))
 
 
 # --------------------------------------------------------------------------- #

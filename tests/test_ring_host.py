@@ -408,3 +408,63 @@ def test_callers_stream_plans_are_kept_per_stream():
     assert runtime._plan_of(bucket, 0x10) is first and runtime._plan_of(bucket, 0x20) is second and len(runtime.plans) == 3
     runtime = HipPipelinedRingRuntime(**common)               # a stream of the ring's own: one plan for a bucket
     assert runtime._plan_of(bucket, 0x10) is runtime._plan_of(bucket, 0x20)
+
+
+def test_a_replay_stands_back_for_every_part_of_a_run_that_is_not_the_executors_own():
+    from types import SimpleNamespace
+
+    from lowbit_comm_amd.hip.library import native_host
+
+    class Recorded(Runtime):
+        def __init__(self):
+            super().__init__()
+            self._replays = SimpleNamespace(own=native_host().own)
+            self.replayed = 0
+
+        def recorded(self, tensor):
+            return ()
+
+        def replay(self, tensor):
+            self.replayed += 1
+
+    def with_runtime(cls=PipelinedRingExecutor):
+        schedule = compile_pipelined_ring_schedule(chunk_plan=compile_chunk_plan(original_numel=15, world_size=3), rank=1)
+        return cls(schedule=schedule, runtime=Recorded(), workspace_session_factory=lambda t: Session(), completion_manager=Works())
+
+    executor = with_runtime()
+    assert executor.replay(object()) and executor._runtime.replayed == 1
+    parts = ("run", "_submit", "_enqueue", "_exchange", "_record", "_finish", "_fail", "_hold", "_release", "_reap")
+    for name in parts + ("_sessions", "_works"):
+        own = getattr(executor, name)
+        setattr(executor, name, (lambda *a, **k: None) if callable(own) else Works())
+        assert not executor.replay(object()) and executor._runtime.replayed == 1, name
+        if name in parts:
+            delattr(executor, name)
+        else:
+            setattr(executor, name, own)
+        assert executor.replay(object()), name
+        executor._runtime.replayed = 1
+    for name in parts:
+        watching = with_runtime(type("Watching", (PipelinedRingExecutor,), {name: lambda *a, **k: None}))
+        assert not watching.replay(object()) and watching._runtime.replayed == 0, name
+    executor._runtime = Runtime()                                     # a runtime that knows nothing of records
+    assert not executor.replay(object())
+
+
+def test_an_executor_with_an_exchange_of_its_own_sees_every_updated_chunk():
+    class Beginning(Runtime):
+        begun = 0
+
+        def begin_schedule(self, context):
+            self.begun += 1
+
+    class Watching(PipelinedRingExecutor):
+        def _exchange(self, submission, step):
+            return super()._exchange(submission, step)
+
+    schedule = compile_pipelined_ring_schedule(chunk_plan=compile_chunk_plan(original_numel=15, world_size=3), rank=1)
+    common = dict(schedule=schedule, workspace_session_factory=lambda t: Session(), completion_manager=Works())
+    plain, watching = PipelinedRingExecutor(runtime=Beginning(), **common), Watching(runtime=Beginning(), **common)
+    plain.run(object())
+    watching.run(object())
+    assert plain._runtime.begun == 1 and watching._runtime.begun == 0

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from lowbit_comm_amd import CompressionConfig
+from lowbit_comm_amd.hip import ring
 
 pytestmark = pytest.mark.gpu
 CONFIG = CompressionConfig()
@@ -49,17 +50,17 @@ def _same(a, b):
     return torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
-def test_replays_give_the_first_calls_bits_and_wait_for_every_hop(hip_device):
+def test_replays_give_the_first_calls_bits_and_wait_for_every_hop(hip_device, monkeypatch):
     transport, source, state = _ring(hip_device)
     bucket = source.clone()
     first = transport(bucket, config=CONFIG).clone()
     (executor,) = transport.executors.values()
-    executor.run = lambda tensor: pytest.fail("a replay makes no submission")
-    for _ in range(3):
-        bucket.copy_(source)
-        Done.waited = 0
-        assert transport(bucket, config=CONFIG) is bucket and _same(bucket, first) and Done.waited == 6
-    del executor.run
+    with monkeypatch.context() as patch:
+        patch.setattr(ring, "_Submission", lambda **kw: pytest.fail("a replay makes no submission"))
+        for _ in range(3):
+            bucket.copy_(source)
+            Done.waited = 0
+            assert transport(bucket, config=CONFIG) is bucket and _same(bucket, first) and Done.waited == 6
     other = source.clone()                                    # another bucket has no record yet: the whole protocol
     assert _same(transport(other, config=CONFIG), first) and len(executor._runtime.plans) == 2
 
@@ -118,6 +119,12 @@ def test_replaced_methods_managers_and_other_tensors_take_the_whole_protocol(hip
     bucket.copy_(source)
     assert _same(transport(bucket, config=CONFIG), first) and seen == [1]
     del runtime.record_completion
+    runs = []
+    executor.run = lambda tensor: (runs.append(tensor), ring.PipelinedRingExecutor.run(executor, tensor))[1]
+    for calls in (1, 2):                                      # an executor's own `run` sees every bucket, not the first alone
+        bucket.copy_(source)
+        assert _same(transport(bucket, config=CONFIG), first) and len(runs) == calls
+    del executor.run
     wide = torch.zeros(source.numel() * 2, dtype=torch.bfloat16, device=hip_device)
     with pytest.raises(RuntimeError, match="contiguous"):
         transport(wide[::2], config=CONFIG)
