@@ -212,6 +212,7 @@ class _Submission:
     context: Any
     resources: list = field(default_factory=list)
     dependencies: list = field(default_factory=list)
+    exchanges: list = field(default_factory=list)      # the handle of every exchange that was started
     completion: Any = None
     record_attempted: bool = False
     failed: bool = False
@@ -230,14 +231,40 @@ class _Submission:
 
     def after_p2p(self, value: Any) -> None:
         self.keep(value)
+        self.exchanges.append(value)
         if _probe(value) is None:
             raise TypeError("P2P dependency must provide nonblocking query() or is_completed()")
         self.dependencies.append(value)
+
+    def started(self, handles: list) -> None:
+        """Exchanges of a replay that failed: waited for as far as they can be."""
+        self.keep(*handles)
+        self.exchanges += handles
+        self.dependencies += [h for h in handles if _probe(h) is not None]
+
+    def drained(self) -> bool:
+        """Whether the exchanges of a failed submission are over, where they can say so: one whose wait was never enqueued
+        may still use the buffers when the stream has run dry."""
+        return all(bool(probe()) for probe in map(_probe, self.exchanges) if probe is not None)
+
+    def has_unordered_exchanges(self) -> bool:
+        ordered = [] if self.completion is None else [d for d in self.dependencies if callable(getattr(d, "wait_stream", None))]
+        return not all(any(handle is d for d in ordered) for handle in self.exchanges)
 
     def keep_workspace_buffers(self) -> None:
         leases = getattr(self.workspace, "leases", ())
         if isinstance(leases, tuple):
             self.keep(*leases)
+
+
+class _NothingLeased:
+    """The workspace session of a replay, whose buffers are its plan's."""
+
+    def release(self, *, completion: Any) -> None:
+        del completion
+
+    def abort(self) -> None:
+        pass
 
 
 class TopologyExecutor:
@@ -332,6 +359,9 @@ class TopologyExecutor:
                 self._record(submission)      # so that there is something to wait for before the buffers go back
             except BaseException:
                 pass
+        abandon = getattr(self._runtime, "abandon_plan", None)
+        if callable(abandon) and submission.has_unordered_exchanges():
+            abandon(submission.context)       # the next run on this tensor must not write into buffers that are on the link
 
     def _hold(self, submission: _Submission) -> None:
         if submission not in self._pending:
@@ -350,7 +380,7 @@ class TopologyExecutor:
             readiness = submission.completion if submission.completion is not None else submission.context
             probe = _probe(readiness)
             try:
-                if probe is None or not probe():
+                if probe is None or not probe() or (submission.failed and not submission.drained()):
                     continue
             except BaseException:
                 continue
@@ -377,7 +407,11 @@ class PipelinedRingExecutor(TopologyExecutor):
         runtime, tensor, context, workspace = self._runtime, submission.tensor, submission.context, submission.workspace
         replay = getattr(runtime, "replay_program", None)
         if callable(replay):
-            handles = replay(context)
+            try:
+                handles = replay(context)
+            except BaseException:
+                submission.started(list(getattr(context, "exchanges", ())))
+                raise
             if handles is not None:          # this tensor's launches and exchanges were recorded by an earlier run
                 for handle in handles:
                     submission.after_p2p(handle)
@@ -402,7 +436,7 @@ class PipelinedRingExecutor(TopologyExecutor):
         exchanges, ordered on that stream and on nothing else, so that there is no work to make, no workspace to lease and no
         completion to record.  ``False``: nothing was done, :meth:`run` takes the tensor - no record, or something else in the place
         of one of the methods, the session factory or the work factory that a run goes through.  A replay that fails is held as
-        a failed run is.
+        a failed run is, with the exchanges that it had started.
 
         Bound by the host: a 13.1 M bf16 bucket of eight ranks spent 34 of its 80 us a pass on the bookkeeping of a submission
         whose buffers belong to the runtime's plan and whose completion is the order of the caller's own stream."""
@@ -417,11 +451,16 @@ class PipelinedRingExecutor(TopologyExecutor):
             recorded = self._runtime.recorded(tensor)
             if recorded is None:
                 return False
+            plan, stream, raw_stream = recorded
+            handles: list = []
             try:
-                self._runtime.replay(tensor, *recorded)
+                self._runtime.replay(tensor, plan["program"], stream, raw_stream, handles)
             except BaseException:
-                context = self._runtime.create_submission_context(tensor)
-                self._fail(_Submission(tensor=tensor, workspace=self._sessions(tensor), context=context))
+                context = RingSubmissionContext(tensor=tensor, stream=stream, producer_completion=known.ordered(stream), plan=plan,
+                                                raw_stream=raw_stream)
+                submission = _Submission(tensor=tensor, workspace=_NothingLeased(), context=context)
+                submission.started(handles)
+                self._fail(submission)
                 raise
             return True
         finally:
@@ -469,6 +508,7 @@ class RingSubmissionContext:
     raw_stream: int = 0
     program: list | None = None        # the launches and exchanges of this run in order, while a plan is being made
     whole_schedule: bool = False       # the steps are those of a ring from its first to its last, in order
+    exchanges: list = field(default_factory=list)      # handles of a replay's exchanges, each from the moment it is started
 
     def query(self) -> bool:
         return bool(self.producer_completion.query())
@@ -488,6 +528,7 @@ class _Replays:
     tensor_type: type
     dtype: Any
     current_stream: Callable[[Any], Any]
+    ordered: Callable[[Any], Any]              # completion of what has been enqueued on a stream
 
 
 def _view(tensor: Any, chunk: ChunkRange) -> Any:
@@ -644,11 +685,21 @@ class HipPipelinedRingRuntime:
 
                 from lowbit_comm_amd.hip import ops
                 from lowbit_comm_amd.hip.library import native_host
+                from lowbit_comm_amd.hip.workspace import StreamOrderedCompletion
 
-                self._replays = _Replays(native_host().own, torch.Tensor, ops.TORCH_DTYPES[self.dtype], torch.cuda.current_stream)
+                self._replays = _Replays(native_host().own, torch.Tensor, ops.TORCH_DTYPES[self.dtype], torch.cuda.current_stream,
+                                         StreamOrderedCompletion)
 
-    def _run_program(self, program: tuple, stream: Any, raw_stream: int) -> list:
-        handles = []
+    def abandon_plan(self, context: RingSubmissionContext) -> None:
+        """A run on this plan failed with an exchange that nothing is ordered after: its buffers stay with the submission that
+        holds them, and the next run on the tensor makes its own."""
+        for key, plan in self.plans.items():
+            if plan is context.plan:
+                del self.plans[key]
+                return
+
+    def _run_program(self, program: tuple, stream: Any, raw_stream: int, handles: list) -> None:
+        """``handles`` receives the handle of each exchange as soon as it is started, so that a failure leaves them all."""
         for op in program:
             kind = op[0]
             if kind == "launch":
@@ -656,8 +707,8 @@ class HipPipelinedRingRuntime:
                     raise RuntimeError("a ring launch has no kernel for this configuration")
             elif kind == "exchange":
                 handle = self._exchange(op[1], op[2], send_peer=op[3], recv_peer=op[4], stream=stream)
-                handle.wait_stream(stream)
                 handles.append(handle)
+                handle.wait_stream(stream)
             else:                                    # "divide": the unfused sequence's in-place mean
                 import torch
 
@@ -665,7 +716,6 @@ class HipPipelinedRingRuntime:
 
                 with torch.cuda.stream(stream):
                     ops.true_divide_(op[1], op[2])
-        return handles
 
     def replay_program(self, context: RingSubmissionContext) -> list | None:
         """Enqueue the recorded launches and exchanges of this tensor's plan; ``None`` when there is no record yet."""
@@ -674,7 +724,8 @@ class HipPipelinedRingRuntime:
         if program is None:
             return None
         if not self.graph_replay:
-            return self._run_program(program, context.stream, context.raw_stream)
+            self._run_program(program, context.stream, context.raw_stream, context.exchanges)
+            return context.exchanges
         import torch
 
         graph = plan.get("graph")
@@ -683,7 +734,7 @@ class HipPipelinedRingRuntime:
             side = torch.cuda.Stream()               # default priority; capture needs a stream of its own
             side.wait_stream(context.stream)
             with torch.cuda.graph(graph, stream=side):
-                self._run_program(program, side, side.cuda_stream)
+                self._run_program(program, side, side.cuda_stream, context.exchanges)
             context.stream.wait_stream(side)
             plan["graph"] = graph
         with torch.cuda.stream(context.stream):
@@ -691,7 +742,7 @@ class HipPipelinedRingRuntime:
         return []
 
     def recorded(self, tensor: Any) -> tuple | None:
-        """``(program, stream, raw stream)`` of a run on ``tensor`` that can be replayed on the caller's stream as it is."""
+        """``(plan, stream, raw stream)`` of a run on ``tensor`` that can be replayed on the caller's stream as it is."""
         known = self._replays
         if known is None or not known.own(self, _REPLAYED) or not isinstance(tensor, known.tensor_type):
             return None
@@ -701,15 +752,15 @@ class HipPipelinedRingRuntime:
         raw_stream = stream.cuda_stream
         key = (tensor.data_ptr(), tensor.numel(), raw_stream)
         plan = self.plans.get(key)
-        program = None if plan is None else plan.get("program")
-        if program is None:
+        if plan is None or "program" not in plan:
             return None
         self.plans.move_to_end(key)
-        return program, stream, raw_stream
+        return plan, stream, raw_stream
 
-    def replay(self, tensor: Any, program: tuple, stream: Any, raw_stream: int) -> None:
+    def replay(self, tensor: Any, program: tuple, stream: Any, raw_stream: int, handles: list) -> None:
         tensor.record_stream(stream)
-        for handle in self._run_program(program, stream, raw_stream):
+        self._run_program(program, stream, raw_stream, handles)
+        for handle in handles:
             if _probe(handle) is None:
                 raise TypeError("P2P dependency must provide nonblocking query() or is_completed()")
 

@@ -422,9 +422,9 @@ def test_a_replay_stands_back_for_every_part_of_a_run_that_is_not_the_executors_
             self.replayed = 0
 
         def recorded(self, tensor):
-            return ()
+            return {"program": ()}, None, 0
 
-        def replay(self, tensor):
+        def replay(self, tensor, program, stream, raw_stream, handles):
             self.replayed += 1
 
     def with_runtime(cls=PipelinedRingExecutor):
@@ -468,3 +468,66 @@ def test_an_executor_with_an_exchange_of_its_own_sees_every_updated_chunk():
     plain.run(object())
     watching.run(object())
     assert plain._runtime.begun == 1 and watching._runtime.begun == 0
+
+
+class _Posted(Endpoint):
+    """An exchange that is on the link until it is told otherwise."""
+
+    def __init__(self, ordered=True):
+        super().__init__(ready=False)
+        self.ordered = ordered
+
+    def wait_stream(self, stream):
+        if not self.ordered:
+            raise OSError("no wait")
+        super().wait_stream(stream)
+
+
+@pytest.mark.parametrize("through", ["replay", "run"])
+@pytest.mark.parametrize("failure", ["exchange", "wait"])
+def test_a_failed_replay_holds_the_exchanges_it_started_and_gives_up_buffers_that_are_on_the_link(through, failure):
+    from types import SimpleNamespace
+
+    from lowbit_comm_amd.config import CompressionConfig
+    from lowbit_comm_amd.hip.library import native_host
+    from lowbit_comm_amd.hip.ring import HipPipelinedRingRuntime, RingSubmissionContext
+
+    posted = []
+
+    def exchange(payload, received, *, send_peer, recv_peer, stream):
+        if failure == "exchange" and len(posted) == 2:
+            raise OSError("link down")
+        posted.append(_Posted(ordered=failure == "exchange" or len(posted) < 2))
+        return posted[-1]
+
+    runtime = HipPipelinedRingRuntime(config=CompressionConfig(), dtype="fp32", world_size=3, rank=1, exchange=exchange)
+    hop = (("launch", lambda raw: True), ("exchange", "payload", "received", 2, 0))
+    plan = runtime.plans["the tensor's"] = {"program": hop * 4}
+    context = RingSubmissionContext(tensor=None, stream="stream", producer_completion=Endpoint(), plan=plan)
+    ended = Endpoint()
+
+    def record_completion(*, context, dependencies):
+        for dependency in dependencies:
+            dependency.wait_stream(context.stream)
+        return ended
+
+    runtime._replays = SimpleNamespace(own=native_host().own, ordered=lambda stream: Endpoint())
+    runtime.recorded = lambda tensor: (plan, "stream", 0)
+    runtime.create_submission_context = lambda tensor: context
+    runtime.wait_for_producer = lambda tensor, *, context: None
+    runtime.record_completion = record_completion
+    _, _, session, executor = make(runtime=runtime)
+    tensor = SimpleNamespace(record_stream=lambda stream: None)
+    with pytest.raises(OSError, match="link down" if failure == "exchange" else "no wait"):
+        getattr(executor, through)(tensor)
+    (submission,) = executor._pending
+    assert len(posted) == (2 if failure == "exchange" else 3)
+    assert all(any(handle is kept for kept in submission.resources) for handle in posted)
+    # every exchange was ordered on the stream: the plan's next launches are behind it; one that was not keeps its buffers
+    assert list(runtime.plans.values()) == ([plan] if failure == "exchange" else []) and submission.context.plan is plan
+    for handle in posted:
+        executor.reap_pending()
+        assert executor.pending_submission_count == 1
+        handle.ready = True
+    executor.reap_pending()
+    assert executor.pending_submission_count == 0 and session.aborts == (through == "run")
