@@ -35,8 +35,9 @@ template <int W> __device__ __forceinline__ constexpr int code_load_mode(int mod
 // hint pays on the direction that carries most of the bytes and costs when both directions carry it:
 //   reads/writes < 0.8  (W = 1, 2 for fp32)  plain code loads, non-temporal stores       (26 M, W = 1: 19.0 us; with
 //                                             non-temporal loads as well 24.8 us)
-//   up to 1.6           (W = 4)               non-temporal loads; stores non-temporal, or written through for
-//                                             outputs beyond the L2s
+//   up to 1.6           (W = 4; for 16-bit    non-temporal loads; stores non-temporal (two 16-bit payloads: written
+//                        outputs W = 2)       through beside the hint), or written through without it for outputs
+//                                             beyond the L2s
 //   above               (W = 8)               non-temporal loads; plain stores while the output fits the L2s
 //                                             (3.3 M: 7.9 us against 8.1 written through, 8.4 non-temporal - the
 //                                             write-back then overlaps the next kernel's ramp), written through
@@ -109,6 +110,10 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
         constexpr int kCodes = code_policy<OT, W, kLike>();
         constexpr int kLoad = policy_of<kLike>();
         constexpr int kStore = reduce_store_policy<OT, W, kLike>();
+        // What the stores without a descriptor take of it.  Two bf16 payloads at an odd output, plain / non-temporal, beyond the
+        // last-level cache: with feedback 1 M elements 4.73 / 4.69 us, 8 M 14.9 / 14.5, 13.1 M 22.4 / 22.4, without it 8 M 8.2 / 7.8,
+        // 26.2 M 21.0 / 19.9.  (Three tensors in rotation, with feedback: 3.2 M 7.1 / 6.6, 13.1 M 19.3 / 22.0.)
+        constexpr bool kStoreNt = (kStore & kNtBit) != 0;
         constexpr int kCodeAlign = MODE == kUnaligned ? 1 : VEC;
         constexpr bool kEarly = BUFFERS && prepared_early<OT, W, MODE>();
         uint32_t words[UNROLL][W][VEC / 4];
@@ -170,8 +175,8 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
             OT o[VEC];
             narrow_all<OT, VEC>(acc, o);
             if constexpr (BUFFERS) buffer_store<OT, VEC, kStore>(out_b, at[u] * sizeof(OT), o);
-            else if constexpr (WHOLE) store_any<OT, VEC, kStore == kNtBit>(out + block_first + at[u], o);
-            else store_live<OT, VEC, kStore == kNtBit>(out + block_first + at[u], live_here - at[u], o);
+            else if constexpr (WHOLE) store_any<OT, VEC, kStoreNt>(out + block_first + at[u], o);
+            else store_live<OT, VEC, kStoreNt>(out + block_first + at[u], live_here - at[u], o);
             if (new_r != nullptr) {
                 OT d[VEC];
                 if constexpr (BUFFERS && !kEarly) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
@@ -179,8 +184,8 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) d[i] = narrow<OT>(widen(pv[u][i]) - acc[i]);
                 if constexpr (BUFFERS) buffer_store<OT, VEC, kStore>(buffer_over(new_r + block_first, T::BLOCK_ELEMS * sizeof(OT)), at[u] * sizeof(OT), d);
-                else if constexpr (WHOLE) store_any<OT, VEC, kStore == kNtBit>(new_r + block_first + at[u], d);
-                else store_live<OT, VEC, kStore == kNtBit>(new_r + block_first + at[u], live_here - at[u], d);
+                else if constexpr (WHOLE) store_any<OT, VEC, kStoreNt>(new_r + block_first + at[u], d);
+                else store_live<OT, VEC, kStoreNt>(new_r + block_first + at[u], live_here - at[u], d);
             }
         }
     };
