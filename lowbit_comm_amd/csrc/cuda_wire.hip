@@ -419,14 +419,18 @@ hipError_t launch_wire_reduce_c(int mode, const WireReduceArgs &a, hipStream_t s
             return hipGetLastError();
         }
     }
-    // Scales apart, four payloads or more and an output below 48 MiB: KEPT.  GPU us of the hook's two launches with error feedback,
-    // non-temporal / KEPT, three states in rotation (and twelve, beyond the last-level cache): eight payloads fp32 2 M 13.9 / 13.1
-    // (14.2 / 13.2), 6.6 M 38.7 / 37.1 (38.6 / 38.9), 13.1 M 72.2 / 71.8 (71.8 / 74.6), 26.2 M 135.6 / 142.8; bf16 2 M 12.0 / 11.1
-    // (12.6 / 12.2), 13.1 M 48.0 / 45.4 (47.7 / 47.6), 21 M 75.0 / 72.1 (74.2 / 74.8); four fp32 6.6 M 35.0 / 33.3 (34.8 / 34.5), bf16
-    // 300,032 5.4 / 4.9 (5.7 / 5.2), 13.1 M 40.0 / 38.0 (39.9 / 39.1); without feedback eight fp32 6.6 M 33.0 / 31.4.  Two payloads
-    // lose beyond the cache (fp32 6.6 M 29.9 / 34.1), interleaved scales everywhere (eight fp32 6.6 M 35.9 / 38.4).
+    // KEPT: scales apart, four payloads or more, with feedback, and an output of a size that gains in rotation and does not lose
+    // beyond the last-level cache, where a training run's buckets are.  GPU us of the hook's two launches, non-temporal / KEPT, three
+    // states in rotation (and beyond the cache): eight payloads fp32 1 MiB 4.87 / 4.55 (5.99 / 5.66), 12 MiB 21.9 / 20.4 (21.7 / 21.3),
+    // 25 MiB 38.9 / 37.2 (38.4 / 38.1), 40 MiB 58.6 / 56.9 (57.8 / 58.5); bf16 0.8 MiB 6.3 / 6.0 (8.6 / 8.4), 15 MiB 31.1 / 29.7 (30.9 /
+    // 30.9), 24 MiB 49.3 / 48.0 (48.0 / 48.6); four bf16 0.1 MiB 5.2 / 5.2 (6.0 / 6.2), 30 MiB 47.6 / 44.9 (47.2 / 46.5).  Four fp32 of 2
+    // to 8 MiB lose either way, 7 MiB 11.1 / 12.2 (11.8 / 12.9).  Without feedback it loses beyond the cache (eight fp32 32 MiB 26.1 / 25.9
+    // (25.8 / 26.9)), with two payloads as well (fp32 6.6 M elements 29.9 / 34.1), with interleaved scales everywhere.
     if constexpr (!COMPACT && WORLD >= 4) {
-        if (mode == kStream && whole_vectors(a.out, a.new_residual) && a.numel * static_cast<int64_t>(sizeof(T)) < int64_t{48} << 20) {
+        const int64_t kib = (a.numel * static_cast<int64_t>(sizeof(T)) + 1023) >> 10;
+        const bool gains = sizeof(T) == 2 ? kib >= 256 && kib < (WORLD <= 6 ? 32 << 10 : 16 << 10)
+                                          : kib <= 1536 || (kib >= 9 << 10 && kib < 32 << 10);
+        if (mode == kStream && a.new_residual != nullptr && gains && whole_vectors(a.out, a.new_residual)) {
             hipLaunchKernelGGL((wire_reduce_kernel<T, G, WORLD, FMA, COMPACT, kNonTemporal, false, true>), grid, dim3(kBlock), 0, stream, a);
             return hipGetLastError();
         }

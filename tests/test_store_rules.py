@@ -38,14 +38,16 @@ def test_decode_around_the_line(hip_device, dtype, wire):
 @pytest.mark.parametrize("world", [3, 4, 8])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_cuda_format_reduce_with_feedback(hip_device, dtype, world, offset):
-    """Aligned and odd outputs, payload counts on both sides of the rule, sizes on both sides of a block and of 48 MiB, against
-    torch in the kernel's own arithmetic: a sum in fp32 of code * (scale / 127), times 1 / world, rounded once."""
+    """Aligned and odd outputs, payload counts on both sides of the rule, sizes on both sides of a block and of the rule's lines,
+    against torch in the kernel's own arithmetic: a sum in fp32 of code * (scale / 127), times 1 / world, rounded once."""
     from lowbit_comm_amd.hip import cuda_wire
 
     config, status = CompressionConfig(), load_hip_extension(wire_format="native")
     name = {torch.float32: "fp32", torch.bfloat16: "bf16"}[dtype]
     item = torch.empty((), dtype=dtype).element_size()
-    sizes = [64 * 5, 4096, 4096 * 9 + 64 * 3] + ([48 * MiB // item - 64, 48 * MiB // item] if world == 4 and offset == 0 else [])
+    lines = [line // item + step for line in ((3 * MiB // 2, 9 * MiB, 32 * MiB) if item == 4 else (MiB // 4, 32 * MiB))
+             for step in (-576, 0, 64)]
+    sizes = [64 * 5, 4096, 4096 * 9 + 64 * 3] + (lines if world == 4 and offset == 0 else [])
     for numel in sizes:
         payloads = [_payload(numel, dtype, config, status, 10 * r + 1, hip_device) for r in range(world)]
         prepared = (torch.randn(numel, device=hip_device) * 1e-3).to(dtype)
