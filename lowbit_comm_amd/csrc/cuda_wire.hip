@@ -548,11 +548,14 @@ hipError_t launch_wire_decode_c(int mode, const WireDecodeArgs &a, int world, hi
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    // One payload of 16 MiB of outputs and more: THROUGH.  us of quantize + decode, nt alone / both, three tensors in rotation (and
-    // twelve, beyond the last-level cache): fp32 6.6 M 14.5 / 14.0 (14.1 / 14.2), 26.2 M 42.3 / 41.6 (42.9 / 42.5), interleaved 6.6 M 15.4 /
-    // 15.0 (13.8 / 13.8); bf16 13.1 M 19.2 / 18.2 (18.6 / 18.0), 4-bit 26.2 M 27.5 / 26.3 (26.4 / 26.1), 1 Mi 4.50 / 4.40 (4.9 / 5.3).
+    // One payload: THROUGH from 16 MiB of outputs on, 8-bit fp32 ones from 32 MiB on.  us of quantize + decode, nt alone / both, three
+    // tensors in rotation (and beyond the last-level cache): bf16 16 MiB 13.7 / 13.3 (13.6 / 13.4), 25 MiB 18.5 / 17.9 (18.7 / 18.2),
+    // interleaved 25 MiB 16.4 / 16.2 (16.8 / 16.6), 4-bit 25 MiB 16.9 / 16.1 (16.0 / 15.8), 1 Mi elements 4.50 / 4.40 (4.9 / 5.3); fp32 20 MiB 12.2 /
+    // 12.1 (11.9 / 12.0), interleaved 12.3 / 12.0 (11.7 / 11.8), 4-bit 11.8 / 11.7 (11.4 / 11.4), 25 MiB 14.5 / 14.4 (14.1 / 14.2), 32 MiB 16.5 / 16.3
+    // (16.4 / 16.4), 100 MiB 41.5 / 41.4 (41.3 / 41.2), 4-bit 39.4 / 38.5 (38.9 / 38.1).
     if constexpr (OP == 0) {
-        if (mode == kStream && world == 1 && whole_vectors(a.out) && a.total_numel * static_cast<int64_t>(sizeof(T)) >= int64_t{16} << 20) {
+        constexpr int64_t kThrough = int64_t{sizeof(T) == 2 || BIT == 4 ? 16 : 32} << 20;
+        if (mode == kStream && world == 1 && whole_vectors(a.out) && a.total_numel * static_cast<int64_t>(sizeof(T)) >= kThrough) {
             hipLaunchKernelGGL((wire_decode_kernel<T, G, BIT, OP, COMPACT, kNonTemporal, true>), grid, dim3(kBlock), 0, stream, a);
             return hipGetLastError();
         }

@@ -133,12 +133,15 @@ hipError_t launch_decode_op(int mode, const DecodeArgs &a, int world, hipStream_
     if (blocks == 0 || world == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL || world > 65535) return hipErrorInvalidValue;
     dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(world));
-    // Outputs of 16 MiB and more leave written through as well as non-temporal, but not several fp32 shards.  us of quantize +
-    // decode, nt alone / both, three tensors in rotation (and twelve, beyond the last-level cache): 6.6 M fp32 elements 14.4 / 13.9
-    // (13.6 / 13.7), 13.1 M bf16 13.5 / 13.3 (18.1 / 17.4), 26.2 M fp32 42.9 / 42.2 (42.7 / 42.7), 1 Mi bf16 4.49 / 4.38 (4.85 /
-    // 5.29); of the plan's three launches on fp32, 8.4 M elements in four shards 20.0 / 20.4, 12.6 M 27.7 / 27.9.
+    // 16-bit outputs of 20 MiB and more, and fp32 ones of one payload from 32 MiB on, leave written through as well as non-temporal.  us
+    // of quantize + decode, nt alone / both, three tensors in rotation (and beyond the last-level cache): one bf16 payload 16 MiB
+    // 12.0 / 12.4 (12.9 / 12.7), 18 MiB 13.5 / 13.7 (14.1 / 13.8), 20 MiB 14.8 / 14.6 (15.1 / 14.8), 32 MiB 21.6 / 20.9 (21.8 / 21.0), 100 MiB 51.0 /
+    // 50.8 (51.4 / 51.3); eight bf16 shards 16 MiB 12.0 / 12.2 (12.7 / 12.8), 20 MiB 14.6 / 14.5 (15.0 / 14.9), 32 MiB 21.3 / 20.9 (21.5 / 20.9);
+    // fp32 22 MiB 12.9 / 12.7 (12.6 / 12.8), 25 MiB 14.1 / 14.0 (13.8 / 13.8), 32 MiB 16.2 / 16.1 (16.1 / 16.0), 100 MiB 41.6 / 41.3 (41.5 / 41.1);
+    // the plan's three launches on fp32, 8.4 M elements in four shards 20.0 / 20.4, 12.6 M 27.7 / 27.9.
     if constexpr (OP == 0) {
-        if (mode == kStream && (sizeof(OT) == 2 || world == 1) && a.total_numel * static_cast<int64_t>(sizeof(OT)) >= int64_t{16} << 20) {
+        constexpr int64_t kThrough = int64_t{sizeof(OT) == 2 ? 20 : 32} << 20;
+        if (mode == kStream && (sizeof(OT) == 2 || world == 1) && a.total_numel * static_cast<int64_t>(sizeof(OT)) >= kThrough) {
             hipLaunchKernelGGL((decode_kernel<OT, G, OP, kStream, kNtBit | kSc1Bit>), grid, dim3(kBlock), 0, stream, a);
             return hipGetLastError();
         }

@@ -22,7 +22,8 @@ def test_decode_around_the_line(hip_device, dtype, wire):
     """A large decode against the decodes of its pieces, which stay below the line (pieces of whole blocks keep their scales)."""
     status, config = load_hip_extension(wire_format=wire), CompressionConfig()
     name, item = {torch.float32: ("fp32", 4), torch.bfloat16: ("bf16", 2)}[dtype]
-    for numel in (16 * MiB // item - 64, 16 * MiB // item, 16 * MiB // item + 64 * 33):
+    line = (32 if item == 4 else 20 if wire == "portable" else 16) * MiB // item
+    for numel in (line - 64, line, line + 64 * 33):
         generator = torch.Generator(device=hip_device).manual_seed(numel)
         values = (torch.randn(numel, generator=generator, device=hip_device) * 1e-3).to(dtype)
         got = dequantize_tensor(quantize_tensor(values, config, extension_status=status), (numel,), config, dtype=name,
