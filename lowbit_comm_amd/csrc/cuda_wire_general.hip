@@ -781,17 +781,18 @@ template <typename T> hipError_t launch_general_quant_t(int g, int bit, const Wi
     }
 }
 
-// The decode waits for one short load per wavefront, so beyond the chip's wavefront slots two tiles each pay - except for large fp32
-// tensors without outliers, whose time is their output's.  us of quantize + decode with one / two tiles, three tensors in rotation
-// (and twelve, beyond the last-level cache): normal book fp32 1 Mi 5.39 / 5.45 (5.69 / 6.29), 6.6 M 13.7 / 11.9 (13.9 / 14.1), 13.1 M
-// 20.6 / 21.5 (22.5 / 23.5), 26.2 M 38.3 / 39.4, bf16 13.1 M 15.9 / 14.7 (16.6 / 16.3), 26.2 M (e2m1) 25.3 / 24.9; with two
-// outliers fp32 6.6 M 17.0 / 15.1 (16.9 / 16.5), 26.2 M 47.1 / 46.1 (47.4 / 46.4), 8-bit bf16 26.2 M 28.4 / 28.0 (30.6 / 30.1), one
-// outlier bf16 1 Mi 5.16 / 5.44, 6.6 M 12.7 / 10.6 (11.8 / 11.1).
+// The decode waits for short loads, the codes and a group's words, so beyond the chip's wavefront slots two tiles a wavefront pay: in 16
+// bits where there is a code book or an outlier to wait for as well, in fp32 with two outliers, or up to 3 Mi elements without one and
+// 4 Mi with one.  us of quantize + decode with one / two tiles, three tensors in rotation (and beyond the last-level cache): two outliers
+// fp32 8-bit 3 Mi 9.4 / 9.0 (10.0 / 9.5), 6.25 Mi 14.6 / 14.1 (15.9 / 15.6), e2m1 25 Mi 48.5 / 47.4 (47.0 / 46.3), bf16 8-bit 5 Mi 9.9 / 9.3 (10.4 / 9.8),
+// 25 Mi 29.1 / 28.2 (30.5 / 29.9); one outlier bf16 6.25 Mi 11.3 / 10.9 (11.8 / 11.4), fp32 3 Mi 9.1 / 8.9 (9.7 / 9.4), 4.6 M 12.4 / 13.0 (13.6 / 14.2),
+// 20 Mi 36.3 / 36.3 (37.4 / 37.6); none, normal book bf16 6.25 Mi 10.3 / 9.7 (10.9 / 10.5), 25 Mi 24.9 / 24.7 (26.9 / 26.6), fp32 2.7 M 7.8 / 7.5 (8.4 /
+// 8.3), 4.7 M 10.6 / 11.3 (11.8 / 12.6), 6.6 M 12.7 / 12.9 (13.8 / 14.1), linear bf16 8 Mi 15.2 / 15.5 (15.2 / 15.4).
 template <typename T, int G, int BIT>
 hipError_t launch_general_decode_b(const WireGeneralDecodeArgs &a, hipStream_t stream) {
     const bool fills = a.numel > kResidentWaves * wire<T, BIT>::TILE;
-    const bool large = sizeof(T) == 4 && a.topk == 0 && a.numel > int64_t{8} << 20;
-    const bool pair = fills && !large;
+    const bool waits = sizeof(T) == 2 ? a.topk > 0 || a.kind != 0 : a.topk == 2 || a.numel <= static_cast<int64_t>(3 + a.topk) << 20;
+    const bool pair = fills && waits;
     const int64_t tile = wire<T, BIT>::TILE * kWavesPerBlock * (pair ? 2 : 1);
     const int64_t blocks = (a.numel + tile - 1) / tile;
     if (blocks == 0) return hipSuccess;

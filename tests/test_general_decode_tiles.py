@@ -16,7 +16,10 @@ def test_large_decodes_equal_the_decodes_of_their_pieces(hip_device, dtype, bit,
     policy = dict(group_size=64, bit=bit, quant_type=quant_type, topk=topk, compact=compact)
     line = (2 if dtype == torch.float32 else 4) * MiB
     generator = torch.Generator(device=hip_device).manual_seed(bit + topk)
-    for numel in (line, line + 64, line + 64 * 1031, 8 * MiB + 64):
+    ends = (line, line + 64, line + 64 * 1031, 8 * MiB + 64)
+    if dtype == torch.float32 and topk < 2:                   # two tiles up to 3 Mi elements, 4 Mi with an outlier
+        ends += ((3 + topk) * MiB, (3 + topk) * MiB + 64)
+    for numel in ends:
         x = (torch.randn(numel, generator=generator, device=hip_device) * 1e-3).to(dtype)
         base = (torch.randn(numel, generator=generator, device=hip_device) * 1e-3).to(dtype)
 
@@ -27,7 +30,7 @@ def test_large_decodes_equal_the_decodes_of_their_pieces(hip_device, dtype, bit,
             assert cuda_wire.bind_dequant_general(payload, out, **policy, **how)()
             return out
 
-        for how in ({}, {"reduce_op": "sum"}):
+        for how in ({}, {"reduce_op": "sum"}, {"reduce_op": "max"}, {"reduce_op": "min"}):
             got = decoded(x, base.clone(), **how)
             for start in range(0, numel, MiB):
                 want = decoded(x[start:start + MiB].clone(), base[start:start + MiB].clone(), **how)
