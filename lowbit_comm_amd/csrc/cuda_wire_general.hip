@@ -638,8 +638,10 @@ __global__ __launch_bounds__(kBlock) void wire_general_decode_kernel(const WireG
     store_elems<Raw, VEC, kNonTemporal>(out, decoded);
 }
 
-// The same with two tiles a wavefront, the loads of both issued before the first is decoded.  (As one kernel for either number the
-// single tile's code comes out 1 to 2 % slower on 13 and 26 M fp32 elements.)
+// The same with two tiles a wavefront, the loads of both issued before the first is decoded.  A text of its own because what the two
+// could share costs the single tile: as one kernel for either number 1 to 2 % on 13 and 26 M fp32 elements, as two kernels that inline the
+// same load and decode functions 5 to 6 % there (normal book, us of quantize + decode: 9 M 15.7 / 16.4, 26.2 M 38.7 / 41.1) and up to 3 % on
+// small ones.  A change to either belongs in both; the tests compare them over codes, outliers and combining decodes.
 template <typename T, int G, int BIT>
 __global__ __launch_bounds__(kBlock) void wire_general_decode_pair_kernel(const WireGeneralDecodeArgs a) {
     constexpr int TILES = 2;
@@ -723,7 +725,7 @@ __global__ __launch_bounds__(kBlock) void wire_general_decode_pair_kernel(const 
         }
         // The decoded tensor is the large stream of this kernel and nothing here reads it again: with the non-temporal
         // hint the decode of 26.2 M fp32 elements takes 19.9 instead of 30.2 us (top-2), 18.0 instead of 31.1 us (code book);
-        // written through as well it loses 1 to 4 %.
+        // written through as well it loses 1 to 6 %.
         store_elems<Raw, VEC, kNonTemporal>(out, decoded);
     }
 }
