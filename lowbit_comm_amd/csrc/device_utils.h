@@ -368,8 +368,8 @@ template <typename T, int N> __device__ __forceinline__ void divide_all(float (&
 // division gives - is checked, not inferred: q1 and RN(q) are equal or neighbouring floats and every half-integer
 // up to 127.5 is a float, so the codes can differ only for a p within a few ulps of (k + 0.5) * scale, and the
 // operations are invariant under a common power of two away from underflow.  tests/native/quotient_check.hip walks
-// all 2^23 scale mantissas x 256 half-integers x 13 neighbouring dividends at three exponents (8*10^10 pairs, every
-// such case) and 2.6*10^10 sampled pairs over the whole exponent range 2^-23 .. 2^120, among them dividends with 8
+// all 2^23 scale mantissas x 256 half-integers x 13 neighbouring dividends at three exponents and the last one's (8*10^10 pairs, every
+// such case) and 2.6*10^10 sampled pairs over the whole exponent range 2^-23 .. 2^121, among them dividends with 8
 // or 11 significant bits: no code and no quotient differs.  The one case outside, a remainder that underflows,
 // needs |p/scale| < 2^-64, where the code is 0 whatever the last bit of the quotient is.  Whole blocks and
 // the block at a chunk's end run the same code, so an element's code does not depend on the block it falls into.

@@ -3,7 +3,7 @@
 // y = 1/s (reciprocal_of_scale there) and q0 = p*y is compared on the device with the division p/s, bit for bit, and so are the codes rint()
 // makes of them.
 //
-// Sampled modes, scale exponents over the whole domain (2^-23 .. 2^120): 0 random, 1 scale mantissa (almost) all
+// Sampled modes, scale exponents over the whole domain (2^-23 .. 2^121, of which the last ends at FLT_MAX / 127): 0 random, 1 scale mantissa (almost) all
 // ones, 2 scales with few mantissa bits, 3 and 4 dividends within four ulps of (k + 0.5) * s, 5 dividends with 8 or
 // 11 significant bits (bf16 / fp16 tensors).
 //
@@ -11,7 +11,8 @@
 // up to 127.5 is a float, so the two can round to different codes only when one of them IS a half-integer, i.e. when
 // p lies within a few ulps of (k + 0.5) * s.  The operations are invariant under multiplying s and p by a power of
 // two as long as nothing underflows or overflows, which cannot happen for |p/s| >= 0.5 in the domain.  So mode 6
-// walks every one of the 2^23 mantissas of s (at exponent 0, and again at both ends of the exponent range), all 256
+// walks every one of the 2^23 mantissas of s (at exponent 0, and again at both ends of the exponent range: 2^-23, 2^120 and what
+// there is of 2^121), all 256
 // half-integers k + 0.5 in (-128, 128) and the 13 dividends within six ulps of RN((k + 0.5) * s): every case in
 // which the refined quotient could change a code.  It also compares y itself, the hardware's reciprocal with one Newton
 // step, with the division 1.0f / s, for every mantissa at every exponent of the scales' range, bit for bit.
@@ -33,7 +34,10 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <string.h>
 __device__ __forceinline__ uint32_t mix(uint64_t x) { x ^= x >> 33; x *= 0xff51afd7ed558ccdULL; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ULL; x ^= x >> 33; return (uint32_t)x; }
+constexpr float kFltMax = 3.402823466e+38f;
+constexpr float kMaxScale = kFltMax / 127.0f;        // biased exponent 248, and its mantissas up to this one's
 struct Tally { unsigned long long tiny, quotient, code; };
 __device__ __forceinline__ float reciprocal(float s) {          // device_utils.h: reciprocal_of_scale
     const float y = __builtin_amdgcn_rcpf(s);
@@ -60,11 +64,11 @@ __global__ void check_all_ties(uint32_t sexp, unsigned long long *bad, float *ex
     const uint32_t sman = blockIdx.x * blockDim.x + threadIdx.x;
     const float s = __uint_as_float((sexp << 23) | sman);
     Tally t = {0, 0, 0};
-    for (int k = -128; k <= 127; ++k) {
+    for (int k = -128; s <= kMaxScale && k <= 127; ++k) {
         const float base = ((float)k + 0.5f) * s;
         for (int ulps = -6; ulps <= 6; ++ulps) {
             const float p = __uint_as_float(__float_as_uint(base) + ulps);
-            if (fabsf(p) <= 127.5f * s) compare(p, s, t, ex);
+            if (fabsf(p) <= 127.5f * s && fabsf(p) <= kFltMax) compare(p, s, t, ex);
         }
     }
     publish(t, bad);
@@ -72,7 +76,7 @@ __global__ void check_all_ties(uint32_t sexp, unsigned long long *bad, float *ex
 __global__ void check_reciprocals(uint32_t sexp, unsigned long long *bad, float *ex) {
     const float s = __uint_as_float((sexp << 23) | (blockIdx.x * blockDim.x + threadIdx.x));
     Tally t = {0, 0, 0};
-    if (__float_as_uint(reciprocal(s)) != __float_as_uint(1.0f / s)) { ++t.quotient; ex[0] = 1.0f; ex[1] = s; }
+    if (s <= kMaxScale && __float_as_uint(reciprocal(s)) != __float_as_uint(1.0f / s)) { ++t.quotient; ex[0] = 1.0f; ex[1] = s; }
     publish(t, bad);
 }
 __global__ void check_shared_reciprocal(uint64_t seed, unsigned long long *bad, float *ex) {
@@ -109,11 +113,12 @@ __global__ void check(uint64_t seed, int mode, unsigned long long *bad, float *e
     for (int it = 0; it < 4096; ++it) {
         uint64_t h = seed * 0x9E3779B97F4A7C15ULL + id * 4096 + it;
         uint32_t a = mix(h), b = mix(h ^ 0xDEADBEEFCAFEULL), c = mix(h + 0x1234567ULL);
-        // scale: random normal float with exponent in [-23+127 .. 120+127]: eps up to FLT_MAX / 127
-        uint32_t sexp = 104 + (a % 144);
+        // scale: random normal float with exponent in [-23+127 .. 121+127]: eps up to FLT_MAX / 127
+        uint32_t sexp = 104 + (a % 145);
         uint32_t sman = b & 0x7FFFFF;
         if (mode == 1) sman = 0x7FFFFF - (b & 7);                 // mantissa (almost) all ones
         if (mode == 2) sman &= 0x7F0000;                           // few mantissa bits (bf16-like scale sources)
+        if (sexp == 248) sman %= (__float_as_uint(kMaxScale) & 0x7FFFFFu) + 1;
         float s = __uint_as_float((sexp << 23) | sman);
         float p;
         if (mode == 3 || mode == 4) {                              // p next to (k + 0.5) * s
@@ -132,7 +137,7 @@ __global__ void check(uint64_t seed, int mode, unsigned long long *bad, float *e
             p = q * s;
             p = __uint_as_float(__float_as_uint(p) ^ ((c >> 24) & 3));
         }
-        if (!(fabsf(p) <= 127.5f * s)) continue;
+        if (!(fabsf(p) <= 127.5f * s && fabsf(p) <= kFltMax)) continue;
         compare(p, s, t, ex);
     }
     publish(t, bad);
@@ -154,10 +159,13 @@ int main(int argc, char **argv) {
             for (int r = 0; r < rounds; ++r) hipLaunchKernelGGL(check_shared_reciprocal, dim3(4096), dim3(256), 0, 0, (uint64_t)(7000 + r), bad, ex);
             n = (unsigned long long)rounds * 4096ULL * 256ULL * 4096ULL;
         } else {
-            const uint32_t exponents[3] = {127, 104, 247};      // 1, the smallest scale, the largest the domain holds
+            const uint32_t exponents[4] = {127, 104, 247, 248};      // 1, the smallest scale, the largest with every mantissa, the last
             for (uint32_t sexp : exponents) hipLaunchKernelGGL(check_all_ties, dim3((1u << 23) / 256), dim3(256), 0, 0, sexp, bad, ex);
-            for (uint32_t sexp = 104; sexp <= 247; ++sexp) hipLaunchKernelGGL(check_reciprocals, dim3((1u << 23) / 256), dim3(256), 0, 0, sexp, bad, ex);
-            n = 3ULL * (1ULL << 23) * 256ULL * 13ULL + 144ULL * (1ULL << 23);
+            for (uint32_t sexp = 104; sexp <= 248; ++sexp) hipLaunchKernelGGL(check_reciprocals, dim3((1u << 23) / 256), dim3(256), 0, 0, sexp, bad, ex);
+            uint32_t last;
+            memcpy(&last, &kMaxScale, 4);
+            const unsigned long long partial = (last & 0x7FFFFFu) + 1ULL;
+            n = (3ULL * (1ULL << 23) + partial) * 256ULL * 13ULL + 144ULL * (1ULL << 23) + partial;
         }
         unsigned long long h[3]; float he[2];
         if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(h, bad, 24, hipMemcpyDeviceToHost) != hipSuccess ||
