@@ -24,9 +24,19 @@ namespace {
 
 using namespace reduce;
 
-template <typename OT, int G, int W, int MODE>
+template <typename OT, int G, int W, int MODE, bool EARLY_SUM>
 __global__ __launch_bounds__(kBlock) void dequant_reduce_kernel(const ReduceArgs a) {
-    dequant_reduce_block<OT, G, W, MODE>(a, blockIdx.x, gridDim.x);
+    dequant_reduce_block<OT, G, W, MODE, EARLY_SUM>(a, blockIdx.x, gridDim.x);
+}
+
+template <typename OT, int G, int W, int MODE> void enqueue_reduce(unsigned blocks, const ReduceArgs &a, hipStream_t stream) {
+    if constexpr (prepared_early<OT, W, MODE>()) {
+        if (a.new_residual != nullptr && takes_early<OT, W, MODE>(a.numel * static_cast<int64_t>(sizeof(OT)))) {
+            hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, MODE, true>), dim3(blocks), dim3(kBlock), 0, stream, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, MODE, false>), dim3(blocks), dim3(kBlock), 0, stream, a);
 }
 
 template <typename OT, int G, int W>
@@ -36,10 +46,10 @@ hipError_t launch_reduce_w(int mode, const ReduceArgs &a, hipStream_t stream) {
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
     switch (mode) {
-        case kStreamThrough: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kStreamThrough>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
-        case kStream: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kStream>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
-        case kVector: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kVector>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
-        default: hipLaunchKernelGGL((dequant_reduce_kernel<OT, G, W, kUnaligned>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a); break;
+        case kStreamThrough: enqueue_reduce<OT, G, W, kStreamThrough>(static_cast<unsigned>(blocks), a, stream); break;
+        case kStream: enqueue_reduce<OT, G, W, kStream>(static_cast<unsigned>(blocks), a, stream); break;
+        case kVector: enqueue_reduce<OT, G, W, kVector>(static_cast<unsigned>(blocks), a, stream); break;
+        default: enqueue_reduce<OT, G, W, kUnaligned>(static_cast<unsigned>(blocks), a, stream); break;
     }
     return hipGetLastError();
 }

@@ -36,8 +36,8 @@ template <int W> __device__ __forceinline__ constexpr int code_load_mode(int mod
 //   reads/writes < 0.8  (W = 1, 2 for fp32)  plain code loads, non-temporal stores       (26 M, W = 1: 19.0 us; with
 //                                             non-temporal loads as well 24.8 us)
 //   up to 1.6           (W = 4; for 16-bit    non-temporal loads; stores non-temporal (two 16-bit payloads: written
-//                        outputs W = 2)       through beside the hint), or written through without it for outputs
-//                                             beyond the L2s
+//                        outputs W = 2)       through beside the hint unless the sum is loaded early), or written
+//                                             through without it for outputs beyond the L2s
 //   above               (W = 8)               non-temporal loads; plain stores while the output fits the L2s
 //                                             (3.3 M: 7.9 us against 8.1 written through, 8.4 non-temporal - the
 //                                             write-back then overlaps the next kernel's ramp), written through
@@ -52,21 +52,27 @@ template <typename OT, int W> constexpr int read_write_class() {
 template <typename OT, int W, int MODE> constexpr int code_policy() {
     return MODE >= kStream && read_write_class<OT, W>() >= 1 ? kNtBit : kCached;
 }
-template <typename OT, int W, int MODE> constexpr int reduce_store_policy() {
+template <typename OT, int W, int MODE, bool EARLY_SUM> constexpr int reduce_store_policy() {
     if (MODE < kStream) return kCached;
     if (read_write_class<OT, W>() == 0) return kNtBit;
     if (MODE == kStreamThrough) return kSc1Bit;
-    return read_write_class<OT, W>() == 1 ? (W <= 2 ? kNtBit | kSc1Bit : kNtBit) : kCached;
+    return read_write_class<OT, W>() == 1 ? (W <= 2 && !EARLY_SUM ? kNtBit | kSc1Bit : kNtBit) : kCached;
 }
 
-// Whether whole blocks issue the load of `prepared` together with the codes' or behind the outputs' stores.  Early it is one
-// round trip to memory less; where reads and writes are about even (class 1) it only pays for outputs within the L2s, of two
-// payloads.  GPU us of the all_gather hook's two launches with error feedback, late / early, three states in rotation (and
-// twelve, beyond the last-level cache): two payloads fp32 4 M 25.3 / 22.7 (25.3 / 23.1), three 1 M 8.8 / 8.4, eight bf16
-// 2 M 11.9 / 11.2 (12.4 / 12.0), 13.1 M 45.2 / 44.9; class 1, two of bf16 1 M 7.7 / 6.8, with the outputs written through as
-// well as non-temporal 6.5 (7.9 / 7.0), 8 M 27.9 / 25.9 (27.3 / 25.0), 13.1 M 34.2 / 34.8; four of fp32 2 M 13.5 / 14.4.
+// Whether a call with error feedback has a kernel whose whole blocks issue the load of `prepared` together with the codes', and takes
+// it for an output of `bytes`; else they load it behind the outputs' stores.  Early it is one round trip to memory less.  A kernel of its
+// own, because the load and its branch cost calls without feedback 3 to 8 % of the reduce (eight bf16 payloads 23,552 elements 2.6 ->
+// 2.8 us, 0.7 M 3.4 -> 3.6).  GPU us of the all_gather hook's two launches, late / early, three states in rotation (and beyond the last-level
+// cache): one payload fp32 1.5 MiB 6.7 / 5.8 (7.0 / 6.1), two of fp32 2 MiB 6.8 / 5.9 (7.3 / 6.5), 50 MiB 60.9 / 58.1 (60.7 / 58.3), eight of bf16 0.5 MiB
+// 5.8 / 5.4 (6.8 / 6.1), 3 MiB 11.1 / 9.9 (12.0 / 10.8), 20 MiB 38.7 / 37.9 (42.4 / 41.7).  Where reads and writes are about even (class 1) only two
+// payloads, up to where the outputs are written through: two of bf16 2.5 MiB 8.3 / 7.4 (8.7 / 7.8), 5 MiB 11.0 / 10.2 (11.2 / 10.9), 10 MiB 17.4 / 17.5
+// (17.5 / 17.6); four of fp32 8 MiB 13.5 / 14.4.  Three fp32 payloads gain to 6 MiB (11.0 / 10.5 (11.6 / 11.2)) and from 24 MiB on, between them
+// they lose (11 MiB 17.5 / 18.3 (18.0 / 18.6)).
 template <typename OT, int W, int MODE> constexpr bool prepared_early() {
-    return read_write_class<OT, W>() != 1 || (W <= 2 && MODE != kStreamThrough);
+    return MODE >= kStream && (read_write_class<OT, W>() != 1 || (W <= 2 && MODE != kStreamThrough));
+}
+template <typename OT, int W, int MODE> bool takes_early(int64_t bytes) {
+    return !(sizeof(OT) == 4 && W == 3 && MODE == kStream && bytes >= int64_t{13} << 19);
 }
 
 // The VEC codes of a lane, from any address under kUnaligned.
@@ -78,8 +84,9 @@ __device__ __forceinline__ void load_codes(const int8_t *__restrict__ p, uint32_
 // ---------------------------------------------------------------------------
 // fused dequant-reduce
 // ---------------------------------------------------------------------------
-// One workgroup's share: block `block_x` of a grid of `grid_x` workgroups.
-template <typename OT, int G, int W, int MODE>
+// One workgroup's share: block `block_x` of a grid of `grid_x` workgroups.  EARLY_SUM: the call has error feedback, and whole blocks load
+// `prepared` with the codes.
+template <typename OT, int G, int W, int MODE, bool EARLY_SUM = false>
 __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsigned block_x, unsigned grid_x) {
     using T = decode_tiling<OT, W>;
     constexpr int VEC = T::VEC;
@@ -96,7 +103,7 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
     const bool mean = a.divisor != 1.0f;
 
     // One pass over the block's tiles with the codes and scales of all of them issued before the arithmetic (`prepared`
-    // with them in the last block; in whole blocks as prepared_early says, else tile by tile after the tile's outputs).  WHOLE:
+    // with them in the last block; in whole blocks under EARLY_SUM, else tile by tile after the tile's outputs).  WHOLE:
     // all of the block's outputs exist.  Whole blocks of aligned tensors use one descriptor per stream over the block's span and 32-bit offsets
     // per lane; the block at the end and tensors at element alignment use 64-bit addresses, a lane's vector cut short
     // at the end.  (A payload holds whole groups, so a lane with one live output may read all of its codes.)  Walked
@@ -109,13 +116,13 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
         constexpr int kLike = MODE == kUnaligned ? static_cast<int>(kStream) : MODE;   // policies as in the streaming mode
         constexpr int kCodes = code_policy<OT, W, kLike>();
         constexpr int kLoad = policy_of<kLike>();
-        constexpr int kStore = reduce_store_policy<OT, W, kLike>();
+        constexpr int kStore = reduce_store_policy<OT, W, kLike, EARLY_SUM>();
         // What the stores without a descriptor take of it.  Two bf16 payloads at an odd output, plain / non-temporal, beyond the
         // last-level cache: with feedback 1 M elements 4.73 / 4.69 us, 8 M 14.9 / 14.5, 13.1 M 22.4 / 22.4, without it 8 M 8.2 / 7.8,
         // 26.2 M 21.0 / 19.9.  (Three tensors in rotation, with feedback: 3.2 M 7.1 / 6.6, 13.1 M 19.3 / 22.0.)
         constexpr bool kStoreNt = (kStore & kNtBit) != 0;
         constexpr int kCodeAlign = MODE == kUnaligned ? 1 : VEC;
-        constexpr bool kEarly = BUFFERS && prepared_early<OT, W, MODE>();
+        constexpr bool kEarly = BUFFERS && EARLY_SUM;
         uint32_t words[UNROLL][W][VEC / 4];
         float scale[UNROLL][W];
         OT pv[UNROLL][VEC];
@@ -147,12 +154,12 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
                 }
             }
         }
-        if (new_r != nullptr) {
+        if constexpr (kEarly) {
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                if constexpr (kEarly) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
-                else if constexpr (!WHOLE) load_live<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], live_here - at[u], pv[u]);
-            }
+            for (int u = 0; u < UNROLL; ++u) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
+        } else if (!WHOLE && (EARLY_SUM || new_r != nullptr)) {   // the end of the tensor: nothing else hides this load
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u) load_live<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], live_here - at[u], pv[u]);
         }
         const buffer_t out_b = buffer_over(out + block_first, T::BLOCK_ELEMS * sizeof(OT));
 #pragma unroll
@@ -177,7 +184,7 @@ __device__ __forceinline__ void dequant_reduce_block(const ReduceArgs &a, unsign
             if constexpr (BUFFERS) buffer_store<OT, VEC, kStore>(out_b, at[u] * sizeof(OT), o);
             else if constexpr (WHOLE) store_any<OT, VEC, kStoreNt>(out + block_first + at[u], o);
             else store_live<OT, VEC, kStoreNt>(out + block_first + at[u], live_here - at[u], o);
-            if (new_r != nullptr) {
+            if (EARLY_SUM || new_r != nullptr) {
                 OT d[VEC];
                 if constexpr (BUFFERS && !kEarly) buffer_load<OT, VEC, kLoad>(prepared_b, at[u] * sizeof(OT), pv[u]);
                 else if constexpr (WHOLE && !BUFFERS) load_any<OT, VEC, kLoad == kNtBit>(prepared + block_first + at[u], pv[u]);

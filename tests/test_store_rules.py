@@ -73,3 +73,34 @@ def _terms(payload, numel, dtype):
     codes = codes.view(-1, width).flip(1).reshape(-1, 64).float()
     step = scales / torch.full_like(scales, 127.0)                    # a division: by a number, torch multiplies by its reciprocal
     return (codes * step[:, None]).reshape(-1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("world", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_portable_reduce_with_and_without_feedback(hip_device, dtype, world, offset):
+    """The kernels that load the sum early and those that load it late or not at all, on both sides of a block's end and of the line of
+    three fp32 payloads, against the oracle's fold."""
+    from lowbit_comm_amd.hip import ops
+    from oracle import codec_torch
+
+    name, item = {torch.float32: ("fp32", 4), torch.bfloat16: ("bf16", 2)}[dtype]
+    bits = torch.int32 if item == 4 else torch.int16
+    block = 256 * 16 // item
+    sizes = [1, 63, block - 1, block, 2 * block, 2 * block + 65, 9 * block + 3]
+    sizes += [13 * MiB // 8 + step for step in (-1, 0)] if world == 3 and item == 4 and offset == 0 else []
+    for numel in sizes:
+        generator = torch.Generator().manual_seed(numel + world)
+        payloads = [codec_torch.quantize((torch.randn(numel, generator=generator) * 1e-3).to(dtype), 64) for _ in range(world)]
+        on_device = [(codes.to(hip_device), scales.to(hip_device)) for codes, scales in payloads]
+        want = codec_torch.reduce_payloads(payloads, numel, 64, name, "mean")
+        prepared = (torch.randn(numel, generator=generator) * 1e-3).to(dtype)
+        for feedback in (False, True):
+            out = torch.zeros(numel + offset, dtype=dtype, device=hip_device)
+            residual = torch.zeros(numel + offset, dtype=dtype, device=hip_device)
+            how = dict(prepared=prepared.to(hip_device), new_residual=residual[offset:]) if feedback else {}
+            assert ops.dequant_reduce_into(on_device, out[offset:], group_size=64, divisor=float(world), **how)
+            assert torch.equal(out[offset:].cpu().view(bits), want.view(bits)), (numel, feedback)
+            if feedback:
+                left = (prepared.float() - want.float()).to(dtype)
+                assert torch.equal(residual[offset:].cpu().view(bits), left.view(bits)), numel
