@@ -99,13 +99,13 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
         constexpr bool kLoadNt = MODE >= kStream || MODE == kUnaligned;
         constexpr bool kStoreNt = MODE >= kStream;
         constexpr int kLoad = policy_of<MODE>();
-        // The compensated sum, and with several tiles a wavefront the other outputs beside the codes, leave with the non-temporal
-        // hint and written through.  nt alone / both, GPU us with three states in rotation (and with twelve, beyond the last-level
-        // cache): local step of 52.4 M bf16 elements 105.9 / 101.4 (117.0 / 111.6), 26.2 M fp32 71.5 / 69.3, of one tile a wavefront
-        // 2 M bf16 6.04 / 5.99 (6.35 / 6.63); the all_gather hook's two launches, whose quantize writes the sum, 2 M bf16 11.7 /
-        // 11.45 (12.7 / 12.3), 13.1 M 45.2 / 45.0.
-        constexpr int kSumStore = MODE >= kStream ? kNtBit | kSc1Bit : kCached;
-        constexpr int kSideStore = TILES > 1 ? kSumStore : policy_of<MODE>();
+        // With several tiles a wavefront the outputs beside the codes leave with the non-temporal hint and written through, else with the
+        // hint alone: the reduce that reads the sum next finds it nearer.  nt alone / both, GPU us with three states in rotation (and
+        // beyond the last-level cache): local step of 52.4 M bf16 elements 105.9 / 101.4 (117.0 / 111.6), 26.2 M fp32 71.5 / 69.3, of one
+        // tile a wavefront 2 M bf16 6.04 / 5.99 (6.35 / 6.63); the quantize that writes the sum, 24 M bf16 28.1 / 27.1 (27.9 / 26.9), 12 M fp32
+        // 26.6 / 25.7 (26.4 / 25.5); with the reduce behind it, of one tile a wavefront, four fp32 payloads of 0.05 MiB 4.5 / 4.9 (5.1 / 5.4), 2 MiB
+        // 6.5 / 7.0 (7.3 / 7.4), three bf16 of 1.6 MiB 6.9 / 7.3 (7.5 / 7.6), eight fp32 of 2.4 MiB 6.9 / 7.4 (7.7 / 8.0).
+        constexpr int kSideStore = TILES > 1 && MODE >= kStream ? kNtBit | kSc1Bit : policy_of<MODE>();
         constexpr int kCodeStore = quant_code_store_policy<HAS_R, MODE>();
         XT xv[UNROLL][VEC];
         RLoad rv[UNROLL][VEC];
@@ -147,9 +147,9 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
         const buffer_t codes_b = buffer_over(codes + block_first, T::BLOCK_ELEMS);
         const buffer_t scales_b = buffer_over(scales + block_first / G, T::BLOCK_ELEMS / G * 4);
         // `out` of element type E, the block's part of the stream at `base`
-        auto store_side = [&](auto policy, auto *base, uint32_t offset, const auto &out) __attribute__((always_inline)) {
+        auto store_side = [&](auto *base, uint32_t offset, const auto &out) __attribute__((always_inline)) {
             using E = typename std::remove_pointer<decltype(base)>::type;
-            if constexpr (BUFFERS) buffer_store<E, VEC, decltype(policy)::value>(buffer_over(base + block_first, T::BLOCK_ELEMS * sizeof(E)), offset * sizeof(E), out);
+            if constexpr (BUFFERS) buffer_store<E, VEC, kSideStore>(buffer_over(base + block_first, T::BLOCK_ELEMS * sizeof(E)), offset * sizeof(E), out);
             else if constexpr (WHOLE) store_any<E, VEC, kStoreNt>(base + block_first + offset, out);
             else store_live<E, VEC, kStoreNt>(base + block_first + offset, live_here - offset, out);
         };
@@ -218,7 +218,7 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
             if (prepared != nullptr) {
                 PT prep_out[VEC];
                 narrow_all<PT, VEC>(p[u], prep_out);
-                store_side(std::integral_constant<int, kSumStore>{}, prepared, at[u], prep_out);
+                store_side(prepared, at[u], prep_out);
             }
             if (new_r != nullptr || restored != nullptr) {
                 float rest[VEC], diff[VEC];
@@ -231,9 +231,8 @@ __device__ __forceinline__ void quant_pack_block(const QuantArgs &a, unsigned bl
                 for (int i = 0; i < VEC; ++i) diff[i] = p[u][i] - rest[i];
                 narrow_all<DT, VEC>(rest, rest_out);
                 narrow_all<NT, VEC>(diff, diff_out);
-                const std::integral_constant<int, kSideStore> side;
-                if (restored != nullptr) store_side(side, restored, at[u], rest_out);
-                if (new_r != nullptr) store_side(side, new_r, at[u], diff_out);
+                if (restored != nullptr) store_side(restored, at[u], rest_out);
+                if (new_r != nullptr) store_side(new_r, at[u], diff_out);
             }
         }
     };
