@@ -441,7 +441,10 @@ class PipelinedRingExecutor(TopologyExecutor):
         Bound by the host: a 13.1 M bf16 bucket of eight ranks spent 34 of its 80 us a pass on the bookkeeping of a submission
         whose buffers belong to the runtime's plan and whose completion is the order of the caller's own stream."""
         known = getattr(self._runtime, "_replays", None)
-        if known is None or not known.own(self, _SUBMITTED) or (self._sessions, self._works) != self._made_with:
+        if known is None or not known.own(self, _SUBMITTED):
+            return False
+        sessions, works = self._made_with
+        if self._sessions is not sessions or self._works is not works:
             return False
         if not self._busy.acquire(blocking=False):
             raise RuntimeError("concurrent run() on one topology executor is unsupported")
@@ -1054,8 +1057,9 @@ class LoopbackRing:
 def policy_beside_group_size(config: CompressionConfig) -> tuple:
     """What of a policy, besides the group size, an executor is made for or refuses: part of the key that a transport keeps its
     executors under, so that a call is answered by its own policy whatever ran before it.  Empty for the default policy."""
-    policy = (config.bit, config.topk, config.quant_type, config.stochastic, config.compact)
-    return () if policy == (8, 0, "linear", False, False) else policy
+    if config.bit == 8 and config.topk == 0 and config.quant_type == "linear" and not config.stochastic and not config.compact:
+        return ()
+    return (config.bit, config.topk, config.quant_type, config.stochastic, config.compact)
 
 
 def make_pipelined_ring_executor(*, config: CompressionConfig, dtype: str, numel: int, world_size: int, rank: int,
