@@ -93,7 +93,7 @@ template <typename T> __device__ __forceinline__ float round_through(float v) {
 // (v_cvt_pk_bf16_f32).  With zero as the pair's lower half the packed register is the rounded value as a float: one
 // instruction an element, where a pair of elements takes one to round and two to take apart.  Kernels that fold payloads
 // round twice an element and payload: the all_gather hook's two launches on 2 M bf16 elements of eight payloads 12.0 -> 11.6 us,
-// the plan's three on 1 M 8.25 -> 8.15, on 9.8 M 18.0 -> 17.8.
+// the plan's three on 1 M 8.25 -> 8.15, on 9.8 M 19.5 -> 19.2.
 template <typename T, int N> __device__ __forceinline__ void round_through_all(float (&v)[N]) {
     if constexpr (same_t<T, float>::value) {
         return;

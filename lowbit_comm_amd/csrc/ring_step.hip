@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kBlock) void ring_step_kernel(const RingStepArgs a)
     auto tiles = [&](auto whole) __attribute__((always_inline)) {
         constexpr bool WHOLE = decltype(whole)::value;
         // Whole blocks of aligned chunks use one descriptor per stream over the block's span and 32-bit offsets per lane: GPU time of
-        // the ring of eight ranks on 13.1 M bf16 elements 46.6 -> 46.0 us, 26.2 M 59.0 -> 58.0, 6.6 M fp32 41.4 -> 41.1.  (Written
+        // the ring of eight ranks on 13.1 M bf16 elements 46.6 -> 46.2 us, 26.2 M 59.0 -> 58.6, 6.6 M fp32 41.5 -> 41.3.  (Written
         // through beside the hint, the chunk's stores are 0.3 us faster on 13.1 M and 0.4 slower on the others; the codes' 1 to 2 us slower.)
         constexpr bool BUFFERS = WHOLE && MODE != kUnaligned;
         constexpr bool kNt = MODE == kStream || MODE == kUnaligned;

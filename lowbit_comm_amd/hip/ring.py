@@ -1108,7 +1108,11 @@ def make_pipelined_ring_transport(*, world_size: int, rank: int, exchange: Calla
 
     A call that is waited for at once (``async_op=False``) runs on the caller's stream: on a stream of the ring's own the
     caller's would wait for all of it, with two events and two stream waits a bucket in between (25 MiB bf16 bucket,
-    eight ranks, 14 hops: 121 -> 84 us a bucket, host time throughout).  ``async_op=True`` has an executor with a stream of its own."""
+    eight ranks, 14 hops: 121 -> 84 us a bucket, host time throughout).  ``async_op=True`` has an executor with a stream of its own.
+
+    Such a call on a bucket that the executor has a record of replays it (84 -> 57 us).  An executor keeps ``max_plans`` records, by
+    address, least recently used first out: more buckets of one shape than that, handed over in turn, never find theirs, and every
+    call costs what a first one does (0.7 ms for 14 hops).  Give ``max_plans`` the number of buckets of the commonest shape."""
     from collections import OrderedDict
 
     from lowbit_comm_amd.exceptions import UnsupportedCollective
