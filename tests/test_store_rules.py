@@ -23,7 +23,7 @@ def test_decode_around_the_line(hip_device, dtype, wire):
     status, config = load_hip_extension(wire_format=wire), CompressionConfig()
     name, item = {torch.float32: ("fp32", 4), torch.bfloat16: ("bf16", 2)}[dtype]
     line = (32 if item == 4 else 20 if wire == "portable" else 16) * MiB // item
-    for numel in (line - 64, line, line + 64 * 33):
+    for numel in sorted({start + step for start in (16 * MiB // item, line) for step in (-64, 0, 64 * 33)}):
         generator = torch.Generator(device=hip_device).manual_seed(numel)
         values = (torch.randn(numel, generator=generator, device=hip_device) * 1e-3).to(dtype)
         got = dequantize_tensor(quantize_tensor(values, config, extension_status=status), (numel,), config, dtype=name,
@@ -47,7 +47,7 @@ def test_cuda_format_reduce_with_feedback(hip_device, dtype, world, offset):
     name = {torch.float32: "fp32", torch.bfloat16: "bf16"}[dtype]
     item = torch.empty((), dtype=dtype).element_size()
     lines = [line // item + step for line in ((3 * MiB // 2, 9 * MiB, 32 * MiB) if item == 4 else (MiB // 4, 32 * MiB))
-             for step in (-576, 0, 64)]
+             for step in (-576, 0, 64)] + [48 * MiB // item - 64, 48 * MiB // item]
     sizes = [64 * 5, 4096, 4096 * 9 + 64 * 3] + (lines if world == 4 and offset == 0 else [])
     for numel in sizes:
         payloads = [_payload(numel, dtype, config, status, 10 * r + 1, hip_device) for r in range(world)]
